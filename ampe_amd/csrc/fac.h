@@ -16,6 +16,41 @@ struct EllOp {
    T Mc = 0;
 };
 
+// Preconditioner blocks that are swept together: each slot holds components
+// [comp, comp + ncomp) of the shared right-hand side and solution vectors and
+// their operator; a kernel over a set runs all slots in one launch.
+template <typename T>
+struct SweepSlot {
+   int kind = 0;  // 0 elliptic (op), 1 orientation (face coefficients D, sm, gamma)
+   int comp = 0, ncomp = 1;
+   const T* D = nullptr;
+   T Dc = 0;
+   const T* C = nullptr;
+   T Cc = 0;
+   const T* M = nullptr;
+   T Mc = 0;
+   const T* sm = nullptr;
+   T gamma = 0;
+};
+constexpr int kMaxSlots = 16;
+template <typename T>
+struct SweepSet {
+   int n = 0;
+   SweepSlot<T> s[kMaxSlots];
+};
+// Appends ncomp components sharing one operator, elliptic ones four to a slot
+// (their coefficients are read once for the four); -1 when no slot is left.
+template <typename T>
+int sweep_add(SweepSet<T>& set, const SweepSlot<T>& proto, int comp, int ncomp);
+
+// One colour of every slot's red-black sweep, and every slot's residual.
+template <typename T>
+int launch_set_sweep(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs, T* x,
+                     int color, hipStream_t s);
+template <typename T>
+int launch_set_residual(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs,
+                        const T* x, T* res, hipStream_t s);
+
 int launch_phase_C(const Level& L, const ampe_model_params& p, double gamma,
                    const double* phi, const double* M, double* C, hipStream_t s);
 

@@ -729,6 +729,130 @@ __global__ void __launch_bounds__(256) k_quat_resrestrict(LevelArgs ca, LevelArg
    }
 }
 
+// ------------------------------------------------------------ block sets
+// The elliptic row's coefficients at one cell, shared by the slot's
+// components: dinv D of the low and high faces, M, C and the diagonal (the
+// products op_residual forms, in its order).
+template <typename T>
+struct EllRowCoef {
+   T wlo[3], whi[3], m, cc, diag;
+};
+
+template <typename T, int NDIM>
+__device__ __forceinline__ EllRowCoef<T> ell_row_coef(const LevelArgs& a, const CellPos& c,
+                                                      const SweepSlot<T>& o, const T* dinv)
+{
+   const int ijk[3] = {c.i, c.j, c.k};
+   EllRowCoef<T> w;
+   T dsum = 0;
+#pragma unroll
+   for (int d = 0; d < NDIM; d++) {
+      T dlo, dhi;
+      if (o.D) {
+         int lo[3] = {ijk[0], ijk[1], ijk[2]};
+         long long flo = face_idx(a, c.pd, d, lo[0], lo[1], lo[2]);
+         lo[d] += 1;
+         long long fhi = face_idx(a, c.pd, d, lo[0], lo[1], lo[2]);
+         dlo = o.D[flo];
+         dhi = o.D[fhi];
+      } else {
+         dlo = dhi = o.Dc;
+      }
+      w.wlo[d] = dinv[d] * dlo;
+      w.whi[d] = dinv[d] * dhi;
+      T ds = dinv[d] * dinv[d] * (dhi + dlo);
+      dsum = (d == 0) ? ds : dsum + ds;
+   }
+   w.m = o.M ? o.M[c.c0] : o.Mc;
+   w.cc = o.C ? o.C[c.c0] : o.Cc;
+   w.diag = w.m * dsum - w.cc;
+   return w;
+}
+
+// rhs - A u of one component from the row's coefficients (op_residual's
+// operations in its order).
+template <typename T, int NDIM>
+__device__ __forceinline__ T ell_row_residual(const EllRowCoef<T>& w, const T* dinv, T rhs,
+                                              const QuatRowVals<T, NDIM>& v)
+{
+   T div = 0;
+#pragma unroll
+   for (int d = 0; d < NDIM; d++) {
+      T flo = w.wlo[d] * (v.zc - v.zl[d]);
+      T fhi = w.whi[d] * (v.zh[d] - v.zc);
+      T t = dinv[d] * (fhi - flo);
+      div = (d == 0) ? t : div + t;
+   }
+   return rhs - w.m * div - w.cc * v.zc;
+}
+
+// One colour of the red-black sweep of every slot: blockIdx.y is the slot, so
+// the phase, orientation and composition blocks (and the components of each)
+// of a level are one launch instead of one per component.  On the small
+// levels of a hierarchy a launch costs 2-4 us whatever it computes, and these
+// sweeps and the ghost fills between them are most of a solve there.
+template <typename T, int NDIM>
+__global__ void __launch_bounds__(128) k_set_sweep(LevelArgs a, SweepSet<T> set, T di0, T di1,
+                                                   T di2, T hi0, T hi1, T hi2,
+                                                   const T* __restrict__ rhs, T* __restrict__ x,
+                                                   int color)
+{
+   CellPos c;
+   if (!cell_pos_color<NDIM>(a, 0, color, c)) return;
+   const SweepSlot<T>& o = set.s[blockIdx.y];
+   const T* b = rhs + o.comp * a.ncg;
+   T* u = x + o.comp * a.ncg;
+   if (o.kind == 1) {
+      const T hinv2[3] = {hi0, hi1, hi2};
+      if (o.ncomp == 4)
+         quat_rbgs_cell<T, NDIM, 4, false>(a, c, o.D, o.sm, o.gamma, hinv2, 4, b, u);
+      else
+         quat_rbgs_cell<T, NDIM, 0, false>(a, c, o.D, o.sm, o.gamma, hinv2, o.ncomp, b, u);
+      return;
+   }
+   const T dinv[3] = {di0, di1, di2};
+   const EllRowCoef<T> w = ell_row_coef<T, NDIM>(a, c, o, dinv);
+   const T dudr = T(1) / w.diag;
+   const QuatIdx q{c.c0, c.c0 - 1, c.c0 + 1};
+   for (int m = 0; m < o.ncomp; m++) {
+      QuatRowVals<T, NDIM> v;
+      quat_row_load<T, NDIM>(c, q, u + m * a.ncg, v);
+      const T res = ell_row_residual<T, NDIM>(w, dinv, b[m * a.ncg + c.c0], v);
+      const T du = -res * dudr;
+      u[m * a.ncg + c.c0] = v.zc + du * T(1);
+   }
+}
+
+// The residual of every slot, in one launch as k_set_sweep.
+template <typename T, int NDIM>
+__global__ void __launch_bounds__(256) k_set_residual(LevelArgs a, SweepSet<T> set, T di0, T di1,
+                                                      T di2, T hi0, T hi1, T hi2,
+                                                      const T* __restrict__ rhs,
+                                                      const T* __restrict__ x,
+                                                      T* __restrict__ res)
+{
+   CellPos c;
+   if (!cell_pos(a, 0, c)) return;
+   const SweepSlot<T>& o = set.s[blockIdx.y];
+   const T* b = rhs + o.comp * a.ncg;
+   const T* u = x + o.comp * a.ncg;
+   T* r = res + o.comp * a.ncg;
+   if (o.kind == 1) {
+      const T hinv2[3] = {hi0, hi1, hi2};
+      (void)quat_residual_cell<T, NDIM, 0, false>(a, c, o.D, o.sm, o.gamma, hinv2, o.ncomp, b, u,
+                                                  r);
+      return;
+   }
+   const T dinv[3] = {di0, di1, di2};
+   const EllRowCoef<T> w = ell_row_coef<T, NDIM>(a, c, o, dinv);
+   const QuatIdx q{c.c0, c.c0 - 1, c.c0 + 1};
+   for (int m = 0; m < o.ncomp; m++) {
+      QuatRowVals<T, NDIM> v;
+      quat_row_load<T, NDIM>(c, q, u + m * a.ncg, v);
+      r[m * a.ncg + c.c0] = ell_row_residual<T, NDIM>(w, dinv, b[m * a.ncg + c.c0], v);
+   }
+}
+
 // ------------------------------------------------------------ launchers
 static dim3 tblock() { return dim3(TX, TY); }
 static dim3 cblock() { return dim3(TX / 2, TY); }
@@ -786,6 +910,59 @@ static void shape(const Level& L, bool reduce, LevelArgs* a, int* grid)
 {
    *a = reduce ? level_args(L) : level_args_col(L);
    *grid = reduce ? L.ncell_tiles : L.ncol_tiles;
+}
+
+template <typename T>
+int sweep_add(SweepSet<T>& set, const SweepSlot<T>& proto, int comp, int ncomp)
+{
+   const int per = proto.kind == 1 ? ncomp : 4;
+   for (int m = 0; m < ncomp; m += per) {
+      if (set.n >= kMaxSlots) {
+         set_error("sweep_add: too many preconditioner blocks");
+         return -1;
+      }
+      SweepSlot<T>& o = set.s[set.n++];
+      o = proto;
+      o.comp = comp + m;
+      o.ncomp = ncomp - m < per ? ncomp - m : per;
+   }
+   return 0;
+}
+
+template <typename T>
+int launch_set_sweep(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs, T* x,
+                     int color, hipStream_t s)
+{
+   T di[3], hi[3];
+   recip(dx, di);
+   recip2(dx, hi);
+   dim3 g(L.ncell_tiles, set.n);
+   if (L.ndim == 3)
+      hipLaunchKernelGGL((k_set_sweep<T, 3>), g, cblock(), 0, s, level_args(L), set, di[0], di[1],
+                         di[2], hi[0], hi[1], hi[2], rhs, x, color);
+   else
+      hipLaunchKernelGGL((k_set_sweep<T, 2>), g, cblock(), 0, s, level_args(L), set, di[0], di[1],
+                         di[2], hi[0], hi[1], hi[2], rhs, x, color);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
+template <typename T>
+int launch_set_residual(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs,
+                        const T* x, T* res, hipStream_t s)
+{
+   T di[3], hi[3];
+   recip(dx, di);
+   recip2(dx, hi);
+   dim3 g(L.ncell_tiles, set.n);
+   if (L.ndim == 3)
+      hipLaunchKernelGGL((k_set_residual<T, 3>), g, tblock(), 0, s, level_args(L), set, di[0],
+                         di[1], di[2], hi[0], hi[1], hi[2], rhs, x, res);
+   else
+      hipLaunchKernelGGL((k_set_residual<T, 2>), g, tblock(), 0, s, level_args(L), set, di[0],
+                         di[1], di[2], hi[0], hi[1], hi[2], rhs, x, res);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
 }
 
 template <typename T>
@@ -973,6 +1150,11 @@ int launch_quat_resrestrict(const Level& coarse, const Level& fine, const T* fc,
 }
 
 #define AMPE_INST(T)                                                                     \
+   template int sweep_add<T>(SweepSet<T>&, const SweepSlot<T>&, int, int);               \
+   template int launch_set_sweep<T>(const Level&, const SweepSet<T>&, const double*,     \
+                                    const T*, T*, int, hipStream_t);                     \
+   template int launch_set_residual<T>(const Level&, const SweepSet<T>&, const double*,  \
+                                       const T*, const T*, T*, hipStream_t);             \
    template int launch_rbgs<T>(const Level&, const EllOp<T>&, const double*, const T*, T*, \
                                int, bool, hipStream_t);                                  \
    template int launch_residual<T>(const Level&, const EllOp<T>&, const double*, const T*, \

@@ -584,7 +584,85 @@ static int hier_psetup(Sim* S, double* y, double gamma)
    return 0;
 }
 
-static int hier_psolve(Sim* S, const double* r, double* z, double delta)
+// The block operators of the last preconditioner setup in element type T.
+template <typename T>
+struct PrecArrays {
+   const T *Cphi, *Mphi, *Dconc, *fc, *sm;
+};
+template <typename T>
+static PrecArrays<T> prec_arrays(const Sim* S);
+template <>
+PrecArrays<float> prec_arrays<float>(const Sim* S)
+{
+   return {S->f_Cphi, S->f_Mphi, S->f_Dconc, S->f_fc, S->f_sqrtm};
+}
+template <>
+PrecArrays<double> prec_arrays<double>(const Sim* S)
+{
+   return {S->Cphi, S->Mphi, S->Dconc, S->fc, S->sqrtm};
+}
+
+// The elliptic blocks (every phase order, every species) or the orientation
+// block (from component comp on) as slots.
+template <typename T>
+static int add_elliptic(const Sim* S, SweepSet<T>& set)
+{
+   const ampe_model_params& p = S->p;
+   const PrecArrays<T> A = prec_arrays<T>(S);
+   SweepSlot<T> ph;
+   ph.Dc = (T)(-S->gamma_setup * p.epsilon_phi * p.epsilon_phi);
+   ph.C = A.Cphi;
+   ph.Cc = T(1);
+   ph.M = p.phi_mobility_type == AMPE_PHI_MOB_KIM ? A.Mphi : nullptr;
+   ph.Mc = (T)p.phi_mobility;
+   if (sweep_add<T>(set, ph, 0, S->nord)) return -1;
+   if (S->ncs == 0) return 0;
+   SweepSlot<T> co;
+   co.D = A.Dconc;
+   co.Cc = T(1);
+   co.Mc = (T)p.conc_mobility;
+   return sweep_add<T>(set, co, S->ic, S->ncs);
+}
+template <typename T>
+static int add_orientation(const Sim* S, SweepSet<T>& set, int comp)
+{
+   const PrecArrays<T> A = prec_arrays<T>(S);
+   SweepSlot<T> q;
+   q.kind = 1;
+   q.D = A.fc;
+   q.sm = A.sm;
+   q.gamma = (T)S->gamma_setup;
+   return sweep_add<T>(set, q, comp, S->p.qlen);
+}
+
+// e = P^-1 r over the hierarchy from e = 0 (zeroed by the caller), one cycle
+// of every block, r used up: all blocks in the same launches when their
+// sweeps on the coarsest level agree, else the orientation block after the
+// elliptic ones.
+template <typename T>
+static int hier_psolve_set(Sim* S, T* r, T* e, T* tmp)
+{
+   const bool q = S->iq >= 0;
+   const bool one = q && S->s.quat_sweeps == S->s.fac_sweeps;
+   const int nell = S->nord + S->ncs;
+   SweepSet<T> set;
+   if (add_elliptic<T>(S, set)) return -1;
+   if (one && add_orientation<T>(S, set, S->iq)) return -1;
+   if (hier_fac_cycle_set<T>(*S->hier, set, S->s.fac_sweeps, (1ULL << nell) - 1, r, e, tmp,
+                             S->stream))
+      return -1;
+   if (!q || one) return 0;
+   const long long off = (long long)S->iq * S->ng;
+   SweepSet<T> qs;
+   if (add_orientation<T>(S, qs, 0)) return -1;
+   return hier_fac_cycle_set<T>(*S->hier, qs, S->s.quat_sweeps, 0, r + off, e + off, tmp + off,
+                                S->stream);
+}
+
+// status: the caller wants to know whether the blocks' residual norms met
+// delta (0 / 1); the integrator does not, and then one cycle per block needs
+// no norm.
+static int hier_psolve(Sim* S, const double* r, double* z, double delta, bool status)
 {
    const ampe_model_params& p = S->p;
    hipStream_t st = S->stream;
@@ -596,6 +674,22 @@ static int hier_psolve(Sim* S, const double* r, double* z, double delta)
    if (!r || !z) {
       set_error("hier_psolve: needs the input and output vectors");
       return -1;
+   }
+   // (60 components of two elliptic operators fit the set's 16 slots of four)
+   if (!status && S->s.fac_max_cycles <= 1 && S->s.quat_max_cycles <= 1 && S->s.fac_tol < 0.0 &&
+       S->nc <= 60) {
+      if (S->s.precision == AMPE_FAC_FP32) {
+         if (psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, S->f_u, st) ||
+             hier_psolve_set<float>(S, S->f_f, S->f_u, S->f_r) ||
+             psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, nullptr, z, st))
+            return -1;
+         return 0;
+      }
+      if (psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, z, st) ||
+          hier_psolve_set<double>(S, S->fac_e, z, S->fac_r))
+         return -1;
+      if (S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql)) return -1;
+      return 0;
    }
    ampe_fac_params fp{S->s.fac_max_cycles, 1, 1, S->s.fac_sweeps, S->s.fac_tol};
    if (S->s.precision == AMPE_FAC_FP32) {
@@ -1079,11 +1173,11 @@ static const Level* qsplit_level(const Sim* S)
 struct PsolveOpts {
    bool f_ready = false;
    bool keep = false;
+   bool status = false;  // hierarchy: return whether the residual norms met delta
 };
-static int hier_psolve(Sim* S, const double* r, double* z, double delta);
 static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o = {})
 {
-   if (S->hier) return hier_psolve(S, r, z, delta);
+   if (S->hier) return hier_psolve(S, r, z, delta, o.status);
    const ampe_model_params& p = S->p;
    hipStream_t st = S->stream;
    long long ng = S->ng;
@@ -1844,7 +1938,9 @@ int sim_cb_psetup(Sim* S, double t, double* y, double gamma)
 
 int sim_cb_psolve(Sim* S, const double* r, double* z, double delta)
 {
-   return psolve(S, r, z, delta);
+   PsolveOpts o;
+   o.status = true;
+   return psolve(S, r, z, delta, o);
 }
 
 int sim_cb_project(Sim* S, const double* y, double* corr, double* err)
