@@ -88,10 +88,8 @@ struct Hier {
    // patch boundary of level l+1
    DevVec<CfFace> fff[kMaxLev];
    DevVec<CfCorr> cfi[kMaxLev];
-   // the face ghosts of level l filled from its own patches (the sweeps and
-   // residuals of the FAC cycle read no edge or corner ghost), the fine faces
-   // cff then fff and the corrections cfc then cfi in one table each
-   DevVec<long long> fg_dst[kMaxLev], fg_src[kMaxLev];
+   // the fine faces cff then fff and the corrections cfc then cfi in one table
+   // each
    DevVec<CfFace> facf[kMaxLev];
    DevVec<CfCorr> facc[kMaxLev];
    // prolongation of level l (l > 0): fine interior cell, coarse parent
@@ -192,8 +190,6 @@ void hier_destroy(Hier* H)
       H->cfc[l].release();
       H->fff[l].release();
       H->cfi[l].release();
-      H->fg_dst[l].release();
-      H->fg_src[l].release();
       H->facf[l].release();
       H->facc[l].release();
       H->pro_dst[l].release();
@@ -293,7 +289,6 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
 
    // ghost tables per level
    std::vector<long long> gd[kMaxLev], gs[kMaxLev], cd[kMaxLev], cs9[kMaxLev];
-   std::vector<long long> fgd[kMaxLev], fgs[kMaxLev];
    std::vector<double> cw[kMaxLev];
    for (int l = 0; l < nlev; l++)
       for (int p = H->pbeg[l]; p < H->pbeg[l + 1]; p++) {
@@ -311,10 +306,6 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
                   if (s >= 0) {
                      gd[l].push_back(dst);
                      gs[l].push_back(s);
-                     if ((i < 0 || i >= n[0]) + (j < 0 || j >= n[1]) + (k < 0 || k >= n[2]) == 1) {
-                        fgd[l].push_back(dst);
-                        fgs[l].push_back(s);
-                     }
                      continue;
                   }
                   if (l == 0) return hier_fail(H, "level 0 leaves a ghost uncovered");
@@ -371,9 +362,6 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
       if (level_create_placed(ndim, H->boxes.data(), np, pl, none, none, &H->comp))
          return hier_fail(H, "composite placement failed");
    }
-   for (int l = 0; l < nlev; l++)
-      if (H->fg_dst[l].upload(fgd[l]) || H->fg_src[l].upload(fgs[l]))
-         return hier_fail(H, "upload failed");
    for (int l = 1; l < nlev; l++) {
       if (H->cf_dst[l].upload(cd[l]) || H->cf_src[l].upload(cs9[l]) || H->cf_w[l].upload(cw[l]))
          return hier_fail(H, "upload failed");
@@ -1591,38 +1579,41 @@ struct SetCtx {
 };
 
 template <typename T>
-static int set_ghosts(const SetCtx<T>& X, int l, T* x)
+static int fac_set_ghosts(const SetCtx<T>& X, int l, T* x)
 {
    const Hier& H = *X.H;
-   const long long ng = H.fg_dst[l].n, nf = l > 0 ? H.cff[l].n : 0;
+   // (the sweeps and residuals of the cycle read no edge or corner ghost)
+   const Level& L = *H.lev[l];
+   const long long ng = L.nghost_face, nf = l > 0 ? H.cff[l].n : 0;
    if (ng + nf == 0) return 0;
    const double tw = tranwt_ref();
    dim3 g = grid1(ng + nf);
    g.y = X.ncomp;
-   hipLaunchKernelGGL(k_set_ghosts<T>, g, dim3(256), 0, X.s, x, H.ncg, H.fg_dst[l].p,
-                      H.fg_src[l].p, ng, H.cff[l].p, nf, X.ewing, (T)tw, (T)(2.0 * tw));
+   hipLaunchKernelGGL(k_set_ghosts<T>, g, dim3(256), 0, X.s, x, H.ncg, L.ghost_dst,
+                      L.ghost_src, ng, H.cff[l].p, nf, X.ewing, (T)tw, (T)(2.0 * tw));
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
 
 // zero: x is zero on the level and its parents, so are its ghosts
 template <typename T>
-static int set_smooth(const SetCtx<T>& X, int l, const T* b, T* x, int sweeps, bool zero)
+static int fac_set_smooth(const SetCtx<T>& X, int l, const T* b, T* x, int sweeps, bool zero)
 {
    const Hier& H = *X.H;
    for (int c = 0; c < 2 * sweeps; c++) {
-      if (!(zero && c == 0) && set_ghosts(X, l, x)) return -1;
-      if (launch_set_sweep<T>(*H.lev[l], *X.set, H.dx[l], b, x, c & 1, X.s)) return -1;
+      if (!(zero && c == 0) && fac_set_ghosts(X, l, x)) return -1;
+      if (launch_set_sweep<T>(*H.lev[l], *X.set, H.dx[l], b, x, c & 1, SetForm{}, X.s)) return -1;
    }
    return 0;
 }
 
 template <typename T>
-static int set_residual(const SetCtx<T>& X, int l, T* res, T* x, const T* b)
+static int fac_set_residual(const SetCtx<T>& X, int l, T* res, T* x, const T* b)
 {
    const Hier& H = *X.H;
-   if (set_ghosts(X, l, x)) return -1;
-   if (launch_set_residual<T>(*H.lev[l], *X.set, H.dx[l], b, x, res, X.s)) return -1;
+   const Level& L = *H.lev[l];
+   if (fac_set_ghosts(X, l, x)) return -1;
+   if (launch_set_residual<T>(L, *X.set, H.dx[l], b, x, res, false, X.s)) return -1;
    if (l + 1 < H.nlev && H.facc[l].n > 0) {
       double af, ac;
       corr_areas(H, l, af, ac);
@@ -1653,14 +1644,14 @@ int hier_fac_cycle_set(const Hier& H, const SweepSet<T>& set, int coarse_its,
    for (int l = top - 1; l >= 0; l--)
       if (coarsen_level_t<T>(H, l, r, r, nc, s)) return -1;
    for (int l = top; l >= 1; l--) {
-      if (set_smooth(X, l, r, e, 1, true)) return -1;
-      if (set_residual(X, l, tmp, e, r)) return -1;
+      if (fac_set_smooth(X, l, r, e, 1, true)) return -1;
+      if (fac_set_residual(X, l, tmp, e, r)) return -1;
       if (coarsen_level_t<T>(H, l - 1, tmp, r, nc, s)) return -1;
    }
-   if (set_smooth(X, 0, r, e, coarse_its, true)) return -1;
+   if (fac_set_smooth(X, 0, r, e, coarse_its, true)) return -1;
    for (int l = 1; l <= top; l++) {
       if (prolong_level_t<T>(H, l, e, nc, s)) return -1;
-      if (set_smooth(X, l, r, e, 1, false)) return -1;
+      if (fac_set_smooth(X, l, r, e, 1, false)) return -1;
    }
    for (int l = top - 1; l >= 0; l--)
       if (coarsen_level_t<T>(H, l, e, e, nc, s)) return -1;

@@ -31,6 +31,16 @@ struct SweepSlot {
    T Mc = 0;
    const T* sm = nullptr;
    T gamma = 0;
+   const T* b = nullptr;  // the slot's own right-hand side instead of the shared one's components
+};
+// How a set's vectors are stored and read: split: the row parity-split layout
+// (every component; coefficients natural); wrap: neighbours across the
+// boundary of a one-patch periodic level read in place (level_wrap_ok), no
+// ghost filled; from 1 / 2: the first red / black colour of a solve from zero
+// (checker_ok levels).
+struct SetForm {
+   bool split = false, wrap = false;
+   int from = 0;
 };
 constexpr int kMaxSlots = 16;
 template <typename T>
@@ -46,10 +56,36 @@ int sweep_add(SweepSet<T>& set, const SweepSlot<T>& proto, int comp, int ncomp);
 // One colour of every slot's red-black sweep, and every slot's residual.
 template <typename T>
 int launch_set_sweep(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs, T* x,
-                     int color, hipStream_t s);
+                     int color, const SetForm& form, hipStream_t s);
 template <typename T>
 int launch_set_residual(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs,
-                        const T* x, T* res, hipStream_t s);
+                        const T* x, T* res, bool split, hipStream_t s);
+// b (on coarse, the fine boxes halved) = the restriction of every slot's
+// residual on fine after sweeps that end with the black colour: the red cells'
+// residuals alone (the caller checks red_residual_ok).
+template <typename T>
+int launch_set_resrestrict(const Level& coarse, const Level& fine, const SweepSet<T>& set,
+                           const double* dx, const T* rhs, const T* x, T* b, const SetForm& form,
+                           hipStream_t s);
+// Algorithmic bytes of one colour of a set's sweep: all solution values read
+// and the colour's written, the colour's right-hand sides, the face and cell
+// coefficients read once.
+template <typename T>
+double set_sweep_bytes(const Level& L, const SweepSet<T>& set, int from)
+{
+   const double n = (double)L.ncell;
+   double v = 0.0;
+   for (int i = 0; i < set.n; i++) {
+      const SweepSlot<T>& o = set.s[i];
+      // the first red colour reads no solution value, the first black one the
+      // red half only
+      const double read = from == 0 ? 1.0 : (from == 1 ? 0.0 : 0.5);
+      v += o.ncomp * n * (read + 0.5 + 0.5);
+      if (o.D) v += (double)L.nside_tot;
+      v += n * ((o.C != nullptr) + (o.M != nullptr) + (o.sm != nullptr));
+   }
+   return v * sizeof(T);
+}
 
 int launch_phase_C(const Level& L, const ampe_model_params& p, double gamma,
                    const double* phi, const double* M, double* C, hipStream_t s);
@@ -65,35 +101,26 @@ template <typename T>
 int launch_residual(const Level& L, const EllOp<T>& op, const double* dx, const T* rhs,
                     const T* u, T* res, double* part, hipStream_t s);
 
-// Orientation block: one colour of the red-black sweep, and the residual.
-// split: the component blocks of rhs, z and res are stored in the row
-// parity-split layout (split_col; fc and sm stay natural).
+// Orientation block: one colour of the red-black sweep, and the residual
+// (split: rhs, z and res in the row parity-split layout).
 template <typename T>
 int launch_quat_rbgs(const Level& L, const T* fc, const T* sm, double gamma, const double* dx,
-                     int ncomp, const T* rhs, T* z, int color, hipStream_t s, bool split = false);
+                     int ncomp, const T* rhs, T* z, int color, hipStream_t s);
 
 template <typename T>
 int launch_quat_residual(const Level& L, const T* fc, const T* sm, double gamma,
                          const double* dx, int ncomp, const T* rhs, const T* z, T* res,
                          double* part, hipStream_t s, bool split = false);
 
-// b (on coarse, the fine boxes halved) = the restriction of the elliptic
-// residual rhs - A u on fine after red-black sweeps ending with the black
-// colour: the red cells' residuals alone, summed per coarse cell (periodic
-// levels with one checkerboard; the caller checks).
+// launch_set_resrestrict of one elliptic block, and of one orientation block
+// of one, two or four components.
 template <typename T>
 int launch_ell_resrestrict(const Level& coarse, const Level& fine, const EllOp<T>& op,
                            const double* dx, const T* rhs, const T* u, T* b, hipStream_t s);
-
-// b (on coarse, the fine boxes halved) = the restriction of the residual
-// rhs - A z on fine when z comes out of red-black sweeps ending with the black
-// colour: the red cells' residuals alone (the black ones vanish), summed per
-// coarse cell.  One, two or four components; valid on periodic levels whose
-// colouring is one checkerboard (the caller checks).
 template <typename T>
 int launch_quat_resrestrict(const Level& coarse, const Level& fine, const T* fc, const T* sm,
                             double gamma, const double* dx, int ncomp, const T* rhs, const T* z,
-                            T* b, hipStream_t s, bool split = false);
+                            T* b, hipStream_t s);
 
 // ------------------------------------------------------------ vectors
 // Flat element-wise ops over n entries (whole ghosted vectors).
@@ -121,17 +148,16 @@ int vec_to_f64(long long n, const float* x, double* y, hipStream_t s);
 int vec_div_f(long long n, const double* x, const double* sm, double* y, hipStream_t s);
 int vec_sqrt(long long n, const double* x, double* y, hipStream_t s);
 // Preconditioner input / output over nc component blocks (orientation blocks
-// [iq, iq+ql) scaled by 1/sqrt(M) on input, sqrt(M) on output); psolve_in
-// also zeroes u.  With f null (FP64) only the orientation blocks go to fq.
-// psolve_out multiplies the result by ewt when ewt is not null.  split (a
-// level): the orientation blocks of f / fq / u are in that level's row
-// parity-split layout.
+// [iq, iq+ql) scaled by 1/sqrt(M) on input, sqrt(M) on output); u, when given,
+// is zeroed by psolve_in.  With f null (FP64) only the orientation blocks go to
+// fq.  split (a level): the blocks from component sp0 on are stored in that
+// level's row parity-split layout.
 template <typename T>
 int psolve_in(long long ng, int nc, int iq, int ql, const double* r, const double* sm, T* f,
-              T* fq, T* u, hipStream_t s, const Level* split = nullptr);
+              T* fq, T* u, hipStream_t s, const Level* split = nullptr, int sp0 = 0);
 template <typename T>
 int psolve_out(long long ng, int nc, int iq, int ql, const T* u, const double* sm,
-               const double* ewt, double* z, hipStream_t s, const Level* split = nullptr);
+               double* z, hipStream_t s, const Level* split = nullptr, int sp0 = 0);
 int vec_scale_comp(long long ng, int ncomp, const double* sm, double* x, hipStream_t s);
 // Reductions over interior cells of ncomp component blocks (host result,
 // synchronises s).

@@ -164,19 +164,6 @@ __global__ void __launch_bounds__(256) k_rbgs(LevelArgs a, OpArgs<T> op, T di0, 
    if (partial) block_store_max<T>(absres, partial);
 }
 
-// The same on the colour-compact mapping (no max-residual partials).
-template <typename T, int NDIM>
-__global__ void __launch_bounds__(128) k_rbgs_c(LevelArgs a, OpArgs<T> op, T di0, T di1, T di2,
-                                                const T* __restrict__ rhs, T* __restrict__ u,
-                                                int color)
-{
-   const T dinv[3] = {di0, di1, di2};
-   for (int kk = 0; kk < a.nz_tile; kk++) {
-      CellPos c;
-      if (cell_pos_color<NDIM>(a, kk, color, c)) (void)rbgs_cell<T, NDIM>(a, c, op, dinv, rhs, u);
-   }
-}
-
 // efo_compres*sca (source/fortran/2d/ellipticfacops.m4:346-446) + sum res^2
 template <typename T, int NDIM>
 __global__ void __launch_bounds__(256) k_residual(LevelArgs a, OpArgs<T> op, T di0, T di1, T di2,
@@ -192,49 +179,6 @@ __global__ void __launch_bounds__(256) k_residual(LevelArgs a, OpArgs<T> op, T d
    sq += (double)r * (double)r;
    AMPE_COLUMN_END
    if (partial) block_store_sum<T>(sq, partial);
-}
-
-// The elliptic residual restricted from the red cells only: after red-black
-// sweeps ending with the black colour each black row's residual vanishes (its
-// update zeroes it, and the row couples the cell to red neighbours only), so
-// the coarse right-hand side is, per coarse cell, the mean of its red
-// children's residuals in k_restrict_cell's summation order.  Periodic levels
-// with one checkerboard (the caller checks).
-template <typename T, int NDIM>
-__global__ void __launch_bounds__(256) k_ell_resrestrict(LevelArgs ca, LevelArgs fa,
-                                                         OpArgs<T> op, T di0, T di1, T di2,
-                                                         const T* __restrict__ rhs,
-                                                         const T* __restrict__ u,
-                                                         T* __restrict__ b)
-{
-   CellPos p;
-   if (!cell_pos(ca, 0, p)) return;
-   const T dinv[3] = {di0, di1, di2};
-   const PatchDev fp = fa.P[ca.T[tile_index(ca)].patch];
-   T pr[4];
-#pragma unroll
-   for (int dz = 0; dz < (NDIM == 3 ? 2 : 1); dz++)
-#pragma unroll
-      for (int dy = 0; dy < 2; dy++) {
-         CellPos c;
-         c.pd = fp;
-         c.j = 2 * p.j + dy;
-         c.k = NDIM == 3 ? 2 * p.k + dz : 0;
-         int gj = fp.lo[1] + c.j;
-         int x = (NDIM == 3) ? fp.lo[0] + gj + (fp.lo[2] + c.k) : fp.lo[1] + gj;
-         int io = ((x - (x / 2) * 2) != 0) ? 1 : 0;  // red cells of the row (cell_pos_color)
-         c.i = 2 * p.i + io;
-         c.st[0] = 1;
-         c.st[1] = fp.sy;
-         c.st[2] = fp.sz;
-         c.c0 = fp.cell_off + (c.i + fa.g) + (long long)(c.j + fa.g) * fp.sy +
-                (long long)(c.k + fa.gz) * fp.sz;
-         T diag;
-         pr[dy + 2 * dz] = op_residual<T, NDIM>(fa, c, op, rhs, u, dinv, &diag);
-      }
-   T sum = pr[0] + pr[1];
-   if (NDIM == 3) sum = sum + (pr[2] + pr[3]);
-   b[p.c0] = sum * (NDIM == 3 ? T(0.125) : T(0.25));
 }
 
 // ------------------------------------------------------------ orientation
@@ -393,59 +337,6 @@ __device__ __forceinline__ T quat_row_apply(const QuatRowCoef<T>& w, const QuatR
    for (int d = 0; d < NDIM; d++) r = r + w.wlo[d] * v.zl[d] + w.whi[d] * v.zh[d];
    return r;
 }
-
-// Gauss-Seidel update of one cell, every component.  QL > 0: QL components,
-// all loads issued before the first update (the updates write only this
-// cell, which no other load of the cell reads); QL = 0: ncomp components one
-// after the other.  SPLIT: z and rhs in the row parity-split layout (fc and
-// sm natural).
-template <typename T, int NDIM, int QL, bool SPLIT>
-__device__ __forceinline__ void quat_rbgs_cell(const LevelArgs& a, const CellPos& c,
-                                               const T* __restrict__ fc, const T* __restrict__ sm,
-                                               T gamma, const T* hinv2, int ncomp,
-                                               const T* __restrict__ rhs, T* __restrict__ z)
-{
-   const QuatRowCoef<T> w = quat_row_coef<T, NDIM>(a, c, fc, sm, gamma, hinv2);
-   const QuatIdx q = quat_idx<SPLIT>(a, c);
-   if (QL > 0) {
-      QuatRowVals<T, NDIM> v[QL > 0 ? QL : 1];
-      T rv[QL > 0 ? QL : 1];
-#pragma unroll
-      for (int m = 0; m < QL; m++) {
-         quat_row_load<T, NDIM>(c, q, z + m * a.ncg, v[m]);
-         rv[m] = rhs[m * a.ncg + q.c];
-      }
-#pragma unroll
-      for (int m = 0; m < QL; m++) {
-         T res = rv[m] - quat_row_apply<T, NDIM>(w, v[m]);
-         z[m * a.ncg + q.c] = v[m].zc + res / w.center;
-      }
-   } else {
-      for (int m = 0; m < ncomp; m++) {
-         QuatRowVals<T, NDIM> v;
-         quat_row_load<T, NDIM>(c, q, z + m * a.ncg, v);
-         T res = rhs[m * a.ncg + q.c] - quat_row_apply<T, NDIM>(w, v);
-         z[m * a.ncg + q.c] = v.zc + res / w.center;
-      }
-   }
-}
-
-// One colour of the sweep on the colour-compact mapping.
-template <typename T, int NDIM, int QL, bool SPLIT>
-__global__ void __launch_bounds__(128) k_quat_rbgs_c(LevelArgs a, const T* __restrict__ fc,
-                                                     const T* __restrict__ sm, T gamma, T hi0,
-                                                     T hi1, T hi2, int ncomp,
-                                                     const T* __restrict__ rhs,
-                                                     T* __restrict__ z, int color)
-{
-   const T hinv2[3] = {hi0, hi1, hi2};
-   for (int kk = 0; kk < a.nz_tile; kk++) {
-      CellPos c;
-      if (cell_pos_color<NDIM>(a, kk, color, c))
-         quat_rbgs_cell<T, NDIM, QL, SPLIT>(a, c, fc, sm, gamma, hinv2, ncomp, rhs, z);
-   }
-}
-
 
 // ------------------------------------------------------------ fused sweep
 // One red-black sweep of the orientation block in one pass, zin -> zout
@@ -647,88 +538,6 @@ __global__ void __launch_bounds__(256) k_quat_residual(LevelArgs a, const T* __r
    if (partial) block_store_sum<T>(sq, partial);
 }
 
-// The residual in the split layout without the reduction, on the pair
-// mapping: a half-wave's cells have one column parity, so its split-layout
-// loads and stores cover contiguous runs.
-template <typename T, int NDIM, int QL>
-__global__ void __launch_bounds__(128) k_quat_residual_p(LevelArgs a, const T* __restrict__ fc,
-                                                         const T* __restrict__ sm, T gamma,
-                                                         T hi0, T hi1, T hi2, int ncomp,
-                                                         const T* __restrict__ rhs,
-                                                         const T* __restrict__ z,
-                                                         T* __restrict__ res)
-{
-   const T hinv2[3] = {hi0, hi1, hi2};
-   for (int kk = 0; kk < a.nz_tile; kk++)
-      for (int io = 0; io < 2; io++) {
-         CellPos c;
-         if (cell_pos_pair(a, kk, io, c))
-            (void)quat_residual_cell<T, NDIM, QL, true>(a, c, fc, sm, gamma, hinv2, ncomp, rhs,
-                                                        z, res);
-      }
-}
-
-// Red residuals restricted.  After a pre-smoothing that ends with the black
-// colour, the residual vanishes on black cells in exact arithmetic (a black
-// update zeroes its own row's residual, and a black row couples its cell to
-// red cells only), so the coarse right-hand side is the restriction of the red
-// residuals: per coarse cell, its 2^(NDIM-1) red children's residuals in the
-// restriction's summation order (each pair of x-children sums to its red
-// member), without storing the fine residual.  Needs one checkerboard across
-// patches and periodic ghosts (a zero-slope ghost would copy a black cell's
-// new value into its own row); the host checks both.
-template <typename T, int NDIM, int QL, bool SPLIT>
-__global__ void __launch_bounds__(256) k_quat_resrestrict(LevelArgs ca, LevelArgs fa,
-                                                          const T* __restrict__ fc,
-                                                          const T* __restrict__ sm, T gamma,
-                                                          T hi0, T hi1, T hi2,
-                                                          const T* __restrict__ rhs,
-                                                          const T* __restrict__ z,
-                                                          T* __restrict__ b)
-{
-   CellPos p;
-   if (!cell_pos(ca, 0, p)) return;
-   const T hinv2[3] = {hi0, hi1, hi2};
-   const PatchDev fp = fa.P[ca.T[tile_index(ca)].patch];
-   T pr[QL][4];
-#pragma unroll
-   for (int dz = 0; dz < (NDIM == 3 ? 2 : 1); dz++)
-#pragma unroll
-      for (int dy = 0; dy < 2; dy++) {
-         CellPos c;
-         c.pd = fp;
-         c.j = 2 * p.j + dy;
-         c.k = NDIM == 3 ? 2 * p.k + dz : 0;
-         int gj = fp.lo[1] + c.j;
-         int x = (NDIM == 3) ? fp.lo[0] + gj + (fp.lo[2] + c.k) : fp.lo[1] + gj;
-         int io = ((x - (x / 2) * 2) != 0) ? 1 : 0;  // red cells of the row (cell_pos_color)
-         c.i = 2 * p.i + io;
-         c.st[0] = 1;
-         c.st[1] = fp.sy;
-         c.st[2] = fp.sz;
-         c.c0 = fp.cell_off + (c.i + fa.g) + (long long)(c.j + fa.g) * fp.sy +
-                (long long)(c.k + fa.gz) * fp.sz;
-         const QuatRowCoef<T> w = quat_row_coef<T, NDIM>(fa, c, fc, sm, gamma, hinv2);
-         const QuatIdx q = quat_idx<SPLIT>(fa, c);
-         QuatRowVals<T, NDIM> v[QL];
-         T rv[QL];
-#pragma unroll
-         for (int m = 0; m < QL; m++) {
-            quat_row_load<T, NDIM>(c, q, z + m * fa.ncg, v[m]);
-            rv[m] = rhs[m * fa.ncg + q.c];
-         }
-#pragma unroll
-         for (int m = 0; m < QL; m++) pr[m][dy + 2 * dz] = rv[m] - quat_row_apply<T, NDIM>(w, v[m]);
-      }
-   const long long co = SPLIT ? split_at(ca, p, 0) : p.c0;
-#pragma unroll
-   for (int m = 0; m < QL; m++) {
-      T s = pr[m][0] + pr[m][1];
-      if (NDIM == 3) s = s + (pr[m][2] + pr[m][3]);
-      b[m * ca.ncg + co] = s * (NDIM == 3 ? T(0.125) : T(0.25));
-   }
-}
-
 // ------------------------------------------------------------ block sets
 // The elliptic row's coefficients at one cell, shared by the slot's
 // components: dinv D of the low and high faces, M, C and the diagonal (the
@@ -786,12 +595,109 @@ __device__ __forceinline__ T ell_row_residual(const EllRowCoef<T>& w, const T* d
    return rhs - w.m * div - w.cc * v.zc;
 }
 
-// One colour of the red-black sweep of every slot: blockIdx.y is the slot, so
-// the phase, orientation and composition blocks (and the components of each)
-// of a level are one launch instead of one per component.  On the small
-// levels of a hierarchy a launch costs 2-4 us whatever it computes, and these
-// sweeps and the ghost fills between them are most of a solve there.
+// Where a cell and its face neighbours sit in one component block.  SPLIT: the
+// row parity-split layout.  WRAP: the one patch of a periodic level, whose
+// neighbours across the boundary are read where they are, at the patch's
+// other side, so that no ghost is filled between two colours (the colours
+// meet across the boundary as inside: the caller checks that the extents are
+// even).
+template <int NDIM>
+struct NbrIdx {
+   long long c, l[NDIM], h[NDIM];
+};
+
+template <int NDIM, bool SPLIT, bool WRAP>
+__device__ __forceinline__ NbrIdx<NDIM> nbr_idx(const LevelArgs& a, const CellPos& c)
+{
+   NbrIdx<NDIM> q;
+   const int nx = c.pd.nx, ig = c.i + a.g;
+   const int il = (WRAP && c.i == 0) ? ig + nx - 1 : ig - 1;
+   const int ih = (WRAP && c.i == nx - 1) ? ig - nx + 1 : ig + 1;
+   const long long row = c.c0 - ig;
+   q.c = SPLIT ? row + split_col(ig, c.pd.sy) : c.c0;
+   q.l[0] = SPLIT ? row + split_col(il, c.pd.sy) : row + il;
+   q.h[0] = SPLIT ? row + split_col(ih, c.pd.sy) : row + ih;
+   const int ijk[3] = {c.i, c.j, c.k}, n[3] = {nx, c.pd.ny, c.pd.nz};
+#pragma unroll
+   for (int d = 1; d < NDIM; d++) {
+      const long long s = c.st[d], w = (long long)(n[d] - 1) * s;
+      q.l[d] = (WRAP && ijk[d] == 0) ? q.c + w : q.c - s;
+      q.h[d] = (WRAP && ijk[d] == n[d] - 1) ? q.c - w : q.c + s;
+   }
+   return q;
+}
+
 template <typename T, int NDIM>
+__device__ __forceinline__ void nbr_load(const NbrIdx<NDIM>& q, const T* __restrict__ x,
+                                         QuatRowVals<T, NDIM>& v)
+{
+#pragma unroll
+   for (int d = 0; d < NDIM; d++) {
+      v.zl[d] = x[q.l[d]];
+      v.zh[d] = x[q.h[d]];
+   }
+}
+
+// Values of a component at the start of a sweep: FROM 0 any, 1 the whole
+// field is zero (a red cell of a solve from zero), 2 the cell itself is zero
+// (a black one after it).
+template <typename T, int NDIM, int FROM>
+__device__ __forceinline__ void nbr_start(const NbrIdx<NDIM>& q, const T* __restrict__ x,
+                                          QuatRowVals<T, NDIM>& v)
+{
+   v.zc = FROM == 0 ? x[q.c] : T(0);
+   if (FROM == 1) {
+#pragma unroll
+      for (int d = 0; d < NDIM; d++) v.zl[d] = v.zh[d] = T(0);
+   } else {
+      nbr_load<T, NDIM>(q, x, v);
+   }
+}
+
+// Gauss-Seidel update of the orientation block at one cell: QL > 0 all loads
+// of QL components before the first update, QL = 0 one component after the
+// other.
+template <typename T, int NDIM, int QL, int FROM>
+__device__ __forceinline__ void set_quat_cell(const QuatRowCoef<T>& w, const NbrIdx<NDIM>& q,
+                                              long long ncg, int ncomp,
+                                              const T* __restrict__ b, T* __restrict__ x)
+{
+   if (QL > 0) {
+      QuatRowVals<T, NDIM> v[QL > 0 ? QL : 1];
+      T rv[QL > 0 ? QL : 1];
+#pragma unroll
+      for (int m = 0; m < QL; m++) {
+         nbr_start<T, NDIM, FROM>(q, x + m * ncg, v[m]);
+         rv[m] = b[m * ncg + q.c];
+      }
+#pragma unroll
+      for (int m = 0; m < QL; m++) {
+         T res = FROM == 1 ? rv[m] : rv[m] - quat_row_apply<T, NDIM>(w, v[m]);
+         x[m * ncg + q.c] = v[m].zc + res / w.center;
+      }
+      return;
+   }
+   for (int m = 0; m < ncomp; m++) {
+      QuatRowVals<T, NDIM> v;
+      nbr_start<T, NDIM, FROM>(q, x + m * ncg, v);
+      T res = b[m * ncg + q.c];
+      if (FROM != 1) res = res - quat_row_apply<T, NDIM>(w, v);
+      x[m * ncg + q.c] = v.zc + res / w.center;
+   }
+}
+
+// One colour of the red-black sweep of every slot on the colour-compact
+// mapping: blockIdx.y is the slot, so the phase, orientation and composition
+// blocks (and the components of each) of a level are one launch instead of one
+// per block; on the small levels of a hierarchy or a V-cycle a launch costs
+// 2-4 us whatever it computes.  FROM 1 and 2: the first red and black colours of
+// a solve from zero, which read no solution values they know to be zero, so
+// that nothing clears the solution first: 32 instead of 48 + 16 bytes a cell for
+// the red colour of the FP32 orientation block.  The large levels are bound by
+// HBM: at 256^3 with six FP32 components about 310 us a colour (80 bytes a
+// cell, 4.3 TB/s; 390 us as separate launches with their ghost fills), the first
+// red one 230 us.
+template <typename T, int NDIM, bool SPLIT, bool WRAP, int FROM>
 __global__ void __launch_bounds__(128) k_set_sweep(LevelArgs a, SweepSet<T> set, T di0, T di1,
                                                    T di2, T hi0, T hi1, T hi2,
                                                    const T* __restrict__ rhs, T* __restrict__ x,
@@ -800,31 +706,33 @@ __global__ void __launch_bounds__(128) k_set_sweep(LevelArgs a, SweepSet<T> set,
    CellPos c;
    if (!cell_pos_color<NDIM>(a, 0, color, c)) return;
    const SweepSlot<T>& o = set.s[blockIdx.y];
-   const T* b = rhs + o.comp * a.ncg;
+   const T* b = o.b ? o.b : rhs + o.comp * a.ncg;
    T* u = x + o.comp * a.ncg;
+   const NbrIdx<NDIM> q = nbr_idx<NDIM, SPLIT, WRAP>(a, c);
    if (o.kind == 1) {
       const T hinv2[3] = {hi0, hi1, hi2};
+      const QuatRowCoef<T> w = quat_row_coef<T, NDIM>(a, c, o.D, o.sm, o.gamma, hinv2);
       if (o.ncomp == 4)
-         quat_rbgs_cell<T, NDIM, 4, false>(a, c, o.D, o.sm, o.gamma, hinv2, 4, b, u);
+         set_quat_cell<T, NDIM, 4, FROM>(w, q, a.ncg, 4, b, u);
       else
-         quat_rbgs_cell<T, NDIM, 0, false>(a, c, o.D, o.sm, o.gamma, hinv2, o.ncomp, b, u);
+         set_quat_cell<T, NDIM, 0, FROM>(w, q, a.ncg, o.ncomp, b, u);
       return;
    }
    const T dinv[3] = {di0, di1, di2};
    const EllRowCoef<T> w = ell_row_coef<T, NDIM>(a, c, o, dinv);
    const T dudr = T(1) / w.diag;
-   const QuatIdx q{c.c0, c.c0 - 1, c.c0 + 1};
    for (int m = 0; m < o.ncomp; m++) {
       QuatRowVals<T, NDIM> v;
-      quat_row_load<T, NDIM>(c, q, u + m * a.ncg, v);
-      const T res = ell_row_residual<T, NDIM>(w, dinv, b[m * a.ncg + c.c0], v);
+      nbr_start<T, NDIM, FROM>(q, u + m * a.ncg, v);
+      const T rv = b[m * a.ncg + q.c];
+      const T res = FROM == 1 ? rv : ell_row_residual<T, NDIM>(w, dinv, rv, v);
       const T du = -res * dudr;
-      u[m * a.ncg + c.c0] = v.zc + du * T(1);
+      u[m * a.ncg + q.c] = v.zc + du * T(1);
    }
 }
 
 // The residual of every slot, in one launch as k_set_sweep.
-template <typename T, int NDIM>
+template <typename T, int NDIM, bool SPLIT>
 __global__ void __launch_bounds__(256) k_set_residual(LevelArgs a, SweepSet<T> set, T di0, T di1,
                                                       T di2, T hi0, T hi1, T hi2,
                                                       const T* __restrict__ rhs,
@@ -834,23 +742,113 @@ __global__ void __launch_bounds__(256) k_set_residual(LevelArgs a, SweepSet<T> s
    CellPos c;
    if (!cell_pos(a, 0, c)) return;
    const SweepSlot<T>& o = set.s[blockIdx.y];
-   const T* b = rhs + o.comp * a.ncg;
+   const T* b = o.b ? o.b : rhs + o.comp * a.ncg;
    const T* u = x + o.comp * a.ncg;
    T* r = res + o.comp * a.ncg;
+   const NbrIdx<NDIM> q = nbr_idx<NDIM, SPLIT, false>(a, c);
    if (o.kind == 1) {
       const T hinv2[3] = {hi0, hi1, hi2};
-      (void)quat_residual_cell<T, NDIM, 0, false>(a, c, o.D, o.sm, o.gamma, hinv2, o.ncomp, b, u,
-                                                  r);
+      const QuatRowCoef<T> w = quat_row_coef<T, NDIM>(a, c, o.D, o.sm, o.gamma, hinv2);
+      for (int m = 0; m < o.ncomp; m++) {
+         QuatRowVals<T, NDIM> v;
+         nbr_start<T, NDIM, 0>(q, u + m * a.ncg, v);
+         r[m * a.ncg + q.c] = b[m * a.ncg + q.c] - quat_row_apply<T, NDIM>(w, v);
+      }
       return;
    }
    const T dinv[3] = {di0, di1, di2};
    const EllRowCoef<T> w = ell_row_coef<T, NDIM>(a, c, o, dinv);
-   const QuatIdx q{c.c0, c.c0 - 1, c.c0 + 1};
    for (int m = 0; m < o.ncomp; m++) {
       QuatRowVals<T, NDIM> v;
-      quat_row_load<T, NDIM>(c, q, u + m * a.ncg, v);
-      r[m * a.ncg + c.c0] = ell_row_residual<T, NDIM>(w, dinv, b[m * a.ncg + c.c0], v);
+      nbr_start<T, NDIM, 0>(q, u + m * a.ncg, v);
+      r[m * a.ncg + q.c] = ell_row_residual<T, NDIM>(w, dinv, b[m * a.ncg + q.c], v);
    }
+}
+
+// Red residuals restricted, every slot in one launch.  After sweeps that end
+// with the black colour the residual vanishes on black cells (a black update
+// zeroes its own row's residual, and a black row couples its cell to red cells
+// only), so the coarse right-hand side is the restriction of the red residuals:
+// per coarse cell, its 2^(NDIM-1) red children's residuals in the
+// restriction's summation order (each pair of x-children sums to its red
+// member), without storing the fine residual.  Needs one checkerboard across
+// patches and periodic ghosts (a zero-slope ghost would copy a black cell's
+// new value into its own row); the host checks both.
+template <typename T, int NDIM, int QL, bool SPLIT, bool WRAP>
+__device__ __forceinline__ void set_resrestrict(const LevelArgs& ca, const LevelArgs& fa,
+                                                const CellPos& p, const SweepSlot<T>& o,
+                                                const T* dinv, const T* hinv2, const T* rhs,
+                                                const T* x, T* bc, int m0)
+{
+   constexpr int N = QL > 0 ? QL : 1;
+   const PatchDev fp = fa.P[ca.T[tile_index(ca)].patch];
+   const T* b = (o.b ? o.b : rhs + o.comp * fa.ncg) + m0 * fa.ncg;
+   const T* u = x + (o.comp + m0) * fa.ncg;
+   T pr[N][4];
+#pragma unroll
+   for (int dz = 0; dz < (NDIM == 3 ? 2 : 1); dz++)
+#pragma unroll
+      for (int dy = 0; dy < 2; dy++) {
+         CellPos c;
+         c.pd = fp;
+         c.j = 2 * p.j + dy;
+         c.k = NDIM == 3 ? 2 * p.k + dz : 0;
+         int gj = fp.lo[1] + c.j;
+         int xs = (NDIM == 3) ? fp.lo[0] + gj + (fp.lo[2] + c.k) : fp.lo[1] + gj;
+         int io = ((xs - (xs / 2) * 2) != 0) ? 1 : 0;  // red cells of the row (cell_pos_color)
+         c.i = 2 * p.i + io;
+         c.st[0] = 1;
+         c.st[1] = fp.sy;
+         c.st[2] = fp.sz;
+         c.c0 = fp.cell_off + (c.i + fa.g) + (long long)(c.j + fa.g) * fp.sy +
+                (long long)(c.k + fa.gz) * fp.sz;
+         const NbrIdx<NDIM> q = nbr_idx<NDIM, SPLIT, WRAP>(fa, c);
+         QuatRowVals<T, NDIM> v[N];
+         T rv[N];
+#pragma unroll
+         for (int m = 0; m < N; m++) {
+            nbr_start<T, NDIM, 0>(q, u + m * fa.ncg, v[m]);
+            rv[m] = b[m * fa.ncg + q.c];
+         }
+         if (o.kind == 1) {
+            const QuatRowCoef<T> w = quat_row_coef<T, NDIM>(fa, c, o.D, o.sm, o.gamma, hinv2);
+#pragma unroll
+            for (int m = 0; m < N; m++)
+               pr[m][dy + 2 * dz] = rv[m] - quat_row_apply<T, NDIM>(w, v[m]);
+         } else {
+            const EllRowCoef<T> w = ell_row_coef<T, NDIM>(fa, c, o, dinv);
+#pragma unroll
+            for (int m = 0; m < N; m++)
+               pr[m][dy + 2 * dz] = ell_row_residual<T, NDIM>(w, dinv, rv[m], v[m]);
+         }
+      }
+   const long long co = (SPLIT ? split_at(ca, p, 0) : p.c0) + (o.comp + m0) * ca.ncg;
+#pragma unroll
+   for (int m = 0; m < N; m++) {
+      T sum = pr[m][0] + pr[m][1];
+      if (NDIM == 3) sum = sum + (pr[m][2] + pr[m][3]);
+      bc[m * ca.ncg + co] = sum * (NDIM == 3 ? T(0.125) : T(0.25));
+   }
+}
+
+template <typename T, int NDIM, bool SPLIT, bool WRAP>
+__global__ void __launch_bounds__(256) k_set_resrestrict(LevelArgs ca, LevelArgs fa,
+                                                         SweepSet<T> set, T di0, T di1, T di2,
+                                                         T hi0, T hi1, T hi2,
+                                                         const T* __restrict__ rhs,
+                                                         const T* __restrict__ x,
+                                                         T* __restrict__ bc)
+{
+   CellPos p;
+   if (!cell_pos(ca, 0, p)) return;
+   const SweepSlot<T>& o = set.s[blockIdx.y];
+   const T dinv[3] = {di0, di1, di2}, hinv2[3] = {hi0, hi1, hi2};
+   if (o.kind == 1 && o.ncomp == 4) {
+      set_resrestrict<T, NDIM, 4, SPLIT, WRAP>(ca, fa, p, o, dinv, hinv2, rhs, x, bc, 0);
+      return;
+   }
+   for (int m = 0; m < o.ncomp; m++)
+      set_resrestrict<T, NDIM, 1, SPLIT, WRAP>(ca, fa, p, o, dinv, hinv2, rhs, x, bc, m);
 }
 
 // ------------------------------------------------------------ launchers
@@ -929,67 +927,154 @@ int sweep_add(SweepSet<T>& set, const SweepSlot<T>& proto, int comp, int ncomp)
    return 0;
 }
 
+// Calls f with the flags as std::integral_constant.
+template <class F>
+static void bool_dispatch(bool v, F&& f)
+{
+   if (v)
+      f(std::true_type());
+   else
+      f(std::false_type());
+}
+
 template <typename T>
 int launch_set_sweep(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs, T* x,
-                     int color, hipStream_t s)
+                     int color, const SetForm& form, hipStream_t s)
 {
    T di[3], hi[3];
    recip(dx, di);
    recip2(dx, hi);
    dim3 g(L.ncell_tiles, set.n);
+   const LevelArgs la = level_args(L);
+   bool quat = false;
+   for (int i = 0; i < set.n; i++) quat |= set.s[i].kind == 1;
+   KernelTimer::Span span(quat ? KernelTimer::QUAT_RBGS : -1, s,
+                          set_sweep_bytes(L, set, form.from));
+   auto go = [&](auto nd, auto sp, auto wr, auto fr) {
+      hipLaunchKernelGGL((k_set_sweep<T, decltype(nd)::value, decltype(sp)::value,
+                                      decltype(wr)::value, decltype(fr)::value>),
+                         g, cblock(), 0, s, la, set, di[0], di[1], di[2], hi[0], hi[1], hi[2],
+                         rhs, x, color);
+   };
+   auto by_from = [&](auto nd, auto sp, auto wr) {
+      if (form.from == 1)
+         go(nd, sp, wr, std::integral_constant<int, 1>());
+      else if (form.from == 2)
+         go(nd, sp, wr, std::integral_constant<int, 2>());
+      else
+         go(nd, sp, wr, std::integral_constant<int, 0>());
+   };
+   auto by_form = [&](auto nd) {
+      bool_dispatch(form.split, [&](auto sp) {
+         bool_dispatch(form.wrap, [&](auto wr) { by_from(nd, sp, wr); });
+      });
+   };
    if (L.ndim == 3)
-      hipLaunchKernelGGL((k_set_sweep<T, 3>), g, cblock(), 0, s, level_args(L), set, di[0], di[1],
-                         di[2], hi[0], hi[1], hi[2], rhs, x, color);
+      by_form(std::integral_constant<int, 3>());
    else
-      hipLaunchKernelGGL((k_set_sweep<T, 2>), g, cblock(), 0, s, level_args(L), set, di[0], di[1],
-                         di[2], hi[0], hi[1], hi[2], rhs, x, color);
+      by_form(std::integral_constant<int, 2>());
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
 
 template <typename T>
 int launch_set_residual(const Level& L, const SweepSet<T>& set, const double* dx, const T* rhs,
-                        const T* x, T* res, hipStream_t s)
+                        const T* x, T* res, bool split, hipStream_t s)
 {
    T di[3], hi[3];
    recip(dx, di);
    recip2(dx, hi);
    dim3 g(L.ncell_tiles, set.n);
-   if (L.ndim == 3)
-      hipLaunchKernelGGL((k_set_residual<T, 3>), g, tblock(), 0, s, level_args(L), set, di[0],
-                         di[1], di[2], hi[0], hi[1], hi[2], rhs, x, res);
-   else
-      hipLaunchKernelGGL((k_set_residual<T, 2>), g, tblock(), 0, s, level_args(L), set, di[0],
-                         di[1], di[2], hi[0], hi[1], hi[2], rhs, x, res);
+   const LevelArgs la = level_args(L);
+   auto go = [&](auto nd, auto sp) {
+      hipLaunchKernelGGL((k_set_residual<T, decltype(nd)::value, decltype(sp)::value>), g,
+                         tblock(), 0, s, la, set, di[0], di[1], di[2], hi[0], hi[1], hi[2], rhs, x,
+                         res);
+   };
+   bool_dispatch(split, [&](auto sp) {
+      if (L.ndim == 3)
+         go(std::integral_constant<int, 3>(), sp);
+      else
+         go(std::integral_constant<int, 2>(), sp);
+   });
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
+}
+
+template <typename T>
+int launch_set_resrestrict(const Level& coarse, const Level& fine, const SweepSet<T>& set,
+                           const double* dx, const T* rhs, const T* x, T* b, const SetForm& form,
+                           hipStream_t s)
+{
+   T di[3], hi[3];
+   recip(dx, di);
+   recip2(dx, hi);
+   dim3 g(coarse.ncell_tiles, set.n);
+   const LevelArgs ca = level_args(coarse), fa = level_args(fine);
+   auto go = [&](auto nd, auto sp, auto wr) {
+      hipLaunchKernelGGL((k_set_resrestrict<T, decltype(nd)::value, decltype(sp)::value,
+                                            decltype(wr)::value>),
+                         g, tblock(), 0, s, ca, fa, set, di[0], di[1], di[2], hi[0], hi[1], hi[2],
+                         rhs, x, b);
+   };
+   bool_dispatch(form.split, [&](auto sp) {
+      bool_dispatch(form.wrap, [&](auto wr) {
+         if (fine.ndim == 3)
+            go(std::integral_constant<int, 3>(), sp, wr);
+         else
+            go(std::integral_constant<int, 2>(), sp, wr);
+      });
+   });
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
+// One block as a set of one slot (component 0 of the arrays passed).
+template <typename T>
+static SweepSet<T> ell_set(const EllOp<T>& op)
+{
+   SweepSet<T> set;
+   set.n = 1;
+   SweepSlot<T>& o = set.s[0];
+   o.D = op.D;
+   o.Dc = op.Dc;
+   o.C = op.C;
+   o.Cc = op.Cc;
+   o.M = op.M;
+   o.Mc = op.Mc;
+   return set;
+}
+template <typename T>
+static SweepSet<T> quat_set(const T* fc, const T* sm, double gamma, int ncomp)
+{
+   SweepSet<T> set;
+   set.n = 1;
+   SweepSlot<T>& o = set.s[0];
+   o.kind = 1;
+   o.ncomp = ncomp;
+   o.D = fc;
+   o.sm = sm;
+   o.gamma = (T)gamma;
+   return set;
 }
 
 template <typename T>
 int launch_rbgs(const Level& L, const EllOp<T>& op, const double* dx, const T* rhs, T* u,
                 int color, bool want_max, hipStream_t s)
 {
+   if (!want_max) return launch_set_sweep<T>(L, ell_set(op), dx, rhs, u, color, SetForm{}, s);
    OpArgs<T> oa{op.D, op.Dc, op.C, op.Cc, op.M, op.Mc};
-   double* part = want_max ? L.partial : nullptr;
-   LevelArgs la;
-   int grid;
-   shape(L, want_max, &la, &grid);
+   double* part = L.partial;
+   LevelArgs la = level_args(L);
+   dim3 g(L.ncell_tiles);
    T di[3];
    recip(dx, di);
-   if (!want_max) {
-      if (L.ndim == 3)
-         hipLaunchKernelGGL((k_rbgs_c<T, 3>), dim3(grid), cblock(), 0, s, la, oa, di[0], di[1],
-                            di[2], rhs, u, color);
-      else
-         hipLaunchKernelGGL((k_rbgs_c<T, 2>), dim3(grid), cblock(), 0, s, la, oa, di[0], di[1],
-                            di[2], rhs, u, color);
-   } else if (L.ndim == 3) {
-      hipLaunchKernelGGL((k_rbgs<T, 3>), dim3(grid), tblock(), 0, s, la, oa, di[0], di[1], di[2],
-                         rhs, u, color, part);
-   } else {
-      hipLaunchKernelGGL((k_rbgs<T, 2>), dim3(grid), tblock(), 0, s, la, oa, di[0], di[1], di[2],
-                         rhs, u, color, part);
-   }
+   if (L.ndim == 3)
+      hipLaunchKernelGGL((k_rbgs<T, 3>), g, tblock(), 0, s, la, oa, di[0], di[1], di[2], rhs, u,
+                         color, part);
+   else
+      hipLaunchKernelGGL((k_rbgs<T, 2>), g, tblock(), 0, s, la, oa, di[0], di[1], di[2], rhs, u,
+                         color, part);
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -1018,42 +1103,14 @@ template <typename T>
 int launch_ell_resrestrict(const Level& coarse, const Level& fine, const EllOp<T>& op,
                            const double* dx, const T* rhs, const T* u, T* b, hipStream_t s)
 {
-   OpArgs<T> oa{op.D, op.Dc, op.C, op.Cc, op.M, op.Mc};
-   T di[3];
-   recip(dx, di);
-   LevelArgs ca = level_args(coarse), fa = level_args(fine);
-   if (fine.ndim == 3)
-      hipLaunchKernelGGL((k_ell_resrestrict<T, 3>), dim3(coarse.ncell_tiles), tblock(), 0, s, ca,
-                         fa, oa, di[0], di[1], di[2], rhs, u, b);
-   else
-      hipLaunchKernelGGL((k_ell_resrestrict<T, 2>), dim3(coarse.ncell_tiles), tblock(), 0, s, ca,
-                         fa, oa, di[0], di[1], di[2], rhs, u, b);
-   AMPE_HIP_CHECK(hipGetLastError());
-   return 0;
+   return launch_set_resrestrict<T>(coarse, fine, ell_set(op), dx, rhs, u, b, SetForm{}, s);
 }
 
 template <typename T>
 int launch_quat_rbgs(const Level& L, const T* fc, const T* sm, double gamma, const double* dx,
-                     int ncomp, const T* rhs, T* z, int color, hipStream_t s, bool split)
+                     int ncomp, const T* rhs, T* z, int color, hipStream_t s)
 {
-   LevelArgs la;
-   int grid;
-   shape(L, false, &la, &grid);
-   T hi[3];
-   recip2(dx, hi);
-   KernelTimer::Span span(KernelTimer::QUAT_RBGS, s, quat_rbgs_bytes(L, ncomp, sizeof(T)));
-   auto go = [&](auto ndim, auto ql) {
-      constexpr int ND = decltype(ndim)::value, Q = decltype(ql)::value;
-      if (split)
-         hipLaunchKernelGGL((k_quat_rbgs_c<T, ND, Q, true>), dim3(grid), cblock(), 0, s, la, fc,
-                            sm, (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, color);
-      else
-         hipLaunchKernelGGL((k_quat_rbgs_c<T, ND, Q, false>), dim3(grid), cblock(), 0, s, la, fc,
-                            sm, (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, color);
-   };
-   quat_dispatch(L.ndim, ncomp, go);
-   AMPE_HIP_CHECK(hipGetLastError());
-   return 0;
+   return launch_set_sweep<T>(L, quat_set(fc, sm, gamma, ncomp), dx, rhs, z, color, SetForm{}, s);
 }
 
 template <typename T>
@@ -1097,22 +1154,20 @@ int launch_quat_residual(const Level& L, const T* fc, const T* sm, double gamma,
                          const double* dx, int ncomp, const T* rhs, const T* z, T* res,
                          double* part, hipStream_t s, bool split)
 {
-   LevelArgs la;
-   int grid;
-   shape(L, part != nullptr, &la, &grid);
+   if (!part)
+      return launch_set_residual<T>(L, quat_set(fc, sm, gamma, ncomp), dx, rhs, z, res, split, s);
+   LevelArgs la = level_args(L);
+   dim3 g(L.ncell_tiles);
    T hi[3];
    recip2(dx, hi);
    auto go = [&](auto ndim, auto ql) {
       constexpr int ND = decltype(ndim)::value, Q = decltype(ql)::value;
-      if (split && !part)
-         hipLaunchKernelGGL((k_quat_residual_p<T, ND, Q>), dim3(grid), cblock(), 0, s, la, fc,
-                            sm, (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res);
-      else if (split)
-         hipLaunchKernelGGL((k_quat_residual<T, ND, Q, true>), dim3(grid), tblock(), 0, s, la, fc,
-                            sm, (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res, part);
+      if (split)
+         hipLaunchKernelGGL((k_quat_residual<T, ND, Q, true>), g, tblock(), 0, s, la, fc, sm,
+                            (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res, part);
       else
-         hipLaunchKernelGGL((k_quat_residual<T, ND, Q, false>), dim3(grid), tblock(), 0, s, la,
-                            fc, sm, (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res, part);
+         hipLaunchKernelGGL((k_quat_residual<T, ND, Q, false>), g, tblock(), 0, s, la, fc, sm,
+                            (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res, part);
    };
    quat_dispatch(L.ndim, ncomp, go);
    AMPE_HIP_CHECK(hipGetLastError());
@@ -1122,45 +1177,27 @@ int launch_quat_residual(const Level& L, const T* fc, const T* sm, double gamma,
 template <typename T>
 int launch_quat_resrestrict(const Level& coarse, const Level& fine, const T* fc, const T* sm,
                             double gamma, const double* dx, int ncomp, const T* rhs, const T* z,
-                            T* b, hipStream_t s, bool split)
+                            T* b, hipStream_t s)
 {
-   if (ncomp != 1 && ncomp != 2 && ncomp != 4) {
-      set_error("launch_quat_resrestrict: one, two or four components");
-      return -1;
-   }
-   T hi[3];
-   recip2(dx, hi);
-   LevelArgs ca = level_args(coarse), fa = level_args(fine);
-   auto go = [&](auto ndim, auto ql) {
-      constexpr int ND = decltype(ndim)::value, Q = decltype(ql)::value;
-      if constexpr (Q > 0) {
-         if (split)
-            hipLaunchKernelGGL((k_quat_resrestrict<T, ND, Q, true>), dim3(coarse.ncell_tiles),
-                               tblock(), 0, s, ca, fa, fc, sm, (T)gamma, hi[0], hi[1], hi[2],
-                               rhs, z, b);
-         else
-            hipLaunchKernelGGL((k_quat_resrestrict<T, ND, Q, false>), dim3(coarse.ncell_tiles),
-                               tblock(), 0, s, ca, fa, fc, sm, (T)gamma, hi[0], hi[1], hi[2],
-                               rhs, z, b);
-      }
-   };
-   quat_dispatch(fine.ndim, ncomp, go);
-   AMPE_HIP_CHECK(hipGetLastError());
-   return 0;
+   return launch_set_resrestrict<T>(coarse, fine, quat_set(fc, sm, gamma, ncomp), dx, rhs, z, b,
+                                    SetForm{}, s);
 }
 
 #define AMPE_INST(T)                                                                     \
    template int sweep_add<T>(SweepSet<T>&, const SweepSlot<T>&, int, int);               \
    template int launch_set_sweep<T>(const Level&, const SweepSet<T>&, const double*,     \
-                                    const T*, T*, int, hipStream_t);                     \
+                                    const T*, T*, int, const SetForm&, hipStream_t);     \
    template int launch_set_residual<T>(const Level&, const SweepSet<T>&, const double*,  \
-                                       const T*, const T*, T*, hipStream_t);             \
+                                       const T*, const T*, T*, bool, hipStream_t);       \
+   template int launch_set_resrestrict<T>(const Level&, const Level&, const SweepSet<T>&, \
+                                          const double*, const T*, const T*, T*,         \
+                                          const SetForm&, hipStream_t);                  \
    template int launch_rbgs<T>(const Level&, const EllOp<T>&, const double*, const T*, T*, \
                                int, bool, hipStream_t);                                  \
    template int launch_residual<T>(const Level&, const EllOp<T>&, const double*, const T*, \
                                    const T*, T*, double*, hipStream_t);                  \
    template int launch_quat_rbgs<T>(const Level&, const T*, const T*, double, const double*, \
-                                    int, const T*, T*, int, hipStream_t, bool);          \
+                                    int, const T*, T*, int, hipStream_t);                \
    template int launch_quat_residual<T>(const Level&, const T*, const T*, double,         \
                                         const double*, int, const T*, const T*, T*,      \
                                         double*, hipStream_t, bool);                     \
@@ -1168,7 +1205,7 @@ int launch_quat_resrestrict(const Level& coarse, const Level& fine, const T* fc,
                                           const double*, const T*, const T*, T*, hipStream_t); \
    template int launch_quat_resrestrict<T>(const Level&, const Level&, const T*, const T*, \
                                            double, const double*, int, const T*,         \
-                                           const T*, T*, hipStream_t, bool);             \
+                                           const T*, T*, hipStream_t);                   \
    template int launch_quat_rbgs_fused<T>(const Level&, const T*, const T*, double,       \
                                           const double*, int, const T*, const T*, T*,    \
                                           hipStream_t);

@@ -89,11 +89,8 @@ __global__ void __launch_bounds__(256) k_gmres_finish(LevelArgs a, int nc, doubl
       double v = kry_dir(x, i) + (-gamma) * jvn;
       if (out) out[i] = v;
       if (pin.f) {
-         bool q = m >= pin.iq && m < pin.iq + pin.ql;
-         if (q)
-            pin.f[pin.split ? m * a.ncg + split_at(a, c, 0) : i] = (float)(v / pin.sm[c.c0]);
-         else
-            pin.f[i] = (float)v;
+         if (m >= pin.iq && m < pin.iq + pin.ql) v = v / pin.sm[c.c0];
+         pin.f[m >= pin.sp0 ? m * a.ncg + split_at(a, c, 0) : i] = (float)v;
       }
    }
 }
@@ -226,12 +223,8 @@ __global__ void __launch_bounds__(256) k_cgs_dots(LevelArgs a, int nc, int ntile
          double v;
          if (src.u) {
             // k_psolve_out's arithmetic, then the ewt scaling
-            if (m >= src.iq && m < src.iq + src.ql) {
-               v = (double)src.u[src.split ? m * a.ncg + split_at(a, c, 0) : i];
-               v = v * src.sm[c.c0];
-            } else {
-               v = (double)src.u[i];
-            }
+            v = (double)src.u[m >= src.sp0 ? m * a.ncg + split_at(a, c, 0) : i];
+            if (m >= src.iq && m < src.iq + src.ql) v = v * src.sm[c.c0];
             v = src.ewt[i] * v;
             out[i] = v;
          } else if (ewt) {

@@ -72,6 +72,7 @@ struct Level {
    long long* ghost_dst = nullptr;  // ghost gather (periodic / neighbours)
    long long* ghost_src = nullptr;
    long long nghost = 0;
+   long long nghost_face = 0;   // the first entries: ghosts next to an interior cell's face
    // the same gather in the row parity-split layout (built on request by
    // level_split_tables)
    long long* ghost_dst_s = nullptr;
@@ -109,6 +110,17 @@ int level_create_placed(int ndim, const ampe_box* boxes, int npatch, const Level
 int ghost_fill(const Level& L, double* f, int ncomp, hipStream_t s, bool split = false);
 int ghost_fill(const Level& L, float* f, int ncomp, hipStream_t s, bool split = false);
 int ghost_fill(const Level& L, int* f, int ncomp, hipStream_t s, bool split = false);
+// The ghosts next to an interior cell's face alone (all that a 7-point or
+// 5-point stencil reads).
+template <typename T>
+int ghost_fill_faces(const Level& L, T* f, int ncomp, hipStream_t s, bool split = false);
+// One red-black checkerboard over the whole level: periodic, covered by its
+// patches, even extents and even, non-negative patch corners, so that every
+// neighbour of a black cell, across patches and the boundary, is red.
+bool checker_ok(const Level& L);
+// A checker_ok level of one patch: a neighbour across the boundary is the
+// cell at the patch's other side.
+bool level_wrap_ok(const Level& L);
 // Builds the split-layout ghost gather of L (once; later calls return 0).
 int level_split_tables(Level& L, hipStream_t s);
 
@@ -138,12 +150,8 @@ struct KernelTimer {
    static int read(int id, double* ms, long long* launches, double* bytes);
 };
 
-// Algorithmic bytes of one colour of the orientation red-black sweep: all z
-// read, the colour's z written and rhs read, every face coefficient and the
-// cell sqrt(M) read once.
-double quat_rbgs_bytes(const Level& L, int ncomp, int elem);
-// The same for one fused sweep (both colours): z read and written, rhs, face
-// coefficients and sqrt(M) read once.
+// Algorithmic bytes of one fused orientation sweep (both colours): z read and
+// written, rhs, face coefficients and sqrt(M) read once.
 double quat_rbgs_fused_bytes(const Level& L, int ncomp, int elem);
 
 }  // namespace ampe

@@ -67,10 +67,37 @@ static void xcd_order(std::vector<Tile>& tiles)
 
 // Work lists, device copies of the patch table and the ghost gather, and
 // the reduction buffers of a level whose patch table L->hp is complete.
-static int level_upload(Level* L, const std::vector<long long>& gd,
-                        const std::vector<long long>& gs, Level** out)
+static int level_upload(Level* L, const std::vector<long long>& gd0,
+                        const std::vector<long long>& gs0, Level** out)
 {
    const int ndim = L->ndim, npatch = L->npatch;
+   // the ghost gather with the face ghosts first (an entry's patch: the last
+   // whose block starts at or before it; the tables list patch after patch)
+   std::vector<long long> gd, gs;
+   {
+      std::vector<long long> rd, rs;
+      int p = 0;
+      for (size_t e = 0; e < gd0.size(); e++) {
+         while (p + 1 < npatch && L->hp[p + 1].cell_off <= gd0[e]) p++;
+         const PatchDev& d = L->hp[p];
+         const long long loc = gd0[e] - d.cell_off;
+         const int x[3] = {(int)(loc % d.sy) - L->g, (int)((loc % d.sz) / d.sy) - L->g,
+                           (int)(loc / d.sz) - L->gz};
+         const int n[3] = {d.nx, d.ny, d.nz};
+         int out_by = 0, outs = 0;
+         for (int a = 0; a < ndim; a++) {
+            const int o = x[a] < 0 ? -x[a] : (x[a] >= n[a] ? x[a] - n[a] + 1 : 0);
+            out_by = std::max(out_by, o);
+            outs += o > 0;
+         }
+         const bool face = outs == 1 && out_by == 1;
+         (face ? gd : rd).push_back(gd0[e]);
+         (face ? gs : rs).push_back(gs0[e]);
+      }
+      L->nghost_face = (long long)gd.size();
+      gd.insert(gd.end(), rd.begin(), rd.end());
+      gs.insert(gs.end(), rs.begin(), rs.end());
+   }
    // work lists
    std::vector<Tile> ct, ft, zt, mt;
    for (int p = 0; p < npatch; p++) {
@@ -382,32 +409,66 @@ __global__ void __launch_bounds__(256) k_ghost_gather(T* __restrict__ f, long lo
 }
 
 template <typename T>
-static int ghost_fill_t(const Level& L, T* f, int ncomp, hipStream_t s, bool split)
+static int ghost_fill_t(const Level& L, T* f, int ncomp, hipStream_t s, bool split,
+                        long long n)
 {
-   if (L.nghost == 0 || ncomp <= 0) return 0;
+   if (n == 0 || ncomp <= 0) return 0;
    if (split && !L.ghost_dst_s) {
       set_error("ghost_fill: the level has no split-layout gather");
       return -1;
    }
-   dim3 grid((unsigned)((L.nghost + 255) / 256), (unsigned)ncomp);
+   dim3 grid((unsigned)((n + 255) / 256), (unsigned)ncomp);
    hipLaunchKernelGGL(k_ghost_gather<T>, grid, dim3(256), 0, s, f, L.ncg,
                       split ? L.ghost_dst_s : L.ghost_dst, split ? L.ghost_src_s : L.ghost_src,
-                      L.nghost);
+                      n);
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
 
+template <typename T>
+int ghost_fill_faces(const Level& L, T* f, int ncomp, hipStream_t s, bool split)
+{
+   return ghost_fill_t(L, f, ncomp, s, split, L.nghost_face);
+}
+template int ghost_fill_faces<double>(const Level&, double*, int, hipStream_t, bool);
+template int ghost_fill_faces<float>(const Level&, float*, int, hipStream_t, bool);
+
+bool checker_ok(const Level& L)
+{
+   if (!L.periodic) return false;
+   long long cells = 1;
+   for (int a = 0; a < L.ndim; a++) {
+      const int ext = L.pbox.hi[a] - L.pbox.lo[a] + 1;
+      if (L.pbox.lo[a] < 0 || (L.pbox.lo[a] & 1) || (ext & 1)) return false;
+      cells *= ext;
+   }
+   for (const PatchDev& d : L.hp)
+      for (int a = 0; a < L.ndim; a++)
+         if (d.lo[a] < 0 || (d.lo[a] & 1)) return false;
+   return cells == L.ncell;
+}
+
+bool level_wrap_ok(const Level& L)
+{
+   if (L.npatch != 1 || !checker_ok(L)) return false;
+   const PatchDev& d = L.hp[0];
+   const int n[3] = {d.nx, d.ny, d.nz};
+   for (int a = 0; a < L.ndim; a++)
+      if (d.lo[a] != L.pbox.lo[a] || n[a] != L.pbox.hi[a] - L.pbox.lo[a] + 1) return false;
+   return true;
+}
+
 int ghost_fill(const Level& L, double* f, int ncomp, hipStream_t s, bool split)
 {
-   return ghost_fill_t(L, f, ncomp, s, split);
+   return ghost_fill_t(L, f, ncomp, s, split, L.nghost);
 }
 int ghost_fill(const Level& L, float* f, int ncomp, hipStream_t s, bool split)
 {
-   return ghost_fill_t(L, f, ncomp, s, split);
+   return ghost_fill_t(L, f, ncomp, s, split, L.nghost);
 }
 int ghost_fill(const Level& L, int* f, int ncomp, hipStream_t s, bool split)
 {
-   return ghost_fill_t(L, f, ncomp, s, split);
+   return ghost_fill_t(L, f, ncomp, s, split, L.nghost);
 }
 
 __global__ void __launch_bounds__(256) k_split_map(const PatchDev* __restrict__ P, int np,
@@ -604,16 +665,6 @@ double quat_rbgs_fused_bytes(const Level& L, int ncomp, int elem)
 {
    double n = (double)L.ncell;
    return (double)elem * (3.0 * ncomp * n + (double)L.nside_tot + n);
-}
-
-double quat_rbgs_bytes(const Level& L, int ncomp, int elem)
-{
-   double n = (double)L.ncell;
-   return (double)elem * (ncomp * n            // z, all cells
-                          + ncomp * 0.5 * n    // rhs, this colour
-                          + ncomp * 0.5 * n    // z written, this colour
-                          + (double)L.nside_tot  // face coefficients
-                          + n);                // sqrt(M)
 }
 
 }  // namespace ampe

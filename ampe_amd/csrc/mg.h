@@ -29,26 +29,20 @@ struct MgLevel {
    T* sm = nullptr;     // orientation sqrt(M) (cell, ghosted), levels >= 1
    T* x = nullptr;      // correction, ncomp_max blocks, levels >= 1
    T* b = nullptr;      // right-hand side, ncomp_max blocks, levels >= 1
-   T* r = nullptr;      // residual, ncomp_max blocks, all levels
-   T* t = nullptr;      // second buffer of the fused orientation sweeps, all levels
+   T* r = nullptr;      // residual, ncomp_max blocks, levels without one checkerboard
 };
 
 template <typename T>
 struct Mg {
    std::vector<MgLevel<T>> lv;  // lv[0] is the fine level (not owned)
    int ncomp_max = 1;
-   bool qsplit = false;         // orientation vectors in the row parity-split layout
+   bool split = false;          // vectors in the row parity-split layout
    int nlev() const { return (int)lv.size(); }
 };
 
 struct MgCycle {
    int nu1 = 2, nu2 = 2;  // pre / post red-black sweeps
    int ncoarse = 16;      // sweeps on the coarsest level
-   // orientation block: one-pass sweeps (same values; measured slower on the
-   // 256^3 workload: 0.32 ms per sweep against 2 x 0.10 ms, averaged over the
-   // levels -- each workgroup walks its column of planes with two barriers per
-   // plane, which leaves too few loads in flight)
-   bool fused = false;
 };
 
 // Build the hierarchy below fine while every patch box and the periodic
@@ -68,24 +62,27 @@ int mg_setup_conc(Mg<T>& m, const T* D0, hipStream_t s);
 template <typename T>
 int mg_setup_quat(Mg<T>& m, const T* fc0, const T* sm0, hipStream_t s);
 
-// One V-cycle on A x = b from x = 0 (x0 zero on entry), fine arrays b0, x0.
-// Elliptic blocks: kind 0 = phase (C field, D constant, M constant or field), kind 1 =
-// composition (D field, C and M constants); op0 is the fine operator.
+// One V-cycle on A x = b from x = 0 for every slot of the set, fine arrays b0,
+// x0 (x0 need not be cleared): the slots' operators are the fine level's, a slot
+// with face coefficients D and no sm is the composition block, one without D the
+// phase block.  The slots number at most ncomp_max components.  split: b0 and x0
+// are in the row parity-split layout.
 template <typename T>
-int mg_vcycle_ell(Mg<T>& m, const EllOp<T>& op0, int kind, const MgCycle& cy, const T* b0,
-                  T* x0, hipStream_t s);
-// Orientation block, ncomp components sharing fc / sqrt(M).
-template <typename T>
-int mg_vcycle_quat(Mg<T>& m, const T* fc0, const T* sm0, double gamma, int ncomp,
-                   const MgCycle& cy, const T* b0, T* x0, hipStream_t s);
+int mg_vcycle(Mg<T>& m, const SweepSet<T>& set, const MgCycle& cy, const T* b0, T* x0, bool split,
+              hipStream_t s);
 
-// Store the orientation block's vectors (b, x, r of every level, and the
-// fine-level b0 / x0 the caller passes) in the row parity-split layout
-// (split_col): one colour of a sweep then reads and writes whole lines.
-// Builds the levels' split ghost gathers; the one-pass sweeps are natural
-// only.
+// Red-black sweeps of a set on one level (ncomp components); zero: x holds
+// nothing yet and stands for zero.
 template <typename T>
-int mg_enable_qsplit(Mg<T>& m, hipStream_t s);
+int set_smooth(const Level& L, const SweepSet<T>& set, const double* dx, int ncomp, const T* b,
+               T* x, int sweeps, bool zero, bool split, hipStream_t s);
+
+// Store the vectors (b, x, r of every level, and the fine-level b0 / x0 the
+// caller passes) in the row parity-split layout (split_col): one colour of a
+// sweep then reads and writes whole lines.  Builds the levels' split ghost
+// gathers.
+template <typename T>
+int mg_enable_split(Mg<T>& m, hipStream_t s);
 
 // Transfer operators (exposed for tests through the C ABI); split: f / c, xc
 // / xf in the row parity-split layout.
@@ -97,7 +94,7 @@ int mg_restrict_side(const Level& coarse, const Level& fine, const T* f, T* c, h
 // order 0: constant refinement, 1: tri/bilinear (coarse ghosts filled).
 template <typename T>
 int mg_prolong_add(const Level& fine, const Level& coarse, int ncomp, int order, const T* xc,
-                   T* xf, hipStream_t s, bool split = false);
+                   T* xf, hipStream_t s, bool split = false, bool wrap = false);
 // coarse holds the boxes of fine halved, patch by patch (even corners/extents)
 bool is_coarsening(const Level& coarse, const Level& fine);
 // After red-black sweeps ending with the black colour, the orientation

@@ -67,103 +67,89 @@ __global__ void __launch_bounds__(256) k_restrict_side(LevelArgs ca, LevelArgs f
 
 // Fine cell += coarse correction: ORDER 1 tri/bilinear interpolation (weights
 // 3/4 toward the parent, 1/4 toward the coarse neighbour on the cell's side in
-// each direction; the coarse field needs filled ghosts), ORDER 0 the parent
-// value (constant refinement).  SPLIT: xc and xf in the row parity-split
-// layout.
-template <typename T, int NDIM, int ORDER, bool SPLIT>
-__device__ __forceinline__ void prolong_cell(const LevelArgs& fa, const LevelArgs& ca,
-                                             const CellPos& p, int ncomp,
-                                             const T* __restrict__ xc, T* __restrict__ xf)
+// each direction; the coarse field needs filled ghosts unless WRAP, the one
+// patch of a periodic level, whose neighbours across the boundary are read at
+// its other side), ORDER 0 the parent value (constant refinement).  One
+// component per blockIdx.y.
+template <typename T, int NDIM, int ORDER>
+__device__ __forceinline__ T prolong_value(const T* __restrict__ x, long long c0, long long c1,
+                                           long long oj, long long ok)
 {
-   const PatchDev cp = ca.P[fa.T[tile_index(fa)].patch];
-   int K = NDIM == 3 ? (p.k >> 1) : 0;
-   const int ig = (p.i >> 1) + ca.g;
-   const long long row = cp.cell_off + (long long)((p.j >> 1) + ca.g) * cp.sy +
-                         (long long)(K + ca.gz) * cp.sz;
-   const int di = (p.i & 1) ? 1 : -1;
-   // the parent and its neighbour across the cell's side in the row
-   const long long c0 = SPLIT ? row + split_col(ig, cp.sy) : row + ig;
-   const long long c1 = SPLIT ? row + split_col(ig + di, cp.sy) : row + ig + di;
-   long long oj = (p.j & 1) ? cp.sy : -cp.sy;
-   long long ok = (NDIM == 3) ? ((p.k & 1) ? cp.sz : -cp.sz) : 0;
-   const long long fo = SPLIT ? split_at(fa, p, 0) : p.c0;
-   for (int m = 0; m < ncomp; m++) {
-      const T* x = xc + m * ca.ncg;
-      T v;
-      if (ORDER == 0) {
-         v = x[c0];
-      } else if (NDIM == 2) {
-         v = T(9.0 / 16.0) * x[c0] + T(3.0 / 16.0) * (x[c1] + x[c0 + oj]) +
+   if (ORDER == 0) return x[c0];
+   if (NDIM == 2)
+      return T(9.0 / 16.0) * x[c0] + T(3.0 / 16.0) * (x[c1] + x[c0 + oj]) +
              T(1.0 / 16.0) * x[c1 + oj];
-      } else {
-         v = T(27.0 / 64.0) * x[c0] +
-             T(9.0 / 64.0) * ((x[c1] + x[c0 + oj]) + x[c0 + ok]) +
-             T(3.0 / 64.0) * ((x[c1 + oj] + x[c1 + ok]) + x[c0 + oj + ok]) +
-             T(1.0 / 64.0) * x[c1 + oj + ok];
-      }
-      T* y = xf + m * fa.ncg;
-      y[fo] = y[fo] + v;
-   }
+   return T(27.0 / 64.0) * x[c0] + T(9.0 / 64.0) * ((x[c1] + x[c0 + oj]) + x[c0 + ok]) +
+          T(3.0 / 64.0) * ((x[c1 + oj] + x[c1 + ok]) + x[c0 + oj + ok]) +
+          T(1.0 / 64.0) * x[c1 + oj + ok];
 }
 
-template <typename T, int NDIM, int ORDER, bool SPLIT>
-__global__ void __launch_bounds__(256) k_prolong_add(LevelArgs fa, LevelArgs ca, int ncomp,
+// Offset from coarse position i of n along a stride st to its neighbour on the
+// low (hi = 0) or high side.
+template <bool WRAP>
+__device__ __forceinline__ long long nbr_off(int i, int n, long long st, int hi)
+{
+   if (hi) return (WRAP && i == n - 1) ? -(long long)(n - 1) * st : st;
+   return (WRAP && i == 0) ? (long long)(n - 1) * st : -st;
+}
+
+template <typename T, int NDIM, int ORDER, bool WRAP>
+__global__ void __launch_bounds__(256) k_prolong_add(LevelArgs fa, LevelArgs ca,
                                                      const T* __restrict__ xc,
                                                      T* __restrict__ xf)
 {
    CellPos p;
-   if (cell_pos(fa, 0, p)) prolong_cell<T, NDIM, ORDER, SPLIT>(fa, ca, p, ncomp, xc, xf);
+   if (!cell_pos(fa, 0, p)) return;
+   const PatchDev cp = ca.P[fa.T[tile_index(fa)].patch];
+   const int I = p.i >> 1, J = p.j >> 1, K = NDIM == 3 ? (p.k >> 1) : 0;
+   const long long c0 = cp.cell_off + (I + ca.g) + (long long)(J + ca.g) * cp.sy +
+                        (long long)(K + ca.gz) * cp.sz;
+   const long long c1 = c0 + nbr_off<WRAP>(I, cp.nx, 1, p.i & 1);
+   const long long oj = nbr_off<WRAP>(J, cp.ny, cp.sy, p.j & 1);
+   const long long ok = NDIM == 3 ? nbr_off<WRAP>(K, cp.nz, cp.sz, p.k & 1) : 0;
+   const T v = prolong_value<T, NDIM, ORDER>(xc + blockIdx.y * ca.ncg, c0, c1, oj, ok);
+   T* y = xf + blockIdx.y * fa.ncg;
+   y[p.c0] = y[p.c0] + v;
 }
 
 // The split-layout prolongation per coarse cell: a thread adds the
 // correction to the 2^NDIM children of its coarse cell (consecutive lanes:
 // consecutive coarse cells, so for each child offset the fine updates are
 // contiguous in the split layout), each child's value by the formula and
-// summation order of prolong_cell.
-template <typename T, int NDIM, int ORDER>
-__global__ void __launch_bounds__(256) k_prolong_add_cc(LevelArgs fa, LevelArgs ca, int ncomp,
+// summation order of the natural form.
+template <typename T, int NDIM, int ORDER, bool WRAP>
+__global__ void __launch_bounds__(256) k_prolong_add_cc(LevelArgs fa, LevelArgs ca,
                                                         const T* __restrict__ xc,
                                                         T* __restrict__ xf)
 {
    CellPos p;
    if (!cell_pos(ca, 0, p)) return;
    const PatchDev fp = fa.P[ca.T[tile_index(ca)].patch];
-   const int sy = p.pd.sy;
-   const long long row = p.c0 - (p.i + ca.g);
+   const int sy = p.pd.sy, nx = p.pd.nx;
    const int ig = p.i + ca.g;
+   const long long row = p.c0 - ig;
    const long long c0 = row + split_col(ig, sy);
-   const long long cm = row + split_col(ig - 1, sy), cp = row + split_col(ig + 1, sy);
-   for (int m = 0; m < ncomp; m++) {
-      const T* x = xc + m * ca.ncg;
-      T* y = xf + m * fa.ncg;
+   const long long cm = row + split_col(ig + (int)nbr_off<WRAP>(p.i, nx, 1, 0), sy);
+   const long long cp = row + split_col(ig + (int)nbr_off<WRAP>(p.i, nx, 1, 1), sy);
+   const T* x = xc + blockIdx.y * ca.ncg;
+   T* y = xf + blockIdx.y * fa.ncg;
+   // every child's old value before the first update: the compiler cannot see
+   // that the children differ, and would wait for each store
+   long long fo[8];
+   T old[8];
 #pragma unroll
-      for (int dz = 0; dz < (NDIM == 3 ? 2 : 1); dz++)
+   for (int e = 0; e < (NDIM == 3 ? 8 : 4); e++) {
+      const int fi = 2 * p.i + (e & 1), fj = 2 * p.j + ((e >> 1) & 1);
+      const int fk = NDIM == 3 ? 2 * p.k + (e >> 2) : 0;
+      fo[e] = fp.cell_off + split_col(fi + fa.g, fp.sy) + (long long)(fj + fa.g) * fp.sy +
+              (long long)(fk + fa.gz) * fp.sz;
+      old[e] = y[fo[e]];
+   }
 #pragma unroll
-         for (int dy = 0; dy < 2; dy++)
-#pragma unroll
-            for (int dx = 0; dx < 2; dx++) {
-               const long long c1 = dx ? cp : cm;
-               const long long oj = dy ? sy : -(long long)sy;
-               const long long ok = NDIM == 3 ? (dz ? p.pd.sz : -p.pd.sz) : 0;
-               T v;
-               if (ORDER == 0) {
-                  v = x[c0];
-               } else if (NDIM == 2) {
-                  v = T(9.0 / 16.0) * x[c0] + T(3.0 / 16.0) * (x[c1] + x[c0 + oj]) +
-                      T(1.0 / 16.0) * x[c1 + oj];
-               } else {
-                  v = T(27.0 / 64.0) * x[c0] +
-                      T(9.0 / 64.0) * ((x[c1] + x[c0 + oj]) + x[c0 + ok]) +
-                      T(3.0 / 64.0) * ((x[c1 + oj] + x[c1 + ok]) + x[c0 + oj + ok]) +
-                      T(1.0 / 64.0) * x[c1 + oj + ok];
-               }
-               const int fi = 2 * p.i + dx, fj = 2 * p.j + dy;
-               const int fk = NDIM == 3 ? 2 * p.k + dz : 0;
-               const long long fo = fp.cell_off + split_col(fi + fa.g, fp.sy) +
-                                    (long long)(fj + fa.g) * fp.sy +
-                                    (long long)(fk + fa.gz) * fp.sz;
-               y[fo] = y[fo] + v;
-            }
+   for (int e = 0; e < (NDIM == 3 ? 8 : 4); e++) {
+      const long long oj = nbr_off<WRAP>(p.j, p.pd.ny, sy, (e >> 1) & 1);
+      const long long ok = NDIM == 3 ? nbr_off<WRAP>(p.k, p.pd.nz, p.pd.sz, e >> 2) : 0;
+      y[fo[e]] = old[e] + prolong_value<T, NDIM, ORDER>(x, c0, (e & 1) ? cp : cm, oj, ok);
    }
 }
 
@@ -204,31 +190,31 @@ int mg_restrict_side(const Level& coarse, const Level& fine, const T* f, T* c, h
 
 template <typename T>
 int mg_prolong_add(const Level& fine, const Level& coarse, int ncomp, int order, const T* xc,
-                   T* xf, hipStream_t s, bool split)
+                   T* xf, hipStream_t s, bool split, bool wrap)
 {
-   dim3 g(fine.ncell_tiles), b(TX, TY);
+   if (ncomp <= 0) return 0;
+   dim3 gf(fine.ncell_tiles, ncomp), gc(coarse.ncell_tiles, ncomp), b(TX, TY);
    LevelArgs fa = level_args(fine), ca = level_args(coarse);
-   auto go = [&](auto nd, auto sp) {
-      constexpr int ND = decltype(nd)::value;
-      constexpr bool SP = decltype(sp)::value;
-      dim3 gc(coarse.ncell_tiles);
-      if (SP && order == 0)
-         hipLaunchKernelGGL((k_prolong_add_cc<T, ND, 0>), gc, b, 0, s, fa, ca, ncomp, xc, xf);
-      else if (SP)
-         hipLaunchKernelGGL((k_prolong_add_cc<T, ND, 1>), gc, b, 0, s, fa, ca, ncomp, xc, xf);
-      else if (order == 0)
-         hipLaunchKernelGGL((k_prolong_add<T, ND, 0, false>), g, b, 0, s, fa, ca, ncomp, xc, xf);
+   auto go = [&](auto nd, auto od, auto wr) {
+      constexpr int ND = decltype(nd)::value, OD = decltype(od)::value;
+      constexpr bool WR = decltype(wr)::value;
+      if (split)
+         hipLaunchKernelGGL((k_prolong_add_cc<T, ND, OD, WR>), gc, b, 0, s, fa, ca, xc, xf);
       else
-         hipLaunchKernelGGL((k_prolong_add<T, ND, 1, false>), g, b, 0, s, fa, ca, ncomp, xc, xf);
+         hipLaunchKernelGGL((k_prolong_add<T, ND, OD, WR>), gf, b, 0, s, fa, ca, xc, xf);
    };
-   using I2 = std::integral_constant<int, 2>;
-   using I3 = std::integral_constant<int, 3>;
-   using ST = std::true_type;
-   using SF = std::false_type;
+   auto by = [&](auto nd) {
+      if (order == 0)
+         go(nd, std::integral_constant<int, 0>(), std::false_type());
+      else if (wrap)
+         go(nd, std::integral_constant<int, 1>(), std::true_type());
+      else
+         go(nd, std::integral_constant<int, 1>(), std::false_type());
+   };
    if (fine.ndim == 3)
-      split ? go(I3(), ST()) : go(I3(), SF());
+      by(std::integral_constant<int, 3>());
    else
-      split ? go(I2(), ST()) : go(I2(), SF());
+      by(std::integral_constant<int, 2>());
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -281,11 +267,7 @@ int mg_create(const Level& fine, const double* dx, int ncomp_max, int max_levels
    MgLevel<T> l0;
    l0.L = const_cast<Level*>(&fine);
    for (int a = 0; a < 3; a++) l0.dx[a] = dx[a];
-   int rc = talloc(&l0.r, (size_t)ncomp_max * fine.ncg);
-   rc |= talloc(&l0.t, (size_t)ncomp_max * fine.ncg);
-   // ghost cells without a gather source are never written: keep them zero,
-   // as in the arrays the sweeps alternate with
-   if (!rc && hipMemset(l0.t, 0, sizeof(T) * (size_t)ncomp_max * fine.ncg) != hipSuccess) rc = -1;
+   int rc = talloc(&l0.r, checker_ok(fine) ? 1 : (size_t)ncomp_max * fine.ncg);
    m->lv.push_back(l0);
    if (max_levels < 1) max_levels = 1;
    while (!rc && (int)m->lv.size() < max_levels && halvable(*m->lv.back().L, min_cells)) {
@@ -318,9 +300,7 @@ int mg_create(const Level& fine, const double* dx, int ncomp_max, int max_levels
       rc |= talloc(&c.sm, ncg);
       rc |= talloc(&c.x, (size_t)ncomp_max * ncg);
       rc |= talloc(&c.b, (size_t)ncomp_max * ncg);
-      rc |= talloc(&c.r, (size_t)ncomp_max * ncg);
-      rc |= talloc(&c.t, (size_t)ncomp_max * ncg);
-      if (!rc && hipMemset(c.t, 0, sizeof(T) * (size_t)ncomp_max * ncg) != hipSuccess) rc = -1;
+      rc |= talloc(&c.r, checker_ok(*c.L) ? 1 : (size_t)ncomp_max * ncg);
       m->lv.push_back(c);
    }
    if (rc) {
@@ -339,7 +319,6 @@ void mg_destroy(Mg<T>* m)
    for (size_t l = 0; l < m->lv.size(); l++) {
       MgLevel<T>& c = m->lv[l];
       (void)hipFree(c.r);
-      (void)hipFree(c.t);
       if (l == 0) continue;
       (void)hipFree(c.C);
       (void)hipFree(c.M);
@@ -393,105 +372,6 @@ int mg_setup_quat(Mg<T>& m, const T* fc0, const T* sm0, hipStream_t s)
 }
 
 // ------------------------------------------------------------ cycles
-template <typename T>
-static int smooth_ell(const Level& L, const EllOp<T>& op, const double* dx, const T* b, T* x,
-                      int sweeps, hipStream_t s)
-{
-   for (int sw = 0; sw < sweeps; sw++) {
-      if (ghost_fill(L, x, 1, s)) return -1;
-      if (launch_rbgs<T>(L, op, dx, b, x, 0, false, s)) return -1;
-      if (ghost_fill(L, x, 1, s)) return -1;
-      if (launch_rbgs<T>(L, op, dx, b, x, 1, false, s)) return -1;
-   }
-   return 0;
-}
-
-template <typename T>
-static int smooth_quat(const Level& L, const T* fc, const T* sm, double gamma, const double* dx,
-                       int ncomp, const T* b, T* x, int sweeps, hipStream_t s, bool split)
-{
-   for (int sw = 0; sw < sweeps; sw++) {
-      if (ghost_fill(L, x, ncomp, s, split)) return -1;
-      if (launch_quat_rbgs<T>(L, fc, sm, gamma, dx, ncomp, b, x, 0, s, split)) return -1;
-      if (ghost_fill(L, x, ncomp, s, split)) return -1;
-      if (launch_quat_rbgs<T>(L, fc, sm, gamma, dx, ncomp, b, x, 1, s, split)) return -1;
-   }
-   return 0;
-}
-
-// nsweeps fused sweeps alternating between *cur and *oth; on return *cur
-// holds the result.
-template <typename T>
-static int smooth_quat_pp(const Level& L, const T* fc, const T* sm, double gamma, const double* dx,
-                          int ncomp, const T* b, T** cur, T** oth, int sweeps, hipStream_t s)
-{
-   for (int sw = 0; sw < sweeps; sw++) {
-      if (ghost_fill(L, *cur, ncomp, s)) return -1;
-      if (launch_quat_rbgs_fused<T>(L, fc, sm, gamma, dx, ncomp, b, *cur, *oth, s)) return -1;
-      std::swap(*cur, *oth);
-   }
-   return 0;
-}
-
-template <typename T>
-static EllOp<T> level_op(const Mg<T>& m, const EllOp<T>& op0, int kind, int l)
-{
-   EllOp<T> op = op0;
-   if (l > 0) {
-      if (kind == 0) {
-         op.C = m.lv[l].C;
-         if (op0.M) op.M = m.lv[l].M;
-      } else {
-         op.D = m.lv[l].D;
-      }
-   }
-   return op;
-}
-
-template <typename T>
-int mg_vcycle_ell(Mg<T>& m, const EllOp<T>& op0, int kind, const MgCycle& cy, const T* b0,
-                  T* x0, hipStream_t s)
-{
-   if (op0.M && kind != 0) {
-      set_error("mg_vcycle_ell: a mobility field is supported for the phase block only");
-      return -1;
-   }
-   int nl = m.nlev();
-   // descend
-   for (int l = 0; l < nl; l++) {
-      MgLevel<T>& c = m.lv[l];
-      const T* b = l == 0 ? b0 : c.b;
-      T* x = l == 0 ? x0 : c.x;
-      EllOp<T> op = level_op(m, op0, kind, l);
-      if (l == nl - 1) {
-         if (smooth_ell<T>(*c.L, op, c.dx, b, x, cy.ncoarse, s)) return -1;
-         break;
-      }
-      if (smooth_ell<T>(*c.L, op, c.dx, b, x, cy.nu1, s)) return -1;
-      if (ghost_fill(*c.L, x, 1, s)) return -1;
-      MgLevel<T>& n = m.lv[l + 1];
-      if (cy.nu1 >= 1 && red_residual_ok(*c.L, 1)) {
-         // the sweeps end with the black colour: restrict the red residuals
-         if (launch_ell_resrestrict<T>(*n.L, *c.L, op, c.dx, b, x, n.b, s)) return -1;
-      } else {
-         if (launch_residual<T>(*c.L, op, c.dx, b, x, c.r, nullptr, s)) return -1;
-         if (mg_restrict_cell<T>(*n.L, *c.L, 1, c.r, n.b, s)) return -1;
-      }
-      if (fill_zero<T>(n.x, n.L->ncg, s)) return -1;
-   }
-   // ascend
-   for (int l = nl - 2; l >= 0; l--) {
-      MgLevel<T>& c = m.lv[l];
-      MgLevel<T>& n = m.lv[l + 1];
-      const T* b = l == 0 ? b0 : c.b;
-      T* x = l == 0 ? x0 : c.x;
-      if (ghost_fill(*n.L, n.x, 1, s)) return -1;
-      if (mg_prolong_add<T>(*c.L, *n.L, 1, 1, n.x, x, s)) return -1;
-      if (smooth_ell<T>(*c.L, level_op(m, op0, kind, l), c.dx, b, x, cy.nu2, s)) return -1;
-   }
-   return 0;
-}
-
 // The residual after red-black sweeps ending with the black colour vanishes
 // on black cells when every black cell's neighbours are red: one checkerboard
 // over the patches (non-negative, even patch corners: the colour rule of the
@@ -510,106 +390,110 @@ bool red_residual_ok(const Level& L, int ncomp)
    return true;
 }
 
+// The set's operators on level l.
 template <typename T>
-int mg_vcycle_quat(Mg<T>& m, const T* fc0, const T* sm0, double gamma, int ncomp,
-                   const MgCycle& cy, const T* b0, T* x0, hipStream_t s)
+static SweepSet<T> level_set(const Mg<T>& m, const SweepSet<T>& set, int l)
 {
-   if (ncomp > m.ncomp_max) {
-      set_error("mg_vcycle_quat: more components than the hierarchy holds");
+   SweepSet<T> r = set;
+   if (l == 0) return r;
+   const MgLevel<T>& c = m.lv[l];
+   for (int i = 0; i < r.n; i++) {
+      SweepSlot<T>& o = r.s[i];
+      o.b = nullptr;
+      if (o.kind == 1) {
+         o.D = c.fc;
+         o.sm = c.sm;
+      } else if (o.D) {
+         o.D = c.D;
+      } else {
+         o.C = c.C;
+         if (o.M) o.M = c.M;
+      }
+   }
+   return r;
+}
+
+// Red-black sweeps of a set on a level.  zero: x holds nothing yet and stands for
+// zero.  On one checkerboard the first two colours then start from what they
+// know (SetForm::from) and nothing is cleared; elsewhere a colour may read its
+// own colour across the boundary, and x is cleared.  A level that wraps fills
+// no ghosts.  nv: length of x.
+template <typename T>
+int set_smooth(const Level& L, const SweepSet<T>& set, const double* dx, int ncomp, const T* b,
+               T* x, int sweeps, bool zero, bool split, hipStream_t s)
+{
+   const bool wrap = level_wrap_ok(L), ck = checker_ok(L);
+   if (zero && (!ck || sweeps == 0) && fill_zero<T>(x, L.ncg * ncomp, s)) return -1;
+   SetForm form;
+   form.split = split;
+   form.wrap = wrap;
+   for (int c = 0; c < 2 * sweeps; c++) {
+      form.from = zero && ck && c < 2 ? 1 + c : 0;
+      if (!wrap && !(zero && c == 0) && ghost_fill_faces(L, x, ncomp, s, split)) return -1;
+      if (launch_set_sweep<T>(L, set, dx, b, x, c & 1, form, s)) return -1;
+   }
+   return 0;
+}
+template int set_smooth<float>(const Level&, const SweepSet<float>&, const double*, int,
+                               const float*, float*, int, bool, bool, hipStream_t);
+template int set_smooth<double>(const Level&, const SweepSet<double>&, const double*, int,
+                                const double*, double*, int, bool, bool, hipStream_t);
+
+template <typename T>
+int mg_vcycle(Mg<T>& m, const SweepSet<T>& set, const MgCycle& cy, const T* b0, T* x0, bool split,
+              hipStream_t s)
+{
+   int nc = 0;
+   for (int i = 0; i < set.n; i++) nc += set.s[i].ncomp;
+   if (nc > m.ncomp_max || (split && !m.split)) {
+      set_error("mg_vcycle: more components than the hierarchy holds, or no split tables");
       return -1;
    }
-   int nl = m.nlev();
-   if (cy.fused && m.qsplit) {
-      set_error("mg_vcycle_quat: the one-pass sweeps use the natural layout");
-      return -1;
-   }
-   if (cy.fused) {
-      // one-pass sweeps alternate between x and t on every level; cur[l] is
-      // the level's current iterate
-      std::vector<T*> cur(nl), oth(nl);
-      for (int l = 0; l < nl; l++) {
-         cur[l] = l == 0 ? x0 : m.lv[l].x;
-         oth[l] = m.lv[l].t;
-      }
-      for (int l = 0; l < nl; l++) {
-         MgLevel<T>& c = m.lv[l];
-         const T* b = l == 0 ? b0 : c.b;
-         const T* fc = l == 0 ? fc0 : c.fc;
-         const T* sm = l == 0 ? sm0 : c.sm;
-         int nsw = (l == nl - 1) ? cy.ncoarse : cy.nu1;
-         if (smooth_quat_pp<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, &cur[l], &oth[l], nsw, s))
-            return -1;
-         if (l == nl - 1) break;
-         if (ghost_fill(*c.L, cur[l], ncomp, s)) return -1;
-         if (launch_quat_residual<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, cur[l], c.r, nullptr,
-                                     s))
-            return -1;
-         MgLevel<T>& n = m.lv[l + 1];
-         if (mg_restrict_cell<T>(*n.L, *c.L, ncomp, c.r, n.b, s)) return -1;
-         if (fill_zero<T>(cur[l + 1], n.L->ncg * ncomp, s)) return -1;
-      }
-      for (int l = nl - 2; l >= 0; l--) {
-         MgLevel<T>& c = m.lv[l];
-         MgLevel<T>& n = m.lv[l + 1];
-         const T* b = l == 0 ? b0 : c.b;
-         const T* fc = l == 0 ? fc0 : c.fc;
-         const T* sm = l == 0 ? sm0 : c.sm;
-         if (ghost_fill(*n.L, cur[l + 1], ncomp, s)) return -1;
-         if (mg_prolong_add<T>(*c.L, *n.L, ncomp, 1, cur[l + 1], cur[l], s)) return -1;
-         if (smooth_quat_pp<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, &cur[l], &oth[l], cy.nu2, s))
-            return -1;
-      }
-      if (cur[0] != x0)
-         AMPE_HIP_CHECK(hipMemcpyAsync(x0, cur[0], sizeof(T) * m.lv[0].L->ncg * ncomp,
-                                       hipMemcpyDeviceToDevice, s));
-      return 0;
-   }
-   const bool sp = m.qsplit;
+   const int nl = m.nlev();
+   SetForm form;
+   form.split = split;
    for (int l = 0; l < nl; l++) {
       MgLevel<T>& c = m.lv[l];
       const T* b = l == 0 ? b0 : c.b;
       T* x = l == 0 ? x0 : c.x;
-      const T* fc = l == 0 ? fc0 : c.fc;
-      const T* sm = l == 0 ? sm0 : c.sm;
-      if (l == nl - 1) {
-         if (smooth_quat<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, x, cy.ncoarse, s, sp)) return -1;
-         break;
-      }
-      if (smooth_quat<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, x, cy.nu1, s, sp)) return -1;
-      if (ghost_fill(*c.L, x, ncomp, s, sp)) return -1;
+      const SweepSet<T> ls = level_set(m, set, l);
+      const int nu = l == nl - 1 ? cy.ncoarse : cy.nu1;
+      if (set_smooth<T>(*c.L, ls, c.dx, nc, b, x, nu, true, split, s)) return -1;
+      if (l == nl - 1) break;
       MgLevel<T>& n = m.lv[l + 1];
-      if (cy.nu1 >= 1 && red_residual_ok(*c.L, ncomp)) {
+      form.wrap = level_wrap_ok(*c.L);
+      if (!form.wrap && ghost_fill_faces(*c.L, x, nc, s, split)) return -1;
+      if (nu >= 1 && checker_ok(*c.L)) {
          // the sweeps end with the black colour: restrict the red residuals
-         if (launch_quat_resrestrict<T>(*n.L, *c.L, fc, sm, gamma, c.dx, ncomp, b, x, n.b, s, sp))
-            return -1;
+         if (launch_set_resrestrict<T>(*n.L, *c.L, ls, c.dx, b, x, n.b, form, s)) return -1;
       } else {
-         if (launch_quat_residual<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, x, c.r, nullptr, s,
-                                     sp))
-            return -1;
-         if (mg_restrict_cell<T>(*n.L, *c.L, ncomp, c.r, n.b, s, sp)) return -1;
+         // (a checkerboard level without sweeps: x is zero, the residual is b)
+         const T* r = checker_ok(*c.L) ? b : c.r;
+         if (r != b && launch_set_residual<T>(*c.L, ls, c.dx, b, x, c.r, split, s)) return -1;
+         if (mg_restrict_cell<T>(*n.L, *c.L, nc, r, n.b, s, split)) return -1;
       }
-      if (fill_zero<T>(n.x, n.L->ncg * ncomp, s)) return -1;
    }
    for (int l = nl - 2; l >= 0; l--) {
       MgLevel<T>& c = m.lv[l];
       MgLevel<T>& n = m.lv[l + 1];
       const T* b = l == 0 ? b0 : c.b;
       T* x = l == 0 ? x0 : c.x;
-      const T* fc = l == 0 ? fc0 : c.fc;
-      const T* sm = l == 0 ? sm0 : c.sm;
-      if (ghost_fill(*n.L, n.x, ncomp, s, sp)) return -1;
-      if (mg_prolong_add<T>(*c.L, *n.L, ncomp, 1, n.x, x, s, sp)) return -1;
-      if (smooth_quat<T>(*c.L, fc, sm, gamma, c.dx, ncomp, b, x, cy.nu2, s, sp)) return -1;
+      // the interpolation reads edge and corner ghosts too
+      const bool wrap = level_wrap_ok(*n.L);
+      if (!wrap && ghost_fill(*n.L, n.x, nc, s, split)) return -1;
+      if (mg_prolong_add<T>(*c.L, *n.L, nc, 1, n.x, x, s, split, wrap)) return -1;
+      if (set_smooth<T>(*c.L, level_set(m, set, l), c.dx, nc, b, x, cy.nu2, false, split, s))
+         return -1;
    }
    return 0;
 }
 
 template <typename T>
-int mg_enable_qsplit(Mg<T>& m, hipStream_t s)
+int mg_enable_split(Mg<T>& m, hipStream_t s)
 {
    for (auto& c : m.lv)
       if (level_split_tables(*c.L, s)) return -1;
-   m.qsplit = true;
+   m.split = true;
    return 0;
 }
 
@@ -619,16 +503,14 @@ int mg_enable_qsplit(Mg<T>& m, hipStream_t s)
    template int mg_setup_phase<T>(Mg<T>&, const T*, const T*, hipStream_t);                  \
    template int mg_setup_conc<T>(Mg<T>&, const T*, hipStream_t);                             \
    template int mg_setup_quat<T>(Mg<T>&, const T*, const T*, hipStream_t);                   \
-   template int mg_vcycle_ell<T>(Mg<T>&, const EllOp<T>&, int, const MgCycle&, const T*, T*, \
-                                 hipStream_t);                                               \
-   template int mg_vcycle_quat<T>(Mg<T>&, const T*, const T*, double, int, const MgCycle&,   \
-                                  const T*, T*, hipStream_t);                                \
+   template int mg_vcycle<T>(Mg<T>&, const SweepSet<T>&, const MgCycle&, const T*, T*, bool,  \
+                             hipStream_t);                                                   \
    template int mg_restrict_cell<T>(const Level&, const Level&, int, const T*, T*,           \
                                     hipStream_t, bool);                                      \
-   template int mg_enable_qsplit<T>(Mg<T>&, hipStream_t);                                    \
+   template int mg_enable_split<T>(Mg<T>&, hipStream_t);                                     \
    template int mg_restrict_side<T>(const Level&, const Level&, const T*, T*, hipStream_t);  \
    template int mg_prolong_add<T>(const Level&, const Level&, int, int, const T*, T*,        \
-                                  hipStream_t, bool);
+                                  hipStream_t, bool, bool);
 AMPE_MG_INST(float)
 AMPE_MG_INST(double)
 

@@ -190,13 +190,13 @@ static int sim_finish(Sim* S, Sim** out)
    if (!rc && s.precond == AMPE_PRECOND_MG) {
       int maxlev = s.mg_max_levels > 0 ? s.mg_max_levels : 32;
       if (s.precision == AMPE_FAC_FP32) {
-         rc = mg_create<float>(L, p.dx, ql, maxlev, 2, &S->mgf);
+         rc = mg_create<float>(L, p.dx, S->nc, maxlev, 2, &S->mgf);
          if (!rc && p.evolve_quat && !s.mg_quat_natural) {
-            rc = mg_enable_qsplit<float>(*S->mgf, nullptr);
+            rc = mg_enable_split<float>(*S->mgf, nullptr);
             if (!rc && hipDeviceSynchronize() != hipSuccess) rc = -1;
          }
       } else
-         rc = mg_create<double>(L, p.dx, ql, maxlev, 2, &S->mgd);
+         rc = mg_create<double>(L, p.dx, S->nc, maxlev, 2, &S->mgd);
    } else if (s.precond != AMPE_PRECOND_REDBLACK) {
       set_error("sim_create: unknown preconditioner");
       rc = -1;
@@ -681,7 +681,7 @@ static int hier_psolve(Sim* S, const double* r, double* z, double delta, bool st
       if (S->s.precision == AMPE_FAC_FP32) {
          if (psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, S->f_u, st) ||
              hier_psolve_set<float>(S, S->f_f, S->f_u, S->f_r) ||
-             psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, nullptr, z, st))
+             psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st))
             return -1;
          return 0;
       }
@@ -734,7 +734,7 @@ static int hier_psolve(Sim* S, const double* r, double* z, double delta, bool st
          if (r2 < 0) return -1;
          ret |= r2;
       }
-      if (psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, nullptr, z, st)) return -1;
+      if (psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st)) return -1;
       return ret;
    }
    // z = 0, fac_u = orientation blocks of r / sqrt(M)
@@ -930,47 +930,94 @@ Mg<double>* mg_of<double>(Sim* S)
    return S->mgd;
 }
 
+// Whether every preconditioner solve runs one cycle per block with no test of a
+// norm or residual: all blocks then share their launches (solve_set), and an
+// FP32 multigrid keeps every component in the split layout.
+static bool set_mode(const Sim* S)
+{
+   return S->s.fac_max_cycles <= 1 && S->s.quat_max_cycles <= 1 &&
+          (S->mgf || S->mgd || S->s.fac_tol < 0.0);
+}
+
+// One cycle of the blocks of a set from x = 0 (x need not be cleared): a
+// multigrid V-cycle, or the red-black sweeps.
+template <typename T>
+static int cycle_set(Sim* S, const SweepSet<T>& set, int ncomp, int sweeps, const T* b, T* x,
+                     bool split)
+{
+   if (Mg<T>* mg = mg_of<T>(S)) {
+      MgCycle cy;
+      cy.nu1 = cy.nu2 = sweeps;
+      cy.ncoarse = S->s.mg_coarse_sweeps;
+      return mg_vcycle<T>(*mg, set, cy, b, x, split, S->stream);
+   }
+   return set_smooth<T>(*S->L, set, S->p.dx, ncomp, b, x, sweeps, true, false, S->stream);
+}
+
+// x = P^-1 b, one cycle of every block: in the same launches when their sweep
+// counts agree, else the orientation block after the elliptic ones.  rown: the
+// phase and composition right-hand sides when b holds the orientation's only.
+template <typename T>
+static int solve_set(Sim* S, const T* b, T* x, const T* rown = nullptr)
+{
+   const bool q = S->iq >= 0, one = q && S->s.quat_sweeps == S->s.fac_sweeps;
+   const bool split = mg_of<T>(S) && mg_of<T>(S)->split;
+   const int nell = S->nord + S->ncs, ql = q ? S->p.qlen : 0;
+   SweepSet<T> set;
+   if (add_elliptic<T>(S, set)) return -1;
+   if (rown)
+      for (int i = 0; i < set.n; i++) set.s[i].b = rown + (long long)set.s[i].comp * S->ng;
+   const long long off = q ? (long long)S->iq * S->ng : 0;
+   const T* bq = rown ? b : b + off;
+   if (one) {
+      if (add_orientation<T>(S, set, S->iq)) return -1;
+      set.s[set.n - 1].b = rown ? bq : nullptr;
+   }
+   if (cycle_set<T>(S, set, nell + (one ? ql : 0), S->s.fac_sweeps, b, x, split)) return -1;
+   if (!q || one) return 0;
+   SweepSet<T> qs;
+   if (add_orientation<T>(S, qs, 0)) return -1;
+   return cycle_set<T>(S, qs, ql, S->s.quat_sweeps, bq, x + off, split);
+}
+
+// One cycle of one block from x = 0 (several cycles per block).
 template <typename T>
 static int block_smooth(Sim* S, PBlock<T>& B, const T* rhs, T* x)
 {
    const Level& L = *S->L;
    hipStream_t st = S->stream;
    const double* dx = S->p.dx;
-   Mg<T>* mg = mg_of<T>(S);
-   if (mg) {
-      // one multigrid V-cycle from x = 0 (x is zero on entry)
-      MgCycle cy;
-      cy.nu1 = cy.nu2 = B.kind == 0 ? S->s.fac_sweeps : S->s.quat_sweeps;
-      cy.ncoarse = S->s.mg_coarse_sweeps;
-      if (B.kind == 0) return mg_vcycle_ell<T>(*mg, B.op, B.comp == 0 ? 0 : 1, cy, rhs, x, st);
-      return mg_vcycle_quat<T>(*mg, B.fc, B.sm, S->gamma_setup, B.ncomp, cy, rhs, x, st);
-   }
-   if (B.kind == 0) {
-      bool want = S->s.fac_tol >= 0.0;
-      if (ghost_fill(L, x, 1, st)) return -1;
+   if (!mg_of<T>(S) && B.kind == 0 && S->s.fac_tol >= 0.0) {
+      if (fill_zero<T>(x, S->ng, st)) return -1;
       for (int sw = 0; sw < S->s.fac_sweeps; sw++) {
          double mr = 0.0, mb = 0.0;
          if (ghost_fill(L, x, 1, st)) return -1;
-         if (launch_rbgs<T>(L, B.op, dx, rhs, x, 0, want, st)) return -1;
-         if (want && reduce_partials(L, L.ncell_tiles, 1, 1, &mr, st)) return -1;
+         if (launch_rbgs<T>(L, B.op, dx, rhs, x, 0, true, st)) return -1;
+         if (reduce_partials(L, L.ncell_tiles, 1, 1, &mr, st)) return -1;
          if (ghost_fill(L, x, 1, st)) return -1;
-         if (launch_rbgs<T>(L, B.op, dx, rhs, x, 1, want, st)) return -1;
-         if (want && reduce_partials(L, L.ncell_tiles, 1, 1, &mb, st)) return -1;
-         if (ghost_fill(L, x, 1, st)) return -1;
-         if (want && (mr > mb ? mr : mb) <= S->s.fac_tol) break;
+         if (launch_rbgs<T>(L, B.op, dx, rhs, x, 1, true, st)) return -1;
+         if (reduce_partials(L, L.ncell_tiles, 1, 1, &mb, st)) return -1;
+         if ((mr > mb ? mr : mb) <= S->s.fac_tol) break;
       }
-   } else {
-      int ql = B.ncomp;
-      if (ghost_fill(L, x, ql, st)) return -1;
-      for (int sw = 0; sw < S->s.quat_sweeps; sw++) {
-         if (ghost_fill(L, x, ql, st)) return -1;
-         if (launch_quat_rbgs<T>(L, B.fc, B.sm, S->gamma_setup, dx, ql, rhs, x, 0, st)) return -1;
-         if (ghost_fill(L, x, ql, st)) return -1;
-         if (launch_quat_rbgs<T>(L, B.fc, B.sm, S->gamma_setup, dx, ql, rhs, x, 1, st)) return -1;
-         if (ghost_fill(L, x, ql, st)) return -1;
-      }
+      return 0;
    }
-   return 0;
+   SweepSet<T> set;
+   if (B.kind == 1) {
+      if (add_orientation<T>(S, set, 0)) return -1;
+   } else {
+      SweepSlot<T> o;
+      o.D = B.op.D;
+      o.Dc = B.op.Dc;
+      o.C = B.op.C;
+      o.Cc = B.op.Cc;
+      o.M = B.op.M;
+      o.Mc = B.op.Mc;
+      if (sweep_add<T>(set, o, 0, 1)) return -1;
+   }
+   // (the elliptic blocks stay natural here: their residuals are)
+   const bool split = B.kind == 1 && mg_of<T>(S) && mg_of<T>(S)->split;
+   return cycle_set<T>(S, set, B.ncomp, B.kind == 0 ? S->s.fac_sweeps : S->s.quat_sweeps, rhs, x,
+                       split);
 }
 
 // residual r = f - A u (ghost fill of u first), per-tile sums into region reg
@@ -981,7 +1028,7 @@ static int block_residual(Sim* S, PBlock<T>& B, int reg)
    hipStream_t st = S->stream;
    double* part = L.partial + (size_t)reg * L.ncell_tiles;
    Mg<T>* mg = mg_of<T>(S);
-   const bool split = B.kind == 1 && mg && mg->qsplit;
+   const bool split = B.kind == 1 && mg && mg->split;
    if (ghost_fill(L, B.u, B.ncomp, st, split)) return -1;
    if (B.kind == 0) return launch_residual<T>(L, B.op, S->p.dx, B.f, B.u, B.r, part, st);
    return launch_quat_residual<T>(L, B.fc, B.sm, S->gamma_setup, S->p.dx, B.ncomp, B.f, B.u,
@@ -1000,7 +1047,7 @@ static int run_blocks(Sim* S, std::vector<PBlock<T>>& blocks, double tol)
    hipStream_t st = S->stream;
    int nb = (int)blocks.size();
    bool multi = S->s.fac_max_cycles > 1 || S->s.quat_max_cycles > 1;
-   // cycle 1 from u = 0 (zeroed by psolve_in)
+   // cycle 1 from u = 0
    for (int b = 0; b < nb; b++) {
       PBlock<T>& B = blocks[b];
       if (block_smooth<T>(S, B, B.f, B.u)) return -1;
@@ -1024,7 +1071,6 @@ static int run_blocks(Sim* S, std::vector<PBlock<T>>& blocks, double tol)
       if (active.empty()) break;
       for (size_t a = 0; a < active.size(); a++) {
          PBlock<T>& B = blocks[active[a]];
-         if (fill_zero<T>(B.e, S->ng * B.ncomp, st)) return -1;
          if (block_smooth<T>(S, B, B.r, B.e)) return -1;
          long long n = S->ng * B.ncomp;
          if (std::is_same<T, double>::value) {
@@ -1097,11 +1143,11 @@ static std::vector<PBlock<T>> make_blocks(Sim* S, double dphi, const T* Cphi, co
    return bl;
 }
 
-// f_u = P^-1 f_f on the FP32 buffers (f_u zeroed first when zero_u).
-static int psolve_f32(Sim* S, double delta, bool zero_u)
+// f_u = P^-1 f_f on the FP32 buffers.
+static int psolve_f32(Sim* S, double delta)
 {
    long long ng = S->ng;
-   if (zero_u && fill_zero<float>(S->f_u, S->nv, S->stream)) return -1;
+   if (set_mode(S)) return solve_set<float>(S, S->f_f, S->f_u);
    double dphi = -S->gamma_setup * S->p.epsilon_phi * S->p.epsilon_phi;
    auto bl = make_blocks<float>(S, dphi, S->f_Cphi, S->f_Mphi, S->f_Dconc, S->f_fc,
                                 S->f_sqrtm);
@@ -1126,7 +1172,7 @@ static bool psolve_graph_ok(const Sim* S)
           S->s.quat_max_cycles <= 1 && (S->mgf || S->s.fac_tol < 0.0);
 }
 
-// psolve_f32(zero_u) captured into a HIP graph (again when gamma changed) and
+// psolve_f32 captured into a HIP graph (again when gamma changed) and
 // replayed: one launch instead of one per kernel of every V-cycle.  The
 // coefficient buffers are read at replay, so a preconditioner setup at the
 // same gamma needs no new capture.
@@ -1140,7 +1186,7 @@ static int psolve_f32_graph(Sim* S)
    if (!S->pgraph) {
       hipGraph_t g = nullptr;
       AMPE_HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
-      int rc = psolve_f32(S, 0.0, true);
+      int rc = psolve_f32(S, 0.0);
       hipError_t e = hipStreamEndCapture(st, &g);
       if (rc < 0 || e != hipSuccess || !g) {
          if (g) (void)hipGraphDestroy(g);
@@ -1160,11 +1206,16 @@ static int psolve_f32_graph(Sim* S)
    return 0;
 }
 
-// The level whose row parity-split layout the FP32 orientation vectors
-// f_f / f_u use (null: natural layout).
-static const Level* qsplit_level(const Sim* S)
+// The level in whose row parity-split layout the FP32 vectors f_f / f_u are
+// stored (null: natural), and the first component that is: all of them when the
+// blocks share their launches, else the orientation's.
+static const Level* split_level(const Sim* S)
 {
-   return S->mgf && S->mgf->qsplit ? S->L : nullptr;
+   return S->mgf && S->mgf->split ? S->L : nullptr;
+}
+static int split_first(const Sim* S)
+{
+   return set_mode(S) || S->iq < 0 ? 0 : S->iq;
 }
 
 // z = P^-1 r.  FP32 preconditioner only: f_ready = the FP32 right-hand side
@@ -1173,7 +1224,9 @@ static const Level* qsplit_level(const Sim* S)
 struct PsolveOpts {
    bool f_ready = false;
    bool keep = false;
-   bool status = false;  // hierarchy: return whether the residual norms met delta
+   // a caller outside the integrator: z's ghosts are filled, and a hierarchy
+   // returns whether the residual norms met delta
+   bool status = false;
 };
 static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o = {})
 {
@@ -1186,39 +1239,55 @@ static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o
    int ql = S->iq >= 0 ? p.qlen : 0;
    int iq = S->iq >= 0 ? S->iq : S->nc;
    if (S->s.precision == AMPE_FAC_FP32) {
-      // f = r (orientation blocks / sqrt(M), FP64 division) in FP32, u = 0
+      // f = r (orientation blocks / sqrt(M), FP64 division) in FP32
       int ret;
       if (o.f_ready) {
-         ret = psolve_graph_ok(S) ? psolve_f32_graph(S) : psolve_f32(S, delta, true);
+         ret = psolve_graph_ok(S) ? psolve_f32_graph(S) : psolve_f32(S, delta);
       } else {
-         if (psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, S->f_u, st,
-                              qsplit_level(S)))
+         if (psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, nullptr, st,
+                              split_level(S), split_first(S)))
             return -1;
-         ret = psolve_f32(S, delta, false);
+         ret = psolve_f32(S, delta);
       }
       if (ret < 0) return -1;
-      if (!o.keep && psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, nullptr, z, st,
-                                       qsplit_level(S)))
+      if (!o.keep && psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st,
+                                       split_level(S), split_first(S)))
          return -1;
+      if (o.status && ghost_fill(*S->L, z, S->nc, st)) return -1;
       return ret;
    }
    if (o.f_ready || o.keep) {
       set_error("psolve: fused input/output is for the FP32 preconditioner");
       return -1;
    }
-   // FP64: z = 0, fac_u = orientation blocks of r / sqrt(M)
-   if (psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, nullptr, S->fac_u, z, st)) return -1;
-   auto bl = make_blocks<double>(S, dphi, S->Cphi, S->Mphi, S->Dconc, S->fc, S->sqrtm);
-   for (auto& B : bl) {
-      long long off = (long long)B.comp * ng;
-      B.f = B.kind == 1 ? S->fac_u : r + off;
-      B.u = z + off;
-      B.e = S->fac_e + off;
-      B.r = S->fac_r + off;
+   int ret = 0;
+   if (set_mode(S) && S->mgd) {
+      // the V-cycle's right-hand side in one vector
+      if (psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, nullptr, st))
+         return -1;
+      if (solve_set<double>(S, S->fac_e, z)) return -1;
+   } else {
+      // fac_u = orientation blocks of r / sqrt(M)
+      if (S->iq >= 0 &&
+          psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, nullptr, S->fac_u, nullptr, st))
+         return -1;
+      if (set_mode(S)) {
+         if (solve_set<double>(S, S->fac_u, z, r)) return -1;
+      } else {
+         auto bl = make_blocks<double>(S, dphi, S->Cphi, S->Mphi, S->Dconc, S->fc, S->sqrtm);
+         for (auto& B : bl) {
+            long long off = (long long)B.comp * ng;
+            B.f = B.kind == 1 ? S->fac_u : r + off;
+            B.u = z + off;
+            B.e = S->fac_e + off;
+            B.r = S->fac_r + off;
+         }
+         ret = run_blocks<double>(S, bl, delta);
+         if (ret < 0) return -1;
+      }
    }
-   int ret = run_blocks<double>(S, bl, delta);
-   if (ret < 0) return -1;
    if (S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql)) return -1;
+   if (o.status && ghost_fill(*S->L, z, S->nc, st)) return -1;
    return ret;
 }
 
@@ -1280,7 +1349,7 @@ static int spgmr(Sim* S, double gamma, const double* bvec, double* x, double del
       pout.ewt = S->ewt;
       pout.iq = pin.iq;
       pout.ql = pin.ql;
-      pin.split = pout.split = qsplit_level(S) ? 1 : 0;
+      if (split_level(S)) pin.sp0 = pout.sp0 = split_first(S);
    }
    double hs[kMaxKrylov + 1];
    if (psolve(S, bvec, S->work, delta) < 0) return -1;

@@ -157,78 +157,76 @@ int vec_sumsq_w(const Level& L, int ncomp, const double* x, const double* w, dou
    return reduce_partials(L, L.ncell_tiles, 1, 0, out, s);
 }
 
-// Preconditioner input over all nc ghosted component blocks: u = 0 and
-// f = r, with the orientation blocks [iq, iq + ql) divided by sqrt(M) (FP64
-// division, then the conversion to T).  For T = double f may be null: then
-// only the orientation blocks are written, to fq (ql blocks).  np > 0: the
-// orientation blocks are stored in the row parity-split layout of the level
-// whose patch table is P (np patches).
+// Preconditioner input over all nc ghosted component blocks, a thread per
+// ghosted cell: f = r, with the orientation blocks [iq, iq + ql) divided by
+// sqrt(M) (FP64 division, then the conversion to T), and u = 0 when given.  For
+// T = double f may be null: then only the orientation blocks are written, to fq
+// (ql blocks).  np > 0: the blocks from sp0 on are stored in the row
+// parity-split layout of the level whose patch table is P (np patches); the
+// position in the row is found once for all components.
 template <typename T>
 __global__ void __launch_bounds__(256) k_psolve_in(long long ng, int nc, int iq, int ql,
                                                    const double* __restrict__ r,
                                                    const double* __restrict__ sm,
                                                    T* __restrict__ f, T* __restrict__ fq,
-                                                   T* __restrict__ u, const PatchDev* P, int np)
+                                                   T* __restrict__ u, const PatchDev* P, int np,
+                                                   int sp0)
 {
-   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= ng * nc) return;
-   long long m = i / ng, c = i - m * ng;
-   u[i] = T(0);
-   bool q = m >= iq && m < iq + ql;
-   if (q) {
-      double v = r[i] / sm[c];
-      long long o = np > 0 ? m * ng + split_index(P, np, c) : i;
-      if (f) f[o] = (T)v;
-      else fq[o - (long long)iq * ng] = (T)v;
-   } else if (f) {
-      f[i] = (T)r[i];
+   const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (c >= ng) return;
+   const long long o = np > 0 ? split_index(P, np, c) : c;
+   const double s = ql > 0 ? sm[c] : 1.0;
+#pragma unroll 2
+   for (int m = 0; m < nc; m++) {
+      if (u) u[m * ng + c] = T(0);
+      const bool q = m >= iq && m < iq + ql;
+      if (!f && !q) continue;
+      double v = r[m * ng + c];
+      if (q) v = v / s;
+      const long long d = m >= sp0 ? o : c;
+      if (f)
+         f[m * ng + d] = (T)v;
+      else
+         fq[(m - iq) * ng + d] = (T)v;
    }
 }
 
-// Preconditioner output: z = u, orientation blocks multiplied by sqrt(M),
-// then by ewt when given (z = ewt u).
+// Preconditioner output: z = u, orientation blocks multiplied by sqrt(M).
 template <typename T>
 __global__ void __launch_bounds__(256) k_psolve_out(long long ng, int nc, int iq, int ql,
                                                     const T* __restrict__ u,
                                                     const double* __restrict__ sm,
-                                                    const double* __restrict__ ewt,
                                                     double* __restrict__ z, const PatchDev* P,
-                                                    int np)
+                                                    int np, int sp0)
 {
-   long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= ng * nc) return;
-   long long m = i / ng, c = i - m * ng;
-   double v;
-   if (m >= iq && m < iq + ql) {
-      v = (double)u[np > 0 ? m * ng + split_index(P, np, c) : i];
-      v = v * sm[c];
-   } else {
-      v = (double)u[i];
+   const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (c >= ng) return;
+   const long long o = np > 0 ? split_index(P, np, c) : c;
+   const double s = ql > 0 ? sm[c] : 1.0;
+#pragma unroll 2
+   for (int m = 0; m < nc; m++) {
+      double v = (double)u[m * ng + (m >= sp0 ? o : c)];
+      if (m >= iq && m < iq + ql) v = v * s;
+      z[m * ng + c] = v;
    }
-   if (ewt) v = ewt[i] * v;
-   z[i] = v;
 }
 
 template <typename T>
 int psolve_in(long long ng, int nc, int iq, int ql, const double* r, const double* sm, T* f,
-              T* fq, T* u, hipStream_t s, const Level* split)
+              T* fq, T* u, hipStream_t s, const Level* split, int sp0)
 {
-   long long n = ng * nc;
-   hipLaunchKernelGGL(k_psolve_in<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ng, nc,
-                      iq, ql, r, sm, f, fq, u, split ? split->dp : nullptr,
-                      split ? split->npatch : 0);
+   hipLaunchKernelGGL(k_psolve_in<T>, dim3(nblk(ng)), dim3(256), 0, s, ng, nc, iq, ql, r, sm, f,
+                      fq, u, split ? split->dp : nullptr, split ? split->npatch : 0, sp0);
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
 
 template <typename T>
-int psolve_out(long long ng, int nc, int iq, int ql, const T* u, const double* sm,
-               const double* ewt, double* z, hipStream_t s, const Level* split)
+int psolve_out(long long ng, int nc, int iq, int ql, const T* u, const double* sm, double* z,
+               hipStream_t s, const Level* split, int sp0)
 {
-   long long n = ng * nc;
-   hipLaunchKernelGGL(k_psolve_out<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ng,
-                      nc, iq, ql, u, sm, ewt, z, split ? split->dp : nullptr,
-                      split ? split->npatch : 0);
+   hipLaunchKernelGGL(k_psolve_out<T>, dim3(nblk(ng)), dim3(256), 0, s, ng, nc, iq, ql, u, sm, z,
+                      split ? split->dp : nullptr, split ? split->npatch : 0, sp0);
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -255,12 +253,10 @@ int vec_scale_comp(long long ng, int ncomp, const double* sm, double* x, hipStre
 }
 
 template int psolve_in<float>(long long, int, int, int, const double*, const double*, float*,
-                              float*, float*, hipStream_t, const Level*);
+                              float*, float*, hipStream_t, const Level*, int);
 template int psolve_in<double>(long long, int, int, int, const double*, const double*, double*,
-                               double*, double*, hipStream_t, const Level*);
-template int psolve_out<float>(long long, int, int, int, const float*, const double*,
-                               const double*, double*, hipStream_t, const Level*);
-template int psolve_out<double>(long long, int, int, int, const double*, const double*,
-                                const double*, double*, hipStream_t, const Level*);
+                               double*, double*, hipStream_t, const Level*, int);
+template int psolve_out<float>(long long, int, int, int, const float*, const double*, double*,
+                               hipStream_t, const Level*, int);
 
 }  // namespace ampe
