@@ -23,18 +23,25 @@ struct KksGuess {
    unsigned* count = nullptr;
 };
 
-// Workgroups of the surrogate pass (each stages the network once and walks
-// the work list with a grid stride).
+// Workgroups of the level-wide call and of the surrogate pass (each of which
+// stages the network once and walks the work list with a grid stride); each
+// has a slot of kKksPart doubles.
+constexpr int kKksGrid = 4096;
 constexpr int kKksSurrGrid = 256;
+constexpr int kKksPart = 5;
+constexpr size_t kKksPartDoubles = (size_t)kKksPart * (kKksGrid + kKksSurrGrid);
 
-// KKS over all ghosted cells of a level.  launch_kks accumulates into device
-// counters dev_acc[6] = {total iterations, max iterations, failure flag,
-// calls, fallbacks, surrogate starts} without synchronising; launch_kks_sync returns max
-// iterations (or -1 on a non-converged cell) and the total, synchronising s.
+// KKS over all ghosted cells of a level.  launch_kks adds its counts to the
+// slots part (kKksPartDoubles doubles, zero at first) without synchronising;
+// kks_finish folds them into the device counters dev_acc[6] = {total iterations,
+// max iterations, failure flag, unused, fallbacks, surrogate starts} and clears
+// them; launch_kks_sync returns max iterations (or -1 on a non-converged cell)
+// and the total, synchronising s.
 constexpr int kKksAcc = 6;
 int launch_kks(const Level& L, const ampe_model_params& p, const double* phi,
                const double* c, const double* clr, const double* csr, double* cl,
-               double* cs, const KksGuess& guess, long long* dev_acc, hipStream_t s);
+               double* cs, const KksGuess& guess, double* part, hipStream_t s);
+int kks_finish(double* part, long long* dev_acc, hipStream_t s);
 int launch_kks_sync(const Level& L, const ampe_model_params& p, const double* phi,
                     const double* c, const double* clr, const double* csr, double* cl,
                     double* cs, int* max_iters, long long* total_iters, hipStream_t s);

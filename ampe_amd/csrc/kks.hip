@@ -10,10 +10,11 @@
 // members evaluated at that temperature, default start (0.5, 0.5)
 // (tests/testCALPHADbinaryKKS.cc:123-127) or the surrogate.
 //
-// Each workgroup writes {sum of updates, max updates or failure marker,
-// fallbacks, failures, surrogate starts} to its partial slot; a one-workgroup finish kernel folds them
-// into device counters in a fixed order (no same-address atomics, no host
-// synchronisation per call).
+// Each workgroup adds {sum of updates, max updates or failure marker,
+// fallbacks, failures, surrogate starts} to its partial slot; a one-workgroup finish
+// kernel folds the slots into device counters in a fixed order when they are
+// read (no same-address atomics, no host synchronisation or extra launch per
+// call).
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -23,12 +24,12 @@
 namespace ampe {
 
 constexpr double kKksFail = 1.0e9;
-constexpr int kKksPart = 5;  // doubles per workgroup
 
 // it: updates, mx: updates or kKksFail, fb: fallback (0/1), nf: failure
 // (0/1), ss: surrogate start (0/1)
+// add: the slot accumulates over calls (until a finish folds it and clears it)
 __device__ inline void kks_block_partial(double it, double mx, double fb, double nf, double ss,
-                                         double* __restrict__ partial)
+                                         double* __restrict__ partial, bool add)
 {
    for (int o = 32; o > 0; o >>= 1) {
       it += __shfl_xor(it, o);
@@ -57,11 +58,19 @@ __device__ inline void kks_block_partial(double it, double mx, double fb, double
          e += sh[kKksPart * k + 3];
          g += sh[kKksPart * k + 4];
       }
-      partial[kKksPart * blockIdx.x] = s;
-      partial[kKksPart * blockIdx.x + 1] = m;
-      partial[kKksPart * blockIdx.x + 2] = f;
-      partial[kKksPart * blockIdx.x + 3] = e;
-      partial[kKksPart * blockIdx.x + 4] = g;
+      double* o = partial + kKksPart * blockIdx.x;
+      if (add) {
+         s += o[0];
+         m = o[1] > m ? o[1] : m;
+         f += o[2];
+         e += o[3];
+         g += o[4];
+      }
+      o[0] = s;
+      o[1] = m;
+      o[2] = f;
+      o[3] = e;
+      o[4] = g;
    }
 }
 
@@ -80,8 +89,12 @@ __device__ inline void kks_surrogate_guess(const MlpDev& m, const u16x8* sf, con
    gs = (double)y[1] * m.out_scale[1] + m.out_shift[1];
 }
 
-// Every cell from the previous-step guess (kks_cell).
-__global__ void __launch_bounds__(256) k_kks(long long n, ampe_model_params p,
+// Every cell from the previous-step guess (kks_cell), a grid stride over the
+// ghosted cells.  CALPHAD is bound by FP64 arithmetic (kks_newton_from), the
+// closed forms by HBM.  256^3 from the composition as the guess (about three
+// updates): 457 us, 966 us with two logarithms and eight divisions an update.
+template <int FE>
+__global__ void __launch_bounds__(256) k_kks(long long n, ampe_model_params p, KksTerms terms,
                                              const double* __restrict__ phi,
                                              const double* __restrict__ c,
                                              const double* __restrict__ clr,
@@ -89,17 +102,21 @@ __global__ void __launch_bounds__(256) k_kks(long long n, ampe_model_params p,
                                              double* __restrict__ cl, double* __restrict__ cs,
                                              double* __restrict__ partial)
 {
-   long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
    double it = 0.0, mx = 0.0;
-   if (t < n) {
+   const long long stride = (long long)gridDim.x * blockDim.x;
+   for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += stride) {
       double xl = clr[t], xs = csr[t];
-      int r = kks_cell(p, c[t], phi[t], xl, xs);
+      int r = kks_cell<FE>(p, terms, c[t], phi[t], xl, xs);
       cl[t] = xl;
       cs[t] = xs;
-      mx = r < 0 ? kKksFail : (double)r;
-      it = r < 0 ? 0.0 : (double)r;
+      if (r < 0) {
+         mx = kKksFail;
+      } else {
+         it += (double)r;
+         mx = (double)r > mx ? (double)r : mx;
+      }
    }
-   kks_block_partial(it, mx, 0.0, mx >= kKksFail ? 1.0 : 0.0, 0.0, partial);
+   kks_block_partial(it, mx, 0.0, mx >= kKksFail ? 1.0 : 0.0, 0.0, partial, true);
 }
 
 // Switch policy, first pass (binary CALPHAD): a cell whose residual at the
@@ -108,7 +125,7 @@ __global__ void __launch_bounds__(256) k_kks(long long n, ampe_model_params p,
 // atomic per wave) and left to k_kks_surr.  Kept free of the network so that
 // it runs at the occupancy of the plain solve.
 __global__ void __launch_bounds__(256) k_kks_defer(long long n, ampe_model_params p,
-                                                   double switch_tol,
+                                                   KksTerms terms, double switch_tol,
                                                    const double* __restrict__ phi,
                                                    const double* __restrict__ c,
                                                    const double* __restrict__ clr,
@@ -119,44 +136,51 @@ __global__ void __launch_bounds__(256) k_kks_defer(long long n, ampe_model_param
                                                    unsigned* __restrict__ count,
                                                    double* __restrict__ partial)
 {
-   long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
    double it = 0.0, mx = 0.0;
-   bool bad = false;
-   if (t < n) {
-      const double T = p.temperature;
-      double ct = c[t];
-      double h = interp(phi[t], p.conc_interp);
-      double xl = clr[t], xs = csr[t];
-      kks_clamp(xl, xs);
-      double f1, f2;
-      kks_residual(p.calphad, T, 1.0 / (kRGas * T), h, ct, xl, xs, f1, f2);
-      bad = switch_tol <= 0.0 || !(dmax(fabs(f1), fabs(f2)) <= switch_tol);
-      if (!bad) {
-         int r = kks_newton_from(p.calphad, T, h, ct, xl, xs, f1, f2, p.newton_max_its,
-                                 p.newton_tol, -1, 0.0);
-         cl[t] = xl;
-         cs[t] = xs;
-         mx = r < 0 ? kKksFail : (double)r;
-         it = r < 0 ? 0.0 : (double)r;
+   const long long stride = (long long)gridDim.x * blockDim.x;
+   for (long long t0 = (long long)blockIdx.x * blockDim.x; t0 < n; t0 += stride) {
+      const long long t = t0 + threadIdx.x;
+      bool bad = false;
+      if (t < n) {
+         double ct = c[t];
+         double h = interp(phi[t], p.conc_interp);
+         double xl = clr[t], xs = csr[t];
+         kks_clamp(xl, xs);
+         double f1, f2;
+         kks_residual(terms, h, ct, xl, xs, f1, f2);
+         bad = switch_tol <= 0.0 || !(dmax(fabs(f1), fabs(f2)) <= switch_tol);
+         if (!bad) {
+            int r = kks_newton_from(terms, h, ct, xl, xs, f1, f2, p.newton_max_its, p.newton_tol,
+                                    -1, 0.0);
+            cl[t] = xl;
+            cs[t] = xs;
+            if (r < 0) {
+               mx = kKksFail;
+            } else {
+               it += (double)r;
+               mx = (double)r > mx ? (double)r : mx;
+            }
+         }
+      }
+      unsigned long long mask = __ballot(bad);
+      if (mask) {
+         const int lane = threadIdx.x & 63;
+         const int first = __ffsll((long long)mask) - 1;
+         unsigned base = 0;
+         if (lane == first) base = atomicAdd(count, (unsigned)__popcll(mask));
+         base = __shfl(base, first);
+         if (bad) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = (int)t;
       }
    }
-   unsigned long long mask = __ballot(bad);
-   if (mask) {
-      const int lane = threadIdx.x & 63;
-      const int first = __ffsll((long long)mask) - 1;
-      unsigned base = 0;
-      if (lane == first) base = atomicAdd(count, (unsigned)__popcll(mask));
-      base = __shfl(base, first);
-      if (bad) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = (int)t;
-   }
-   kks_block_partial(it, mx, 0.0, mx >= kKksFail ? 1.0 : 0.0, 0.0, partial);
+   kks_block_partial(it, mx, 0.0, mx >= kKksFail ? 1.0 : 0.0, 0.0, partial, true);
 }
 
 // Switch policy, second pass: the listed cells start from the surrogate and
 // restart from the previous-step guess when the residual after probe_its
 // updates exceeds probe_tol.  Grid-stride over the list, whole waves at a
 // time (the network's MFMA inference needs all 64 lanes).
-__global__ void __launch_bounds__(256) k_kks_surr(ampe_model_params p, MlpDev m, int probe_its,
+__global__ void __launch_bounds__(256) k_kks_surr(ampe_model_params p, KksTerms terms, MlpDev m,
+                                                  int probe_its,
                                                   double probe_tol,
                                                   const double* __restrict__ phi,
                                                   const double* __restrict__ c,
@@ -189,16 +213,16 @@ __global__ void __launch_bounds__(256) k_kks_surr(ampe_model_params p, MlpDev m,
       kks_surrogate_guess(m, sf, sb, ct, pt, T, gl, gs);
       if (in) {
          double h = interp(pt, p.conc_interp);
-         int r = kks_newton(p.calphad, T, h, ct, gl, gs, p.newton_max_its, p.newton_tol,
-                            probe_its, probe_tol);
+         int r = kks_newton(terms, h, ct, gl, gs, p.newton_max_its, p.newton_tol, probe_its,
+                            probe_tol);
          if (r == -2) {
             fb += 1.0;
             double xl = clr[t], xs = csr[t];
             kks_clamp(xl, xs);
             double f1, f2;
-            kks_residual(p.calphad, T, 1.0 / (kRGas * T), h, ct, xl, xs, f1, f2);
-            int r2 = kks_newton_from(p.calphad, T, h, ct, xl, xs, f1, f2, p.newton_max_its,
-                                     p.newton_tol, -1, 0.0);
+            kks_residual(terms, h, ct, xl, xs, f1, f2);
+            int r2 = kks_newton_from(terms, h, ct, xl, xs, f1, f2, p.newton_max_its, p.newton_tol,
+                                     -1, 0.0);
             r = r2 < 0 ? -1 : r2 + probe_its;
             gl = xl;
             gs = xs;
@@ -214,23 +238,26 @@ __global__ void __launch_bounds__(256) k_kks_surr(ampe_model_params p, MlpDev m,
          }
       }
    }
-   kks_block_partial(it, mx, fb, mx >= kKksFail ? 1.0 : 0.0, ss, partial);
+   kks_block_partial(it, mx, fb, mx >= kKksFail ? 1.0 : 0.0, ss, partial, true);
 }
 
 // acc[0] += updates, acc[1] = max(acc[1], max updates), acc[2] |= failure,
-// acc[3] += 1 (calls), acc[4] += fallbacks, acc[5] += surrogate starts.
-// One workgroup.
-__global__ void __launch_bounds__(1024) k_kks_finish(const double* __restrict__ partial, int nb,
-                                                     long long* __restrict__ acc,
-                                                     unsigned* __restrict__ count)
+// acc[4] += fallbacks, acc[5] += surrogate starts from the nb accumulated
+// partials, which it clears (acc[3] is unused).  One workgroup, once per
+// reading of the counters: after every call it took 43 us of a 256^3 right-hand
+// side and a launch of every small one.
+__global__ void __launch_bounds__(1024) k_kks_finish(double* __restrict__ partial, int nb,
+                                                     long long* __restrict__ acc)
 {
    __shared__ double ss[1024], sm[1024], sf[1024], sg[1024];
    double s = 0.0, m = 0.0, f = 0.0, g = 0.0;
    for (int i = threadIdx.x; i < nb; i += 1024) {
-      s += partial[kKksPart * i];
-      m = partial[kKksPart * i + 1] > m ? partial[kKksPart * i + 1] : m;
-      f += partial[kKksPart * i + 2];
-      g += partial[kKksPart * i + 4];
+      double* o = partial + kKksPart * i;
+      s += o[0];
+      m = o[1] > m ? o[1] : m;
+      f += o[2];
+      g += o[4];
+      for (int k = 0; k < kKksPart; k++) o[k] = 0.0;
    }
    ss[threadIdx.x] = s;
    sm[threadIdx.x] = m;
@@ -253,12 +280,12 @@ __global__ void __launch_bounds__(1024) k_kks_finish(const double* __restrict__ 
       long long mxi = fail ? 0 : (long long)sm[0];
       acc[1] = mxi > acc[1] ? mxi : acc[1];
       if (fail) acc[2] = 1;
-      acc[3] += 1;
       acc[4] += (long long)sf[0];
       acc[5] += (long long)sg[0];
-      if (count) *count = 0u;  // the work list is empty again for the next call
    }
 }
+
+__global__ void k_kks_list_clear(unsigned* count) { *count = 0u; }
 
 MlpDev Surrogate::dev() const
 {
@@ -278,13 +305,20 @@ MlpDev Surrogate::dev() const
    return d;
 }
 
+// Workgroups of the level-wide call: enough to fill the chip several times
+// over, few enough that the partials stay a few pages (4096 walk 16 cells a
+// thread at 256^3).
+static unsigned kks_grid(const Level& L)
+{
+   return (unsigned)std::min<long long>((L.ncg + 255) / 256, kKksGrid);
+}
+
 int launch_kks(const Level& L, const ampe_model_params& p, const double* phi,
                const double* c, const double* clr, const double* csr, double* cl,
-               double* cs, const KksGuess& guess, long long* dev_acc, hipStream_t s)
+               double* cs, const KksGuess& guess, double* part, hipStream_t s)
 {
-   unsigned nb = (unsigned)((L.ncg + 255) / 256);
-   unsigned nparts = nb;
-   unsigned* count = nullptr;
+   const unsigned nb = kks_grid(L);
+   const KksTerms terms = kks_terms(p.calphad, p.temperature);
    if (guess.surrogate && p.fe_model == AMPE_FE_CALPHAD_BINARY) {
       const Surrogate& S = *guess.surrogate;
       if (S.hid != kMlpHidden || S.nin != 3 || S.nout != 2) {
@@ -296,22 +330,34 @@ int launch_kks(const Level& L, const ampe_model_params& p, const double* phi,
          return -1;
       }
       MlpDev m = S.dev();
-      count = guess.count;
-      hipLaunchKernelGGL(k_kks_defer, dim3(nb), dim3(256), 0, s, L.ncg, p, guess.switch_tol,
-                         phi, c, clr, csr, cl, cs, guess.list, count, L.kks_part);
+      hipLaunchKernelGGL(k_kks_defer, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
+                         guess.switch_tol, phi, c, clr, csr, cl, cs, guess.list, guess.count, part);
       AMPE_HIP_CHECK(hipGetLastError());
       unsigned g = std::min<unsigned>(kKksSurrGrid, nb);
-      hipLaunchKernelGGL(k_kks_surr, dim3(g), dim3(256), 0, s, p, m, guess.probe_its,
-                         guess.probe_tol, phi, c, clr, csr, cl, cs, guess.list, count,
-                         L.kks_part + (size_t)kKksPart * nb);
-      nparts = nb + g;
+      hipLaunchKernelGGL(k_kks_surr, dim3(g), dim3(256), 0, s, p, terms, m, guess.probe_its,
+                         guess.probe_tol, phi, c, clr, csr, cl, cs, guess.list, guess.count,
+                         part + (size_t)kKksPart * kKksGrid);
+      AMPE_HIP_CHECK(hipGetLastError());
+      // the work list is empty again for the next call
+      hipLaunchKernelGGL(k_kks_list_clear, dim3(1), dim3(1), 0, s, guess.count);
+   } else if (p.fe_model == AMPE_FE_QUADRATIC) {
+      hipLaunchKernelGGL(k_kks<AMPE_FE_QUADRATIC>, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
+                         phi, c, clr, csr, cl, cs, part);
+   } else if (p.fe_model == AMPE_FE_KKS_DILUTE) {
+      hipLaunchKernelGGL(k_kks<AMPE_FE_KKS_DILUTE>, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
+                         phi, c, clr, csr, cl, cs, part);
    } else {
-      hipLaunchKernelGGL(k_kks, dim3(nb), dim3(256), 0, s, L.ncg, p, phi, c, clr, csr, cl, cs,
-                         L.kks_part);
+      hipLaunchKernelGGL(k_kks<AMPE_FE_CALPHAD_BINARY>, dim3(nb), dim3(256), 0, s, L.ncg, p,
+                         terms, phi, c, clr, csr, cl, cs, part);
    }
    AMPE_HIP_CHECK(hipGetLastError());
-   hipLaunchKernelGGL(k_kks_finish, dim3(1), dim3(1024), 0, s, L.kks_part, (int)nparts, dev_acc,
-                      count);
+   return 0;
+}
+
+int kks_finish(double* part, long long* dev_acc, hipStream_t s)
+{
+   hipLaunchKernelGGL(k_kks_finish, dim3(1), dim3(1024), 0, s, part, kKksGrid + kKksSurrGrid,
+                      dev_acc);
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -322,7 +368,8 @@ int launch_kks_sync(const Level& L, const ampe_model_params& p, const double* ph
 {
    long long* acc = reinterpret_cast<long long*>(L.iscratch);
    AMPE_HIP_CHECK(hipMemsetAsync(acc, 0, sizeof(long long) * kKksAcc, s));
-   if (launch_kks(L, p, phi, c, clr, csr, cl, cs, KksGuess{}, acc, s)) return -1;
+   if (launch_kks(L, p, phi, c, clr, csr, cl, cs, KksGuess{}, L.kks_part, s)) return -1;
+   if (kks_finish(L.kks_part, acc, s)) return -1;
    AMPE_HIP_CHECK(hipMemcpyAsync(L.hpinned, acc, sizeof(long long) * kKksAcc,
                                  hipMemcpyDeviceToHost, s));
    AMPE_HIP_CHECK(hipStreamSynchronize(s));
@@ -371,23 +418,22 @@ __global__ void __launch_bounds__(256) k_kks_batch(long long n, ampe_model_param
       double gl = 0.5, gs = 0.5;
       if (SURR) kks_surrogate_guess(m, sf, sb, ct, pt, Tt, gl, gs);
       if (!in) continue;
-      ampe_calphad_phase ph[2];
-      calphad_at(tab, Tt, ph);
+      const KksTerms terms = kks_terms_at(tab, Tt);
       double h = interp(pt, p.conc_interp);
       int r;
       if (SURR) {
          ss += 1.0;
-         r = kks_newton(ph, Tt, h, ct, gl, gs, p.newton_max_its, p.newton_tol, probe_its,
+         r = kks_newton(terms, h, ct, gl, gs, p.newton_max_its, p.newton_tol, probe_its,
                         probe_tol);
          if (r == -2) {
             fb += 1.0;
             gl = 0.5;
             gs = 0.5;
-            int r2 = kks_newton(ph, Tt, h, ct, gl, gs, p.newton_max_its, p.newton_tol, -1, 0.0);
+            int r2 = kks_newton(terms, h, ct, gl, gs, p.newton_max_its, p.newton_tol, -1, 0.0);
             r = r2 < 0 ? -1 : r2 + probe_its;
          }
       } else {
-         r = kks_newton(ph, Tt, h, ct, gl, gs, p.newton_max_its, p.newton_tol, -1, 0.0);
+         r = kks_newton(terms, h, ct, gl, gs, p.newton_max_its, p.newton_tol, -1, 0.0);
       }
       cl[t] = gl;
       cs[t] = gs;
@@ -399,7 +445,7 @@ __global__ void __launch_bounds__(256) k_kks_batch(long long n, ampe_model_param
          mx = (double)r > mx ? (double)r : mx;
       }
    }
-   kks_block_partial(it, mx, fb, nf, ss, partial);
+   kks_block_partial(it, mx, fb, nf, ss, partial, false);
 }
 
 // Fixed-order fold of nb workgroup partials into {updates, largest count,

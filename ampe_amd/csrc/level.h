@@ -81,7 +81,7 @@ struct Level {
    double* dred = nullptr;     // reduction results (16 doubles)
    double* hpinned = nullptr;  // pinned host scalars
    int* iscratch = nullptr;    // device integer flags
-   double* kks_part = nullptr; // KKS per-workgroup partials (8 per 256 ghosted cells)
+   double* kks_part = nullptr; // KKS per-workgroup partials (kKksPartDoubles)
    // control-volume weights of the cells in dot products and norms (a
    // hierarchy's composite level: zero under a finer level); null: 1
    const double* wt = nullptr;

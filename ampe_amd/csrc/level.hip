@@ -1,6 +1,7 @@
 // Level layout, ghost gather and deterministic reductions.
 #include "level.h"
 #include "kernels.h"
+#include "kks.h"
 
 #include <algorithm>
 #include <cstring>
@@ -142,11 +143,8 @@ static int level_upload(Level* L, const std::vector<long long>& gd0,
    if (e == hipSuccess) e = hipMalloc(&L->dred, sizeof(double) * 16);
    if (e == hipSuccess) e = hipHostMalloc(&L->hpinned, sizeof(double) * 64);
    if (e == hipSuccess) e = hipMalloc(&L->iscratch, sizeof(int) * 64);
-   if (e == hipSuccess)
-      // KKS partials: one slot per 256 ghosted cells plus 256 slots of the
-      // surrogate pass
-      e = hipMalloc(&L->kks_part,
-                    sizeof(double) * 8 * ((size_t)((L->ncg + 255) / 256 + 1) + 256));
+   if (e == hipSuccess) e = hipMalloc(&L->kks_part, sizeof(double) * kKksPartDoubles);
+   if (e == hipSuccess) e = hipMemset(L->kks_part, 0, sizeof(double) * kKksPartDoubles);
    if (e == hipSuccess)
       e = hipMemcpy(L->dp, L->hp.data(), sizeof(PatchDev) * npatch, hipMemcpyHostToDevice);
    if (e == hipSuccess)

@@ -51,4 +51,41 @@ AMPE_HD double log_pos(double x)
    return dk * ln2_hi - ((h - (s * (h + R) + dk * ln2_lo)) - f);
 }
 
+// ln(n / d) for positive n and d with one division: both scaled into [1/2, 1)
+// (their exponents apart), one of them doubled when the quotient lies outside
+// [sqrt(1/2), sqrt(2)], then 2 atanh s with s = (n - d) / (n + d): the
+// difference is exact, so s and the series are right to an ulp or two of the
+// result's leading part however close n and d are.  The series is log_pos's.
+// NaN unless both are positive and finite.
+AMPE_HD double log_ratio(double n, double d)
+{
+   if (!(n > 0.0 && d > 0.0 && n < HUGE_VAL && d < HUGE_VAL)) return __builtin_nan("");
+   const double ln2_hi = 0.6931471803691238;
+   const double ln2_lo = 1.9082149292705877e-10;
+   int en, ed;
+   double a = std::frexp(n, &en), b = std::frexp(d, &ed);
+   int e = en - ed;
+   if (a < 0.7071067811865476 * b) {
+      a = a + a;
+      e -= 1;
+   } else if (0.7071067811865476 * a > b) {
+      b = b + b;
+      e += 1;
+   }
+   const double s = (a - b) / (a + b);
+   const double z = s * s;
+   double t = 2.0 / 21.0;
+   t = std::fma(t, z, 2.0 / 19.0);
+   t = std::fma(t, z, 2.0 / 17.0);
+   t = std::fma(t, z, 2.0 / 15.0);
+   t = std::fma(t, z, 2.0 / 13.0);
+   t = std::fma(t, z, 2.0 / 11.0);
+   t = std::fma(t, z, 2.0 / 9.0);
+   t = std::fma(t, z, 2.0 / 7.0);
+   t = std::fma(t, z, 2.0 / 5.0);
+   t = std::fma(t, z, 2.0 / 3.0);
+   const double dk = (double)e;
+   return std::fma(dk, ln2_hi, s + (s + std::fma(s, t * z, dk * ln2_lo)));
+}
+
 }  // namespace ampe

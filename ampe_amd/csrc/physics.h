@@ -176,6 +176,29 @@ AMPE_HD double calphad_d2(const ampe_calphad_phase& cp, double T, double c)
           4.0 * c * (1.0 - c) * d2P;
 }
 
+// Driving force (f_L(cl) - f_S(cs)) - mu_S(cs) (cl - cs) [J/mol] of the two
+// CALPHAD phases.  With w(c) = f - c f' = G_B + RT ln(1 - c) + excess it is
+// w_L(cl) - w_S(cs) + (mu_L(cl) - mu_S(cs)) cl: the logarithms pair up into two
+// of quotients, where the energies and the potential one by one take five and
+// cancel most of their digits against each other.
+AMPE_HD double calphad_drive(const ampe_calphad_phase* ph, double T, double cl, double cs)
+{
+   const double RT = kRGas * T;
+   const double l0 = log_ratio(1.0 - cl, 1.0 - cs), l1 = log_ratio(cl, cs);
+   double w[2], mu[2];
+   for (int k = 0; k < 2; k++) {
+      const ampe_calphad_phase& q = ph[k];
+      const double c = k == 0 ? cl : cs;
+      const double x = 2.0 * c - 1.0;
+      const double P = q.L[0] + x * (q.L[1] + x * (q.L[2] + x * q.L[3]));
+      const double dP = q.L[1] + x * (2.0 * q.L[2] + x * 3.0 * q.L[3]);
+      const double e = 2.0 * c * (1.0 - c) * dP - x * P;
+      mu[k] = (q.gA - q.gB) + e;
+      w[k] = q.gB + (c * (1.0 - c) * P - c * e);
+   }
+   return (w[0] - w[1]) + RT * l0 + ((mu[0] - mu[1]) + RT * (l1 - l0)) * cl;
+}
+
 // Dilute binary solution (c = solute fraction):
 //   f_L(c) = RT (c ln c - c),
 //   f_S(c) = RT (c ln c - c) - RT ln(k_e) c + dG(T),
@@ -361,13 +384,92 @@ AMPE_HD void calphad_at(const ampe_calphad_tdep& tab, double T, ampe_calphad_pha
    }
 }
 
-// Residual of the binary CALPHAD KKS system at (xl, xs):
-// F = [(mu_L(xl) - mu_S(xs))/RT, (1-h) xl + h xs - c].
-AMPE_HD void kks_residual(const ampe_calphad_phase* ph, double T, double RTinv, double h,
-                          double c, double xl, double xs, double& f1, double& f2)
+// What the binary CALPHAD KKS system needs of the two phases at one
+// temperature, over RT: the difference of the end members' G_A - G_B, and the
+// excess part of dG/dc as a polynomial in u = 2c - 1 (with P the Redlich-Kister
+// sum, (1 - 2c) P + 2c(1 - c) P' = -u P + (1 - u^2)/2 P').
+struct KksTerms {
+   double k0;
+   double e[2][5];
+};
+
+AMPE_HD void kks_excess(const double* L, double RTinv, double* e)
 {
-   f1 = (calphad_mu(ph[0], T, xl) - calphad_mu(ph[1], T, xs)) * RTinv;
+   e[0] = 0.5 * L[1] * RTinv;
+   e[1] = (L[2] - L[0]) * RTinv;
+   e[2] = 1.5 * (L[3] - L[1]) * RTinv;
+   e[3] = -2.0 * L[2] * RTinv;
+   e[4] = -2.5 * L[3] * RTinv;
+}
+
+AMPE_HD KksTerms kks_terms(const ampe_calphad_phase* ph, double T)
+{
+   const double RTinv = 1.0 / (kRGas * T);
+   KksTerms t;
+   t.k0 = ((ph[0].gA - ph[0].gB) - (ph[1].gA - ph[1].gB)) * RTinv;
+   for (int k = 0; k < 2; k++) kks_excess(ph[k].L, RTinv, t.e[k]);
+   return t;
+}
+
+// Residual of the binary CALPHAD KKS system at (xl, xs):
+// F = [(mu_L(xl) - mu_S(xs))/RT, (1-h) xl + h xs - c].  The two ideal parts
+// are one logarithm, ln(xl (1 - xs) / ((1 - xl) xs)).
+AMPE_HD void kks_residual(const KksTerms& t, double h, double c, double xl, double xs, double& f1,
+                          double& f2)
+{
+   const double u = std::fma(2.0, xl, -1.0), v = std::fma(2.0, xs, -1.0);
+   const double* a = t.e[0];
+   const double* b = t.e[1];
+   const double el =
+       std::fma(u, std::fma(u, std::fma(u, std::fma(u, a[4], a[3]), a[2]), a[1]), a[0]);
+   const double es =
+       std::fma(v, std::fma(v, std::fma(v, std::fma(v, b[4], b[3]), b[2]), b[1]), b[0]);
+   f1 = (t.k0 + (el - es)) + log_ratio(xl * (1.0 - xs), (1.0 - xl) * xs);
    f2 = (1.0 - h) * xl + h * xs - c;
+}
+
+// The terms at a cell's temperature from a tdep table, the end members by
+// calphad_gfun's intervals and terms.  The interval loop is uniform and a
+// lane enters the intervals its temperature lies in (one or two over a wave), so
+// that the coefficients are scalars; indexing them by the lane's interval
+// costs 32 gathered loads a cell.  (The terms are summed as calphad_gfun sums
+// them: those of one end member reach 10^6 J/mol and cancel, and another order
+// moves the potentials by 1e-14 RT.)
+AMPE_HD KksTerms kks_terms_at(const ampe_calphad_tdep& tab, double T)
+{
+   const double Ti = 1.0 / T, lnT = log_pos(T);
+   const double T2 = T * T, T3 = T2 * T, T7 = T3 * T3 * T;
+   const double Tm9 = 1.0 / (T3 * T3 * T3);
+   double g[2][2];
+   for (int ph = 0; ph < 2; ph++)
+      for (int sp = 0; sp < 2; sp++) {
+         const ampe_calphad_gfun& f = tab.g[ph][sp];
+         bool above = true;  // T >= Tc[1..k]
+         double v = 0.0;
+         for (int k = 0; k < f.nrange; k++) {
+            const bool next = k < f.nrange - 1 && T >= f.Tc[k + 1];
+            if (above && !next) {
+               const double* a = f.coef[k];
+               v = a[0] + a[1] * T + a[2] * T * lnT;
+               v = v + a[3] * T2;
+               v = v + a[4] * T3;
+               v = v + a[5] * T7;
+               v = v + a[6] * Ti;
+               v = v + a[7] * Tm9;
+            }
+            above = above && next;
+         }
+         g[ph][sp] = v;
+      }
+   const double RTinv = 1.0 / (kRGas * T);
+   KksTerms t;
+   t.k0 = ((g[0][0] - g[0][1]) - (g[1][0] - g[1][1])) * RTinv;
+   for (int ph = 0; ph < 2; ph++) {
+      double L[4];
+      for (int i = 0; i < 4; i++) L[i] = std::fma(tab.L[ph][i][1], T, tab.L[ph][i][0]);
+      kks_excess(L, RTinv, t.e[ph]);
+   }
+   return t;
 }
 
 // Start of a KKS Newton: the guess clamped into [1e-12, 1-1e-12].
@@ -384,16 +486,23 @@ AMPE_HD void kks_clamp(double& xl, double& xs)
 // given; step halving keeps the iterate inside (0,1); converged when both
 // |F_i| < tol.  Returns the number of updates, -1 after maxits updates
 // without convergence, or -2 when probe_its >= 0 and max|F| > probe_tol after
-// probe_its updates (the caller restarts).
-AMPE_HD int kks_newton_from(const ampe_calphad_phase* ph, double T, double h, double c,
-                            double& cl, double& cs, double f1, double f2, int maxits,
-                            double tol, int probe_its, double probe_tol)
+// probe_its updates (the caller restarts).  The test stops a hundredth short of
+// tol: the residual's rounding (about 1e-15 of the ideal and excess parts)
+// depends on the order of its terms, and a solution accepted here is within tol
+// in any order.
+// The solve is bound by FP64 arithmetic: an update is one logarithm and two
+// divisions (the Jacobian 1/(x (1 - x)) + E'(x) of each phase enters multiplied by
+// both x (1 - x)), against two logarithms of quotients and eight divisions with
+// each phase's potential and second derivative evaluated by itself.
+AMPE_HD int kks_newton_from(const KksTerms& t, double h, double c, double& cl, double& cs,
+                            double f1, double f2, int maxits, double tol, int probe_its,
+                            double probe_tol)
 {
-   double RTinv = 1.0 / (kRGas * T);
    double xl = cl, xs = cs;
+   const double accept = 0.99 * tol;
    for (int it = 0; it <= maxits; it++) {
-      if (it > 0) kks_residual(ph, T, RTinv, h, c, xl, xs, f1, f2);
-      if (fabs(f1) < tol && fabs(f2) < tol) {
+      if (it > 0) kks_residual(t, h, c, xl, xs, f1, f2);
+      if (fabs(f1) < accept && fabs(f2) < accept) {
          cl = xl;
          cs = xs;
          return it;
@@ -404,12 +513,20 @@ AMPE_HD int kks_newton_from(const ampe_calphad_phase* ph, double T, double h, do
          cs = xs;
          return -2;
       }
-      double a = calphad_d2(ph[0], T, xl) * RTinv;
-      double b = -calphad_d2(ph[1], T, xs) * RTinv;
-      double cc = 1.0 - h, d = h;
-      double det = a * d - b * cc;
-      double dl = -(d * f1 - b * f2) / det;
-      double ds = -(a * f2 - cc * f1) / det;
+      const double u = std::fma(2.0, xl, -1.0), v = std::fma(2.0, xs, -1.0);
+      const double* a = t.e[0];
+      const double* b = t.e[1];
+      // dE/dc = 2 dE/du
+      const double dl2 =
+          std::fma(u, std::fma(u, std::fma(u, 8.0 * a[4], 6.0 * a[3]), 4.0 * a[2]), 2.0 * a[1]);
+      const double ds2 =
+          std::fma(v, std::fma(v, std::fma(v, 8.0 * b[4], 6.0 * b[3]), 4.0 * b[2]), 2.0 * b[1]);
+      const double pl = xl * (1.0 - xl), ps = xs * (1.0 - xs);
+      const double A = ps * std::fma(pl, dl2, 1.0), S = pl * std::fma(ps, ds2, 1.0);
+      const double q1 = pl * ps * f1;
+      const double inv = 1.0 / std::fma(A, h, S * (1.0 - h));
+      const double dl = -std::fma(h, q1, S * f2) * inv;
+      const double ds = -std::fma(A, f2, -(1.0 - h) * q1) * inv;
       double alpha = 1.0;
       for (int k = 0; k < 60; k++) {
          double nl = xl + alpha * dl, ns = xs + alpha * ds;
@@ -425,13 +542,13 @@ AMPE_HD int kks_newton_from(const ampe_calphad_phase* ph, double T, double h, do
 }
 
 // Binary CALPHAD KKS Newton from the guess (cl, cs) (see kks_newton_from).
-AMPE_HD int kks_newton(const ampe_calphad_phase* ph, double T, double h, double c, double& cl,
-                       double& cs, int maxits, double tol, int probe_its, double probe_tol)
+AMPE_HD int kks_newton(const KksTerms& t, double h, double c, double& cl, double& cs, int maxits,
+                       double tol, int probe_its, double probe_tol)
 {
    kks_clamp(cl, cs);
    double f1, f2;
-   kks_residual(ph, T, 1.0 / (kRGas * T), h, c, cl, cs, f1, f2);
-   return kks_newton_from(ph, T, h, c, cl, cs, f1, f2, maxits, tol, probe_its, probe_tol);
+   kks_residual(t, h, c, cl, cs, f1, f2);
+   return kks_newton_from(t, h, c, cl, cs, f1, f2, maxits, tol, probe_its, probe_tol);
 }
 
 // Quadratic wells: closed form of mu_L = mu_S with mass balance.
@@ -447,25 +564,25 @@ AMPE_HD void kks_quadratic(const ampe_model_params& p, double h, double c, doubl
 
 // Per-cell KKS at the model temperature: mu_L(cL) = mu_S(cS),
 // (1-h) cL + h cS = c.  Quadratic wells and the dilute solution: closed
-// forms.  CALPHAD: kks_newton from the guess in (cl, cs).  Returns the
-// iteration count or -1.
-AMPE_HD int kks_cell(const ampe_model_params& p, double c, double phi, double& cl,
-                     double& cs)
+// forms.  CALPHAD: kks_newton from the guess in (cl, cs) with the phases' terms
+// t.  Returns the iteration count or -1.
+template <int FE>
+AMPE_HD int kks_cell(const ampe_model_params& p, const KksTerms& t, double c, double phi,
+                     double& cl, double& cs)
 {
    double h = interp(phi, p.conc_interp);
-   if (p.fe_model == AMPE_FE_QUADRATIC) {
+   if (FE == AMPE_FE_QUADRATIC) {
       kks_quadratic(p, h, c, cl, cs);
       return 0;
    }
-   if (p.fe_model == AMPE_FE_KKS_DILUTE) {
+   if (FE == AMPE_FE_KKS_DILUTE) {
       double k = p.dilute_keq;
       double xl = c / (1.0 - h + h * k);
       cl = xl;
       cs = k * xl;
       return 0;
    }
-   return kks_newton(p.calphad, p.temperature, h, c, cl, cs, p.newton_max_its, p.newton_tol,
-                     -1, 0.0);
+   return kks_newton(t, h, c, cl, cs, p.newton_max_its, p.newton_tol, -1, 0.0);
 }
 
 }  // namespace ampe

@@ -342,12 +342,16 @@ __device__ __forceinline__ void phase_rhs_tail(const LevelArgs& a, const ampe_mo
    if (FE != kFeNone) {
       double convL = k.convL, convA = k.convA;
       double c_l = cl[c0], c_a = cs[c0];
-      double f_l = fenergy_t<FE>(p, c_l, 0) * convL;
-      double f_a = fenergy_t<FE>(p, c_a, 1) * convA;
-      double mu = (FE == AMPE_FE_QUADRATIC) ? dfenergy_t<FE>(p, c_l, 0) * convL
-                                            : dfenergy_t<FE>(p, c_a, 1) * convA;
       double hp = dinterp(ph, p.energy_interp);
-      r += hp * ((f_l - f_a) - mu * (c_l - c_a));
+      if (FE == AMPE_FE_CALPHAD_BINARY && convL == convA) {
+         r += hp * (calphad_drive(p.calphad, p.temperature, c_l, c_a) * convL);
+      } else {
+         double f_l = fenergy_t<FE>(p, c_l, 0) * convL;
+         double f_a = fenergy_t<FE>(p, c_a, 1) * convA;
+         double mu = (FE == AMPE_FE_QUADRATIC) ? dfenergy_t<FE>(p, c_l, 0) * convL
+                                               : dfenergy_t<FE>(p, c_a, 1) * convA;
+         r += hp * ((f_l - f_a) - mu * (c_l - c_a));
+      }
       if (p.phi_mobility_type == AMPE_PHI_MOB_KIM) mob = phase_mobility_t<FE>(p, c_l, c_a);
    }
    rhs[c0] = mob * r;

@@ -69,7 +69,9 @@ struct Sim {
          *f_Mphi = nullptr;
    hipStream_t stream = nullptr;
    hipEvent_t ev0 = nullptr, ev1 = nullptr;
-   long long* kks_acc = nullptr;  // device KKS counters (launch_kks)
+   long long* kks_acc = nullptr;  // device KKS counters (kks_finish)
+   double* kks_part = nullptr;    // and the partials they are folded from (launch_kks)
+   long long kks_calls = 0;
    KksGuess guess;                // surrogate guess when kks_guess is surrogate
    Mg<double>* mgd = nullptr;     // multigrid hierarchy (precond = MG, FP64)
    Mg<float>* mgf = nullptr;      // multigrid hierarchy (precond = MG, FP32)

@@ -203,6 +203,8 @@ static int sim_finish(Sim* S, Sim** out)
    }
    if (!rc && hipMalloc(&S->kks_acc, sizeof(long long) * kKksAcc) != hipSuccess) rc = -1;
    if (!rc && hipMemset(S->kks_acc, 0, sizeof(long long) * kKksAcc) != hipSuccess) rc = -1;
+   if (!rc && hipMalloc(&S->kks_part, sizeof(double) * kKksPartDoubles) != hipSuccess) rc = -1;
+   if (!rc && hipMemset(S->kks_part, 0, sizeof(double) * kKksPartDoubles) != hipSuccess) rc = -1;
    if (rc || hipStreamCreate(&S->stream) != hipSuccess ||
        hipEventCreate(&S->ev0) != hipSuccess || hipEventCreate(&S->ev1) != hipSuccess) {
       if (!rc) set_error("sim_create: stream/event creation failed");
@@ -267,6 +269,7 @@ void sim_destroy(Sim* S)
                     S->f_sqrtm, S->f_Dconc, S->f_fc, S->f_Mphi};
    for (float* v : fall) (void)hipFree(v);
    (void)hipFree(S->kks_acc);
+   (void)hipFree(S->kks_part);
    (void)hipFree(S->guess.list);
    (void)hipFree(S->guess.count);
    mg_destroy(S->mgf);
@@ -325,20 +328,22 @@ static int kks(Sim* S, const double* y)
       }
       g = S->guess;
    }
-   return launch_kks(*S->L, S->p, y, c, S->clr, S->csr, S->cl, S->cs, g, S->kks_acc, S->stream);
+   S->kks_calls++;
+   return launch_kks(*S->L, S->p, y, c, S->clr, S->csr, S->cl, S->cs, g, S->kks_part, S->stream);
 }
 
 // Read the KKS device counters into the stats; -1 if a cell failed.
 static int kks_collect(Sim* S)
 {
    if (S->ic < 0) return 0;
+   if (!S->tern && kks_finish(S->kks_part, S->kks_acc, S->stream)) return -1;
    AMPE_HIP_CHECK(hipMemcpyAsync(S->L->hpinned, S->kks_acc, sizeof(long long) * kKksAcc,
                                  hipMemcpyDeviceToHost, S->stream));
    AMPE_HIP_CHECK(hipStreamSynchronize(S->stream));
    long long h[kKksAcc];
    std::memcpy(h, S->L->hpinned, sizeof(h));
    S->st.kks_iters = h[0];
-   S->st.kks_calls = h[3];
+   S->st.kks_calls = S->kks_calls;
    S->st.kks_fallbacks = h[4];
    S->st.kks_surrogate_starts = h[5];
    S->st.kks_cells = S->st.kks_calls * S->L->ncg;
@@ -386,9 +391,11 @@ int sim_set_state(Sim* S, const double* phi, const double* c, const double* q)
       AMPE_HIP_CHECK(hipMemcpyAsync(S->csr, cc, sizeof(double) * S->ng,
                                     hipMemcpyDeviceToDevice, st));
       AMPE_HIP_CHECK(hipMemsetAsync(S->kks_acc, 0, sizeof(long long) * kKksAcc, st));
+      AMPE_HIP_CHECK(hipMemsetAsync(S->kks_part, 0, sizeof(double) * kKksPartDoubles, st));
       if (kks(S, S->y)) return -1;
       if (kks_collect(S)) return -1;
       std::memset(&S->st, 0, sizeof(S->st));
+      S->kks_calls = 0;
       AMPE_HIP_CHECK(hipMemsetAsync(S->kks_acc, 0, sizeof(long long) * kKksAcc, st));
    }
    S->t = 0.0;
@@ -420,9 +427,11 @@ int sim_set_state_composite(Sim* S, const double* y_host)
       AMPE_HIP_CHECK(hipMemcpyAsync(S->csr, cc, sizeof(double) * S->ng,
                                     hipMemcpyDeviceToDevice, st));
       AMPE_HIP_CHECK(hipMemsetAsync(S->kks_acc, 0, sizeof(long long) * kKksAcc, st));
+      AMPE_HIP_CHECK(hipMemsetAsync(S->kks_part, 0, sizeof(double) * kKksPartDoubles, st));
       if (kks(S, S->y)) return -1;
       if (kks_collect(S)) return -1;
       std::memset(&S->st, 0, sizeof(S->st));
+      S->kks_calls = 0;
       AMPE_HIP_CHECK(hipMemsetAsync(S->kks_acc, 0, sizeof(long long) * kKksAcc, st));
    }
    S->t = 0.0;
