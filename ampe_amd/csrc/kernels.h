@@ -181,6 +181,12 @@ struct RhsConst {
    double Dl, Ds;     // D_L0 exp(-Q_L/RT), D_S0 exp(-Q_S/RT)
 };
 RhsConst rhs_const(const ampe_model_params& p);
+// The constants of every level of a hierarchy (PatchDev::lev), so that one
+// launch covers all levels; rhs_lev: the same for each.
+struct RhsLev {
+   RhsConst k[4];
+};
+RhsLev rhs_lev(const ampe_model_params& p);
 
 // Index of face (i,j,k) of direction d of patch pd in a side field.
 __device__ __forceinline__ long long face_idx(const LevelArgs& a, const PatchDev& pd,
@@ -205,6 +211,26 @@ __device__ __forceinline__ long long int_idx(const CellPos& c)
 // ------------------------------------------------------------ launchers
 int launch_quat_grad(const Level& L, const ampe_model_params& p, const double* q,
                      double* gmod, double* face_norm2, hipStream_t s);
+// The faces' 1 / |grad q| (grad_normi of the face norm), and the face
+// coefficients from them.
+int launch_quat_gni(const Level& L, const ampe_model_params& p, const RhsLev& k, const double* q,
+                    double* gni, hipStream_t s);
+int launch_quat_face_coef_gni(const Level& L, const ampe_model_params& p, const double* phi,
+                              const double* gni, double* fc, hipStream_t s);
+// Phase and orientation right-hand sides, and the composition's (KKS form) with
+// conc, in one launch (rhs_all.hip): q null for no orientation, cl / cs null for
+// no composition; conc 0: none, 1: from the stored Dc and Dphi, 2: Dc and Dphi
+// formed and stored too.  rhs: the state vector's components, iq and ic the
+// orientation's and the composition's.
+int launch_rhs_all(const Level& L, const ampe_model_params& p, const RhsLev& k, const double* y,
+                   int iq, int ic, const double* cl, const double* cs, const double* gni,
+                   double* Dc, double* Dphi, int conc, double* rhs, hipStream_t s);
+int launch_conc_coeffs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
+                           const double* phi, const double* cl, const double* cs, double* Dc,
+                           double* Dphi, hipStream_t s);
+int launch_conc_rhs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
+                        const double* c, const double* phi, const double* Dc, const double* Dphi,
+                        double* rhs, hipStream_t s);
 int launch_phase_rhs(const Level& L, const ampe_model_params& p, const double* phi,
                      const double* q, const double* cl, const double* cs, double* rhs,
                      hipStream_t s);

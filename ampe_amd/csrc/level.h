@@ -42,6 +42,7 @@ struct PatchDev {
    long long side_off[3];  // patch faces offset inside direction block d
    long long int_off;      // compact interior offset (host I/O, tags)
    int lo[3];              // box lower corner (global index space)
+   int lev;                // level of a hierarchy's composite (0 otherwise)
    int physb;              // bit 2d / 2d+1: lower / upper side in direction d lies on a
                            // physical (non-periodic) boundary of the level's bounding box
 };
@@ -99,6 +100,7 @@ void level_destroy(Level* L);
 struct LevelPlacement {
    long long cell_base = 0, ncg_total = 0, int_base = 0, ncell_total = 0;
    long long side_base[3] = {0, 0, 0}, nside_total[3] = {0, 0, 0};
+   const int* patch_lev = nullptr;  // PatchDev::lev per patch (null: 0)
 };
 int level_create_placed(int ndim, const ampe_box* boxes, int npatch, const LevelPlacement& pl,
                         const std::vector<long long>& gd, const std::vector<long long>& gs,

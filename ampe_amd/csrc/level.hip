@@ -208,6 +208,7 @@ int level_create(int ndim, const ampe_box* boxes, int npatch, int ghost,
          delete L;
          return -1;
       }
+      d.lev = 0;
       d.nx = n[0];
       d.ny = n[1];
       d.nz = n[2];
@@ -353,6 +354,7 @@ int level_create_placed(int ndim, const ampe_box* boxes, int npatch, const Level
       d.int_off = ioff;
       ioff += (long long)n[0] * n[1] * n[2];
       d.physb = 0;
+      d.lev = pl.patch_lev ? pl.patch_lev[p] : 0;
       for (int a = 0; a < 3; a++) {
          d.side_off[a] = soff[a];
          if (a < ndim)

@@ -7,16 +7,13 @@
 // arrays, so each kernel reads its cell fields once and writes its outputs
 // once; the arithmetic of each face is the reference's, in its order.
 #include "kernels.h"
+#include "rhs_dev.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
 
 namespace ampe {
-
-// Single precision literal 1.e-12 of anisotropic_gradient_flux promoted to
-// double (source/fortran/2d/quatrhs.m4:193, 3d/quatrhs.m4:184).
-#define AMPE_ANISO_THRESHOLD ((double)1.e-12f)
 
 // Launch-uniform quantities derived from the model on the host: IEEE division
 // gives the device's value, and the kernels do no per-cell division or exp
@@ -39,95 +36,6 @@ RhsConst rhs_const(const ampe_model_params& p)
    k.Dl = p.D_liquid * std::exp(-(p.Q0_liquid / kRGas) * invT);
    k.Ds = p.D_solid * std::exp(-(p.Q0_solid / kRGas) * invT);
    return k;
-}
-
-// ------------------------------------------------------------ phase flux
-// Face between cells cm = c0 - st[d] and c0, direction d.
-// Simple: gradient_flux (source/fortran/2d/quatrhs.m4:12-53).
-// Isotropic (2-D): compute_flux_isotropic (2d/quatrhs.m4:106-151).
-// Anisotropic: anisotropic_gradient_flux (2d/quatrhs.m4:154-256,
-// 3d/quatrhs.m4:149-356).
-__device__ __forceinline__ void quatmult4(const double* a, const double* b, double* r)
-{
-   r[0] = a[0] * b[0] - a[1] * b[1] - a[2] * b[2] - a[3] * b[3];
-   r[1] = a[0] * b[1] + a[1] * b[0] + a[2] * b[3] - a[3] * b[2];
-   r[2] = a[0] * b[2] + a[2] * b[0] + a[3] * b[1] - a[1] * b[3];
-   r[3] = a[0] * b[3] + a[3] * b[0] + a[1] * b[2] - a[2] * b[1];
-}
-
-// FLUX < 0 reads p.flux_type at run time.
-template <int NDIM, int FLUX = -1>
-__device__ double phase_face_flux(const ampe_model_params& p, const RhsConst& k,
-                                  const double* __restrict__ ph, const double* __restrict__ q,
-                                  long long ncg, const long long* st, int d, long long cm,
-                                  long long c0)
-{
-   const int ft = (FLUX < 0) ? p.flux_type : FLUX;
-   if (ft == AMPE_FLUX_ANISOTROPIC) {
-      if (NDIM == 2) {
-         double eps = p.epsilon_phi, nu = p.aniso_nu;
-         int kn = p.aniso_knumber;
-         double pi = 4.0 * atan(1.0);
-         double dinv0 = k.dxinv[0], dinv1 = k.dxinv[1];
-         int t = 1 - d;  // transverse direction
-         double gn = (ph[c0] - ph[cm]) * (d == 0 ? dinv0 : dinv1);
-         double gt = 0.25 * (ph[cm + st[t]] - ph[cm - st[t]] + ph[c0 + st[t]] - ph[c0 - st[t]]) *
-                     (d == 0 ? dinv1 : dinv0);
-         double dphidx = (d == 0) ? gn : gt;
-         double dphidy = (d == 0) ? gt : gn;
-         double theta = (fabs(dphidx) > AMPE_ANISO_THRESHOLD) ? atan(dphidy / dphidx) : 0.5 * pi;
-         double qa = 0.5 * (q[cm] + q[c0]);
-         if (qa > 1.0) qa = 1.0;
-         if (qa < -1.0) qa = -1.0;
-         double phia = (p.qlen == 4) ? 2.0 * acos(qa) : acos(qa);
-         double epst = eps * (1.0 + nu * cos(kn * (theta - phia)));
-         double deps = -kn * eps * nu * sin(kn * (theta - phia));
-         if (d == 0) return epst * epst * dphidx - epst * deps * dphidy;
-         return epst * epst * dphidy + epst * deps * dphidx;
-      } else {
-         double eps = p.epsilon_phi, eps4 = p.aniso_nu;
-         const double* dinv = k.dxinv;
-         double factor = 4.0 * eps4 / (1.0 - 3.0 * eps4);
-         double gr[3];
-#pragma unroll
-         for (int e = 0; e < 3; e++) {
-            if (e == d)
-               gr[e] = (ph[c0] - ph[cm]) * dinv[e];
-            else
-               gr[e] = 0.25 * (ph[cm + st[e]] - ph[cm - st[e]] + ph[c0 + st[e]] - ph[c0 - st[e]]) *
-                       dinv[e];
-         }
-         double gphi2 = gr[0] * gr[0] + gr[1] * gr[1] + gr[2] * gr[2];
-         double dg[4], n4;
-         if (fabs(gphi2) > AMPE_ANISO_THRESHOLD) {
-            double nni = 1.0 / sqrt(gphi2);
-            double n[4] = {0.0, gr[0] * nni, gr[1] * nni, gr[2] * nni};
-            double qa[4];
-#pragma unroll
-            for (int m = 0; m < 4; m++) qa[m] = 0.5 * (q[m * ncg + cm] + q[m * ncg + c0]);
-            double qp[4] = {qa[0], -qa[1], -qa[2], -qa[3]}, tq[4], np[4];
-            quatmult4(n, qp, tq);
-            quatmult4(qa, tq, np);
-            double a1 = np[1] * np[1], a2 = np[2] * np[2], a3 = np[3] * np[3];
-            n4 = a1 * a1 + a2 * a2 + a3 * a3;
-            double dd[4] = {0.0, np[1] * (np[1] * np[1] - n4), np[2] * (np[2] * np[2] - n4),
-                            np[3] * (np[3] * np[3] - n4)};
-            quatmult4(dd, qa, tq);
-            quatmult4(qp, tq, dg);
-         } else {
-            dg[0] = dg[1] = dg[2] = dg[3] = 0.0;
-            n4 = 0.0;
-         }
-         double gamma = eps * (1.0 - 3.0 * eps4) * (1.0 + factor * n4);
-         return gamma * gamma * gr[d] + 16.0 * eps * gamma * eps4 * sqrt(gphi2) * dg[d + 1];
-      }
-   }
-   if (ft == AMPE_FLUX_ISOTROPIC && NDIM == 2) {
-      double dinv = k.e2dx12[d];
-      long long t = st[1 - d];
-      return dinv * ((ph[c0 - t] - ph[cm - t]) + (ph[c0] - ph[cm]) * 10.0 + (ph[c0 + t] - ph[cm + t]));
-   }
-   return (ph[c0] - ph[cm]) * k.e2dx[d];
 }
 
 // |grad q| from cell-centred gradients: quatdiffs -> quatgrad_cell ->
@@ -164,116 +72,153 @@ __global__ void __launch_bounds__(256) k_quat_modulus(LevelArgs a, ampe_model_pa
    gmod[c.c0] = quat_cell_modulus<NDIM>(p, k, q, a.ncg, c.st, c.c0);
 }
 
-// |grad q|^2 on faces from the full side gradient (quatgrad_side
-// 2d/quatgrad.m4:157-229, summed as compute_face_coef2d quatfacops.m4:83-92).
-// QL > 0: the component count as a compile-time constant (loops unrolled);
-// QL = 0 reads p.qlen.
-template <int NDIM, int QL = 0>
-__device__ __forceinline__ double quat_face_norm2(const ampe_model_params& p, const RhsConst& k,
-                                                  const double* __restrict__ q, long long ncg,
-                                                  const long long* st, int d, long long cm,
-                                                  long long c0)
-{
-   double s = 0.0;
-   const int ql = QL > 0 ? QL : p.qlen;
-#pragma unroll
-   for (int n = 0; n < NDIM; n++) {
-      double dinv = k.dxinv[n];
-      double p25 = 0.25 * dinv;
-#pragma unroll
-      for (int m = 0; m < ql; m++) {
-         const double* aa = q + m * ncg;
-         double gv;
-         if (n == d) {
-            gv = dinv * (aa[c0] - aa[cm]);
-         } else {
-            long long t = st[n];
-            gv = p25 * ((aa[cm + t] - aa[cm]) + (aa[cm] - aa[cm - t]) + (aa[c0 + t] - aa[c0]) +
-                        (aa[c0] - aa[c0 - t]));
-         }
-         s = s + gv * gv;
-      }
-   }
-   return s;
-}
-
-template <int NDIM, int QL>
+// GNI: store 1 / |grad q| of the face (grad_normi) instead of |grad q|^2.
+template <int NDIM, int QL, bool GNI>
 __global__ void __launch_bounds__(256) k_quat_face_norm2(LevelArgs a, ampe_model_params p,
-                                                         RhsConst k, const double* __restrict__ q,
+                                                         RhsLev kl, const double* __restrict__ q,
                                                          double* __restrict__ n2)
 {
    CellPos c;
    if (!cell_pos(a, 1, c)) return;
    if (NDIM == 2 && c.k > 0) return;
+   const RhsConst& k = kl.k[c.pd.lev];
    for (int d = 0; d < NDIM; d++) {
       bool ok = (c.i < c.pd.nx + (d == 0)) && (c.j < c.pd.ny + (d == 1)) &&
                 (NDIM == 2 || c.k < c.pd.nz + (d == 2));
       if (!ok) continue;
-      n2[face_idx(a, c.pd, d, c.i, c.j, c.k)] =
-          quat_face_norm2<NDIM, QL>(p, k, q, a.ncg, c.st, d, c.c0 - c.st[d], c.c0);
+      const double v = quat_face_norm2<NDIM, QL>(p, k, q, a.ncg, c.st, d, c.c0 - c.st[d], c.c0);
+      n2[face_idx(a, c.pd, d, c.i, c.j, c.k)] = GNI ? face_gni(p, k, v) : v;
    }
 }
 
-// The same face norms in 3-D with the workgroup's q values staged in LDS: the
-// tile's cells grown by one in each direction (planes k-1, k, k+1) are read
-// once, coalesced along i, and every face of the tile takes its values from
-// LDS in quat_face_norm2's order (the global-memory form reads up to ten
-// neighbours per component per face).  Halo cells outside the ghost box are
-// only needed by faces that do not exist; they are set to zero.
-template <int QL>
-__global__ void __launch_bounds__(256) k_quat_face_norm2_lds(LevelArgs a, ampe_model_params p,
-                                                             RhsConst k,
-                                                             const double* __restrict__ q,
-                                                             double* __restrict__ n2)
+// The same in 3-D for four components.  A workgroup marches up a column of KM
+// planes of its tile: four planes of the tile's q with a one-cell halo sit in
+// LDS (k - 1, k, k + 1 and the one being loaded), so that each value is read
+// once, and a cell's centred differences serve all its faces: across a face
+// between cells A and B the transverse gradient is (D(A) + D(B)) / 4h with D(c)
+// = q(c + 1) - q(c - 1).  A thread evaluates its cell's low faces, the last cell
+// of a row, column or stack the high one too.  256^3: 413 us (56 bytes a cell,
+// 2.3 TB/s; bound by the LDS reads and the square root and division of each
+// face at three workgroups a CU); 681 us with three planes loaded per plane and
+// ten neighbour values per component and face.
+template <bool GNI>
+__global__ void __launch_bounds__(256) k_quat_face_norm2_march(LevelArgs a, ampe_model_params p,
+                                                               RhsLev kl,
+                                                               const double* __restrict__ q,
+                                                               double* __restrict__ n2)
 {
-   constexpr int HX = TX + 2, HY = TY + 2;
-   __shared__ double sq[QL][3][HY][HX];
+   constexpr int QL = 4, HX = TX + 2, HY = TY + 2, NH = HX * HY;
+   __shared__ double sq[4][QL][HY][HX];
    const Tile t = a.T[tile_index(a)];
    const PatchDev pd = a.P[t.patch];
+   const RhsConst& k = kl.k[pd.lev];
    const int tid = (int)threadIdx.y * TX + (int)threadIdx.x;
-   for (int e = tid; e < 3 * HY * HX; e += TX * TY) {
-      const int ii = e % HX, r = e / HX;
-      const int jj = r % HY, kk = r / HY;
-      const int ci = t.i0 - 1 + ii, cj = t.j0 - 1 + jj, ck = t.k - 1 + kk;
-      const bool ok = ci >= -a.g && ci < pd.nx + a.g && cj >= -a.g && cj < pd.ny + a.g &&
-                      ck >= -a.gz && ck < pd.nz + a.gz;
-      const long long idx = pd.cell_off + (ci + a.g) + (long long)(cj + a.g) * pd.sy +
-                            (long long)(ck + a.gz) * pd.sz;
+   // the (at most two) halo-tile positions this thread loads, in every plane
+   long long off[2];
+   int hx[2], hy[2];
+   bool ok[2];
 #pragma unroll
-      for (int m = 0; m < QL; m++) sq[m][kk][jj][ii] = ok ? q[m * a.ncg + idx] : 0.0;
+   for (int r = 0; r < 2; r++) {
+      const int e = tid + r * TX * TY;
+      hx[r] = e % HX;
+      hy[r] = e / HX;
+      const int ci = t.i0 - 1 + hx[r], cj = t.j0 - 1 + hy[r];
+      ok[r] = e < NH && ci < pd.nx + a.g && cj < pd.ny + a.g;
+      off[r] = pd.cell_off + (ci + a.g) + (long long)(cj + a.g) * pd.sy;
    }
-   __syncthreads();
-   const int i = t.i0 + (int)threadIdx.x, j = t.j0 + (int)threadIdx.y, kc = t.k;
-   if (i >= pd.nx + 1 || j >= pd.ny + 1) return;
-   const int x0 = (int)threadIdx.x + 1, y0 = (int)threadIdx.y + 1;
+   const int kend = min(t.k + a.nz_tile, pd.nz);  // one past the column's last plane
+   double v[2][QL];
+   auto fetch = [&](int kc) {
 #pragma unroll
-   for (int d = 0; d < 3; d++) {
-      const bool ok = (i < pd.nx + (d == 0)) && (j < pd.ny + (d == 1)) && (kc < pd.nz + (d == 2));
-      if (!ok) continue;
-      // cm = the cell across the low face of direction d
-      const int mx = x0 - (d == 0), my = y0 - (d == 1), mz = 1 - (d == 2);
-      double s = 0.0;
+      for (int r = 0; r < 2; r++) {
+         const long long o = off[r] + (long long)(kc + a.gz) * pd.sz;
 #pragma unroll
-      for (int n = 0; n < 3; n++) {
-         const double dinv = k.dxinv[n];
-         const double p25 = 0.25 * dinv;
-         const int tx = (n == 0), ty = (n == 1), tz = (n == 2);
-#pragma unroll
-         for (int m = 0; m < QL; m++) {
-            const double c0v = sq[m][1][y0][x0], cmv = sq[m][mz][my][mx];
-            double gv;
-            if (n == d) {
-               gv = dinv * (c0v - cmv);
-            } else {
-               gv = p25 * ((sq[m][mz + tz][my + ty][mx + tx] - cmv) +
-                           (cmv - sq[m][mz - tz][my - ty][mx - tx]) +
-                           (sq[m][1 + tz][y0 + ty][x0 + tx] - c0v) +
-                           (c0v - sq[m][1 - tz][y0 - ty][x0 - tx]));
-            }
-            s = s + gv * gv;
-         }
+         for (int m = 0; m < QL; m++) v[r][m] = ok[r] ? q[m * a.ncg + o] : 0.0;
       }
-      n2[face_idx(a, pd, d, i, j, kc)] = s;
+   };
+   auto put = [&](int kc) {
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+         if (ok[r])
+#pragma unroll
+            for (int m = 0; m < QL; m++) sq[kc & 3][m][hy[r]][hx[r]] = v[r][m];
+   };
+   // planes kc - 1 .. kc + 1 (planes are numbered from -1; & 3 of -1 is 3)
+   for (int kc = t.k - 1; kc <= t.k + 1; kc++) {
+      fetch(kc);
+      put(kc);
+   }
+   const int i = t.i0 + (int)threadIdx.x, j = t.j0 + (int)threadIdx.y;
+   const bool in = i < pd.nx && j < pd.ny;
+   const int x = (int)threadIdx.x + 1, y = (int)threadIdx.y + 1;
+   const double dx = k.dxinv[0], dy = k.dxinv[1], dz = k.dxinv[2];
+   const double qx = 0.25 * dx, qy = 0.25 * dy, qz = 0.25 * dz;
+   for (int kc = t.k; kc < kend; kc++) {
+      __syncthreads();
+      const int P0 = (kc - 1) & 3, P1 = kc & 3, P2 = (kc + 1) & 3;
+      const bool more = kc + 1 < kend;
+      if (more) fetch(kc + 2);  // in flight while this plane is worked on
+      if (in) {
+         // face between cells A (x - ex, y - ey, plane PA) and B (x, y, plane PB)
+         auto store = [&](int d, int ii, int jj, int kk, double s) {
+            n2[face_idx(a, pd, d, ii, jj, kk)] = GNI ? face_gni(p, k, s) : s;
+         };
+         auto xface = [&](int xb) {
+            double s = 0.0;
+#pragma unroll
+            for (int m = 0; m < QL; m++) {
+               const auto& c = sq[P1][m];
+               const double g0 = dx * (c[y][xb] - c[y][xb - 1]);
+               const double g1 = qy * ((c[y + 1][xb - 1] - c[y - 1][xb - 1]) +
+                                       (c[y + 1][xb] - c[y - 1][xb]));
+               const double g2 = qz * ((sq[P2][m][y][xb - 1] - sq[P0][m][y][xb - 1]) +
+                                       (sq[P2][m][y][xb] - sq[P0][m][y][xb]));
+               s += g0 * g0;
+               s += g1 * g1;
+               s += g2 * g2;
+            }
+            return s;
+         };
+         auto yface = [&](int yb) {
+            double s = 0.0;
+#pragma unroll
+            for (int m = 0; m < QL; m++) {
+               const auto& c = sq[P1][m];
+               const double g0 = qx * ((c[yb - 1][x + 1] - c[yb - 1][x - 1]) +
+                                       (c[yb][x + 1] - c[yb][x - 1]));
+               const double g1 = dy * (c[yb][x] - c[yb - 1][x]);
+               const double g2 = qz * ((sq[P2][m][yb - 1][x] - sq[P0][m][yb - 1][x]) +
+                                       (sq[P2][m][yb][x] - sq[P0][m][yb][x]));
+               s += g0 * g0;
+               s += g1 * g1;
+               s += g2 * g2;
+            }
+            return s;
+         };
+         auto zface = [&](int PA, int PB) {
+            double s = 0.0;
+#pragma unroll
+            for (int m = 0; m < QL; m++) {
+               const auto& A = sq[PA][m];
+               const auto& B = sq[PB][m];
+               const double g0 = qx * ((A[y][x + 1] - A[y][x - 1]) + (B[y][x + 1] - B[y][x - 1]));
+               const double g1 = qy * ((A[y + 1][x] - A[y - 1][x]) + (B[y + 1][x] - B[y - 1][x]));
+               const double g2 = dz * (B[y][x] - A[y][x]);
+               s += g0 * g0;
+               s += g1 * g1;
+               s += g2 * g2;
+            }
+            return s;
+         };
+         store(0, i, j, kc, xface(x));
+         store(1, i, j, kc, yface(y));
+         store(2, i, j, kc, zface(P0, P1));
+         if (i == pd.nx - 1) store(0, i + 1, j, kc, xface(x + 1));
+         if (j == pd.ny - 1) store(1, i, j + 1, kc, yface(y + 1));
+         if (kc == pd.nz - 1) store(2, i, j, kc + 1, zface(P1, P2));
+      }
+      // its slot held plane kc - 2, which no wave reads any more
+      if (more) put(kc + 2);
    }
 }
 
@@ -284,7 +229,6 @@ __global__ void __launch_bounds__(256) k_quat_face_norm2_lds(LevelArgs a, ampe_m
 // :393-511 / CALPHADFreeEnergyStrategyBinary.cc:521-651), times M_phi.
 // Specialised on the flux type FLUX and the free-energy model FE (kFeNone: no
 // composition field) so that each instance holds only its own path's registers.
-constexpr int kFeNone = 3;
 
 template <int NDIM, int FE>
 __device__ __forceinline__ void phase_rhs_tail(const LevelArgs& a, const ampe_model_params& p,
@@ -340,19 +284,8 @@ __device__ __forceinline__ void phase_rhs_tail(const LevelArgs& a, const ampe_mo
    }
    double mob = p.phi_mobility;
    if (FE != kFeNone) {
-      double convL = k.convL, convA = k.convA;
-      double c_l = cl[c0], c_a = cs[c0];
-      double hp = dinterp(ph, p.energy_interp);
-      if (FE == AMPE_FE_CALPHAD_BINARY && convL == convA) {
-         r += hp * (calphad_drive(p.calphad, p.temperature, c_l, c_a) * convL);
-      } else {
-         double f_l = fenergy_t<FE>(p, c_l, 0) * convL;
-         double f_a = fenergy_t<FE>(p, c_a, 1) * convA;
-         double mu = (FE == AMPE_FE_QUADRATIC) ? dfenergy_t<FE>(p, c_l, 0) * convL
-                                               : dfenergy_t<FE>(p, c_a, 1) * convA;
-         r += hp * ((f_l - f_a) - mu * (c_l - c_a));
-      }
-      if (p.phi_mobility_type == AMPE_PHI_MOB_KIM) mob = phase_mobility_t<FE>(p, c_l, c_a);
+      r += phase_drive<FE>(p, k, ph, cl[c0], cs[c0]);
+      if (p.phi_mobility_type == AMPE_PHI_MOB_KIM) mob = phase_mobility_t<FE>(p, cl[c0], cs[c0]);
    }
    rhs[c0] = mob * r;
 }
@@ -441,22 +374,6 @@ __global__ void __launch_bounds__(256) k_phase_rhs_faces(LevelArgs a, ampe_model
 }
 
 // ------------------------------------------------------------ quat RHS
-// compute_face_coef2d/3d (2d/quatfacops.m4:14-122) from the face |grad q|^2
-__device__ __forceinline__ double quat_face_coef(const ampe_model_params& p, const RhsConst& k,
-                                                 double phm, double ph0, double n2f)
-{
-   double floor2 = p.gradient_floor * p.gradient_floor;
-   double maxgni = k.maxgni;
-   double eps2 = p.epsilon_q * p.epsilon_q;
-   double mf = 2.0 * p.H_parameter;
-   double phia = face_avg(phm, ph0, p.avg_type);
-   double tempa = 0.5 * (p.temperature + p.temperature);
-   double diff = mf * tempa * interp(phia, p.orient_interp1);
-   double hphi2 = interp(phia, p.orient_interp2);
-   double gni = grad_normi(n2f, p.floor_type, floor2, maxgni);
-   return -gni * diff - eps2 * hphi2;
-}
-
 // QuatFACOps::evaluateRHS with use_gradq_for_flux and projection
 // (source/QuatFACOps.cc:1861-1890, 2089-2108): flux = fc dq/dh
 // (compute_flux2d_from_gradq), lambda (compute_lambda_flux2d/3d),
@@ -547,10 +464,8 @@ __global__ void __launch_bounds__(256) k_quat_project(LevelArgs a, int ql,
 }
 
 // ------------------------------------------------------------ composition
-// concentration_pfmdiffusion (2d/concentrationdiffusion.m4:14-96) and
-// setDiffCoeffForPhaseOnPatch (source/KKSCompositionRHSStrategy.cc:210-373)
 template <int NDIM>
-__global__ void __launch_bounds__(256) k_conc_coeffs(LevelArgs a, ampe_model_params p, RhsConst k,
+__global__ void __launch_bounds__(256) k_conc_coeffs(LevelArgs a, ampe_model_params p, RhsLev kl,
                                                      const double* __restrict__ phi,
                                                      const double* __restrict__ cl,
                                                      const double* __restrict__ cs,
@@ -560,29 +475,21 @@ __global__ void __launch_bounds__(256) k_conc_coeffs(LevelArgs a, ampe_model_par
    CellPos c;
    if (!cell_pos(a, 1, c)) return;
    if (NDIM == 2 && c.k > 0) return;
+   const RhsConst& k = kl.k[c.pd.lev];
    for (int d = 0; d < NDIM; d++) {
       bool ok = (c.i < c.pd.nx + (d == 0)) && (c.j < c.pd.ny + (d == 1)) &&
                 (NDIM == 2 || c.k < c.pd.nz + (d == 2));
       if (!ok) continue;
       long long c0 = c.c0, cm = c0 - c.st[d];
       long long fi = face_idx(a, c.pd, d, c.i, c.j, c.k);
-      double vphi = face_avg(phi[cm], phi[c0], p.avg_type);
-      double hphi = interp(vphi, p.energy_interp);
-      double dl = k.Dl, ds = k.Ds;
-      double dd = (1.0 - hphi) * dl + hphi * ds;
-      Dc[fi] = dd;
-      double ph = face_avg(phi[c0], phi[cm], p.avg_type);
-      double c_l = 0.5 * (cl[c0] + cl[cm]);
-      double c_a = 0.5 * (cs[c0] + cs[cm]);
-      double hp = dinterp(ph, p.energy_interp);
-      Dphi[fi] = dd * hp * (c_l - c_a);
+      conc_face_coeffs(p, k, phi[cm], phi[c0], cl[cm], cl[c0], cs[cm], cs[c0], Dc[fi], Dphi[fi]);
    }
 }
 
 // concentrationflux (2d/concentrationrhs.m4:15-82) + computerhsconcentration
 // (2d/concentrationrhs.m4:326-367)
 template <int NDIM>
-__global__ void __launch_bounds__(256) k_conc_rhs(LevelArgs a, ampe_model_params p, RhsConst k,
+__global__ void __launch_bounds__(256) k_conc_rhs(LevelArgs a, ampe_model_params p, RhsLev kl,
                                                   const double* __restrict__ cc,
                                                   const double* __restrict__ phi,
                                                   const double* __restrict__ Dc,
@@ -590,6 +497,7 @@ __global__ void __launch_bounds__(256) k_conc_rhs(LevelArgs a, ampe_model_params
                                                   double* __restrict__ rhs)
 {
    AMPE_COLUMN_BEGIN(a, c)
+   const RhsConst& k = kl.k[c.pd.lev];
    const long long c0 = c.c0;
    const int ijk[3] = {c.i, c.j, c.k};
    double s = 0.0;
@@ -905,25 +813,43 @@ static dim3 tile_block() { return dim3(TX, TY); }
       AMPE_HIP_CHECK(hipGetLastError());                                       \
    } while (0)
 
+RhsLev rhs_lev(const ampe_model_params& p)
+{
+   RhsLev l;
+   l.k[0] = l.k[1] = l.k[2] = l.k[3] = rhs_const(p);
+   return l;
+}
+
+template <bool GNI>
+static int quat_face_norms(const Level& L, const ampe_model_params& p, const RhsLev& k,
+                           const double* q, double* n2, hipStream_t s)
+{
+   dim3 g(L.nface_tiles), b = tile_block();
+   LevelArgs a = level_args(L, true);
+   if (L.ndim == 3 && p.qlen == 4)
+      hipLaunchKernelGGL(k_quat_face_norm2_march<GNI>, dim3(L.nmarch_tiles), b, 0, s,
+                         level_args_march(L), p, k, q, n2);
+   else if (L.ndim == 3)
+      hipLaunchKernelGGL((k_quat_face_norm2<3, 0, GNI>), g, b, 0, s, a, p, k, q, n2);
+   else if (p.qlen == 4)
+      hipLaunchKernelGGL((k_quat_face_norm2<2, 4, GNI>), g, b, 0, s, a, p, k, q, n2);
+   else
+      hipLaunchKernelGGL((k_quat_face_norm2<2, 0, GNI>), g, b, 0, s, a, p, k, q, n2);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
 int launch_quat_grad(const Level& L, const ampe_model_params& p, const double* q,
                      double* gmod, double* face_norm2, hipStream_t s)
 {
    if (gmod) AMPE_DISPATCH(L, k_quat_modulus, L.ncell_tiles, level_args(L), p, rhs_const(p), q, gmod);
-   if (face_norm2) {
-      dim3 g(L.nface_tiles), b = tile_block();
-      LevelArgs a = level_args(L, true);
-      RhsConst k = rhs_const(p);
-      if (L.ndim == 3 && p.qlen == 4)
-         hipLaunchKernelGGL((k_quat_face_norm2_lds<4>), g, b, 0, s, a, p, k, q, face_norm2);
-      else if (L.ndim == 3)
-         hipLaunchKernelGGL((k_quat_face_norm2<3, 0>), g, b, 0, s, a, p, k, q, face_norm2);
-      else if (p.qlen == 4)
-         hipLaunchKernelGGL((k_quat_face_norm2<2, 4>), g, b, 0, s, a, p, k, q, face_norm2);
-      else
-         hipLaunchKernelGGL((k_quat_face_norm2<2, 0>), g, b, 0, s, a, p, k, q, face_norm2);
-      AMPE_HIP_CHECK(hipGetLastError());
-   }
-   return 0;
+   return face_norm2 ? quat_face_norms<false>(L, p, rhs_lev(p), q, face_norm2, s) : 0;
+}
+
+int launch_quat_gni(const Level& L, const ampe_model_params& p, const RhsLev& k, const double* q,
+                    double* gni, hipStream_t s)
+{
+   return quat_face_norms<true>(L, p, k, q, gni, s);
 }
 
 template <int NDIM, int FLUX>
@@ -1037,11 +963,26 @@ int launch_quat_project(const Level& L, const ampe_model_params& p, const double
    return 0;
 }
 
+int launch_conc_coeffs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
+                           const double* phi, const double* cl, const double* cs, double* Dc,
+                           double* Dphi, hipStream_t s)
+{
+   AMPE_DISPATCH(L, k_conc_coeffs, L.nface_tiles, level_args(L, true), p, k, phi, cl, cs, Dc, Dphi);
+   return 0;
+}
+
 int launch_conc_coeffs(const Level& L, const ampe_model_params& p, const double* phi,
                        const double* cl, const double* cs, double* Dc, double* Dphi,
                        hipStream_t s)
 {
-   AMPE_DISPATCH(L, k_conc_coeffs, L.nface_tiles, level_args(L, true), p, rhs_const(p), phi, cl, cs, Dc, Dphi);
+   return launch_conc_coeffs_lev(L, p, rhs_lev(p), phi, cl, cs, Dc, Dphi, s);
+}
+
+int launch_conc_rhs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
+                        const double* c, const double* phi, const double* Dc, const double* Dphi,
+                        double* rhs, hipStream_t s)
+{
+   AMPE_DISPATCH(L, k_conc_rhs, L.ncol_tiles, level_args_col(L), p, k, c, phi, Dc, Dphi, rhs);
    return 0;
 }
 
@@ -1049,8 +990,7 @@ int launch_conc_rhs(const Level& L, const ampe_model_params& p, const double* c,
                     const double* phi, const double* Dc, const double* Dphi, double* rhs,
                     hipStream_t s)
 {
-   AMPE_DISPATCH(L, k_conc_rhs, L.ncol_tiles, level_args_col(L), p, rhs_const(p), c, phi, Dc, Dphi, rhs);
-   return 0;
+   return launch_conc_rhs_lev(L, p, rhs_lev(p), c, phi, Dc, Dphi, rhs, s);
 }
 
 int launch_ebs_coeffs(const Level& L, const ampe_model_params& p, const double* phi, double* DL,
@@ -1112,7 +1052,8 @@ namespace ampe {
 // Face coefficients of the orientation operator on every face (used by the
 // preconditioner; QuatFACOps::setOperatorCoefficients,
 // source/QuatFACOps.cc:735-829).
-template <int NDIM>
+// GNI: n2 holds the faces' 1 / |grad q|.
+template <int NDIM, bool GNI>
 __global__ void __launch_bounds__(256) k_quat_face_coef(LevelArgs a, ampe_model_params p, RhsConst k,
                                                         const double* __restrict__ phi,
                                                         const double* __restrict__ n2,
@@ -1126,7 +1067,8 @@ __global__ void __launch_bounds__(256) k_quat_face_coef(LevelArgs a, ampe_model_
                 (NDIM == 2 || c.k < c.pd.nz + (d == 2));
       if (!ok) continue;
       long long fi = face_idx(a, c.pd, d, c.i, c.j, c.k);
-      fc[fi] = quat_face_coef(p, k, phi[c.c0 - c.st[d]], phi[c.c0], n2[fi]);
+      const double pm = phi[c.c0 - c.st[d]], p0 = phi[c.c0];
+      fc[fi] = GNI ? quat_face_coef_gni(p, pm, p0, n2[fi]) : quat_face_coef(p, k, pm, p0, n2[fi]);
    }
 }
 
@@ -1143,7 +1085,28 @@ __global__ void __launch_bounds__(256) k_sqrt_quat_mobility(long long n, ampe_mo
 int launch_quat_face_coef(const Level& L, const ampe_model_params& p, const double* phi,
                           const double* n2, double* fc, hipStream_t s)
 {
-   AMPE_DISPATCH(L, k_quat_face_coef, L.nface_tiles, level_args(L, true), p, rhs_const(p), phi, n2, fc);
+   const dim3 g(L.nface_tiles), b = tile_block();
+   const LevelArgs a = level_args(L, true);
+   const RhsConst k = rhs_const(p);
+   if (L.ndim == 3)
+      hipLaunchKernelGGL((k_quat_face_coef<3, false>), g, b, 0, s, a, p, k, phi, n2, fc);
+   else
+      hipLaunchKernelGGL((k_quat_face_coef<2, false>), g, b, 0, s, a, p, k, phi, n2, fc);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
+int launch_quat_face_coef_gni(const Level& L, const ampe_model_params& p, const double* phi,
+                              const double* gni, double* fc, hipStream_t s)
+{
+   const dim3 g(L.nface_tiles), b = tile_block();
+   const LevelArgs a = level_args(L, true);
+   const RhsConst k = rhs_const(p);
+   if (L.ndim == 3)
+      hipLaunchKernelGGL((k_quat_face_coef<3, true>), g, b, 0, s, a, p, k, phi, gni, fc);
+   else
+      hipLaunchKernelGGL((k_quat_face_coef<2, true>), g, b, 0, s, a, p, k, phi, gni, fc);
+   AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
 

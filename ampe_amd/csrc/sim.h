@@ -58,7 +58,7 @@ struct Sim {
    // phase concentrations and their per-step Newton guesses (ghosted)
    double *cl = nullptr, *cs = nullptr, *clr = nullptr, *csr = nullptr;
    // lagged face data and preconditioner coefficients
-   double *n2 = nullptr, *Dc = nullptr, *Dphi = nullptr, *Dconc = nullptr, *fc = nullptr;
+   double *gni = nullptr, *Dc = nullptr, *Dphi = nullptr, *Dconc = nullptr, *fc = nullptr;
    double* fcq = nullptr;  // orientation face coefficients of the current RHS evaluation
    double *Cphi = nullptr, *sqrtm = nullptr, *Mphi = nullptr;
    double* phid = nullptr;  // phase field of the EBS isotropic stencil's diffusivities

@@ -170,7 +170,7 @@ static int sim_finish(Sim* S, Sim** out)
    rc |= dalloc(&S->fac_u, S->ng * ql);
    rc |= dalloc(&S->fac_e, S->nv);
    rc |= dalloc(&S->fac_r, S->nv);
-   double** sides[] = {&S->n2, &S->Dc, &S->Dphi, &S->Dconc, &S->fc, &S->fcq};
+   double** sides[] = {&S->gni, &S->Dc, &S->Dphi, &S->Dconc, &S->fc, &S->fcq};
    for (auto v : sides) rc |= dalloc(v, S->nf);
    if (S->tern) {
       rc |= dalloc(&S->ph6, 6 * S->ng);
@@ -260,7 +260,7 @@ void sim_destroy(Sim* S)
    double* all[] = {S->y, S->yprev, S->ypred, S->ycur, S->ahist, S->fcur, S->b, S->del,
                     S->ewt, S->work, S->work2, S->jv, S->xk, S->corr, S->acor, S->cl, S->cs,
                     S->clr, S->csr, S->Cphi, S->sqrtm, S->Mphi, S->fac_u, S->fac_e, S->fac_r,
-                    S->n2,
+                    S->gni,
                     S->Dc, S->Dphi, S->Dconc, S->fc, S->fcq, S->phid, S->z1, S->z2,
                     S->ph6, S->Db};
    for (double* v : all) (void)hipFree(v);
@@ -537,10 +537,10 @@ static int hier_rhs_eval(Sim* S, double* y, double* ydot, bool fd)
                                 ydot + (long long)S->ic * S->ng, st);
    }
    if (S->nord > 1) return hier_phase_rhs_multiorder(*S->hier, p, S->nord, phi, ydot, st);
-   if (q && recompute && hier_quat_face_norm2(*S->hier, p, q, S->n2, st)) return -1;
+   if (q && recompute && hier_quat_face_norm2(*S->hier, p, q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
    if (hier_phase_rhs(*S->hier, p, phi, q, S->cl, S->cs, ydot, st)) return -1;
-   if (q && hier_quat_rhs(*S->hier, p, phi, q, S->n2, S->fcq, ydot + (long long)S->iq * S->ng,
+   if (q && hier_quat_rhs(*S->hier, p, phi, q, S->gni, S->fcq, ydot + (long long)S->iq * S->ng,
                           st))
       return -1;
    if (c) {
@@ -563,12 +563,12 @@ static int hier_psetup(Sim* S, double* y, double gamma)
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
-   if (q && hier_quat_face_norm2(*S->hier, p, q, S->n2, st)) return -1;
+   if (q && hier_quat_face_norm2(*S->hier, p, q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
    // several orders: the well scale passed is 0, so C = 1
    ampe_model_params pw = p;
    if (S->nord > 1) pw.phi_well_scale = 0.0;
-   if (hier_precond_coeffs(*S->hier, pw, gamma, phi, S->cl, S->cs, S->n2, S->Mphi, S->Cphi,
+   if (hier_precond_coeffs(*S->hier, pw, gamma, phi, S->cl, S->cs, S->gni, S->Mphi, S->Cphi,
                            q ? S->fc : nullptr, q ? S->sqrtm : nullptr, st))
       return -1;
    if (c && S->tern) {
@@ -803,14 +803,14 @@ static int rhs_eval(Sim* S, double* y, double* ydot, bool fd)
                                   ydot + (long long)S->ic * S->ng, st);
    }
    if (S->nord > 1) return launch_phase_rhs_multiorder(L, p, S->nord, phi, nullptr, ydot, st);
-   if (q && recompute && launch_quat_grad(L, p, q, nullptr, S->n2, st)) return -1;
+   const RhsLev k = rhs_lev(p);
+   if (q && recompute && launch_quat_gni(L, p, k, q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
-   if (launch_phase_rhs(L, p, phi, q, S->cl, S->cs, ydot, st)) return -1;
-   // face coefficients once per face, then the orientation RHS from them
-   if (q && launch_quat_face_coef(L, p, phi, S->n2, S->fcq, st)) return -1;
-   if (q && launch_quat_rhs_fc(L, p, phi, q, S->fcq, ydot + (long long)S->iq * S->ng, st))
+   const bool ebs = c && p.conc_rhs_form == AMPE_CONC_RHS_EBS;
+   if (launch_rhs_all(L, p, k, y, S->iq, S->ic, S->cl, S->cs, S->gni, S->Dc, S->Dphi,
+                      !c || ebs ? 0 : (recompute ? 2 : 1), ydot, st))
       return -1;
-   if (c && p.conc_rhs_form == AMPE_CONC_RHS_EBS) {
+   if (ebs) {
       // Dc, Dphi hold the liquid and solid face diffusivities
       if (recompute) {
          if (p.conc_diffusion_type == AMPE_CONC_DIFF_COMPOSITION) {
@@ -837,10 +837,6 @@ static int rhs_eval(Sim* S, double* y, double* ydot, bool fd)
                                      ydot + (long long)S->ic * S->ng, st)) {
          return -1;
       }
-   } else if (c) {
-      if (recompute && launch_conc_coeffs(L, p, phi, S->cl, S->cs, S->Dc, S->Dphi, st)) return -1;
-      if (launch_conc_rhs(L, p, c, phi, S->Dc, S->Dphi, ydot + (long long)S->ic * S->ng, st))
-         return -1;
    }
    return 0;
 }
@@ -857,7 +853,7 @@ static int psetup(Sim* S, double* y, double gamma)
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
-   if (q && launch_quat_grad(L, p, q, nullptr, S->n2, st)) return -1;
+   if (q && launch_quat_gni(L, p, rhs_lev(p), q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
    // phase block: C = 1 + gamma M w g'' (source/PhaseFACOps.cc:33-51)
    // phase mobility after the phase concentrations (QuatIntegrator::
@@ -883,7 +879,7 @@ static int psetup(Sim* S, double* y, double gamma)
    }
    // orientation block (source/QuatFACOps.cc:735-829)
    if (q) {
-      if (launch_quat_face_coef(L, p, phi, S->n2, S->fc, st)) return -1;
+      if (launch_quat_face_coef_gni(L, p, phi, S->gni, S->fc, st)) return -1;
       if (launch_sqrt_quat_mobility(L, p, phi, S->sqrtm, st)) return -1;
    }
    if (S->s.precision == AMPE_FAC_FP32) {
