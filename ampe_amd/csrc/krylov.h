@@ -8,67 +8,57 @@ namespace ampe {
 
 constexpr int kMaxKrylov = 32;
 
-// FP32 preconditioner right-hand side written next to a Krylov vector r:
-// f = r, orientation components [iq, iq + ql) divided by sqrt(M) = sm
-// (f == nullptr: none).
+// How a preconditioner right-hand side r is written: the orientation components
+// [iq, iq + ql) divided by sqrt(M) = sm (null: none), and with f in FP32 to f.
 struct PrecIn {
    float* f = nullptr;
    const double* sm = nullptr;
    int iq = 0, ql = 0;
-   int sp0 = 1 << 30;  // components from sp0 on are in the row parity-split layout
+   int sp0 = 1 << 30;  // components of f from sp0 on are in the row parity-split layout
 };
 
-// A Krylov vector read from the FP32 preconditioner solution u: v = ewt u,
-// orientation components multiplied by sm first (u == nullptr: read v).
+// A preconditioned vector as the solve left it: FP32 u, or FP64 z; orientation
+// components to be multiplied by sm (null: none).
 struct PrecOut {
    const float* u = nullptr;
+   const double* z = nullptr;
    const double* sm = nullptr;
-   const double* ewt = nullptr;
    int iq = 0, ql = 0;
-   int sp0 = 1 << 30;  // components from sp0 on are in the row parity-split layout
+   int sp0 = 1 << 30;  // components of u from sp0 on are in the row parity-split layout
 };
 
+// Basis vectors (not scaled by ewt, not normalised) and a factor for each.
 struct VecList {
    int n;
    const double* v[kMaxKrylov];
    double y[kMaxKrylov];
 };
 
-int kry_prep(const Level& L, int nc, double hinv, double* V, const double* ewt, double* xk,
-             double* sumsq, hipStream_t s);
-int kry_mid(const Level& L, int nc, double sig, const double* xk, const double* ycur,
+// work2 = sig (z h) + ycur
+int kry_mid(const Level& L, int nc, double sig, const double* z, double h, const double* ycur,
             double* work2, hipStream_t s);
-// The same with the direction (V h) / ewt computed on the fly from an
-// unnormalised basis vector V and its scale h (no xk array).
-int kry_mid_scaled(const Level& L, int nc, double sig, const double* V, double h,
-                   const double* ewt, const double* ycur, double* work2, hipStream_t s);
-// (out may be null when pin.f receives the FP32 preconditioner input.)
-int kry_finish_scaled(const Level& L, int nc, double siginv, double gamma, const double* V,
-                      double h, const double* ewt, const double* jv, const double* fcur,
-                      double* out, const PrecIn& pin, hipStream_t s);
-int kry_finish(const Level& L, int nc, double siginv, double gamma, const double* xk,
-               const double* jv, const double* fcur, double* out, hipStream_t s);
-int kry_scale_dot(const Level& L, int nc, const double* ewt, const double* work, double* out,
-                  const double* other, double* dot, hipStream_t s);
-int kry_mgs(const Level& L, int nc, double* w, const double* Vi, double h, const double* Vnext,
-            double* dot, hipStream_t s);
-int kry_lincomb(const Level& L, int nc, const VecList& vl, const double* ewt, double* x,
-                hipStream_t s);
+// v = z h + (-gamma) (siginv jv + (-siginv) fcur), written as pin says; with
+// pin.f out may be null.
+int kry_finish(const Level& L, int nc, double siginv, double gamma, const double* z, double h,
+               const double* jv, const double* fcur, double* out, const PrecIn& pin,
+               hipStream_t s);
+// b = gamma f - (y - a), written as pin says (out may be null with pin.f).
 int kry_newton_rhs(const Level& L, int nc, double gamma, const double* f, const double* y,
-                   const double* ah, double* b, hipStream_t s);
-// Classical Gram-Schmidt (at most kMaxCgs dots per pass, so maxl <= 14).
+                   const double* ah, double* out, const PrecIn& pin, hipStream_t s);
+// z = src, *sumsq = (ewt z) . (ewt z)
+int kry_start(const Level& L, int nc, const PrecOut& src, const double* ewt, double* z,
+              double* sumsq, hipStream_t s);
+// z = src orthogonalised against the vectors of vl (vl.y: their normalisation
+// factors) by classical (at most kMaxCgs - 1 vectors) or modified Gram-Schmidt in
+// the ewt-weighted product.  sums[k] = src . v[k] of the products taken,
+// sums[vl.n] = z . z, and with classical sums[vl.n + 1] = src . src.
 constexpr int kMaxCgs = 16;
-// out = ewt * work (ewt != null) or out as is; sums[k] = out . vl.v[k]
-// (k < vl.n) and sums[vl.n] = out . out, one pass and one synchronisation.
-int kry_cgs_dots(const Level& L, int nc, const double* ewt, const double* work, double* out,
-                 const VecList& vl, double* sums, hipStream_t s);
-// The same with out = ewt u formed from the FP32 preconditioner solution.
-int kry_cgs_dots_from(const Level& L, int nc, const PrecOut& src, double* out,
-                      const VecList& vl, double* sums, hipStream_t s);
-// w = w + sum_k vl.y[k] vl.v[k] (k in order); *sumsq = w . w.
-int kry_cgs_update(const Level& L, int nc, double* w, const VecList& vl, double* sumsq,
-                   hipStream_t s);
-int kry_newton_update(const Level& L, int nc, const double* del, const double* ewt, double* y,
+int kry_cgs(const Level& L, int nc, const PrecOut& src, const VecList& vl, double cv,
+            const double* ewt, double* z, double* sums, hipStream_t s);
+int kry_mgs(const Level& L, int nc, const PrecOut& src, const VecList& vl, double cv,
+            const double* ewt, double* z, double* sums, hipStream_t s);
+// x = sum_k vl.y[k] vl.v[k] (k in order); y = y + x; *sumsq = (ewt x) . (ewt x)
+int kry_newton_update(const Level& L, int nc, const VecList& vl, const double* ewt, double* y,
                       double* sumsq, hipStream_t s);
 
 }  // namespace ampe

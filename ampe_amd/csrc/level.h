@@ -79,7 +79,7 @@ struct Level {
    long long* ghost_dst_s = nullptr;
    long long* ghost_src_s = nullptr;
    double* partial = nullptr;  // per-workgroup reduction partials (16 per tile)
-   double* dred = nullptr;     // reduction results (16 doubles)
+   double* dred = nullptr;     // reduction results (64 doubles)
    double* hpinned = nullptr;  // pinned host scalars
    int* iscratch = nullptr;    // device integer flags
    double* kks_part = nullptr; // KKS per-workgroup partials (kKksPartDoubles)
@@ -134,6 +134,12 @@ int reduce_partials(const Level& L, int nparts, int ncol, int op,
 // Sums of nreg consecutive regions of nparts partials each (region r starts at
 // L.partial + r * nparts), one launch and one synchronisation.
 int reduce_regions(const Level& L, int nparts, int nreg, double* host_out, hipStream_t s);
+// The sums of nreg regions at part left on the device at out; and the sum of one
+// region returned to the host behind the nhead values at L.dred.
+int reduce_regions_dev(const Level& L, const double* part, int nparts, int nreg, double* out,
+                       hipStream_t s);
+int reduce_last(const Level& L, const double* part, int nparts, int nhead, double* host_out,
+                hipStream_t s);
 
 // Optional event timing of selected kernels, process-wide.  While a kernel
 // class is enabled, each of its launches is bracketed by two events recorded

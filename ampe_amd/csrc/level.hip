@@ -140,7 +140,7 @@ static int level_upload(Level* L, const std::vector<long long>& gd0,
       if (e == hipSuccess) e = hipMalloc(&L->ghost_src, sizeof(long long) * gs.size());
    }
    if (e == hipSuccess) e = hipMalloc(&L->partial, sizeof(double) * (size_t)maxparts * 16);
-   if (e == hipSuccess) e = hipMalloc(&L->dred, sizeof(double) * 16);
+   if (e == hipSuccess) e = hipMalloc(&L->dred, sizeof(double) * 64);
    if (e == hipSuccess) e = hipHostMalloc(&L->hpinned, sizeof(double) * 64);
    if (e == hipSuccess) e = hipMalloc(&L->iscratch, sizeof(int) * 64);
    if (e == hipSuccess) e = hipMalloc(&L->kks_part, sizeof(double) * kKksPartDoubles);
@@ -499,62 +499,98 @@ int level_split_tables(Level& L, hipStream_t s)
    return 0;
 }
 
-// Single-workgroup fixed-order reduction of nparts x ncol partials
-// (column-interleaved).  Each lane walks a fixed stride, then a fixed tree.
+// Fixed-order reduction of nparts values `stride` apart by a workgroup of 1024:
+// eight loads of a lane in flight (65536 values one after the other took 31 us),
+// then a tree.
+__device__ __forceinline__ double reduce_1024(const double* __restrict__ p, int nparts, int stride,
+                                              int op, double* sh)
+{
+   double acc[8];  // sums start at 0; maxima are of non-negative values
+#pragma unroll
+   for (int u = 0; u < 8; u++) acc[u] = 0.0;
+   for (int i = threadIdx.x; i < nparts; i += 8192) {
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+         const int k = i + 1024 * u;
+         const double v = k < nparts ? p[(long long)k * stride] : 0.0;
+         acc[u] = (op == 0) ? acc[u] + v : (v > acc[u] ? v : acc[u]);
+      }
+   }
+#pragma unroll
+   for (int w = 4; w > 0; w >>= 1)
+#pragma unroll
+      for (int u = 0; u < w; u++) {
+         const double b = acc[u + w];
+         acc[u] = (op == 0) ? acc[u] + b : (b > acc[u] ? b : acc[u]);
+      }
+   double v = acc[0];
+   for (int o = 32; o > 0; o >>= 1) {
+      const double b = __shfl_xor(v, o);
+      v = (op == 0) ? v + b : (b > v ? b : v);
+   }
+   __syncthreads();  // sh may still be read from the reduction before
+   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+   __syncthreads();
+   v = sh[0];
+#pragma unroll
+   for (int k = 1; k < 16; k++) v = (op == 0) ? v + sh[k] : (sh[k] > v ? sh[k] : v);
+   return v;
+}
+
+// nparts x ncol partials (column-interleaved), one workgroup.  out may be pinned
+// host memory: the result is there when the stream has been waited for.
 __global__ void __launch_bounds__(1024) k_reduce_partials(const double* __restrict__ part,
                                                           int nparts, int ncol, int op,
                                                           double* __restrict__ out)
 {
-   __shared__ double sh[1024];
+   __shared__ double sh[16];
    for (int c = 0; c < ncol; c++) {
-      double acc = 0.0;  // sums start at 0; maxima are of non-negative values
-      for (int i = threadIdx.x; i < nparts; i += 1024) {
-         double v = part[(long long)i * ncol + c];
-         acc = (op == 0) ? acc + v : (v > acc ? v : acc);
-      }
-      sh[threadIdx.x] = acc;
-      __syncthreads();
-      for (int w = 512; w > 0; w >>= 1) {
-         if (threadIdx.x < w) {
-            double a = sh[threadIdx.x], b = sh[threadIdx.x + w];
-            sh[threadIdx.x] = (op == 0) ? a + b : (b > a ? b : a);
-         }
-         __syncthreads();
-      }
-      if (threadIdx.x == 0) out[c] = sh[0];
-      __syncthreads();
+      const double v = reduce_1024(part + c, nparts, ncol, op, sh);
+      if (threadIdx.x == 0) out[c] = v;
    }
 }
 
-// One workgroup per region r: the sum of part[r * nparts .. + nparts) in the
-// fixed order of k_reduce_partials.
+// One workgroup per region r: the sum of part[r * nparts .. + nparts).  With head
+// the nhead values there are put before the sums.
 __global__ void __launch_bounds__(1024) k_reduce_regions(const double* __restrict__ part,
-                                                         int nparts, double* __restrict__ out)
+                                                         int nparts,
+                                                         const double* __restrict__ head,
+                                                         int nhead, double* __restrict__ out)
 {
-   __shared__ double sh[1024];
-   const double* p = part + (long long)blockIdx.x * nparts;
-   double acc = 0.0;
-   for (int i = threadIdx.x; i < nparts; i += 1024) acc = acc + p[i];
-   sh[threadIdx.x] = acc;
-   __syncthreads();
-   for (int w = 512; w > 0; w >>= 1) {
-      if (threadIdx.x < w) sh[threadIdx.x] = sh[threadIdx.x] + sh[threadIdx.x + w];
-      __syncthreads();
-   }
-   if (threadIdx.x == 0) out[blockIdx.x] = sh[0];
+   __shared__ double sh[16];
+   const double v = reduce_1024(part + (long long)blockIdx.x * nparts, nparts, 1, 0, sh);
+   if (threadIdx.x == 0) out[nhead + blockIdx.x] = v;
+   if (blockIdx.x == 0 && (int)threadIdx.x < nhead) out[threadIdx.x] = head[threadIdx.x];
 }
 
 int reduce_partials(const Level& L, int nparts, int ncol, int op,
                     double* host_out, hipStream_t s)
 {
-   double* dout = L.dred;
    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(1024), 0, s, L.partial, nparts,
-                      ncol, op, dout);
+                      ncol, op, L.hpinned);
    AMPE_HIP_CHECK(hipGetLastError());
-   AMPE_HIP_CHECK(hipMemcpyAsync(L.hpinned, dout, sizeof(double) * ncol,
-                                 hipMemcpyDeviceToHost, s));
    AMPE_HIP_CHECK(hipStreamSynchronize(s));
    for (int c = 0; c < ncol; c++) host_out[c] = L.hpinned[c];
+   return 0;
+}
+
+int reduce_regions_dev(const Level& L, const double* part, int nparts, int nreg, double* out,
+                       hipStream_t s)
+{
+   hipLaunchKernelGGL(k_reduce_regions, dim3(nreg), dim3(1024), 0, s, part, nparts, nullptr, 0,
+                      out);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
+int reduce_last(const Level& L, const double* part, int nparts, int nhead, double* host_out,
+                hipStream_t s)
+{
+   hipLaunchKernelGGL(k_reduce_regions, dim3(1), dim3(1024), 0, s, part, nparts, L.dred, nhead,
+                      L.hpinned);
+   AMPE_HIP_CHECK(hipGetLastError());
+   AMPE_HIP_CHECK(hipStreamSynchronize(s));
+   for (int r = 0; r <= nhead; r++) host_out[r] = L.hpinned[r];
    return 0;
 }
 
@@ -564,11 +600,7 @@ int reduce_regions(const Level& L, int nparts, int nreg, double* host_out, hipSt
       set_error("reduce_regions: at most 16 regions");
       return -1;
    }
-   hipLaunchKernelGGL(k_reduce_regions, dim3(nreg), dim3(1024), 0, s, L.partial, nparts,
-                      L.dred);
-   AMPE_HIP_CHECK(hipGetLastError());
-   AMPE_HIP_CHECK(hipMemcpyAsync(L.hpinned, L.dred, sizeof(double) * nreg,
-                                 hipMemcpyDeviceToHost, s));
+   if (reduce_regions_dev(L, L.partial, nparts, nreg, L.hpinned, s)) return -1;
    AMPE_HIP_CHECK(hipStreamSynchronize(s));
    for (int r = 0; r < nreg; r++) host_out[r] = L.hpinned[r];
    return 0;

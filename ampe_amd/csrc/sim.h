@@ -46,8 +46,8 @@ struct Sim {
    bool have_prev = false;
    // state and Newton-Krylov work vectors (nc ghosted component blocks)
    double *y = nullptr, *yprev = nullptr, *ypred = nullptr, *ycur = nullptr,
-          *ahist = nullptr, *fcur = nullptr, *b = nullptr, *del = nullptr, *ewt = nullptr,
-          *work = nullptr, *work2 = nullptr, *jv = nullptr, *xk = nullptr, *corr = nullptr,
+          *ahist = nullptr, *fcur = nullptr, *b = nullptr, *ewt = nullptr,
+          *work = nullptr, *work2 = nullptr, *jv = nullptr, *corr = nullptr,
           *acor = nullptr;
    std::vector<double*> V;
    // adaptive mode: Nordsieck columns h y' and h^2 y''/2 (the state y is the

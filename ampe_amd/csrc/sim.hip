@@ -155,7 +155,7 @@ static int sim_finish(Sim* S, Sim** out)
    int ql = p.evolve_quat ? p.qlen : 1;
    int rc = 0;
    double** vecs[] = {&S->y, &S->yprev, &S->ypred, &S->ycur, &S->ahist, &S->fcur, &S->b,
-                      &S->del, &S->ewt, &S->work, &S->work2, &S->jv, &S->xk, &S->corr,
+                      &S->ewt, &S->work, &S->work2, &S->jv, &S->corr,
                       &S->acor};
    for (auto v : vecs) rc |= dalloc(v, S->nv);
    if (s.adaptive) {
@@ -257,8 +257,8 @@ int sim_create_hier(const ampe_model_params& p, const ampe_solver_params& s, Hie
 void sim_destroy(Sim* S)
 {
    if (!S) return;
-   double* all[] = {S->y, S->yprev, S->ypred, S->ycur, S->ahist, S->fcur, S->b, S->del,
-                    S->ewt, S->work, S->work2, S->jv, S->xk, S->corr, S->acor, S->cl, S->cs,
+   double* all[] = {S->y, S->yprev, S->ypred, S->ycur, S->ahist, S->fcur, S->b,
+                    S->ewt, S->work, S->work2, S->jv, S->corr, S->acor, S->cl, S->cs,
                     S->clr, S->csr, S->Cphi, S->sqrtm, S->Mphi, S->fac_u, S->fac_e, S->fac_r,
                     S->gni,
                     S->Dc, S->Dphi, S->Dconc, S->fc, S->fcq, S->phid, S->z1, S->z2,
@@ -553,17 +553,18 @@ static int hier_rhs_eval(Sim* S, double* y, double* ydot, bool fd)
    return 0;
 }
 
-static int hier_psetup(Sim* S, double* y, double gamma)
+static int hier_psetup(Sim* S, double* y, double gamma, bool fresh)
 {
    const ampe_model_params& p = S->p;
    hipStream_t st = S->stream;
    S->st.npe++;
    int ql = S->iq >= 0 ? p.qlen : 0;
-   if (hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ic, S->ncs, S->iq, ql, st)) return -1;
+   if (!fresh && hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ic, S->ncs, S->iq, ql, st))
+      return -1;
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
-   if (q && hier_quat_face_norm2(*S->hier, p, q, S->gni, st)) return -1;
+   if (q && !fresh && hier_quat_face_norm2(*S->hier, p, q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
    // several orders: the well scale passed is 0, so C = 1
    ampe_model_params pw = p;
@@ -668,10 +669,32 @@ static int hier_psolve_set(Sim* S, T* r, T* e, T* tmp)
                                 S->stream);
 }
 
+// Of the preconditioner solve.  f_ready: the right-hand side is formed already
+// (orientation components divided by sqrt(M)), with the FP32 preconditioner in
+// S->f_f, else in r, which the solve may overwrite.  keep: the solution is left
+// as the blocks have it (orientation components without sqrt(M)), in S->f_u or z.
+struct PsolveOpts {
+   bool f_ready = false;
+   bool keep = false;
+   // the solve may be captured into a graph
+   bool graph = false;
+   // a caller outside the integrator: z's ghosts are filled, and a hierarchy
+   // returns whether the residual norms met delta
+   bool status = false;
+};
+
+// Every block of the hierarchy in the same launches (60 components of two
+// elliptic operators fit the set's 16 slots of four): one cycle a block.
+static bool hier_set_ok(const Sim* S)
+{
+   return S->s.fac_max_cycles <= 1 && S->s.quat_max_cycles <= 1 && S->s.fac_tol < 0.0 &&
+          S->nc <= 60;
+}
+
 // status: the caller wants to know whether the blocks' residual norms met
 // delta (0 / 1); the integrator does not, and then one cycle per block needs
 // no norm.
-static int hier_psolve(Sim* S, const double* r, double* z, double delta, bool status)
+static int hier_psolve(Sim* S, const double* r, double* z, double delta, const PsolveOpts& o)
 {
    const ampe_model_params& p = S->p;
    hipStream_t st = S->stream;
@@ -680,25 +703,27 @@ static int hier_psolve(Sim* S, const double* r, double* z, double delta, bool st
    int ql = S->iq >= 0 ? p.qlen : 0;
    int iq = S->iq >= 0 ? S->iq : S->nc;
    int ret = 0;
-   if (!r || !z) {
+   if (!o.status && hier_set_ok(S)) {
+      if (S->s.precision == AMPE_FAC_FP32) {
+         if (o.f_ready ? fill_zero(S->f_u, S->nv, st)
+                       : psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, S->f_u,
+                                          st))
+            return -1;
+         if (hier_psolve_set<float>(S, S->f_f, S->f_u, S->f_r)) return -1;
+         return o.keep ? 0 : psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st);
+      }
+      if (o.f_ready ? fill_zero(z, S->nv, st)
+                    : psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, z, st))
+         return -1;
+      if (hier_psolve_set<double>(S, o.f_ready ? const_cast<double*>(r) : S->fac_e, z, S->fac_r))
+         return -1;
+      if (!o.keep && S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql))
+         return -1;
+      return 0;
+   }
+   if (!r || !z || o.f_ready || o.keep) {
       set_error("hier_psolve: needs the input and output vectors");
       return -1;
-   }
-   // (60 components of two elliptic operators fit the set's 16 slots of four)
-   if (!status && S->s.fac_max_cycles <= 1 && S->s.quat_max_cycles <= 1 && S->s.fac_tol < 0.0 &&
-       S->nc <= 60) {
-      if (S->s.precision == AMPE_FAC_FP32) {
-         if (psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, S->f_u, st) ||
-             hier_psolve_set<float>(S, S->f_f, S->f_u, S->f_r) ||
-             psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st))
-            return -1;
-         return 0;
-      }
-      if (psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, z, st) ||
-          hier_psolve_set<double>(S, S->fac_e, z, S->fac_r))
-         return -1;
-      if (S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql)) return -1;
-      return 0;
    }
    ampe_fac_params fp{S->s.fac_max_cycles, 1, 1, S->s.fac_sweeps, S->s.fac_tol};
    if (S->s.precision == AMPE_FAC_FP32) {
@@ -841,19 +866,21 @@ static int rhs_eval(Sim* S, double* y, double* ydot, bool fd)
    return 0;
 }
 
-// CVSpgmrPrecondSet (source/QuatIntegrator.cc:3300-3376)
-static int psetup(Sim* S, double* y, double gamma)
+// CVSpgmrPrecondSet (source/QuatIntegrator.cc:3300-3376).  fresh: the last
+// evaluation was a full one of the right-hand side at y, which filled y's ghosts
+// and the face gradients.
+static int psetup(Sim* S, double* y, double gamma, bool fresh = false)
 {
-   if (S->hier) return hier_psetup(S, y, gamma);
+   if (S->hier) return hier_psetup(S, y, gamma, fresh);
    const Level& L = *S->L;
    const ampe_model_params& p = S->p;
    hipStream_t st = S->stream;
    S->st.npe++;
-   if (ghost_fill(L, y, S->nc, st)) return -1;
+   if (!fresh && ghost_fill(L, y, S->nc, st)) return -1;
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
-   if (q && launch_quat_gni(L, p, rhs_lev(p), q, S->gni, st)) return -1;
+   if (q && !fresh && launch_quat_gni(L, p, rhs_lev(p), q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
    // phase block: C = 1 + gamma M w g'' (source/PhaseFACOps.cc:33-51)
    // phase mobility after the phase concentrations (QuatIntegrator::
@@ -1223,19 +1250,10 @@ static int split_first(const Sim* S)
    return set_mode(S) || S->iq < 0 ? 0 : S->iq;
 }
 
-// z = P^-1 r.  FP32 preconditioner only: f_ready = the FP32 right-hand side
-// S->f_f was already formed from r (by the Krylov kernel that produced r);
-// keep = the solution is left in S->f_u for the caller (z untouched).
-struct PsolveOpts {
-   bool f_ready = false;
-   bool keep = false;
-   // a caller outside the integrator: z's ghosts are filled, and a hierarchy
-   // returns whether the residual norms met delta
-   bool status = false;
-};
+// z = P^-1 r.
 static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o = {})
 {
-   if (S->hier) return hier_psolve(S, r, z, delta, o.status);
+   if (S->hier) return hier_psolve(S, r, z, delta, o);
    const ampe_model_params& p = S->p;
    hipStream_t st = S->stream;
    long long ng = S->ng;
@@ -1246,14 +1264,10 @@ static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o
    if (S->s.precision == AMPE_FAC_FP32) {
       // f = r (orientation blocks / sqrt(M), FP64 division) in FP32
       int ret;
-      if (o.f_ready) {
-         ret = psolve_graph_ok(S) ? psolve_f32_graph(S) : psolve_f32(S, delta);
-      } else {
-         if (psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, nullptr, st,
-                              split_level(S), split_first(S)))
-            return -1;
-         ret = psolve_f32(S, delta);
-      }
+      if (!o.f_ready && psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, nullptr,
+                                         st, split_level(S), split_first(S)))
+         return -1;
+      ret = o.graph && psolve_graph_ok(S) ? psolve_f32_graph(S) : psolve_f32(S, delta);
       if (ret < 0) return -1;
       if (!o.keep && psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st,
                                        split_level(S), split_first(S)))
@@ -1261,28 +1275,26 @@ static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o
       if (o.status && ghost_fill(*S->L, z, S->nc, st)) return -1;
       return ret;
    }
-   if (o.f_ready || o.keep) {
-      set_error("psolve: fused input/output is for the FP32 preconditioner");
-      return -1;
-   }
    int ret = 0;
    if (set_mode(S) && S->mgd) {
       // the V-cycle's right-hand side in one vector
-      if (psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, nullptr, st))
+      if (!o.f_ready &&
+          psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, nullptr, st))
          return -1;
-      if (solve_set<double>(S, S->fac_e, z)) return -1;
+      if (solve_set<double>(S, o.f_ready ? const_cast<double*>(r) : S->fac_e, z)) return -1;
    } else {
-      // fac_u = orientation blocks of r / sqrt(M)
-      if (S->iq >= 0 &&
+      // fq: orientation blocks of r / sqrt(M)
+      if (!o.f_ready && S->iq >= 0 &&
           psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, nullptr, S->fac_u, nullptr, st))
          return -1;
+      double* fq = o.f_ready ? const_cast<double*>(r) + iq * ng : S->fac_u;
       if (set_mode(S)) {
-         if (solve_set<double>(S, S->fac_u, z, r)) return -1;
+         if (solve_set<double>(S, fq, z, r)) return -1;
       } else {
          auto bl = make_blocks<double>(S, dphi, S->Cphi, S->Mphi, S->Dconc, S->fc, S->sqrtm);
          for (auto& B : bl) {
             long long off = (long long)B.comp * ng;
-            B.f = B.kind == 1 ? S->fac_u : r + off;
+            B.f = B.kind == 1 ? fq : r + off;
             B.u = z + off;
             B.e = S->fac_e + off;
             B.r = S->fac_r + off;
@@ -1291,7 +1303,8 @@ static int psolve(Sim* S, const double* r, double* z, double delta, PsolveOpts o
          if (ret < 0) return -1;
       }
    }
-   if (S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql)) return -1;
+   if (!o.keep && S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql))
+      return -1;
    if (o.status && ghost_fill(*S->L, z, S->nc, st)) return -1;
    return ret;
 }
@@ -1316,11 +1329,41 @@ static double cellvol(const Sim* S)
    return dx[0] * dx[1] * (S->p.ndim == 3 ? dx[2] : 1.0);
 }
 
-// SPGMR, left preconditioned, MGS, x0 = 0, scaling by ewt, difference-quotient
-// Jv (sigma = 1/||v||_wrms) and A v = v - gamma Jv.  V[l] is normalised lazily
-// by the next iteration's first kernel.  Returns 0 converged, 1 residual
-// reduced, 2 failure, -1 fatal.
-static int spgmr(Sim* S, double gamma, const double* bvec, double* x, double delta)
+// How the Krylov kernels pass vectors to and from the preconditioner solve: in
+// its own form, except for a hierarchy solved block by block.
+struct KryIo {
+   PrecIn in;
+   PrecOut out;
+   PsolveOpts o;
+};
+
+static KryIo kry_io(const Sim* S)
+{
+   KryIo io;
+   const bool f32 = S->s.precision == AMPE_FAC_FP32;
+   io.out.z = S->work;
+   if (S->hier && !hier_set_ok(S)) return io;
+   io.o.f_ready = io.o.keep = true;
+   if (S->iq >= 0) {
+      io.in.sm = io.out.sm = S->sqrtm;
+      io.in.iq = io.out.iq = S->iq;
+      io.in.ql = io.out.ql = S->p.qlen;
+   }
+   if (f32) {
+      io.in.f = S->f_f;
+      io.out.u = S->f_u;
+      if (split_level(S)) io.in.sp0 = io.out.sp0 = split_first(S);
+   }
+   return io;
+}
+
+// SPGMR, left preconditioned, x0 = 0, scaling by ewt, difference-quotient Jv and
+// A v = v - gamma Jv, on the right-hand side kry_newton_rhs formed (in S->b or the
+// preconditioner's input).  Basis vector i is ewt V[i] hs[i], so that its WRMS norm
+// over ewt is sqrt(wfac / cv) and the difference-quotient increment
+// 1 / ||v||_wrms is sqrt(cv / wfac).  The solution is *x, a combination of V.
+// Returns 0 converged, 1 residual reduced, 2 failure, -1 fatal.
+static int spgmr(Sim* S, double gamma, const KryIo& io, VecList* x, double delta)
 {
    const Level& L = *S->L;
    hipStream_t st = S->stream;
@@ -1332,123 +1375,57 @@ static int spgmr(Sim* S, double gamma, const double* bvec, double* x, double del
    int ld = maxl + 1;
 #define HH(i, j) Hm[(size_t)(i) * ld + (j)]
    double givens[2 * kMaxKrylov], g[kMaxKrylov + 1], yv[kMaxKrylov];
-   // Classical Gram-Schmidt keeps the basis unnormalised: basis vector i is
-   // V[i] hs[i].  The difference-quotient increment then needs no norm pass:
-   // the normalised vector has sum(v^2) cv = 1, so its WRMS norm over ewt is
-   // sqrt(wfac / cv) and sigma = sqrt(cv / wfac).  With the FP32
-   // preconditioner, the kernel that forms A v also writes the FP32
-   // preconditioner input, and the dot kernel reads the FP32 solution.
    const bool cgs = S->s.gstype == AMPE_GS_CLASSICAL;
-   // (one level only: the hierarchy's FP32 block solves take the FP64 input
-   // and write the FP64 output)
-   const bool fuse_out = cgs && S->s.precision == AMPE_FAC_FP32 && !S->hier;
-   PrecIn pin;
-   PrecOut pout;
-   if (fuse_out) {
-      pin.f = S->f_f;
-      pin.sm = S->sqrtm;
-      pin.iq = S->iq >= 0 ? S->iq : nc;
-      pin.ql = S->iq >= 0 ? S->p.qlen : 0;
-      pout.u = S->f_u;
-      pout.sm = S->sqrtm;
-      pout.ewt = S->ewt;
-      pout.iq = pin.iq;
-      pout.ql = pin.ql;
-      if (split_level(S)) pin.sp0 = pout.sp0 = split_first(S);
-   }
    double hs[kMaxKrylov + 1];
-   if (psolve(S, bvec, S->work, delta) < 0) return -1;
+   x->n = 0;
+   PsolveOpts o = io.o;
+   if (psolve(S, S->b, S->work, delta, o) < 0) return -1;
+   o.graph = true;
    double rho;
-   if (kry_scale_dot(L, nc, S->ewt, S->work, S->V[0], S->V[0], &rho, st)) return -1;
+   if (kry_start(L, nc, io.out, S->ewt, S->V[0], &rho, st)) return -1;
    rho = std::sqrt(rho * cv);
    double rho0 = rho;
-   if (rho <= delta) {
-      AMPE_HIP_CHECK(hipMemsetAsync(x, 0, sizeof(double) * S->nv, st));
-      return 0;
-   }
-   double hinv = 1.0 / rho;
-   hs[0] = hinv;
+   if (rho <= delta) return 0;
+   hs[0] = 1.0 / rho;
    std::memset(g, 0, sizeof(g));
    g[0] = rho;
    int lused = 0;
    bool converged = false;
+   const double sig = std::sqrt(cv / wfac), siginv = 1.0 / sig;
    for (int l = 0; l < maxl; l++) {
       S->st.nli++;
-      if (cgs) {
-         double sig = std::sqrt(cv / wfac);
-         if (kry_mid_scaled(L, nc, sig, S->V[l], hs[l], S->ewt, S->ycur, S->work2, st))
-            return -1;
-         if (rhs_eval(S, S->work2, S->jv, true)) return -1;
-         double siginv = 1.0 / sig;
-         // with the fused FP32 preconditioner input the FP64 (I - gamma J) v is
-         // not stored: the dot kernel writes V[l+1] from the preconditioned vector
-         if (kry_finish_scaled(L, nc, siginv, gamma, S->V[l], hs[l], S->ewt, S->jv, S->fcur,
-                               fuse_out ? nullptr : S->V[l + 1], pin, st))
-            return -1;
-      } else {
-         double ss;
-         // V[l] *= hinv; xk = V[l] / ewt; ||xk||_wrms
-         if (kry_prep(L, nc, hinv, S->V[l], S->ewt, S->xk, &ss, st)) return -1;
-         double sig = 1.0 / std::sqrt(ss * wfac);
-         if (kry_mid(L, nc, sig, S->xk, S->ycur, S->work2, st)) return -1;
-         if (rhs_eval(S, S->work2, S->jv, true)) return -1;
-         double siginv = 1.0 / sig;
-         if (kry_finish(L, nc, siginv, gamma, S->xk, S->jv, S->fcur, S->V[l + 1], st))
-            return -1;
-      }
-      if (fuse_out) {
-         // input formed by the finish kernel, solution left in f_u
-         PsolveOpts o;
-         o.f_ready = true;
-         o.keep = true;
-         if (psolve(S, S->V[l + 1], nullptr, delta, o) < 0) return -1;
-      } else if (psolve(S, S->V[l + 1], S->work, delta) < 0) {
+      if (kry_mid(L, nc, sig, S->V[l], hs[l], S->ycur, S->work2, st)) return -1;
+      if (rhs_eval(S, S->work2, S->jv, true)) return -1;
+      // the solve's right-hand side: FP32, or FP64 in V[l + 1]
+      if (kry_finish(L, nc, siginv, gamma, S->V[l], hs[l], S->jv, S->fcur,
+                     io.in.f ? nullptr : S->V[l + 1], io.in, st))
          return -1;
+      if (psolve(S, S->V[l + 1], S->work, delta, o) < 0) return -1;
+      double hn, sums[kMaxKrylov + 2];
+      VecList vl;
+      vl.n = l + 1;
+      for (int i = 0; i <= l; i++) {
+         vl.v[i] = S->V[i];
+         vl.y[i] = hs[i];
       }
-      double hn;
-      if (S->s.gstype == AMPE_GS_CLASSICAL) {
-         // V[l+1] = ewt work with all its dots in one pass, one linear
-         // combination, re-orthogonalised when the norm dropped by > 1000
-         // (SUNClassicalGS)
-         VecList vl;
-         vl.n = l + 1;
-         for (int i = 0; i <= l; i++) vl.v[i] = S->V[i];
-         double sums[kMaxCgs];
-         if (fuse_out) {
-            // V[l+1] = ewt P^-1 (...) from the FP32 solution, with its dots
-            if (kry_cgs_dots_from(L, nc, pout, S->V[l + 1], vl, sums, st)) return -1;
-         } else if (kry_cgs_dots(L, nc, S->ewt, S->work, S->V[l + 1], vl, sums, st)) {
-            return -1;
-         }
-         double vk_norm = std::sqrt(sums[l + 1] * cv);
-         for (int i = 0; i <= l; i++) {
-            HH(i, l) = (sums[i] * hs[i]) * cv;
-            vl.y[i] = -HH(i, l) * hs[i];
-         }
-         double ss;
-         if (kry_cgs_update(L, nc, S->V[l + 1], vl, &ss, st)) return -1;
-         hn = std::sqrt(ss * cv);
+      if (cgs) {
+         // all dots in one pass, one linear combination, re-orthogonalised when
+         // the norm dropped by > 1000 (SUNClassicalGS)
+         if (kry_cgs(L, nc, io.out, vl, cv, S->ewt, S->V[l + 1], sums, st)) return -1;
+         const double vk_norm = std::sqrt(sums[l + 2] * cv);
+         for (int i = 0; i <= l; i++) HH(i, l) = (sums[i] * hs[i]) * cv;
+         hn = std::sqrt(sums[l + 1] * cv);
          if (1000.0 * hn < vk_norm) {
-            if (kry_cgs_dots(L, nc, nullptr, nullptr, S->V[l + 1], vl, sums, st)) return -1;
-            for (int i = 0; i <= l; i++) {
-               double d = (sums[i] * hs[i]) * cv;
-               HH(i, l) += d;
-               vl.y[i] = -d * hs[i];
-            }
-            if (kry_cgs_update(L, nc, S->V[l + 1], vl, &ss, st)) return -1;
-            hn = std::sqrt(ss * cv);
+            PrecOut again;
+            again.z = S->V[l + 1];
+            if (kry_cgs(L, nc, again, vl, cv, S->ewt, S->V[l + 1], sums, st)) return -1;
+            for (int i = 0; i <= l; i++) HH(i, l) += (sums[i] * hs[i]) * cv;
+            hn = std::sqrt(sums[l + 1] * cv);
          }
       } else {
-         // V[l+1] = ewt work; modified Gram-Schmidt, each step fused with the next dot
-         double dot;
-         if (kry_scale_dot(L, nc, S->ewt, S->work, S->V[l + 1], S->V[0], &dot, st)) return -1;
-         for (int i = 0; i <= l; i++) {
-            double hij = dot * cv;
-            HH(i, l) = hij;
-            const double* nxt = (i < l) ? S->V[i + 1] : nullptr;
-            if (kry_mgs(L, nc, S->V[l + 1], S->V[i], hij, nxt, &dot, st)) return -1;
-         }
-         hn = std::sqrt(dot * cv);
+         if (kry_mgs(L, nc, io.out, vl, cv, S->ewt, S->V[l + 1], sums, st)) return -1;
+         for (int i = 0; i <= l; i++) HH(i, l) = (sums[i] * hs[i]) * cv;
+         hn = std::sqrt(sums[l + 1] * cv);
       }
       HH(l + 1, l) = hn;
       for (int i = 0; i < l; i++) {
@@ -1483,21 +1460,18 @@ static int spgmr(Sim* S, double gamma, const double* bvec, double* x, double del
          break;
       }
       if (hn == 0.0) break;
-      hinv = 1.0 / hn;
-      hs[l + 1] = hinv;
+      hs[l + 1] = 1.0 / hn;
    }
    for (int i = lused - 1; i >= 0; i--) {
       double sacc = g[i];
       for (int j = i + 1; j < lused; j++) sacc -= HH(i, j) * yv[j];
       yv[i] = sacc / HH(i, i);
    }
-   VecList vl;
-   vl.n = lused;
+   x->n = lused;
    for (int i = 0; i < lused; i++) {
-      vl.v[i] = S->V[i];
-      vl.y[i] = cgs ? yv[i] * hs[i] : yv[i];
+      x->v[i] = S->V[i];
+      x->y[i] = yv[i] * hs[i];
    }
-   if (kry_lincomb(L, nc, vl, S->ewt, x, st)) return -1;
 #undef HH
    if (converged) return 0;
    return rho < rho0 ? 1 : 2;
@@ -1523,21 +1497,25 @@ static int newton(Sim* S, double gamma, double delta, double tq4, bool force_set
    for (int m = 0; m < S->s.max_newton; m++) {
       S->st.nni++;
       if (rhs_eval(S, S->ycur, S->fcur, false)) return -1;
-      if (kry_newton_rhs(L, S->nc, gamma, S->fcur, S->ycur, S->ahist, S->b, st)) return -1;
       if (m == 0 && call_setup) {
-         if (psetup(S, S->ycur, gamma)) return -1;
+         if (psetup(S, S->ycur, gamma, true)) return -1;
          S->nstlp = S->nst;
          S->crate = 1.0;
          *did_setup = true;
       }
-      int ls = spgmr(S, gamma, S->b, S->del, delta);
+      const KryIo io = kry_io(S);
+      if (kry_newton_rhs(L, S->nc, gamma, S->fcur, S->ycur, S->ahist, io.in.f ? nullptr : S->b,
+                         io.in, st))
+         return -1;
+      VecList del_v;
+      int ls = spgmr(S, gamma, io, &del_v, delta);
       if (ls < 0) return -1;
       if (ls == 2 || (ls == 1 && m > 0)) {
          S->st.nlcf++;
          return 1;
       }
       double ss;
-      if (kry_newton_update(L, S->nc, S->del, S->ewt, S->ycur, &ss, st)) return -1;
+      if (kry_newton_update(L, S->nc, del_v, S->ewt, S->ycur, &ss, st)) return -1;
       double del = std::sqrt(ss * wfac);
       if (m > 0) {
          double r = del / delp;
