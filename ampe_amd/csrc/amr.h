@@ -53,6 +53,13 @@ int hier_sim_sync_fill(Hier* H, double* y, int nc, int nord, int ic, int ncs, in
                        hipStream_t s);
 int hier_ghost_fill(const Hier& H, double* f, int ncomp, int cf, hipStream_t s);
 int hier_coarsen(const Hier& H, double* f, int ncomp, int quatnorm, hipStream_t s);
+// The integrator's right-hand side over all levels (amr.hip); recompute: the lagged
+// face data (gni, Dc, Dphi) too.  hier_quat_gni: the faces' 1 / |grad q| alone.
+int hier_rhs_all(const Hier& H, const ampe_model_params& p, const double* y, int iq, int ic,
+                 bool recompute, const double* cl, const double* cs, double* gni, double* Dc,
+                 double* Dphi, double* rhs, hipStream_t s);
+int hier_quat_gni(const Hier& H, const ampe_model_params& p, const double* q, double* gni,
+                  hipStream_t s);
 int hier_phase_rhs(const Hier& H, const ampe_model_params& p0, const double* phi,
                    const double* q, const double* cl, const double* cs, double* rhs,
                    hipStream_t s);
@@ -95,11 +102,10 @@ int hier_fac_solve_f32(Hier& H, const HBlock<float>& B, const ampe_fac_params& P
 template <typename T>
 int hier_fac_cycle_set(const Hier& H, const SweepSet<T>& set, int coarse_its,
                        unsigned long long ewing, T* r, T* e, T* tmp, hipStream_t s);
-// Per-level coefficient passes of the preconditioner setup: phase C and
-// mobility, orientation face coefficients and sqrt(M_q), each level with its
-// own spacing.
+// Coefficients of the preconditioner setup, all levels: phase C and mobility,
+// orientation face coefficients (gni: the faces' 1 / |grad q|) and sqrt(M_q).
 int hier_precond_coeffs(const Hier& H, const ampe_model_params& p0, double gamma,
-                        const double* phi, const double* cl, const double* cs, const double* n2,
+                        const double* phi, const double* cl, const double* cs, const double* gni,
                         double* Mphi, double* Cphi, double* fc, double* sqrtm, hipStream_t s);
 
 }  // namespace ampe

@@ -359,6 +359,10 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
       pl.ncell_total = H->ncell;
       for (int a = 0; a < 3; a++) pl.nside_total[a] = H->nside[a];
       std::vector<long long> none;
+      std::vector<int> patch_lev((size_t)np);
+      for (int l = 0; l < nlev; l++)
+         for (int q = H->pbeg[l]; q < H->pbeg[l + 1]; q++) patch_lev[q] = l;
+      pl.patch_lev = patch_lev.data();
       if (level_create_placed(ndim, H->boxes.data(), np, pl, none, none, &H->comp))
          return hier_fail(H, "composite placement failed");
    }
@@ -668,6 +672,21 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
 // ------------------------------------------------------------ kernels
 namespace {
 
+// The value of coarse-fine ghost e: its parent cell (mode 1) or the linear
+// refinement of the coarse cells around it.
+template <typename T>
+__device__ __forceinline__ T cf_value(const T* __restrict__ a, const long long* __restrict__ s,
+                                      const double* __restrict__ w, int mode, int ndim)
+{
+   if (mode == 1) return a[s[0]];
+   double x = w[0], y = w[1], z = w[2];
+   T q1 = a[s[1]], q2 = a[s[2]], q3 = a[s[3]], q4 = a[s[4]];
+   if (ndim == 2) return (q1 + (q3 - q1) * x) * (1.0 - y) + (q2 + (q4 - q2) * x) * y;
+   T q5 = a[s[5]], q6 = a[s[6]], q7 = a[s[7]], q8 = a[s[8]];
+   return ((q1 + (q3 - q1) * x) * (1.0 - y) + (q2 + (q4 - q2) * x) * y) * (1.0 - z) +
+          ((q5 + (q7 - q5) * x) * (1.0 - y) + (q6 + (q8 - q6) * x) * y) * z;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) k_cf_fill(T* __restrict__ f, long long ncg, int ncomp,
                                                  const long long* __restrict__ dst,
@@ -677,24 +696,40 @@ __global__ void __launch_bounds__(256) k_cf_fill(T* __restrict__ f, long long nc
 {
    long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
    if (e >= n) return;
-   const long long* s = src + 9 * e;
    for (int m = 0; m < ncomp; m++) {
       T* a = f + m * ncg;
-      T v;
-      if (mode == 1) {
-         v = a[s[0]];
-      } else {
-         double x = w[3 * e], y = w[3 * e + 1], z = w[3 * e + 2];
-         T q1 = a[s[1]], q2 = a[s[2]], q3 = a[s[3]], q4 = a[s[4]];
-         if (ndim == 2) {
-            v = (q1 + (q3 - q1) * x) * (1.0 - y) + (q2 + (q4 - q2) * x) * y;
-         } else {
-            T q5 = a[s[5]], q6 = a[s[6]], q7 = a[s[7]], q8 = a[s[8]];
-            v = ((q1 + (q3 - q1) * x) * (1.0 - y) + (q2 + (q4 - q2) * x) * y) * (1.0 - z) +
-                ((q5 + (q7 - q5) * x) * (1.0 - y) + (q6 + (q8 - q6) * x) * y) * z;
-         }
-      }
-      a[dst[e]] = v;
+      a[dst[e]] = cf_value(a, src + 9 * e, w + 3 * e, mode, ndim);
+   }
+}
+
+// Average of a coarse cell's children: components [m0, m1) of the cell dst, the
+// children in x-fastest order from base with the fine strides; with quatnorm (at
+// most four components) the average is normalised.
+template <typename T>
+__device__ __forceinline__ void coarsen_cell(const T* __restrict__ fsrc, T* __restrict__ f,
+                                             long long ncg, int m0, int m1, long long dst,
+                                             long long base, long long packed, double dvf,
+                                             double dvc, int nchild, int quatnorm)
+{
+   const long long sy = packed & 0xffffffffLL, sz = packed >> 32;
+   T acc[4];
+   for (int m = m0; m < m1; m++) {
+      const T* a = fsrc + m * ncg + base;
+      T s = 0.0;
+      for (int c = 0; c < 8; c++)
+         if (c < nchild) s = s + a[(c & 1) + ((c >> 1) & 1) * sy + (c >> 2) * sz] * dvf;
+      T v = s / (T)dvc;
+      if (!quatnorm)
+         f[m * ncg + dst] = v;
+      else if (m - m0 < 4)
+         acc[m - m0] = v;
+   }
+   if (quatnorm) {
+      double s = 0.0;
+      for (int m = 0; m < m1 - m0; m++) s = s + acc[m] * acc[m];
+      double mg = sqrt(s);
+      double minv = mg < 1.0e-15 ? 0.0 : 1.0 / mg;
+      for (int m = m0; m < m1; m++) f[m * ncg + dst] = acc[m - m0] * minv;
    }
 }
 
@@ -708,31 +743,85 @@ __global__ void __launch_bounds__(256) k_coarsen(const T* __restrict__ fsrc,
 {
    long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
    if (e >= n) return;
-   // children in x-fastest order from the first child and the fine strides
-   const long long base = src[2 * e], packed = src[2 * e + 1];
-   const long long sy = packed & 0xffffffffLL, sz = packed >> 32;
    // without the normalisation the components are independent: one per
    // blockIdx.y
    const int m0 = quatnorm ? 0 : (int)blockIdx.y, m1 = quatnorm ? ncomp : m0 + 1;
-   T acc[4];
-   for (int m = m0; m < m1; m++) {
-      const T* a = fsrc + m * ncg + base;
-      T s = 0.0;
-      for (int c = 0; c < 8; c++)
-         if (c < nchild) s = s + a[(c & 1) + ((c >> 1) & 1) * sy + (c >> 2) * sz] * dvf;
-      T v = s / (T)dvc;
-      if (!quatnorm)
-         f[m * ncg + dst[e]] = v;
-      else if (m < 4)
-         acc[m] = v;
+   coarsen_cell(fsrc, f, ncg, m0, m1, dst[e], src[2 * e], src[2 * e + 1], dvf, dvc, nchild,
+                quatnorm);
+}
+
+// A state vector's components at once: blockIdx.y counts its plain components,
+// the four of the orientation (from iq on, normalised) are its last row.
+__global__ void __launch_bounds__(256) k_coarsen_state(double* __restrict__ y, long long ncg,
+                                                       int iq, const long long* __restrict__ dst,
+                                                       const long long* __restrict__ src,
+                                                       long long n, double dvf, double dvc,
+                                                       int nchild)
+{
+   long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (e >= n) return;
+   const bool q = iq >= 0 && blockIdx.y == gridDim.y - 1;
+   // the plain components lie before and after the orientation's
+   int m0 = (int)blockIdx.y;
+   if (q)
+      m0 = iq;
+   else if (iq >= 0 && m0 >= iq)
+      m0 += 4;
+   coarsen_cell(y, y, ncg, m0, m0 + (q ? 4 : 1), dst[e], src[2 * e], src[2 * e + 1], dvf, dvc,
+                nchild, q ? 1 : 0);
+}
+
+// The ghosts of every level in one launch, one component per blockIdx.y: the
+// levels' own gathers and the linear refinements (k_cf_fill), which all read
+// interior cells only.
+struct HierGhosts {
+   int nlev;
+   const long long *gd[kMaxLev], *gs[kMaxLev], *cd[kMaxLev], *cs[kMaxLev];
+   const double* cw[kMaxLev];
+   long long ng[kMaxLev], nc[kMaxLev];
+};
+
+__global__ void __launch_bounds__(256) k_hier_ghosts(double* __restrict__ f, long long ncg,
+                                                     HierGhosts h, int ndim)
+{
+   long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+   double* a = f + (long long)blockIdx.y * ncg;
+   for (int l = 0; l < h.nlev; l++) {
+      if (t < h.ng[l]) {
+         a[h.gd[l][t]] = a[h.gs[l][t]];
+         return;
+      }
+      t -= h.ng[l];
+      if (t < h.nc[l]) {
+         a[h.cd[l][t]] = cf_value(a, h.cs[l] + 9 * t, h.cw[l] + 3 * t, 2, ndim);
+         return;
+      }
+      t -= h.nc[l];
    }
-   if (quatnorm) {
-      double s = 0.0;
-      for (int m = 0; m < ncomp; m++) s = s + acc[m] * acc[m];
-      double mg = sqrt(s);
-      double minv = mg < 1.0e-15 ? 0.0 : 1.0 / mg;
-      for (int m = 0; m < ncomp; m++) f[m * ncg + dst[e]] = acc[m] * minv;
-   }
+}
+
+// face arrays of the same layout, coarsened together (one per blockIdx.y)
+struct FaceSet {
+   double* f[3];
+};
+
+__global__ void __launch_bounds__(256) k_face_coarsen_set(FaceSet fs, const long long* __restrict__ fd,
+                                                          const long long* __restrict__ fsrc,
+                                                          const int* __restrict__ dir, long long n,
+                                                          double af0, double af1, double af2,
+                                                          double ac0, double ac1, double ac2,
+                                                          int nfine)
+{
+   long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+   if (e >= n) return;
+   int d = dir[e];
+   double af = d == 0 ? af0 : (d == 1 ? af1 : af2);
+   double ac = d == 0 ? ac0 : (d == 1 ? ac1 : ac2);
+   double* a = fs.f[blockIdx.y];
+   double acc = 0.0;
+   for (int r = 0; r < 4; r++)
+      if (r < nfine) acc = acc + a[fsrc[4 * e + r]] * af;
+   a[fd[e]] = acc / ac;
 }
 
 __global__ void __launch_bounds__(256) k_face_coarsen(const double* __restrict__ src,
@@ -1074,6 +1163,68 @@ static void corr_areas(const Hier& H, int l, double& af, double& ac)
 }
 
 // ------------------------------------------------------------ composite RHS
+static int coarsen_faces_set(const Hier& H, const FaceSet& fs, int n, hipStream_t s)
+{
+   for (int l = H.nlev - 2; l >= 0; l--) {
+      if (H.fcrs_dst[l].n == 0) continue;
+      double af[3], ac[3];
+      face_areas(H, l, af, ac);
+      dim3 g = grid1(H.fcrs_dst[l].n);
+      g.y = n;
+      hipLaunchKernelGGL(k_face_coarsen_set, g, dim3(256), 0, s, fs, H.fcrs_dst[l].p,
+                         H.fcrs_src[l].p, H.fcrs_dir[l].p, H.fcrs_dst[l].n, af[0], af[1], af[2],
+                         ac[0], ac[1], ac[2], H.ndim == 3 ? 4 : 2);
+      AMPE_HIP_CHECK(hipGetLastError());
+   }
+   return 0;
+}
+
+static RhsLev hier_rhs_lev(const Hier& H, const ampe_model_params& p)
+{
+   static_assert(kMaxLev == sizeof(RhsLev) / sizeof(RhsConst), "RhsLev holds every level");
+   RhsLev k = rhs_lev(p);
+   for (int l = 0; l < H.nlev; l++) k.k[l] = rhs_const(lev_params(H, p, l));
+   return k;
+}
+
+// The integrator's right-hand side of the state y (coarsened, ghosts filled, phase
+// concentrations set) over all levels: each kernel runs once over all patches with
+// its level's constants, then the coarse-fine corrections, six launches with the
+// coarsening and the ghosts for a lagged evaluation; level by level and field by
+// field it took 25.
+int hier_rhs_all(const Hier& H, const ampe_model_params& p, const double* y, int iq, int ic,
+                 bool recompute, const double* cl, const double* cs, double* gni, double* Dc,
+                 double* Dphi, double* rhs, hipStream_t s)
+{
+   const Level& L = *H.comp;
+   const RhsLev k = hier_rhs_lev(H, p);
+   if (recompute) {
+      if (iq >= 0 && launch_quat_gni(L, p, k, y + (long long)iq * H.ncg, gni, s)) return -1;
+      if (ic >= 0) {
+         if (launch_conc_coeffs_lev(L, p, k, y, cl, cs, Dc, Dphi, s)) return -1;
+         FaceSet fs{{Dc, Dphi, nullptr}};
+         if (coarsen_faces_set(H, fs, 2, s)) return -1;
+      }
+   }
+   if (launch_rhs_all(L, p, k, y, iq, ic, cl, cs, gni, Dc, Dphi, ic >= 0 ? 1 : 0, rhs, s))
+      return -1;
+   HierCorr hc;
+   hc.n = H.nlev - 1;
+   for (int l = 0; l < hc.n; l++) {
+      hc.cc[l] = H.cfc[l].p;
+      hc.ff[l] = H.cff[l + 1].p;
+      hc.count[l] = (int)H.cfc[l].n;
+      corr_areas(H, l, hc.af[l], hc.ac[l]);
+   }
+   return launch_hier_corr(H.ndim, hc, p, k, H.ncg, y, iq, ic, cl, cs, gni, Dc, Dphi, rhs, s);
+}
+
+int hier_quat_gni(const Hier& H, const ampe_model_params& p, const double* q, double* gni,
+                  hipStream_t s)
+{
+   return launch_quat_gni(*H.comp, p, hier_rhs_lev(H, p), q, gni, s);
+}
+
 int hier_phase_rhs(const Hier& H, const ampe_model_params& p0, const double* phi,
                    const double* q, const double* cl, const double* cs, double* rhs,
                    hipStream_t s)
@@ -1125,11 +1276,8 @@ int hier_conc_coeffs(const Hier& H, const ampe_model_params& p0, const double* p
    for (int l = 0; l < H.nlev; l++)
       if (launch_conc_coeffs(*H.lev[l], lev_params(H, p0, l), phi, cl, cs, Dc, Dphi, s))
          return -1;
-   for (int l = H.nlev - 2; l >= 0; l--) {
-      if (hier_coarsen_faces_level(H, l, Dc, Dc, 1, s)) return -1;
-      if (hier_coarsen_faces_level(H, l, Dphi, Dphi, 1, s)) return -1;
-   }
-   return 0;
+   FaceSet fs{{Dc, Dphi, nullptr}};
+   return coarsen_faces_set(H, fs, 2, s);
 }
 
 int hier_conc_rhs(const Hier& H, const ampe_model_params& p0, const double* c, const double* phi,
@@ -1198,12 +1346,8 @@ int hier_ebs3_coeffs(const Hier& H, const ampe_model_params& p0, int norder, con
    for (int l = 0; l < H.nlev; l++)
       if (launch_ebs3_coeffs(*H.lev[l], lev_params(H, p0, l), norder, phi, DL, DA, DB, s))
          return -1;
-   for (int l = H.nlev - 2; l >= 0; l--) {
-      if (hier_coarsen_faces_level(H, l, DL, DL, 1, s)) return -1;
-      if (hier_coarsen_faces_level(H, l, DA, DA, 1, s)) return -1;
-      if (hier_coarsen_faces_level(H, l, DB, DB, 1, s)) return -1;
-   }
-   return 0;
+   FaceSet fs{{DL, DA, DB}};
+   return coarsen_faces_set(H, fs, 3, s);
 }
 
 int hier_conc_rhs_ebs3(const Hier& H, const ampe_model_params& p0, const double* ph6,
@@ -1699,24 +1843,53 @@ int hier_weight_sum(Hier* H, double* sum)
 int hier_sim_sync_fill(Hier* H, double* y, int nc, int nord, int ic, int ncs, int iq, int qlen,
                        hipStream_t s)
 {
-   if (hier_coarsen(*H, y, nord, 0, s)) return -1;
-   if (ic >= 0 && hier_coarsen(*H, y + (long long)ic * H->ncg, ncs, 0, s)) return -1;
-   if (iq >= 0 && hier_coarsen(*H, y + (long long)iq * H->ncg, qlen, 1, s)) return -1;
-   return hier_ghost_fill(*H, y, nc, 2, s);
+   if (iq >= 0 && qlen != 4) {
+      set_error("hier_sim_sync_fill: four orientation components");
+      return -1;
+   }
+   (void)ic;
+   const int rows = nord + ncs + (iq >= 0 ? 1 : 0);
+   for (int l = H->nlev - 2; l >= 0; l--) {
+      if (H->crs_dst[l].n == 0) continue;
+      dim3 g = grid1(H->crs_dst[l].n);
+      g.y = rows;
+      hipLaunchKernelGGL(k_coarsen_state, g, dim3(256), 0, s, y, H->ncg, iq, H->crs_dst[l].p,
+                         H->crs_src[l].p, H->crs_dst[l].n, cell_vol(*H, l + 1), cell_vol(*H, l),
+                         H->ndim == 3 ? 8 : 4);
+      AMPE_HIP_CHECK(hipGetLastError());
+   }
+   HierGhosts h;
+   h.nlev = H->nlev;
+   long long n = 0;
+   for (int l = 0; l < H->nlev; l++) {
+      const Level& L = *H->lev[l];
+      h.gd[l] = L.ghost_dst;
+      h.gs[l] = L.ghost_src;
+      h.ng[l] = L.nghost;
+      h.cd[l] = H->cf_dst[l].p;
+      h.cs[l] = H->cf_src[l].p;
+      h.cw[l] = H->cf_w[l].p;
+      h.nc[l] = l > 0 ? H->cf_dst[l].n : 0;
+      n += h.ng[l] + h.nc[l];
+   }
+   if (n == 0) return 0;
+   dim3 g = grid1(n);
+   g.y = nc;
+   hipLaunchKernelGGL(k_hier_ghosts, g, dim3(256), 0, s, y, H->ncg, h, H->ndim);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
 }
 
 int hier_precond_coeffs(const Hier& H, const ampe_model_params& p0, double gamma,
-                        const double* phi, const double* cl, const double* cs, const double* n2,
+                        const double* phi, const double* cl, const double* cs, const double* gni,
                         double* Mphi, double* Cphi, double* fc, double* sqrtm, hipStream_t s)
 {
    bool kim = p0.phi_mobility_type == AMPE_PHI_MOB_KIM;
-   for (int l = 0; l < H.nlev; l++) {
-      ampe_model_params p = lev_params(H, p0, l);
-      const Level& L = *H.lev[l];
-      if (kim && launch_phase_mobility(L, p, cl, cs, Mphi, s)) return -1;
-      if (launch_phase_C(L, p, gamma, phi, kim ? Mphi : nullptr, Cphi, s)) return -1;
-      if (fc && launch_quat_face_coef(L, p, phi, n2, fc, s)) return -1;
-   }
+   // none of them depends on the spacing
+   const Level& L = *H.comp;
+   if (kim && launch_phase_mobility(L, p0, cl, cs, Mphi, s)) return -1;
+   if (launch_phase_C(L, p0, gamma, phi, kim ? Mphi : nullptr, Cphi, s)) return -1;
+   if (fc && launch_quat_face_coef_gni(L, p0, phi, gni, fc, s)) return -1;
    // sqrt(M_q) of every ghosted entry (cell-wise, no spacing)
    if (sqrtm && launch_sqrt_quat_mobility(*H.comp, p0, phi, sqrtm, s)) return -1;
    return 0;

@@ -319,6 +319,19 @@ struct CfCorr {
 // Composite right-hand sides: the coarse level's fused kernel has run; each
 // listed coarse cell's divergence takes the finer level's fluxes (their
 // area-weighted average, af / ac) on its coarse-fine faces.
+// All levels and fields at once: the records of the coarser levels 0 .. n - 1 with
+// the finer level's faces.
+struct HierCorr {
+   int n = 0;
+   const CfCorr* cc[4];
+   const CfFace* ff[4];
+   int count[4];
+   double af[4], ac[4];
+};
+int launch_hier_corr(int ndim, const HierCorr& hc, const ampe_model_params& p, const RhsLev& k,
+                     long long ncg, const double* y, int iq, int ic, const double* cl,
+                     const double* cs, const double* gni, const double* Dc, const double* Dphi,
+                     double* rhs, hipStream_t s);
 int launch_hier_phase_corr(int ndim, const CfCorr* cc, int ncorr, const CfFace* ff,
                            const ampe_model_params& pc, const ampe_model_params& pf,
                            long long ncg, const double* phi, const double* q, const double* cl,

@@ -1247,6 +1247,137 @@ __global__ void __launch_bounds__(256) k_hier_quat_corr(const CfCorr* __restrict
    }
 }
 
+// The corrections of every level and field in one launch: blockIdx.y the field
+// (phase; orientation; composition), the records of all levels one after the
+// other.  They read the state and the lagged face data only, so that no order
+// between the levels is needed.  The orientation's face coefficients are formed
+// from the face's 1 / |grad q| as in the level kernel, once per face for its four
+// components.  Bound by the latency of one thread's chain of dependent loads: a
+// three-level 2-D dendrite takes 11 us; one launch per level and
+// field with stored coefficients took 64 us.
+template <int NDIM>
+__global__ void __launch_bounds__(64) k_hier_corr(HierCorr hc, ampe_model_params p, RhsLev kl,
+                                                  long long ncg, const double* __restrict__ phi,
+                                                  const double* __restrict__ q,
+                                                  const double* __restrict__ c,
+                                                  const double* __restrict__ cl,
+                                                  const double* __restrict__ cs,
+                                                  const double* __restrict__ gni,
+                                                  const double* __restrict__ Dc,
+                                                  const double* __restrict__ Dphi,
+                                                  double* __restrict__ yp, double* __restrict__ yq,
+                                                  double* __restrict__ yc)
+{
+   int t = blockIdx.x * blockDim.x + threadIdx.x, l = 0;
+   for (; l < hc.n && t >= hc.count[l]; l++) t -= hc.count[l];
+   if (l >= hc.n) return;
+   const CfCorr& e = hc.cc[l][t];
+   const CfFace* ff = hc.ff[l];
+   const RhsConst &kc = kl.k[l], &kf = kl.k[l + 1];
+   const double af = hc.af[l], ac = hc.ac[l];
+   constexpr int nf = NDIM == 3 ? 4 : 2;
+   const long long c0 = e.cell;
+   const int field = blockIdx.y == 0 ? 0 : (q && blockIdx.y == 1 ? 1 : 2);
+   if (field == 0) {
+      const long long stc[3] = {1, e.sy, e.sz};
+      double delta = 0.0;
+      for (int f = 0; f < e.nface; f++) {
+         const int d = e.d[f];
+         const double fold = phase_face_flux<NDIM>(p, kc, phi, q, ncg, stc, d, e.cm[f], e.c0[f]);
+         double acc = 0.0;
+         for (int r = 0; r < nf; r++) {
+            const CfFace& g = ff[e.fine[f] + r];
+            const long long stf[3] = {1, g.sy, g.sz};
+            acc = acc + phase_face_flux<NDIM>(p, kf, phi, q, ncg, stf, d, g.cm, g.c0) * af;
+         }
+         const double t1 = (acc / ac - fold) * kc.dxinv[d];
+         delta = delta + (e.side[f] ? t1 : -t1);
+      }
+      double mob = p.phi_mobility;
+      if (p.with_conc && p.phi_mobility_type == AMPE_PHI_MOB_KIM)
+         mob = phase_mobility(p, cl[c0], cs[c0]);
+      yp[c0] = yp[c0] + mob * delta;
+   } else if (field == 1) {
+      double ddv[4] = {0.0, 0.0, 0.0, 0.0}, dl[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int f = 0; f < e.nface; f++) {
+         const int d = e.d[f];
+         const long long m0 = e.cm[f], p0 = e.c0[f];
+         const double fcc = quat_face_coef_gni(p, phi[m0], phi[p0], gni[e.face[f]]);
+         double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+         for (int r = 0; r < nf; r++) {
+            const CfFace& g = ff[e.fine[f] + r];
+            const double fcf = quat_face_coef_gni(p, phi[g.cm], phi[g.c0], gni[g.face]);
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+               acc[m] = acc[m] +
+                        fcf * (kf.dxinv[d] * (q[m * ncg + g.c0] - q[m * ncg + g.cm])) * af;
+         }
+#pragma unroll
+         for (int m = 0; m < 4; m++) {
+            const double fold = fcc * (kc.dxinv[d] * (q[m * ncg + p0] - q[m * ncg + m0]));
+            const double fnew = acc[m] / ac;
+            const double dif = e.side[f] ? (fnew - fold) : -(fnew - fold);
+            ddv[m] = ddv[m] + dif * kc.dxinv[d];
+            dl[m] = dl[m] + dif * kc.hdxinv[d];
+         }
+      }
+      double dlam = 0.0, sumq2 = 0.0, qv[4];
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+         qv[m] = q[m * ncg + c0];
+         dlam = dlam - qv[m] * dl[m];
+         sumq2 = sumq2 + qv[m] * qv[m];
+      }
+      dlam = dlam / sumq2;
+      const double mq = quat_mobility(p, phi[c0]);
+#pragma unroll
+      for (int m = 0; m < 4; m++)
+         yq[m * ncg + c0] = yq[m * ncg + c0] - mq * (ddv[m] + 2.0 * qv[m] * dlam);
+   } else {
+      double delta = 0.0;
+      for (int f = 0; f < e.nface; f++) {
+         const int d = e.d[f];
+         const long long fo = e.face[f], m0 = e.cm[f], p0 = e.c0[f];
+         const double fold = kc.dxinv[d] * (Dc[fo] * (c[p0] - c[m0]) + Dphi[fo] * (phi[p0] - phi[m0]));
+         double acc = 0.0;
+#pragma unroll
+         for (int r = 0; r < nf; r++) {
+            const CfFace& g = ff[e.fine[f] + r];
+            const double jf = kf.dxinv[d] * (Dc[g.face] * (c[g.c0] - c[g.cm]) +
+                                             Dphi[g.face] * (phi[g.c0] - phi[g.cm]));
+            acc = acc + jf * af;
+         }
+         const double t1 = kc.dxinv[d] * (acc / ac - fold);
+         delta = delta + (e.side[f] ? t1 : -t1);
+      }
+      yc[c0] = yc[c0] + p.conc_mobility * delta;
+   }
+}
+
+int launch_hier_corr(int ndim, const HierCorr& hc, const ampe_model_params& p, const RhsLev& k,
+                     long long ncg, const double* y, int iq, int ic, const double* cl,
+                     const double* cs, const double* gni, const double* Dc, const double* Dphi,
+                     double* rhs, hipStream_t s)
+{
+   int n = 0;
+   for (int l = 0; l < hc.n; l++) n += hc.count[l];
+   if (n <= 0) return 0;
+   const double* q = iq >= 0 ? y + (long long)iq * ncg : nullptr;
+   const double* c = ic >= 0 ? y + (long long)ic * ncg : nullptr;
+   double* yq = iq >= 0 ? rhs + (long long)iq * ncg : nullptr;
+   double* yc = ic >= 0 ? rhs + (long long)ic * ncg : nullptr;
+   const dim3 g((n + 63) / 64, 1 + (q ? 1 : 0) + (c ? 1 : 0)), b(64);
+   if (ndim == 3)
+      hipLaunchKernelGGL(k_hier_corr<3>, g, b, 0, s, hc, p, k, ncg, y, q, c, cl, cs, gni, Dc, Dphi,
+                         rhs, yq, yc);
+   else
+      hipLaunchKernelGGL(k_hier_corr<2>, g, b, 0, s, hc, p, k, ncg, y, q, c, cl, cs, gni, Dc, Dphi,
+                         rhs, yq, yc);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
 int launch_hier_phase_corr(int ndim, const CfCorr* cc, int ncorr, const CfFace* ff,
                            const ampe_model_params& pc, const ampe_model_params& pf,
                            long long ncg, const double* phi, const double* q, const double* cl,

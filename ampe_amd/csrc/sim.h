@@ -59,7 +59,6 @@ struct Sim {
    double *cl = nullptr, *cs = nullptr, *clr = nullptr, *csr = nullptr;
    // lagged face data and preconditioner coefficients
    double *gni = nullptr, *Dc = nullptr, *Dphi = nullptr, *Dconc = nullptr, *fc = nullptr;
-   double* fcq = nullptr;  // orientation face coefficients of the current RHS evaluation
    double *Cphi = nullptr, *sqrtm = nullptr, *Mphi = nullptr;
    double* phid = nullptr;  // phase field of the EBS isotropic stencil's diffusivities
    double *fac_u = nullptr, *fac_e = nullptr, *fac_r = nullptr;

@@ -170,7 +170,7 @@ static int sim_finish(Sim* S, Sim** out)
    rc |= dalloc(&S->fac_u, S->ng * ql);
    rc |= dalloc(&S->fac_e, S->nv);
    rc |= dalloc(&S->fac_r, S->nv);
-   double** sides[] = {&S->gni, &S->Dc, &S->Dphi, &S->Dconc, &S->fc, &S->fcq};
+   double** sides[] = {&S->gni, &S->Dc, &S->Dphi, &S->Dconc, &S->fc};
    for (auto v : sides) rc |= dalloc(v, S->nf);
    if (S->tern) {
       rc |= dalloc(&S->ph6, 6 * S->ng);
@@ -261,7 +261,7 @@ void sim_destroy(Sim* S)
                     S->ewt, S->work, S->work2, S->jv, S->corr, S->acor, S->cl, S->cs,
                     S->clr, S->csr, S->Cphi, S->sqrtm, S->Mphi, S->fac_u, S->fac_e, S->fac_r,
                     S->gni,
-                    S->Dc, S->Dphi, S->Dconc, S->fc, S->fcq, S->phid, S->z1, S->z2,
+                    S->Dc, S->Dphi, S->Dconc, S->fc, S->phid, S->z1, S->z2,
                     S->ph6, S->Db};
    for (double* v : all) (void)hipFree(v);
    for (double* v : S->V) (void)hipFree(v);
@@ -526,7 +526,6 @@ static int hier_rhs_eval(Sim* S, double* y, double* ydot, bool fd)
    int ql = S->iq >= 0 ? p.qlen : 0;
    if (hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ic, S->ncs, S->iq, ql, st)) return -1;
    const double* phi = y;
-   const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
    if (S->tern) {
       if (kks(S, y)) return -1;
@@ -537,20 +536,9 @@ static int hier_rhs_eval(Sim* S, double* y, double* ydot, bool fd)
                                 ydot + (long long)S->ic * S->ng, st);
    }
    if (S->nord > 1) return hier_phase_rhs_multiorder(*S->hier, p, S->nord, phi, ydot, st);
-   if (q && recompute && hier_quat_face_norm2(*S->hier, p, q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
-   if (hier_phase_rhs(*S->hier, p, phi, q, S->cl, S->cs, ydot, st)) return -1;
-   if (q && hier_quat_rhs(*S->hier, p, phi, q, S->gni, S->fcq, ydot + (long long)S->iq * S->ng,
-                          st))
-      return -1;
-   if (c) {
-      if (recompute && hier_conc_coeffs(*S->hier, p, phi, S->cl, S->cs, S->Dc, S->Dphi, st))
-         return -1;
-      if (hier_conc_rhs(*S->hier, p, c, phi, S->Dc, S->Dphi, ydot + (long long)S->ic * S->ng,
-                        st))
-         return -1;
-   }
-   return 0;
+   return hier_rhs_all(*S->hier, p, y, S->iq, S->ic, recompute, S->cl, S->cs, S->gni, S->Dc,
+                       S->Dphi, ydot, st);
 }
 
 static int hier_psetup(Sim* S, double* y, double gamma, bool fresh)
@@ -564,7 +552,7 @@ static int hier_psetup(Sim* S, double* y, double gamma, bool fresh)
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
-   if (q && !fresh && hier_quat_face_norm2(*S->hier, p, q, S->gni, st)) return -1;
+   if (q && !fresh && hier_quat_gni(*S->hier, p, q, S->gni, st)) return -1;
    if (c && kks(S, y)) return -1;
    // several orders: the well scale passed is 0, so C = 1
    ampe_model_params pw = p;

@@ -274,7 +274,8 @@ __global__ void __launch_bounds__(256) k_hier_tern3_phase_corr(
    const int nf = NDIM == 3 ? 4 : 2;
    const double e2c[3] = {e2c0, e2c1, e2c2}, e2f[3] = {e2f0, e2f1, e2f2};
    const double dxi[3] = {dxi0, dxi1, dxi2};
-   for (int ip = 0; ip < norder; ip++) {
+   {
+      const int ip = blockIdx.y;
       const double* f = phi + (long long)ip * ncg;
       double delta = 0.0;
       for (int k = 0; k < e.nface; k++) {
@@ -317,7 +318,8 @@ __global__ void __launch_bounds__(256) k_hier_ebs3_corr(
    const CfCorr& e = cc[t];
    const int nf = NDIM == 3 ? 4 : 2;
    const double dic[3] = {dxc0, dxc1, dxc2}, dif[3] = {dxf0, dxf1, dxf2};
-   for (int sp = 0; sp < 2; sp++) {
+   {
+      const int sp = blockIdx.y;
       const double* cl = ph + (long long)sp * ncg;
       const double* ca = ph + (long long)(2 + sp) * ncg;
       const double* cb = ph + (long long)(4 + sp) * ncg;
@@ -458,7 +460,7 @@ int launch_hier_tern3_phase_corr(int ndim, const CfCorr* cc, int ncorr, const Cf
    double ec[3], ef[3], dc[3], df[3];
    tern3_e2dx(pc, ndim, ec, dc);
    tern3_e2dx(pf, ndim, ef, df);
-   dim3 g((ncorr + 255) / 256), b(256);
+   dim3 g((ncorr + 255) / 256, norder), b(256);
    if (ndim == 3)
       hipLaunchKernelGGL(k_hier_tern3_phase_corr<3>, g, b, 0, s, cc, ncorr, ff, norder, ncg,
                          ec[0], ec[1], ec[2], ef[0], ef[1], ef[2], dc[0], dc[1], dc[2],
@@ -482,7 +484,7 @@ int launch_hier_ebs3_corr(int ndim, const CfCorr* cc, int ncorr, const CfFace* f
       dc[d] = 1.0 / pc.dx[d];
       df[d] = 1.0 / pf.dx[d];
    }
-   dim3 g((ncorr + 255) / 256), b(256);
+   dim3 g((ncorr + 255) / 256, 2), b(256);
    if (ndim == 3)
       hipLaunchKernelGGL(k_hier_ebs3_corr<3>, g, b, 0, s, cc, ncorr, ff, ncg, dc[0], dc[1],
                          dc[2], df[0], df[1], df[2], pc.conc_mobility, af, ac, ph, DL, DA, DB,
