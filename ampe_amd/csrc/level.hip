@@ -76,22 +76,40 @@ static int level_upload(Level* L, const std::vector<long long>& gd0,
    // whose block starts at or before it; the tables list patch after patch)
    std::vector<long long> gd, gs;
    {
+      const size_t ne = gd0.size();
       std::vector<long long> rd, rs;
-      int p = 0;
-      for (size_t e = 0; e < gd0.size(); e++) {
+      gd.reserve(ne);
+      gs.reserve(ne);
+      rd.reserve(ne);
+      rs.reserve(ne);
+      int p = 0, x = 0, y = 0, z = 0;  // the entry's position in its patch's ghosted box
+      long long at = -1;               // and the entry before it
+      for (size_t e = 0; e < ne; e++) {
+         const bool same = at >= 0 && gd0[e] >= at &&
+                           (p + 1 == npatch || gd0[e] < L->hp[p + 1].cell_off);
          while (p + 1 < npatch && L->hp[p + 1].cell_off <= gd0[e]) p++;
          const PatchDev& d = L->hp[p];
-         const long long loc = gd0[e] - d.cell_off;
-         const int x[3] = {(int)(loc % d.sy) - L->g, (int)((loc % d.sz) / d.sy) - L->g,
-                           (int)(loc / d.sz) - L->gz};
-         const int n[3] = {d.nx, d.ny, d.nz};
-         int out_by = 0, outs = 0;
-         for (int a = 0; a < ndim; a++) {
-            const int o = x[a] < 0 ? -x[a] : (x[a] >= n[a] ? x[a] - n[a] + 1 : 0);
-            out_by = std::max(out_by, o);
-            outs += o > 0;
+         if (same && gd0[e] - at <= d.sy) {
+            // the tables run through a box row by row: mostly one step or one row
+            x += (int)(gd0[e] - at);
+            if (x >= d.sy) {
+               x -= d.sy;
+               if (++y == d.ny + 2 * L->g) {
+                  y = 0;
+                  z++;
+               }
+            }
+         } else {
+            const long long loc = gd0[e] - d.cell_off, row = loc % d.sz;
+            x = (int)(row % d.sy);
+            y = (int)(row / d.sy);
+            z = (int)(loc / d.sz);
          }
-         const bool face = outs == 1 && out_by == 1;
+         at = gd0[e];
+         auto outside = [](int i, int n) { return i < 0 ? -i : (i >= n ? i - n + 1 : 0); };
+         const int ox = outside(x - L->g, d.nx), oy = outside(y - L->g, d.ny),
+                   oz = ndim == 3 ? outside(z - L->gz, d.nz) : 0;
+         const bool face = ox + oy + oz == 1;
          (face ? gd : rd).push_back(gd0[e]);
          (face ? gs : rs).push_back(gs0[e]);
       }
