@@ -95,13 +95,13 @@ int hier_fac_solve(Hier& H, const ampe_hier_block& B, const ampe_fac_params& P, 
 int hier_fac_solve_f32(Hier& H, const HBlock<float>& B, const ampe_fac_params& P, const float* f,
                        float* u, int ncomp, double tol, double* norm, int* cycles, hipStream_t s);
 // One FAC cycle over the levels for all blocks of a set at once, from e = 0
-// (zero on entry): e = the correction, covered cells averaged from the finer
-// level; r = the right-hand side on entry, used up; tmp: work.  All three hold
+// (zero on entry): e = the correction, with covered also on covered cells, averaged
+// from the finer level; r = the right-hand side on entry, used up; tmp: work.  All three hold
 // the set's components.  coarse_its sweeps on level 0, no tolerance test, no
 // norm; bit (component) of ewing selects Ewing's fix for it.
 template <typename T>
 int hier_fac_cycle_set(const Hier& H, const SweepSet<T>& set, int coarse_its,
-                       unsigned long long ewing, T* r, T* e, T* tmp, hipStream_t s);
+                       unsigned long long ewing, T* r, T* e, T* tmp, bool covered, hipStream_t s);
 // Coefficients of the preconditioner setup, all levels: phase C and mobility,
 // orientation face coefficients (gni: the faces' 1 / |grad q|) and sqrt(M_q).
 int hier_precond_coeffs(const Hier& H, const ampe_model_params& p0, double gamma,

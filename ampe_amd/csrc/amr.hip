@@ -1026,9 +1026,12 @@ __global__ void __launch_bounds__(256) k_set_ghosts(T* __restrict__ x, long long
 
 // k_fac_corr for every component of a block set in one launch, the fine face
 // fluxes formed from the fine level's cells here (k_oflux_save's arithmetic)
-// instead of being saved by a launch of their own and read back.
+// instead of being saved by a launch of their own and read back.  One component
+// per blockIdx.y: the chain of dependent loads of a thread, not the bandwidth, is
+// what it takes (three-level 2-D dendrite: 9 us; 33 us with a slot's components
+// one after the other).
 template <typename T>
-__global__ void __launch_bounds__(256) k_set_corr(T* __restrict__ res, const T* __restrict__ x,
+__global__ void __launch_bounds__(64) k_set_corr(T* __restrict__ res, const T* __restrict__ x,
                                                   long long ncg, SweepSet<T> set,
                                                   const CfCorr* __restrict__ cc, long long n,
                                                   const CfFace* __restrict__ ff, int nfine,
@@ -1038,33 +1041,34 @@ __global__ void __launch_bounds__(256) k_set_corr(T* __restrict__ res, const T* 
    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
    if (t >= n) return;
    const CfCorr& e = cc[t];
-   const SweepSlot<T>& o = set.s[blockIdx.y];
-   for (int m = o.comp; m < o.comp + o.ncomp; m++) {
-      const T* u = x + m * ncg;
-      T delta = 0.0;
-      for (int f = 0; f < e.nface; f++) {
-         const int d = e.d[f];
-         const T dinv = d == 0 ? di0 : (d == 1 ? di1 : di2);
-         const T dfin = d == 0 ? df0 : (d == 1 ? df1 : df2);
-         const T dd = o.D ? o.D[e.face[f]] : o.Dc;
-         const T wc = o.kind == 1 ? o.sm[e.c0[f]] * u[e.c0[f]] : u[e.c0[f]];
-         const T wm = o.kind == 1 ? o.sm[e.cm[f]] * u[e.cm[f]] : u[e.cm[f]];
-         const T fold = dinv * dd * (wc - wm);
-         T acc = 0.0;
-         for (int r = 0; r < nfine; r++) {
-            const CfFace& g = ff[e.fine[f] + r];
-            const T gd = o.D ? o.D[g.face] : o.Dc;
-            const T gc = o.kind == 1 ? o.sm[g.c0] * u[g.c0] : u[g.c0];
-            const T gm = o.kind == 1 ? o.sm[g.cm] * u[g.cm] : u[g.cm];
-            acc = acc + dfin * gd * (gc - gm) * af;
-         }
-         const T fnew = acc / ac;
-         const T t1 = dinv * (fnew - fold);
-         delta = delta + (e.side[f] ? t1 : -t1);
+   int i = 0, m = (int)blockIdx.y;  // the m-th component of the set
+   while (m >= set.s[i].ncomp) m -= set.s[i++].ncomp;
+   const SweepSlot<T>& o = set.s[i];
+   m += o.comp;
+   const T* u = x + m * ncg;
+   T delta = 0.0;
+   for (int f = 0; f < e.nface; f++) {
+      const int d = e.d[f];
+      const T dinv = d == 0 ? di0 : (d == 1 ? di1 : di2);
+      const T dfin = d == 0 ? df0 : (d == 1 ? df1 : df2);
+      const T dd = o.D ? o.D[e.face[f]] : o.Dc;
+      const T wc = o.kind == 1 ? o.sm[e.c0[f]] * u[e.c0[f]] : u[e.c0[f]];
+      const T wm = o.kind == 1 ? o.sm[e.cm[f]] * u[e.cm[f]] : u[e.cm[f]];
+      const T fold = dinv * dd * (wc - wm);
+      T acc = 0.0;
+      for (int r = 0; r < nfine; r++) {
+         const CfFace& g = ff[e.fine[f] + r];
+         const T gd = o.D ? o.D[g.face] : o.Dc;
+         const T gc = o.kind == 1 ? o.sm[g.c0] * u[g.c0] : u[g.c0];
+         const T gm = o.kind == 1 ? o.sm[g.cm] * u[g.cm] : u[g.cm];
+         acc = acc + dfin * gd * (gc - gm) * af;
       }
-      const T mm = o.kind == 1 ? o.gamma * o.sm[e.cell] : (o.M ? o.M[e.cell] : o.Mc);
-      res[m * ncg + e.cell] = res[m * ncg + e.cell] - mm * delta;
+      const T fnew = acc / ac;
+      const T t1 = dinv * (fnew - fold);
+      delta = delta + (e.side[f] ? t1 : -t1);
    }
+   const T mm = o.kind == 1 ? o.gamma * o.sm[e.cell] : (o.M ? o.M[e.cell] : o.Mc);
+   res[m * ncg + e.cell] = res[m * ncg + e.cell] - mm * delta;
 }
 
 }  // namespace
@@ -1708,11 +1712,11 @@ static int fac_solve_t(Hier& H, const HBlock<T>& B, const ampe_fac_params& P, co
 // residual follows the cycle (its norm is only reported), ghosts are filled
 // once between two uses, and the fine fluxes of the composite residual are
 // formed where they are used.  Same operations on the same values as
-// fac_solve_t with one cycle.  Three-level 2-D dendrite of 1.5 10^5 cells: 36
-// launches a solve instead of 660, four integrator steps in 31 ms instead of
-// 165; the launches, not the sweeps, are what a solve of this size costs.  Two
-// 3-D levels of 96^3 cells, nine orders and two species: two steps in 124 ms
-// instead of 259.
+// fac_solve_t with one cycle.  Three-level 2-D dendrite of 1.5 10^5 cells: 32
+// launches a solve instead of 660; the launches, not the sweeps, are what a solve
+// of this size costs.  Four integrator steps of it take 18 ms, with solves and
+// right-hand sides block by block and level by level 155 ms; two steps on two 3-D
+// levels of 96^3 cells, nine orders and two species, 108 ms and 256 ms.
 template <typename T>
 struct SetCtx {
    const Hier* H;
@@ -1766,9 +1770,8 @@ static int fac_set_residual(const SetCtx<T>& X, int l, T* res, T* x, const T* b)
          di[d] = (T)(1.0 / H.dx[l][d]);
          df[d] = (T)(1.0 / H.dx[l + 1][d]);
       }
-      dim3 g = grid1(H.facc[l].n);
-      g.y = X.set->n;
-      hipLaunchKernelGGL(k_set_corr<T>, g, dim3(256), 0, X.s, res, x, H.ncg, *X.set, H.facc[l].p,
+      dim3 g((unsigned)((H.facc[l].n + 63) / 64), X.ncomp);
+      hipLaunchKernelGGL(k_set_corr<T>, g, dim3(64), 0, X.s, res, x, H.ncg, *X.set, H.facc[l].p,
                          H.facc[l].n, H.facf[l + 1].p, H.ndim == 3 ? 4 : 2, di[0], di[1], di[2],
                          df[0], df[1], df[2], (T)af, (T)ac);
       AMPE_HIP_CHECK(hipGetLastError());
@@ -1778,15 +1781,14 @@ static int fac_set_residual(const SetCtx<T>& X, int l, T* res, T* x, const T* b)
 
 template <typename T>
 int hier_fac_cycle_set(const Hier& H, const SweepSet<T>& set, int coarse_its,
-                       unsigned long long ewing, T* r, T* e, T* tmp, hipStream_t s)
+                       unsigned long long ewing, T* r, T* e, T* tmp, bool covered, hipStream_t s)
 {
    int nc = 0;
    for (int i = 0; i < set.n; i++) nc += set.s[i].ncomp;
    SetCtx<T> X{&H, &set, nc, ewing, s};
    const int top = H.nlev - 1;
-   // the residual of e = 0: the right-hand side, averaged onto covered cells
-   for (int l = top - 1; l >= 0; l--)
-      if (coarsen_level_t<T>(H, l, r, r, nc, s)) return -1;
+   // the residual of e = 0 is the right-hand side; on covered cells the finer
+   // level's residual takes its place before it is read
    for (int l = top; l >= 1; l--) {
       if (fac_set_smooth(X, l, r, e, 1, true)) return -1;
       if (fac_set_residual(X, l, tmp, e, r)) return -1;
@@ -1797,15 +1799,15 @@ int hier_fac_cycle_set(const Hier& H, const SweepSet<T>& set, int coarse_its,
       if (prolong_level_t<T>(H, l, e, nc, s)) return -1;
       if (fac_set_smooth(X, l, r, e, 1, false)) return -1;
    }
-   for (int l = top - 1; l >= 0; l--)
+   for (int l = top - 1; covered && l >= 0; l--)
       if (coarsen_level_t<T>(H, l, e, e, nc, s)) return -1;
    return 0;
 }
 template int hier_fac_cycle_set<float>(const Hier&, const SweepSet<float>&, int,
-                                       unsigned long long, float*, float*, float*, hipStream_t);
+                                       unsigned long long, float*, float*, float*, bool, hipStream_t);
 template int hier_fac_cycle_set<double>(const Hier&, const SweepSet<double>&, int,
                                         unsigned long long, double*, double*, double*,
-                                        hipStream_t);
+                                        bool, hipStream_t);
 
 static HBlock<double> hblock_of(const ampe_hier_block& B)
 {

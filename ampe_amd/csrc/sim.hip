@@ -462,13 +462,10 @@ int sim_set_time(Sim* S, double t, double h0)
 
 // The state with every finer level coarsened onto the cells it covers (the
 // output QuatIntegrator coarsens after each step, source/QuatIntegrator.cc:
-// 2190-2196); the integrator's own state is left as it is.
-int sim_get_state_composite(Sim* S, double* y_host)
+// 2190-2196), in S->work; the integrator's own state, whose covered cells are
+// undefined between evaluations, is left as it is.
+static int covered_state(Sim* S)
 {
-   if (!S->hier) {
-      set_error("get_state_composite: not a hierarchy sim");
-      return -1;
-   }
    hipStream_t st = S->stream;
    AMPE_HIP_CHECK(hipMemcpyAsync(S->work, S->y, sizeof(double) * S->nv, hipMemcpyDeviceToDevice,
                                  st));
@@ -476,27 +473,37 @@ int sim_get_state_composite(Sim* S, double* y_host)
    if (S->ic >= 0 &&
        hier_coarsen(*S->hier, S->work + (long long)S->ic * S->ng, S->ncs, 0, st))
       return -1;
-   if (S->iq >= 0 &&
-       hier_coarsen(*S->hier, S->work + (long long)S->iq * S->ng, S->p.qlen, 1, st))
+   return S->iq >= 0 ? hier_coarsen(*S->hier, S->work + (long long)S->iq * S->ng, S->p.qlen, 1, st)
+                     : 0;
+}
+
+int sim_get_state_composite(Sim* S, double* y_host)
+{
+   if (!S->hier) {
+      set_error("get_state_composite: not a hierarchy sim");
       return -1;
+   }
+   if (covered_state(S)) return -1;
    AMPE_HIP_CHECK(hipMemcpyAsync(y_host, S->work, sizeof(double) * S->nv, hipMemcpyDeviceToHost,
-                                 st));
-   AMPE_HIP_CHECK(hipStreamSynchronize(st));
+                                 S->stream));
+   AMPE_HIP_CHECK(hipStreamSynchronize(S->stream));
    return 0;
 }
 
 int sim_get_state(Sim* S, double* phi, double* c, double* q, double* cl, double* cs)
 {
    const Level& L = *S->L;
+   if (S->hier && covered_state(S)) return -1;
+   const double* y = S->hier ? S->work : S->y;
    AMPE_HIP_CHECK(hipStreamSynchronize(S->stream));
    for (int m = 0; phi && m < S->nord; m++)
-      if (gather_interior(S, S->y + (long long)m * S->ng, phi + (long long)m * L.ncell)) return -1;
+      if (gather_interior(S, y + (long long)m * S->ng, phi + (long long)m * L.ncell)) return -1;
    for (int m = 0; c && m < S->ncs; m++)
-      if (gather_interior(S, S->y + (long long)(S->ic + m) * S->ng, c + (long long)m * L.ncell))
+      if (gather_interior(S, y + (long long)(S->ic + m) * S->ng, c + (long long)m * L.ncell))
          return -1;
    if (q && S->iq >= 0)
       for (int m = 0; m < S->p.qlen; m++)
-         if (gather_interior(S, S->y + (long long)(S->iq + m) * S->ng, q + (long long)m * L.ncell))
+         if (gather_interior(S, y + (long long)(S->iq + m) * S->ng, q + (long long)m * L.ncell))
             return -1;
    // the three-phase model: cl = liquid, cs = solid A, two species each
    for (int m = 0; S->ic >= 0 && m < S->ncs; m++) {
@@ -638,7 +645,7 @@ static int add_orientation(const Sim* S, SweepSet<T>& set, int comp)
 // sweeps on the coarsest level agree, else the orientation block after the
 // elliptic ones.
 template <typename T>
-static int hier_psolve_set(Sim* S, T* r, T* e, T* tmp)
+static int hier_psolve_set(Sim* S, T* r, T* e, T* tmp, bool covered)
 {
    const bool q = S->iq >= 0;
    const bool one = q && S->s.quat_sweeps == S->s.fac_sweeps;
@@ -647,20 +654,22 @@ static int hier_psolve_set(Sim* S, T* r, T* e, T* tmp)
    if (add_elliptic<T>(S, set)) return -1;
    if (one && add_orientation<T>(S, set, S->iq)) return -1;
    if (hier_fac_cycle_set<T>(*S->hier, set, S->s.fac_sweeps, (1ULL << nell) - 1, r, e, tmp,
-                             S->stream))
+                             covered, S->stream))
       return -1;
    if (!q || one) return 0;
    const long long off = (long long)S->iq * S->ng;
    SweepSet<T> qs;
    if (add_orientation<T>(S, qs, 0)) return -1;
    return hier_fac_cycle_set<T>(*S->hier, qs, S->s.quat_sweeps, 0, r + off, e + off, tmp + off,
-                                S->stream);
+                                covered, S->stream);
 }
 
 // Of the preconditioner solve.  f_ready: the right-hand side is formed already
 // (orientation components divided by sqrt(M)), with the FP32 preconditioner in
 // S->f_f, else in r, which the solve may overwrite.  keep: the solution is left
-// as the blocks have it (orientation components without sqrt(M)), in S->f_u or z.
+// as the blocks have it (orientation components without sqrt(M)), in S->f_u or z,
+// a hierarchy's covered cells undefined: a state is averaged onto them before it is
+// used, and sums give them no weight.
 struct PsolveOpts {
    bool f_ready = false;
    bool keep = false;
@@ -697,13 +706,14 @@ static int hier_psolve(Sim* S, const double* r, double* z, double delta, const P
                        : psolve_in<float>(ng, S->nc, iq, ql, r, S->sqrtm, S->f_f, nullptr, S->f_u,
                                           st))
             return -1;
-         if (hier_psolve_set<float>(S, S->f_f, S->f_u, S->f_r)) return -1;
+         if (hier_psolve_set<float>(S, S->f_f, S->f_u, S->f_r, !o.keep)) return -1;
          return o.keep ? 0 : psolve_out<float>(ng, S->nc, iq, ql, S->f_u, S->sqrtm, z, st);
       }
       if (o.f_ready ? fill_zero(z, S->nv, st)
                     : psolve_in<double>(ng, S->nc, iq, ql, r, S->sqrtm, S->fac_e, nullptr, z, st))
          return -1;
-      if (hier_psolve_set<double>(S, o.f_ready ? const_cast<double*>(r) : S->fac_e, z, S->fac_r))
+      if (hier_psolve_set<double>(S, o.f_ready ? const_cast<double*>(r) : S->fac_e, z, S->fac_r,
+                                   !o.keep))
          return -1;
       if (!o.keep && S->iq >= 0 && vec_mul_comp(S, z + (long long)S->iq * ng, S->sqrtm, ql))
          return -1;

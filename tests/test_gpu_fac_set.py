@@ -7,6 +7,8 @@ patches with the orientation block, with equal and unequal sweep counts
 (one set, or the orientation after the elliptic blocks), nine orders and two
 species on two periodic 3-D levels (slots of four, four and one component)
 and fifty orders in 2-D (thirteen slots), in FP64 and FP32."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -91,3 +93,34 @@ def test_set_solve_matches_block_by_block(dev, case, fp32):
     for m in range(sim.nc):
         for (*_, a), (*_, b) in zip(h.patch_blocks(got[0][0], m), h.patch_blocks(got[1][0], m)):
             assert np.array_equal(a, b), (case, m, float(np.max(np.abs(a - b))))
+
+
+def test_state_after_steps_is_averaged(dev):
+    """The integrator's solve leaves covered cells undefined: both state outputs
+    hold the averages there, and the steps do not depend on what was there."""
+    from ampe_amd import hip as H
+    nd, levels, dom0, periodic = 2, [[((0, 0), (15, 15))], [((8, 8), (23, 23))]], (16, 16), True
+    p = P.two_grain_params(ndim=nd)
+    p.quad_ceq[0], p.quad_ceq[1] = 0.40, 0.45
+    h = H.Hier(nd, levels, dom0, (1.0,) * 3, periodic)
+    sim = H.HierSim(p, P.solver_defaults(dt=1e-3), h)
+    rng = np.random.Generator(np.random.Philox(2))
+    y = rng.uniform(0.4, 0.6, (sim.nc, h.ncg))
+    y[sim.nc - 4:] /= np.sqrt((y[sim.nc - 4:] ** 2).sum(0))
+    sim.set_state(y.ravel())
+    rc, _ = sim.advance(2)
+    assert rc == 0
+    a = sim.get_state().reshape(sim.nc, -1)
+    ncell = 16 * 16 + 16 * 16
+    f = [np.zeros(ncell), np.zeros(ncell), np.zeros((4, ncell))]
+    ptr = lambda v: v.ctypes.data_as(C.c_void_p)  # noqa: E731
+    H.check(H.lib().ampe_sim_get_state(sim.h, ptr(f[0]), ptr(f[1]), ptr(f[2]), None, None))
+    # level 0's interior of the composite layout, cells 4..11 covered
+    for m, v in enumerate([f[0], f[1], *f[2]]):
+        c = a[m, :18 * 18].reshape(18, 18)[1:-1, 1:-1]
+        fine = a[m, 18 * 18:].reshape(18, 18)[1:-1, 1:-1]
+        assert np.array_equal(v[:256].reshape(16, 16), c)
+        assert np.array_equal(v[256:].reshape(16, 16), fine)
+        if m < 2:
+            avg = 0.25 * (fine[::2, ::2] + fine[1::2, ::2] + fine[::2, 1::2] + fine[1::2, 1::2])
+            assert np.max(np.abs(c[4:12, 4:12] - avg)) <= 8 * 2.0 ** -53
