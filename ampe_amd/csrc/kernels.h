@@ -178,6 +178,7 @@ struct RhsConst {
    double e2dx12[3];  // eps_phi^2/(12 dx)
    double convL, convA;  // 1e-6/v_m of the liquid and the solid
    double maxgni;     // 1/gradient_floor
+   double logk, dG;   // dilute solution: log k_e, dilute_dG
    double Dl, Ds;     // D_L0 exp(-Q_L/RT), D_S0 exp(-Q_S/RT)
 };
 RhsConst rhs_const(const ampe_model_params& p);

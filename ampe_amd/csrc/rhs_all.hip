@@ -18,7 +18,8 @@
 // (155 registers): a bound of 128 registers spills (1736 us), and a thread that
 // goes on to the next planes holds back the loads behind its stores (2671 us for
 // one plane a thread in that form).  Lagged on 151 x 93 x 67: 71 us.  Anisotropic
-// dilute alloy, 1500 x 1130: 98 us.
+// dilute alloy, 1500 x 1130: 81 us (98 with a face angle from four transcendentals
+// and the logarithm of k_e taken in every cell).
 #include <type_traits>
 
 #include "rhs_dev.h"

