@@ -222,10 +222,13 @@ int launch_quat_face_coef_gni(const Level& L, const ampe_model_params& p, const 
 // conc, in one launch (rhs_all.hip): q null for no orientation, cl / cs null for
 // no composition; conc 0: none, 1: from the stored Dc and Dphi, 2: Dc and Dphi
 // formed and stored too.  rhs: the state vector's components, iq and ic the
-// orientation's and the composition's.
+// orientation's and the composition's.  fin (conc 0 or 1): the values go on to the
+// preconditioner's input (krylov.h), rhs is not written.
+struct KryFin;
 int launch_rhs_all(const Level& L, const ampe_model_params& p, const RhsLev& k, const double* y,
                    int iq, int ic, const double* cl, const double* cs, const double* gni,
-                   double* Dc, double* Dphi, int conc, double* rhs, hipStream_t s);
+                   double* Dc, double* Dphi, int conc, double* rhs, hipStream_t s,
+                   const KryFin* fin = nullptr);
 int launch_conc_coeffs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
                            const double* phi, const double* cl, const double* cs, double* Dc,
                            double* Dphi, hipStream_t s);

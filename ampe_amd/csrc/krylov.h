@@ -34,14 +34,37 @@ struct VecList {
    double y[kMaxKrylov];
 };
 
-// work2 = sig (z h) + ycur
+// What makes the next preconditioner right-hand side of a difference quotient's
+// jv: v = z h + (-gamma) (siginv jv + (-siginv) f), written to out and as pin says
+// (with pin.f out may be null).
+struct KryFin {
+   const double* z = nullptr;
+   double h = 0.0, siginv = 0.0, gamma = 0.0;
+   const double* f = nullptr;
+   double* out = nullptr;
+   PrecIn pin;
+};
+
+__device__ __forceinline__ bool in_range(int m, int iq, int ql) { return m >= iq && m < iq + ql; }
+
+__device__ __forceinline__ void prec_in(const LevelArgs& a, const PrecIn& pin, const CellPos& c,
+                                        long long sp, int m, double v, double sm, double* out)
+{
+   if (pin.sm && in_range(m, pin.iq, pin.ql)) v = v / sm;
+   if (out) out[m * a.ncg + c.c0] = v;
+   if (pin.f) pin.f[m * a.ncg + (m >= pin.sp0 ? sp : c.c0)] = (float)v;
+}
+
+__device__ __forceinline__ double kry_fin(const KryFin& k, long long i, double jv)
+{
+   return k.z[i] * k.h + (-k.gamma) * (k.siginv * jv + (-k.siginv) * k.f[i]);
+}
+
+// work2 = sig (z h) + ycur; with ghosts also on the level's ghost cells, from the
+// cells they copy.
 int kry_mid(const Level& L, int nc, double sig, const double* z, double h, const double* ycur,
-            double* work2, hipStream_t s);
-// v = z h + (-gamma) (siginv jv + (-siginv) fcur), written as pin says; with
-// pin.f out may be null.
-int kry_finish(const Level& L, int nc, double siginv, double gamma, const double* z, double h,
-               const double* jv, const double* fcur, double* out, const PrecIn& pin,
-               hipStream_t s);
+            double* work2, bool ghosts, hipStream_t s);
+int kry_finish(const Level& L, int nc, const KryFin& fin, const double* jv, hipStream_t s);
 // b = gamma f - (y - a), written as pin says (out may be null with pin.f).
 int kry_newton_rhs(const Level& L, int nc, double gamma, const double* f, const double* y,
                    const double* ah, double* out, const PrecIn& pin, hipStream_t s);

@@ -70,8 +70,6 @@ __device__ __forceinline__ Pair pair_of(const LevelArgs& a, const CellPos& c, in
    return p;
 }
 
-__device__ __forceinline__ bool in_range(int m, int iq, int ql) { return m >= iq && m < iq + ql; }
-
 // Component m of the vector src describes, at cell c.
 __device__ __forceinline__ double prec_out(const LevelArgs& a, const PrecOut& src, const CellPos& c,
                                            long long sp, int m, double sm)
@@ -82,46 +80,46 @@ __device__ __forceinline__ double prec_out(const LevelArgs& a, const PrecOut& sr
    return v;
 }
 
-__device__ __forceinline__ void prec_in(const LevelArgs& a, const PrecIn& pin, const CellPos& c,
-                                        long long sp, int m, double v, double sm, double* out)
-{
-   if (pin.sm && in_range(m, pin.iq, pin.ql)) v = v / sm;
-   if (out) out[m * a.ncg + c.c0] = v;
-   if (pin.f) pin.f[m * a.ncg + (m >= pin.sp0 ? sp : c.c0)] = (float)v;
-}
-
-__global__ void __launch_bounds__(256) k_kry_mid(LevelArgs a, int nc, double sig,
+// Workgroups from ntiles on take the ghosts (dst a copy of src), so that the
+// stencils that follow need no launch of their own for them.
+__global__ void __launch_bounds__(256) k_kry_mid(LevelArgs a, int nc, int ntiles, double sig,
                                                  const double* __restrict__ z, double h,
                                                  const double* __restrict__ ycur,
-                                                 double* __restrict__ work2)
+                                                 double* __restrict__ work2,
+                                                 const long long* __restrict__ dst,
+                                                 const long long* __restrict__ src, long long ng)
 {
-   CellPos c;
-   if (!cell_pos(a, 0, c)) return;
-#pragma unroll 2
-   for (int m = 0; m < nc; m++) {
-      const long long i = m * a.ncg + c.c0;
-      work2[i] = sig * (z[i] * h) + ycur[i];
+   long long from, to;
+   if ((int)blockIdx.x < ntiles) {
+      CellPos c;
+      if (!cell_pos(a, 0, c)) return;
+      from = to = c.c0;
+   } else {
+      const long long e = (long long)((int)blockIdx.x - ntiles) * (TX * TY) +
+                          (int)(threadIdx.x + TX * threadIdx.y);
+      if (e >= ng) return;
+      to = dst[e];
+      from = src[e];
    }
+#pragma unroll 2
+   for (int m = 0; m < nc; m++)
+      work2[m * a.ncg + to] = sig * (z[m * a.ncg + from] * h) + ycur[m * a.ncg + from];
 }
 
-__global__ void __launch_bounds__(256) k_kry_finish(LevelArgs a, int nc, double siginv,
-                                                    double gamma, const double* __restrict__ z,
-                                                    double h, const double* __restrict__ jv,
-                                                    const double* __restrict__ fcur,
-                                                    double* out, PrecIn pin)
+__global__ void __launch_bounds__(256) k_kry_finish(LevelArgs a, int nc, KryFin fin,
+                                                    const double* __restrict__ jv)
 {
    CellPos c;
    if (!cell_pos(a, 0, c)) return;
-   const long long sp = pin.sp0 < nc ? split_at(a, c, 0) : 0;
-   const double sm = pin.sm ? pin.sm[c.c0] : 1.0;
+   const long long sp = fin.pin.sp0 < nc ? split_at(a, c, 0) : 0;
+   const double sm = fin.pin.sm ? fin.pin.sm[c.c0] : 1.0;
    for (int m = 0; m < nc; m += 2) {
       const Pair p = pair_of(a, c, nc, m);
       double v[2];
 #pragma unroll
-      for (int e = 0; e < 2; e++)
-         v[e] = z[p.i[e]] * h + (-gamma) * (siginv * jv[p.i[e]] + (-siginv) * fcur[p.i[e]]);
-      prec_in(a, pin, c, sp, m, v[0], sm, out);
-      if (m + 1 < nc) prec_in(a, pin, c, sp, m + 1, v[1], sm, out);
+      for (int e = 0; e < 2; e++) v[e] = kry_fin(fin, p.i[e], jv[p.i[e]]);
+      prec_in(a, fin.pin, c, sp, m, v[0], sm, fin.out);
+      if (m + 1 < nc) prec_in(a, fin.pin, c, sp, m + 1, v[1], sm, fin.out);
    }
 }
 
@@ -346,17 +344,19 @@ __global__ void __launch_bounds__(256) k_newton_update(LevelArgs a, int nc, VecL
    } while (0)
 
 int kry_mid(const Level& L, int nc, double sig, const double* z, double h, const double* ycur,
-            double* work2, hipStream_t s)
+            double* work2, bool ghosts, hipStream_t s)
 {
-   AMPE_TILE_LAUNCH(k_kry_mid, nc, sig, z, h, ycur, work2);
+   const long long ng = ghosts ? L.nghost : 0;
+   hipLaunchKernelGGL(k_kry_mid, dim3(L.ncell_tiles + (unsigned)((ng + TX * TY - 1) / (TX * TY))),
+                      dim3(TX, TY), 0, s, level_args(L), nc, L.ncell_tiles, sig, z, h, ycur, work2,
+                      L.ghost_dst, L.ghost_src, ng);
+   AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
 
-int kry_finish(const Level& L, int nc, double siginv, double gamma, const double* z, double h,
-               const double* jv, const double* fcur, double* out, const PrecIn& pin,
-               hipStream_t s)
+int kry_finish(const Level& L, int nc, const KryFin& fin, const double* jv, hipStream_t s)
 {
-   AMPE_TILE_LAUNCH(k_kry_finish, nc, siginv, gamma, z, h, jv, fcur, out, pin);
+   AMPE_TILE_LAUNCH(k_kry_finish, nc, fin, jv);
    return 0;
 }
 

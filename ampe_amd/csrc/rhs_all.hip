@@ -22,13 +22,19 @@
 // and the logarithm of k_e taken in every cell).
 #include <type_traits>
 
+#include "krylov.h"
 #include "rhs_dev.h"
 
 namespace ampe {
 
 namespace {
 
-template <int NDIM, int FE, int CONC>
+// FIN: the right-hand side is a difference quotient's, and goes on to the
+// preconditioner's input (KryFin) without being stored.  128^3, six components:
+// 43 us less per Krylov iteration than storing it for a launch that reads it (of
+// some 800 us), 128^2: two launches fewer of thirteen with the ghosts filled by
+// the kernel that forms the state.
+template <int NDIM, int FE, int CONC, bool FIN>
 __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_params& p,
                                          const RhsConst& k, const CellPos& c, double r,
                                          const double* __restrict__ phi,
@@ -38,9 +44,23 @@ __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_pa
                                          const double* __restrict__ cs,
                                          const double* __restrict__ gni, double* __restrict__ Dc,
                                          double* __restrict__ Dphi, double* __restrict__ yp,
-                                         double* __restrict__ yq, double* __restrict__ yc)
+                                         double* __restrict__ yq, double* __restrict__ yc,
+                                         const KryFin& fin, int iq, int ic)
 {
    const long long c0 = c.c0, ncg = a.ncg;
+   long long sp = 0;
+   double sm = 1.0;
+   if (FIN) {
+      if (fin.pin.sp0 < (1 << 30)) sp = split_at(a, c, 0);
+      if (fin.pin.sm) sm = fin.pin.sm[c0];
+   }
+   // component m of the state vector, at field y's entry i
+   auto put = [&](double* y, long long i, int m, double v) {
+      if (FIN)
+         prec_in(a, fin.pin, c, sp, m, kry_fin(fin, m * ncg + c0, v), sm, fin.out);
+      else
+         y[i] = v;
+   };
    const double* dinv = k.dxinv;
    const double* hd = k.hdxinv;
    constexpr int NF = 2 * NDIM;  // faces: low of direction d at d, high at NDIM + d
@@ -102,7 +122,7 @@ __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_pa
       const double mq = quat_mobility(p, ph);
 #pragma unroll
       for (int m = 0; m < 4; m++)
-         yq[m * ncg + c0] = 0.0 - mq * (dv[m] + 2.0 * qv[m] * lam);
+         put(yq, m * ncg + c0, iq + m, 0.0 - mq * (dv[m] + 2.0 * qv[m] * lam));
       const double mf = 2.0 * p.H_parameter, T = p.temperature;
       const double eq2 = 0.5 * p.epsilon_q * p.epsilon_q;
       const double gm = sqrt(g2);
@@ -114,7 +134,7 @@ __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_pa
       r += phase_drive<FE>(p, k, ph, cl[c0], cs[c0]);
       if (p.phi_mobility_type == AMPE_PHI_MOB_KIM) mob = phase_mobility_t<FE>(p, cl[c0], cs[c0]);
    }
-   yp[c0] = mob * r;
+   put(yp, c0, 0, mob * r);
    if (CONC == 0) return;
    const double cv = cc[c0];
    double Df[NF], Ef[NF];  // Dc and Dphi of the faces
@@ -151,12 +171,12 @@ __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_pa
       const double t = dinv[d] * (jh - jl);
       s = (d == 0) ? t : s + t;
    }
-   yc[c0] = p.conc_mobility * s;
+   put(yc, c0, ic, p.conc_mobility * s);
 }
 
 // One cell per thread; the anisotropic flux (four transcendentals a face) is
 // evaluated once per x and y face through LDS (k_phase_rhs_faces).
-template <int NDIM, int FLUX, int FE, int CONC>
+template <int NDIM, int FLUX, int FE, int CONC, bool FIN>
 __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params p, RhsLev kl,
                                                  const double* __restrict__ phi,
                                                  const double* __restrict__ q,
@@ -167,7 +187,8 @@ __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params 
                                                  double* __restrict__ Dc,
                                                  double* __restrict__ Dphi,
                                                  double* __restrict__ yp, double* __restrict__ yq,
-                                                 double* __restrict__ yc)
+                                                 double* __restrict__ yc, KryFin fin, int iq,
+                                                 int ic)
 {
    if constexpr (FLUX == AMPE_FLUX_ANISOTROPIC) {
       __shared__ double fx[TY][TX + 1];
@@ -211,8 +232,9 @@ __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params 
          double fhi = phase_face_flux<NDIM, FLUX>(p, k, phi, q, a.ncg, c.st, 2, c0, c0 + sz);
          r = r + (fhi - flo) * k.dxinv[2];
       }
-      rhs_tail<NDIM, FE, CONC>(a, p, k, c, r, phi, q, cc, cl, cs, gni, Dc, Dphi,
-                               yp, yq, yc);
+      rhs_tail<NDIM, FE, CONC, FIN>(a, p, k, c, r, phi, q, cc, cl, cs, gni, Dc, Dphi,
+                               yp, yq, yc, fin, iq,
+                                    ic);
    } else {
       CellPos c;
       if (!cell_pos(a, 0, c)) return;
@@ -226,7 +248,8 @@ __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params 
          double dt = (fhi - flo) * k.dxinv[d];
          r = (d == 0) ? dt : r + dt;
       }
-      rhs_tail<NDIM, FE, CONC>(a, p, k, c, r, phi, q, cc, cl, cs, gni, Dc, Dphi, yp, yq, yc);
+      rhs_tail<NDIM, FE, CONC, FIN>(a, p, k, c, r, phi, q, cc, cl, cs, gni, Dc, Dphi, yp, yq, yc, fin, iq,
+                                    ic);
    }
 }
 
@@ -234,19 +257,30 @@ __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params 
 
 int launch_rhs_all(const Level& L, const ampe_model_params& p, const RhsLev& k, const double* y,
                    int iq, int ic, const double* cl, const double* cs, const double* gni,
-                   double* Dc, double* Dphi, int conc, double* rhs, hipStream_t s)
+                   double* Dc, double* Dphi, int conc, double* rhs, hipStream_t s, const KryFin* fin)
 {
+   if (fin && conc > 1) {
+      set_error("rhs: a full evaluation's values are stored");
+      return -1;
+   }
+   const KryFin kf = fin ? *fin : KryFin{};
    const int fe = ic >= 0 ? p.fe_model : kFeNone;
    const double* q = iq >= 0 ? y + (long long)iq * L.ncg : nullptr;
    const double* cc = ic >= 0 ? y + (long long)ic * L.ncg : nullptr;
    double* yq = iq >= 0 ? rhs + (long long)iq * L.ncg : nullptr;
    double* yc = ic >= 0 ? rhs + (long long)ic * L.ncg : nullptr;
    const LevelArgs a = level_args(L);
-   auto go = [&](auto nd, auto fl, auto f, auto cn) {
+   auto go2 = [&](auto nd, auto fl, auto f, auto cn, auto fi) {
       hipLaunchKernelGGL((k_rhs_all<decltype(nd)::value, decltype(fl)::value, decltype(f)::value,
-                                    decltype(cn)::value>),
+                                    decltype(cn)::value, decltype(fi)::value>),
                          dim3(L.ncell_tiles), dim3(TX, TY), 0, s, a, p, k, y, q, cc, cl, cs, gni,
-                         Dc, Dphi, rhs, yq, yc);
+                         Dc, Dphi, rhs, yq, yc, kf, iq, ic);
+   };
+   auto go = [&](auto nd, auto fl, auto f, auto cn) {
+      if constexpr (decltype(cn)::value < 2) {
+         if (fin) return go2(nd, fl, f, cn, std::true_type());
+      }
+      go2(nd, fl, f, cn, std::false_type());
    };
    using I0 = std::integral_constant<int, 0>;
    using I1 = std::integral_constant<int, 1>;

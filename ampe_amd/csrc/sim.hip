@@ -803,7 +803,18 @@ static int hier_psolve(Sim* S, const double* r, double* z, double delta, const P
    return ret;
 }
 
-static int rhs_eval(Sim* S, double* y, double* ydot, bool fd)
+// A lagged evaluation of the KKS or pure phase form on one level, whose values one
+// launch forms, so that they can go on to the preconditioner's input.
+static bool rhs_fin_ok(const Sim* S)
+{
+   return !S->hier && !S->tern && S->nord == 1 && S->s.lag_quat_sidegrad &&
+          !(S->ic >= 0 && S->p.conc_rhs_form == AMPE_CONC_RHS_EBS);
+}
+
+// ghosts: y's are filled.  fin (rhs_fin_ok, fd): ydot is not written, the
+// preconditioner's input is.
+static int rhs_eval(Sim* S, double* y, double* ydot, bool fd, bool ghosts = false,
+                    const KryFin* fin = nullptr)
 {
    if (S->hier) return hier_rhs_eval(S, y, ydot, fd);
    const Level& L = *S->L;
@@ -811,7 +822,7 @@ static int rhs_eval(Sim* S, double* y, double* ydot, bool fd)
    hipStream_t st = S->stream;
    bool recompute = !fd || !S->s.lag_quat_sidegrad;
    S->st.nfe++;
-   if (ghost_fill(L, y, S->nc, st)) return -1;
+   if (!ghosts && ghost_fill(L, y, S->nc, st)) return -1;
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
@@ -831,7 +842,7 @@ static int rhs_eval(Sim* S, double* y, double* ydot, bool fd)
    if (c && kks(S, y)) return -1;
    const bool ebs = c && p.conc_rhs_form == AMPE_CONC_RHS_EBS;
    if (launch_rhs_all(L, p, k, y, S->iq, S->ic, S->cl, S->cs, S->gni, S->Dc, S->Dphi,
-                      !c || ebs ? 0 : (recompute ? 2 : 1), ydot, st))
+                      !c || ebs ? 0 : (recompute ? 2 : 1), ydot, st, fin))
       return -1;
    if (ebs) {
       // Dc, Dphi hold the liquid and solid face diffusivities
@@ -1392,12 +1403,18 @@ static int spgmr(Sim* S, double gamma, const KryIo& io, VecList* x, double delta
    const double sig = std::sqrt(cv / wfac), siginv = 1.0 / sig;
    for (int l = 0; l < maxl; l++) {
       S->st.nli++;
-      if (kry_mid(L, nc, sig, S->V[l], hs[l], S->ycur, S->work2, st)) return -1;
-      if (rhs_eval(S, S->work2, S->jv, true)) return -1;
+      if (kry_mid(L, nc, sig, S->V[l], hs[l], S->ycur, S->work2, !S->hier, st)) return -1;
       // the solve's right-hand side: FP32, or FP64 in V[l + 1]
-      if (kry_finish(L, nc, siginv, gamma, S->V[l], hs[l], S->jv, S->fcur,
-                     io.in.f ? nullptr : S->V[l + 1], io.in, st))
-         return -1;
+      KryFin fin;
+      fin.z = S->V[l];
+      fin.h = hs[l];
+      fin.siginv = siginv;
+      fin.gamma = gamma;
+      fin.f = S->fcur;
+      fin.out = io.in.f ? nullptr : S->V[l + 1];
+      fin.pin = io.in;
+      if (rhs_eval(S, S->work2, S->jv, true, !S->hier, rhs_fin_ok(S) ? &fin : nullptr)) return -1;
+      if (!rhs_fin_ok(S) && kry_finish(L, nc, fin, S->jv, st)) return -1;
       if (psolve(S, S->V[l + 1], S->work, delta, o) < 0) return -1;
       double hn, sums[kMaxKrylov + 2];
       VecList vl;

@@ -103,3 +103,50 @@ def test_classical_matches_modified(dev, n, cuts, fp32, mg, model):
     size = np.concatenate([b / (s.rtol * np.abs(b) + s.atol) for b in res[1]])
     bound = 100 * np.sqrt(np.mean(size ** 2)) * 2.0 ** (-24 if fp32 else -53)
     assert np.sqrt(np.mean(ew ** 2)) <= bound, (np.sqrt(np.mean(ew ** 2)), bound)
+
+
+@pytest.mark.parametrize("n,cuts,fp32,mg", [((48, 40, 1), (), False, False),
+                                            ((66, 34, 1), (33,), True, False),
+                                            ((64, 32, 1), (), True, True),
+                                            ((16, 12, 8), (), True, True),
+                                            ((17, 6, 5), (9,), False, False)])
+@pytest.mark.parametrize("make,kw", [
+    (P.two_grain_params, {}), (P.two_grain_params, dict(evolve_quat=0)),
+    (P.two_grain_params, dict(with_conc=0)), (P.two_grain_params, dict(with_conc=0, evolve_quat=0)),
+    (P.two_grain_params, dict(flux_type=P.FLUX_ISOTROPIC)),
+    (P.dilute_params, dict(flux_type=P.FLUX_ANISOTROPIC, aniso_nu=0.03))])
+def test_values_passed_on_match_stored(dev, n, cuts, fp32, mg, make, kw):
+    """A lagged evaluation passes its values on to the preconditioner's input, an
+    unlagged one stores them for a launch of their own.  Where nothing that is
+    lagged varies (gradients below the floor, equal phases) the two take the same
+    steps to the last bit."""
+    from ampe_amd import hip as H
+    nd = 3 if n[2] > 1 else 2
+    shape = (n[2], n[1], n[0]) if nd == 3 else (n[1], n[0])
+    rng = np.random.Generator(np.random.Philox(8))
+    p = make(ndim=nd, **kw)
+    p.gradient_floor = 1e6
+    p.D_solid, p.Q0_solid = p.D_liquid, p.Q0_liquid
+    p.quad_ceq[0] = p.quad_ceq[1] = 0.4
+    p.dilute_keq = 1.0
+    phi, c = rng.uniform(0.3, 0.7, shape), rng.uniform(0.35, 0.45, shape)
+    q = rng.normal(size=(4,) + shape) * 0.1 + 1.0
+    q /= np.sqrt((q ** 2).sum(0))
+    boxes, dom = _boxes(n, cuts)
+    cut = lambda a: np.concatenate([a[..., b.lo[0]:b.hi[0] + 1].reshape(*a.shape[:a.ndim - nd], -1)  # noqa: E731
+                                    for b in boxes], -1)
+    res = []
+    for lag in (0, 1):
+        s = P.solver_defaults(maxl=5, max_newton=5, dt=1e-8, lag_quat_sidegrad=lag,
+                              gstype=P.GS_CLASSICAL if fp32 else P.GS_MODIFIED,
+                              precision=P.FAC_FP32 if fp32 else P.FP64,
+                              precond=P.PRECOND_MG if mg else P.PRECOND_REDBLACK)
+        sim = H.Sim(p, s, boxes, periodic=dom)
+        sim.set_state(cut(phi), cut(c) if p.with_conc else None, cut(q) if p.evolve_quat else None)
+        rc, st = sim.advance(2)
+        assert rc == 0 and st["nli"] > 0, (rc, st)
+        f = sim.get_state((sim.ncell,))
+        res.append([f[0]] + ([f[1], f[3], f[4]] if p.with_conc else []) +
+                   ([f[2]] if p.evolve_quat else []))
+    for a, b in zip(*res):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b), float(np.max(np.abs(a - b)))
