@@ -824,29 +824,6 @@ __global__ void __launch_bounds__(256) k_face_coarsen_set(FaceSet fs, const long
    a[fd[e]] = acc / ac;
 }
 
-__global__ void __launch_bounds__(256) k_face_coarsen(const double* __restrict__ src,
-                                                      double* __restrict__ dst, long long nside,
-                                                      int ncomp, const long long* __restrict__ fd,
-                                                      const long long* __restrict__ fs,
-                                                      const int* __restrict__ dir, long long n,
-                                                      double af0, double af1, double af2,
-                                                      double ac0, double ac1, double ac2,
-                                                      int nfine)
-{
-   long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-   if (e >= n) return;
-   int d = dir[e];
-   double af = d == 0 ? af0 : (d == 1 ? af1 : af2);
-   double ac = d == 0 ? ac0 : (d == 1 ? ac1 : ac2);
-   for (int m = 0; m < ncomp; m++) {
-      const double* a = src + m * nside;
-      double acc = 0.0;
-      for (int r = 0; r < 4; r++)
-         if (r < nfine) acc = acc + a[fs[4 * e + r]] * af;
-      dst[m * nside + fd[e]] = acc / ac;
-   }
-}
-
 template <typename T>
 __global__ void __launch_bounds__(256) k_prolong_const_add(T* __restrict__ e, long long ncg,
                                                            const long long* __restrict__ dst,
@@ -1133,20 +1110,6 @@ static void face_areas(const Hier& H, int l, double af[3], double ac[3])
             ac[d] = ac[d] * H.dx[l][a];
          }
    }
-}
-
-int hier_coarsen_faces_level(const Hier& H, int l, const double* src, double* dst, int ncomp,
-                             hipStream_t s)
-{
-   if (l + 1 >= H.nlev || H.fcrs_dst[l].n == 0) return 0;
-   double af[3], ac[3];
-   face_areas(H, l, af, ac);
-   hipLaunchKernelGGL(k_face_coarsen, grid1(H.fcrs_dst[l].n), dim3(256), 0, s, src, dst,
-                      H.nside_tot, ncomp, H.fcrs_dst[l].p, H.fcrs_src[l].p, H.fcrs_dir[l].p,
-                      H.fcrs_dst[l].n, af[0], af[1], af[2], ac[0], ac[1], ac[2],
-                      H.ndim == 3 ? 4 : 2);
-   AMPE_HIP_CHECK(hipGetLastError());
-   return 0;
 }
 
 static ampe_model_params lev_params(const Hier& H, const ampe_model_params& p0, int l)

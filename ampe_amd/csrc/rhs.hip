@@ -1130,6 +1130,9 @@ __global__ void __launch_bounds__(256) k_quat_face_coef(LevelArgs a, ampe_model_
    CellPos c;
    if (!cell_pos(a, 1, c)) return;
    if (NDIM == 2 && c.k > 0) return;
+   // unrolled: the strides indexed by a running d go to scratch memory (256^3: 1.03
+   // ms so, 0.21 ms)
+#pragma unroll
    for (int d = 0; d < NDIM; d++) {
       bool ok = (c.i < c.pd.nx + (d == 0)) && (c.j < c.pd.ny + (d == 1)) &&
                 (NDIM == 2 || c.k < c.pd.nz + (d == 2));

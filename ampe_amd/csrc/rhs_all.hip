@@ -31,9 +31,9 @@ namespace {
 
 // FIN: the right-hand side is a difference quotient's, and goes on to the
 // preconditioner's input (KryFin) without being stored.  128^3, six components:
-// 43 us less per Krylov iteration than storing it for a launch that reads it (of
-// some 800 us), 128^2: two launches fewer of thirteen with the ghosts filled by
-// the kernel that forms the state.
+// 85 us less per Krylov iteration of 1.2 ms than storing it for a launch that reads
+// it; 128^2: two launches fewer of nineteen with the ghosts filled by the kernel
+// that forms the state.
 template <int NDIM, int FE, int CONC, bool FIN>
 __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_params& p,
                                          const RhsConst& k, const CellPos& c, double r,

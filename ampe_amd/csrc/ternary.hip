@@ -188,6 +188,8 @@ __global__ void __launch_bounds__(256) k_ebs3_coeffs(LevelArgs a, Ebs3Const k, l
    CellPos c;
    if (!cell_pos(a, 1, c)) return;
    if (NDIM == 2 && c.k > 0) return;
+   // unrolled: the strides indexed by a running d went to scratch memory
+#pragma unroll
    for (int d = 0; d < NDIM; d++) {
       bool ok = (c.i < c.pd.nx + (d == 0)) && (c.j < c.pd.ny + (d == 1)) &&
                 (NDIM == 2 || c.k < c.pd.nz + (d == 2));
