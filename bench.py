@@ -19,8 +19,8 @@ same solver at --truth-atol, untimed) at the same t, which measures each
 form's Newton-tolerance error; fp64_reference (red-black block solves) is kept
 as context: it is the oracle-parity path and a different algorithm.
 
-Roofline: the headline form's dominant kernel, the FP32 orientation red-black
-sweep k_quat_rbgs_c<float,3,4> (all MG levels), is event-timed on the integrator's
+Roofline: the headline form's dominant kernel, the FP32 red-black sweep of all
+blocks k_set_sweep<float,3> (all MG levels), is event-timed on the integrator's
 stream during the timed steps; achieved = its algorithmic bytes / its time;
 traffic = its HBM bytes per launch from the committed rocprofv3 counter summary.
 
@@ -67,7 +67,7 @@ from ampe_amd import params as P  # noqa: E402
 HBM_PEAK_GBS = 8000.0
 BF16_MFMA_PEAK_TFLOPS = 2500.0
 FP64_PEAK_TFLOPS = 78.6
-TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "quat_rbgs_f32_polycrystal256_traffic.txt")
+TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "set_sweep_f32_polycrystal256_traffic.txt")
 
 
 def measured_traffic(path=TRAFFIC_PROFILE):
@@ -857,11 +857,11 @@ def main():
                  "Newton updates; the surrogate starts only the cells whose previous-step "
                  "residual exceeds 1e-2, so it cannot save time here (its gain is at cold "
                  "starts: the surrogate report)")
-    # dominant kernel of the headline form: the FP32 orientation red-black
-    # sweep, event-timed on the integrator's stream over the timed steps
+    # dominant kernel of the headline form: the FP32 red-black sweep of all
+    # blocks, event-timed on the integrator's stream over the timed steps
     kt = H["ktime"]
     quat_gbs = kt["bytes"] / (kt["ms"] * 1e-3) / 1e9
-    roof_quat = dict(kernel="k_quat_rbgs_c<float,3,4>", launches=kt["launches"],
+    roof_quat = dict(kernel="k_set_sweep<float,3>", launches=kt["launches"],
                      avg_ms=kt["ms"] / kt["launches"],
                      bytes_per_launch=kt["bytes"] / kt["launches"], achieved=quat_gbs)
     log(f"[bench] roofline {roof_quat}")
