@@ -21,7 +21,8 @@
 // and no longer waits for the host), finish 78 us (97), mid
 // 54 us (77).  Vectors are loaded two components at a time and for a compiled
 // count of basis vectors (up to ten): behind a branch per vector the loads of
-// the dots waited for each other.
+// the dots waited for each other.  Modified Gram-Schmidt takes two basis vectors
+// a pass (k_mgs).
 #include "krylov.h"
 
 namespace ampe {
@@ -239,66 +240,116 @@ __global__ void __launch_bounds__(256) k_cgs_update(LevelArgs a, int nc, PrecOut
    tile_store_sum(acc, partial);
 }
 
-// Sum of np values by the whole workgroup, the same in every one (fixed order).
-__device__ __forceinline__ double sum_parts(const double* __restrict__ p, int np)
+// Sums of N runs of np values, ps apart, by the whole workgroup, the same in every
+// one (fixed order).
+template <int N>
+__device__ __forceinline__ void sum_parts(const double* __restrict__ p, int np, int ps,
+                                          double (&s)[N])
 {
-   if (np == 1) return p[0];
-   __shared__ double sh[4];
+   if (np == 1) {
+#pragma unroll
+      for (int k = 0; k < N; k++) s[k] = p[k * ps];
+      return;
+   }
+   __shared__ double sh[4][N];
    const int t = threadIdx.x + TX * threadIdx.y;
-   double v = 0.0;
-   for (int i = t; i < np; i += TX * TY) v += p[i];
-   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-   if ((t & 63) == 0) sh[t >> 6] = v;
+   double v[N];
+#pragma unroll
+   for (int k = 0; k < N; k++) v[k] = 0.0;
+   for (int i = t; i < np; i += TX * TY)
+#pragma unroll
+      for (int k = 0; k < N; k++) v[k] += p[(long long)k * ps + i];
+#pragma unroll
+   for (int k = 0; k < N; k++) {
+      for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+      if ((t & 63) == 0) sh[t >> 6][k] = v[k];
+   }
    __syncthreads();
-   return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+#pragma unroll
+   for (int k = 0; k < N; k++) s[k] = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
 }
 
-// One step of modified Gram-Schmidt and the product of the next:
-// z = src + c v, c = -((s hv) cv) hv with s the sum of the np values at parts
-// (stored to *dot); partial = sum (ewt z)(ewt next), or (ewt z)^2 (next null).
-// v null: no update (z is not written), the first product.
-__global__ void __launch_bounds__(256) k_mgs(LevelArgs a, int nc, PrecOut src,
-                                             const double* __restrict__ v, double hv, double cv,
-                                             const double* __restrict__ parts, int np, double* dot,
-                                             const double* __restrict__ next,
+// Two basis vectors and their normalisation factors.
+struct VecPair {
+   const double* v[2];
+   double h[2];
+};
+
+// Modified Gram-Schmidt, two vectors a pass: z = src + c0 v0 + c1 v1 with
+// c_k = -((s_k h_k) cv) h_k, s0 = src . v0 and s1 = (src + c0 v0) . v1 =
+// src . v1 + c0 (v0 . v1), stored to dot[0] and dot[1].  parts: the np partial
+// sums, ps apart, of src . v0, src . v1 and v0 . v1.  partial: the same sums of z and
+// the next pair (NEXT 2), z . next (NEXT 1) or z . z (NEXT 0).  CUR 1: one vector;
+// CUR 0: none, the first products (z is not written).
+// Bound by memory.  One vector a pass reads z, ewt, the vector and the next one and
+// writes z: five vectors' traffic for one; two a pass cost seven.  256^3, six
+// components (805 MB a vector): 1114 us for two (5.1 TB/s), 742 us for one by
+// itself; with the scaled basis (no ewt, one vector a pass) 596 us, and two
+// passes more per iteration (1.3 ms).  An iteration at maxl = 30: 17.1 ms, 20.2 in the
+// scaled form.
+template <int CUR, int NEXT>
+__global__ void __launch_bounds__(256) k_mgs(LevelArgs a, int nc, int ntiles, PrecOut src,
+                                             VecPair cur, VecPair next, double cv,
+                                             const double* __restrict__ parts, int np, int ps,
+                                             double* __restrict__ dot,
                                              const double* __restrict__ ewt, double* z,
                                              double* __restrict__ partial)
 {
-   double co = 0.0;
-   if (v) {
-      const double s = sum_parts(parts, np);
-      if (np > 1 && blockIdx.x == 0 && threadIdx.x + threadIdx.y == 0) *dot = s;
-      co = -((s * hv) * cv) * hv;
+   double co[2] = {0.0, 0.0};
+   if (CUR > 0) {
+      double s[CUR == 2 ? 3 : 1];
+      sum_parts(parts, np, ps, s);
+      co[0] = -((s[0] * cur.h[0]) * cv) * cur.h[0];
+      if (CUR == 2) {
+         s[1] = s[1] + co[0] * s[CUR == 2 ? 2 : 0];
+         co[1] = -((s[1] * cur.h[1]) * cv) * cur.h[1];
+      }
+      if (blockIdx.x == 0 && threadIdx.x + threadIdx.y == 0)
+         for (int k = 0; k < CUR; k++) dot[k] = s[k];
    }
+   constexpr int NS = NEXT == 2 ? 3 : 1;
    CellPos c;
-   double acc = 0.0;
+   double acc[NS];
+#pragma unroll
+   for (int k = 0; k < NS; k++) acc[k] = 0.0;
    if (cell_pos(a, 0, c)) {
       const double w = red_w(a, c.c0);
       const long long sp = src.sp0 < nc ? split_at(a, c, 0) : 0;
       const double sm = src.sm ? src.sm[c.c0] : 1.0;
       for (int m = 0; m < nc; m += 2) {
          const Pair p = pair_of(a, c, nc, m);
-         double e[2], t[2], b[2], x[2];
+         double e[2], t[2], b[2][2], x[2][2];
 #pragma unroll
          for (int j = 0; j < 2; j++) {
             e[j] = ewt[p.i[j]];
             t[j] = prec_out(a, src, c, sp, m + 1 < nc ? m + j : m, sm);
-            b[j] = v ? v[p.i[j]] : 0.0;
-            x[j] = next ? next[p.i[j]] : 0.0;
+#pragma unroll
+            for (int k = 0; k < CUR; k++) b[j][k] = cur.v[k][p.i[j]];
+#pragma unroll
+            for (int k = 0; k < NEXT; k++) x[j][k] = next.v[k][p.i[j]];
          }
 #pragma unroll
          for (int j = 0; j < 2; j++) {
-            if (v) t[j] = t[j] + co * b[j];
-            const double u = e[j] * t[j];
-            acc += (next ? (u * e[j]) * x[j] : u * u) * (j ? w * p.on : w);
+#pragma unroll
+            for (int k = 0; k < CUR; k++) t[j] = t[j] + co[k] * b[j][k];
+            const double u = e[j] * t[j], wj = j ? w * p.on : w;
+            if (NEXT == 0) {
+               acc[0] += (u * u) * wj;
+            } else {
+               acc[0] += ((u * e[j]) * x[j][0]) * wj;
+               if (NEXT == 2) {
+                  acc[1] += ((u * e[j]) * x[j][1]) * wj;
+                  acc[NS - 1] += (((e[j] * e[j]) * x[j][0]) * x[j][1]) * wj;
+               }
+            }
          }
-         if (v) {
+         if (CUR > 0) {
             z[p.i[0]] = t[0];
             if (m + 1 < nc) z[p.i[1]] = t[1];
          }
       }
    }
-   tile_store_sum(acc, partial);
+   tile_store_sums(acc, NS, ntiles, partial);
 }
 
 __global__ void __launch_bounds__(256) k_newton_update(LevelArgs a, int nc, VecList vl,
@@ -428,9 +479,9 @@ int kry_cgs(const Level& L, int nc, const PrecOut& src, const VecList& vl, doubl
    return 0;
 }
 
-// Up to this many tiles a step sums the partial products of the step before by
-// itself, in every workgroup: four loads a thread (128^2 has 64 tiles: 5.1 us a
-// step); above, a reduction launch comes between (about 2 us and its gap).
+// Up to this many tiles a pass sums the partial products of the pass before by
+// itself, in every workgroup: at most twelve loads a thread; above, a reduction
+// launch comes between (about 2 us and its gap).
 constexpr int kSelfSumTiles = 1024;
 
 int kry_mgs(const Level& L, int nc, const PrecOut& src, const VecList& vl, double cv,
@@ -441,19 +492,45 @@ int kry_mgs(const Level& L, int nc, const PrecOut& src, const VecList& vl, doubl
       set_error("kry_mgs: too many vectors");
       return -1;
    }
-   const bool self = nt > 1 && nt <= kSelfSumTiles;
-   PrecOut in;
-   in.z = z;
-   AMPE_TILE_LAUNCH(k_mgs, nc, src, nullptr, 0.0, 0.0, nullptr, 0, nullptr, vl.v[0], ewt, nullptr,
-                    L.partial);
-   for (int i = 0; i < n; i++) {
-      double* from = L.partial + (long long)(i & 1) * nt;
-      double* to = L.partial + (long long)((i + 1) & 1) * nt;
-      if (!self && reduce_regions_dev(L, from, nt, 1, L.dred + i, s)) return -1;
-      AMPE_TILE_LAUNCH(k_mgs, nc, i ? in : src, vl.v[i], vl.y[i], cv, self ? from : L.dred + i,
-                       self ? nt : 1, L.dred + i, i + 1 < n ? vl.v[i + 1] : nullptr, ewt, z, to);
+   const bool self = nt <= kSelfSumTiles;
+   // L.dred: the n products, and behind them the sums a pass starts from
+   double* start = L.dred + kMaxKrylov;
+   PrecOut from = src;
+   VecPair cur{}, next{};
+   // pass i takes vectors i - 2 and i - 1 out and forms the products of i and i + 1
+   for (int i = 0; i < n + 2; i += 2) {
+      const int take = i == 0 ? 0 : (i <= n ? 2 : 1), form = i >= n ? 0 : (i + 1 < n ? 2 : 1);
+      cur = next;
+      for (int k = 0; k < form; k++) {
+         next.v[k] = vl.v[i + k];
+         next.h[k] = vl.y[i + k];
+      }
+      const int half = (i >> 1) & 1;
+      double* out = L.partial + 3LL * half * nt;
+      const double* in = L.partial + 3LL * (1 - half) * nt;
+      if (take && !self) {
+         if (reduce_regions_dev(L, in, nt, take == 2 ? 3 : 1, start, s)) return -1;
+         in = start;
+      }
+      const int np = self ? nt : 1, ps = self ? nt : 1;
+      double* dot = L.dred + (i ? i - 2 : 0);
+#define AMPE_MGS_CASE(CUR, NEXT)                                                             \
+   if (take == CUR && form == NEXT)                                                          \
+   AMPE_TILE_LAUNCH((k_mgs<CUR, NEXT>), nc, nt, from, cur, next, cv, in, np, ps, dot, ewt, z, out)
+      AMPE_MGS_CASE(0, 1);
+      AMPE_MGS_CASE(0, 2);
+      AMPE_MGS_CASE(1, 0);
+      AMPE_MGS_CASE(2, 0);
+      AMPE_MGS_CASE(2, 1);
+      AMPE_MGS_CASE(2, 2);
+#undef AMPE_MGS_CASE
+      if (take) {
+         from = PrecOut{};
+         from.z = z;
+      }
+      if (form == 0) return reduce_last(L, out, nt, n, sums, s);
    }
-   return reduce_last(L, L.partial + (long long)(n & 1) * nt, nt, n, sums, s);
+   return -1;
 }
 
 int kry_newton_update(const Level& L, int nc, const VecList& vl, const double* ewt, double* y,

@@ -34,15 +34,19 @@ def _boxes(n, cuts):
     return out, dom
 
 
-@pytest.mark.parametrize("gstype", [P.GS_MODIFIED, P.GS_CLASSICAL])
-def test_long_spaces_match_oracle(dev, gstype):
+@pytest.mark.parametrize("gstype,maxl,eplifac,model", [
+    (P.GS_MODIFIED, 14, 1e-5, {}), (P.GS_CLASSICAL, 14, 1e-5, {}),
+    # two vectors a pass: both remainders up to the longest space, odd component counts
+    (P.GS_MODIFIED, 30, 1e-11, {}), (P.GS_MODIFIED, 29, 1e-11, dict(with_conc=0))])
+def test_long_spaces_match_oracle(dev, gstype, maxl, eplifac, model):
     from oracle import oracle as O
     from ampe_amd import hip as H
     n = 48
-    p = P.two_grain_params(ndim=2)
+    p = P.two_grain_params(ndim=2, **model)
     p.quad_ceq[0], p.quad_ceq[1] = 0.40, 0.45
     phi, c, q = P.two_grain_state(n=n, radius=n / 4, ndim=2)
-    s = P.solver_defaults(maxl=14, max_newton=5, gstype=gstype, eplifac=1e-5)
+    c = c if p.with_conc else None
+    s = P.solver_defaults(maxl=maxl, max_newton=5, gstype=gstype, eplifac=eplifac)
     osim = O.Sim(p, s, n)
     osim.set_state(phi, c, q)
     box = H.boxes_of((n, n), 2)
@@ -52,8 +56,10 @@ def test_long_spaces_match_oracle(dev, gstype):
         ro, _ = osim.advance(1)
         rg, st = gsim.advance(1)
         assert ro == rg == 0
-    assert st["nli"] > 10 * st["nni"], st  # long spaces occurred
+    assert st["nli"] > (10 if maxl == 14 else 20) * st["nni"], st  # long spaces occurred
     for a, b in zip(gsim.get_state((n, n))[:3], osim.get_state()[:3]):
+        if not b.any():
+            continue  # a field the model does not have
         assert np.max(np.abs(a - b)) <= 1e-10 * np.max(np.abs(b))
 
 
