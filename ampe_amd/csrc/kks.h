@@ -33,15 +33,15 @@ constexpr size_t kKksPartDoubles = (size_t)kKksPart * (kKksGrid + kKksSurrGrid);
 
 // KKS over all ghosted cells of a level.  launch_kks adds its counts to the
 // slots part (kKksPartDoubles doubles, zero at first) without synchronising;
-// kks_finish folds them into the device counters dev_acc[6] = {total iterations,
-// max iterations, failure flag, unused, fallbacks, surrogate starts} and clears
-// them; launch_kks_sync returns max iterations (or -1 on a non-converged cell)
+// kks_finish folds them (those of the surrogate pass with surrogate) into the
+// device counters dev_acc[6] = {total iterations, max iterations, failure flag,
+// unused, fallbacks, surrogate starts} and clears them; launch_kks_sync returns max iterations (or -1 on a non-converged cell)
 // and the total, synchronising s.
 constexpr int kKksAcc = 6;
 int launch_kks(const Level& L, const ampe_model_params& p, const double* phi,
                const double* c, const double* clr, const double* csr, double* cl,
                double* cs, const KksGuess& guess, double* part, hipStream_t s);
-int kks_finish(double* part, long long* dev_acc, hipStream_t s);
+int kks_finish(const Level& L, double* part, bool surrogate, long long* dev_acc, hipStream_t s);
 int launch_kks_sync(const Level& L, const ampe_model_params& p, const double* phi,
                     const double* c, const double* clr, const double* csr, double* cl,
                     double* cs, int* max_iters, long long* total_iters, hipStream_t s);

@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(256) k_kks(long long n, ampe_model_params p, K
                                              const double* __restrict__ clr,
                                              const double* __restrict__ csr,
                                              double* __restrict__ cl, double* __restrict__ cs,
-                                             double* __restrict__ partial)
+                                             double* __restrict__ partial, bool add)
 {
    double it = 0.0, mx = 0.0;
    const long long stride = (long long)gridDim.x * blockDim.x;
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(256) k_kks(long long n, ampe_model_params p, K
          mx = (double)r > mx ? (double)r : mx;
       }
    }
-   kks_block_partial(it, mx, 0.0, mx >= kKksFail ? 1.0 : 0.0, 0.0, partial, true);
+   kks_block_partial(it, mx, 0.0, mx >= kKksFail ? 1.0 : 0.0, 0.0, partial, add);
 }
 
 // Switch policy, first pass (binary CALPHAD): a cell whose residual at the
@@ -313,14 +313,35 @@ static unsigned kks_grid(const Level& L)
    return (unsigned)std::min<long long>((L.ncg + 255) / 256, kKksGrid);
 }
 
+// The level-wide call from the previous-step guess; add: its counts go on top of
+// those in the slots.
+static int kks_level(const Level& L, const ampe_model_params& p, const double* phi,
+                     const double* c, const double* clr, const double* csr, double* cl,
+                     double* cs, double* part, bool add, hipStream_t s)
+{
+   const unsigned nb = kks_grid(L);
+   const KksTerms terms = kks_terms(p.calphad, p.temperature);
+   if (p.fe_model == AMPE_FE_QUADRATIC)
+      hipLaunchKernelGGL(k_kks<AMPE_FE_QUADRATIC>, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
+                         phi, c, clr, csr, cl, cs, part, add);
+   else if (p.fe_model == AMPE_FE_KKS_DILUTE)
+      hipLaunchKernelGGL(k_kks<AMPE_FE_KKS_DILUTE>, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
+                         phi, c, clr, csr, cl, cs, part, add);
+   else
+      hipLaunchKernelGGL(k_kks<AMPE_FE_CALPHAD_BINARY>, dim3(nb), dim3(256), 0, s, L.ncg, p,
+                         terms, phi, c, clr, csr, cl, cs, part, add);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
 int launch_kks(const Level& L, const ampe_model_params& p, const double* phi,
                const double* c, const double* clr, const double* csr, double* cl,
                double* cs, const KksGuess& guess, double* part, hipStream_t s)
 {
-   const unsigned nb = kks_grid(L);
-   const KksTerms terms = kks_terms(p.calphad, p.temperature);
    if (guess.surrogate && p.fe_model == AMPE_FE_CALPHAD_BINARY) {
       const Surrogate& S = *guess.surrogate;
+      const unsigned nb = kks_grid(L);
+      const KksTerms terms = kks_terms(p.calphad, p.temperature);
       if (S.hid != kMlpHidden || S.nin != 3 || S.nout != 2) {
          set_error("launch_kks: the surrogate must map (c, phi, T) -> (cL, cS) with 64 hidden");
          return -1;
@@ -336,28 +357,21 @@ int launch_kks(const Level& L, const ampe_model_params& p, const double* phi,
       unsigned g = std::min<unsigned>(kKksSurrGrid, nb);
       hipLaunchKernelGGL(k_kks_surr, dim3(g), dim3(256), 0, s, p, terms, m, guess.probe_its,
                          guess.probe_tol, phi, c, clr, csr, cl, cs, guess.list, guess.count,
-                         part + (size_t)kKksPart * kKksGrid);
+                         part + (size_t)kKksPart * nb);
       AMPE_HIP_CHECK(hipGetLastError());
       // the work list is empty again for the next call
       hipLaunchKernelGGL(k_kks_list_clear, dim3(1), dim3(1), 0, s, guess.count);
-   } else if (p.fe_model == AMPE_FE_QUADRATIC) {
-      hipLaunchKernelGGL(k_kks<AMPE_FE_QUADRATIC>, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
-                         phi, c, clr, csr, cl, cs, part);
-   } else if (p.fe_model == AMPE_FE_KKS_DILUTE) {
-      hipLaunchKernelGGL(k_kks<AMPE_FE_KKS_DILUTE>, dim3(nb), dim3(256), 0, s, L.ncg, p, terms,
-                         phi, c, clr, csr, cl, cs, part);
-   } else {
-      hipLaunchKernelGGL(k_kks<AMPE_FE_CALPHAD_BINARY>, dim3(nb), dim3(256), 0, s, L.ncg, p,
-                         terms, phi, c, clr, csr, cl, cs, part);
+      AMPE_HIP_CHECK(hipGetLastError());
+      return 0;
    }
-   AMPE_HIP_CHECK(hipGetLastError());
-   return 0;
+   return kks_level(L, p, phi, c, clr, csr, cl, cs, part, true, s);
 }
 
-int kks_finish(double* part, long long* dev_acc, hipStream_t s)
+int kks_finish(const Level& L, double* part, bool surrogate, long long* dev_acc, hipStream_t s)
 {
-   hipLaunchKernelGGL(k_kks_finish, dim3(1), dim3(1024), 0, s, part, kKksGrid + kKksSurrGrid,
-                      dev_acc);
+   // only the slots the level's calls write: all 4352 take 6 us of a small call
+   const int n = (int)kks_grid(L) + (surrogate ? kKksSurrGrid : 0);
+   hipLaunchKernelGGL(k_kks_finish, dim3(1), dim3(1024), 0, s, part, n, dev_acc);
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -368,8 +382,9 @@ int launch_kks_sync(const Level& L, const ampe_model_params& p, const double* ph
 {
    long long* acc = reinterpret_cast<long long*>(L.iscratch);
    AMPE_HIP_CHECK(hipMemsetAsync(acc, 0, sizeof(long long) * kKksAcc, s));
-   if (launch_kks(L, p, phi, c, clr, csr, cl, cs, KksGuess{}, L.kks_part, s)) return -1;
-   if (kks_finish(L.kks_part, acc, s)) return -1;
+   // (the slots are written, whatever is in them)
+   if (kks_level(L, p, phi, c, clr, csr, cl, cs, L.kks_part, false, s)) return -1;
+   if (kks_finish(L, L.kks_part, false, acc, s)) return -1;
    AMPE_HIP_CHECK(hipMemcpyAsync(L.hpinned, acc, sizeof(long long) * kKksAcc,
                                  hipMemcpyDeviceToHost, s));
    AMPE_HIP_CHECK(hipStreamSynchronize(s));

@@ -336,7 +336,9 @@ static int kks(Sim* S, const double* y)
 static int kks_collect(Sim* S)
 {
    if (S->ic < 0) return 0;
-   if (!S->tern && kks_finish(S->kks_part, S->kks_acc, S->stream)) return -1;
+   if (!S->tern && kks_finish(*S->L, S->kks_part, S->s.kks_guess == AMPE_GUESS_SURROGATE, S->kks_acc,
+                              S->stream))
+      return -1;
    AMPE_HIP_CHECK(hipMemcpyAsync(S->L->hpinned, S->kks_acc, sizeof(long long) * kKksAcc,
                                  hipMemcpyDeviceToHost, S->stream));
    AMPE_HIP_CHECK(hipStreamSynchronize(S->stream));
