@@ -39,10 +39,18 @@ namespace ampe {
 
 constexpr int kMaxLev = 4;
 
+// part of another table
+template <typename T>
+struct DevSpan {
+   const T* p = nullptr;
+   long long n = 0;
+};
+
 template <typename T>
 struct DevVec {
    T* p = nullptr;
    long long n = 0;
+   DevSpan<T> part(size_t from, size_t count) const { return {p + from, (long long)count}; }
    int upload(const std::vector<T>& h)
    {
       n = (long long)h.size();
@@ -80,16 +88,16 @@ struct Hier {
    DevVec<long long> fcrs_dst[kMaxLev], fcrs_src[kMaxLev];
    DevVec<int> fcrs_dir[kMaxLev];
    // coarse-fine faces of level l (l > 0) and corrections of level l (< nlev-1)
-   DevVec<CfFace> cff[kMaxLev];
-   DevVec<CfCorr> cfc[kMaxLev];
+   DevSpan<CfFace> cff[kMaxLev];
+   DevSpan<CfCorr> cfc[kMaxLev];
    // the FAC composite residual replaces every coarse face on a fine patch
    // boundary: fine faces of level l on fine-fine patch boundaries (saved
    // after cff[l]) and the covered coarse cells of level l next to a fine
    // patch boundary of level l+1
-   DevVec<CfFace> fff[kMaxLev];
-   DevVec<CfCorr> cfi[kMaxLev];
-   // the fine faces cff then fff and the corrections cfc then cfi in one table
-   // each
+   DevSpan<CfFace> fff[kMaxLev];
+   DevSpan<CfCorr> cfi[kMaxLev];
+   // the tables they are parts of: the fine faces cff then fff, the corrections
+   // cfc then cfi
    DevVec<CfFace> facf[kMaxLev];
    DevVec<CfCorr> facc[kMaxLev];
    // prolongation of level l (l > 0): fine interior cell, coarse parent
@@ -186,10 +194,6 @@ void hier_destroy(Hier* H)
       H->fcrs_dst[l].release();
       H->fcrs_src[l].release();
       H->fcrs_dir[l].release();
-      H->cff[l].release();
-      H->cfc[l].release();
-      H->fff[l].release();
-      H->cfi[l].release();
       H->facf[l].release();
       H->facc[l].release();
       H->pro_dst[l].release();
@@ -288,9 +292,22 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
    H->nside_tot = so[0] + so[1] + so[2];
 
    // ghost tables per level
-   std::vector<long long> gd[kMaxLev], gs[kMaxLev], cd[kMaxLev], cs9[kMaxLev];
+   GhostTable gt[kMaxLev];
+   std::vector<long long> cd[kMaxLev], cs9[kMaxLev];
    std::vector<double> cw[kMaxLev];
-   for (int l = 0; l < nlev; l++)
+   for (int l = 0; l < nlev; l++) {
+      long long ng = 0;
+      for (int p = H->pbeg[l]; p < H->pbeg[l + 1]; p++) {
+         const ampe_box& b = H->boxes[p];
+         long long n[3], in = 1, all = 1;
+         for (int a = 0; a < ndim; a++) {
+            n[a] = box_n(b, a, ndim);
+            in *= n[a];
+            all *= n[a] + 2;
+         }
+         ng += all - in;
+      }
+      gt[l].reserve(ng);
       for (int p = H->pbeg[l]; p < H->pbeg[l + 1]; p++) {
          const ampe_box& b = H->boxes[p];
          int n[3] = {box_n(b, 0, ndim), box_n(b, 1, ndim), box_n(b, 2, ndim)};
@@ -304,8 +321,9 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
                   long long dst = cidx(*H, p, i, j, k);
                   long long s = find_cell(*H, l, g);
                   if (s >= 0) {
-                     gd[l].push_back(dst);
-                     gs[l].push_back(s);
+                     gt[l].add(GhostTable::outside(i, n[0]) + GhostTable::outside(j, n[1]) +
+                                   GhostTable::outside(k, n[2]) == 1,
+                               dst, s);
                      continue;
                   }
                   if (l == 0) return hier_fail(H, "level 0 leaves a ghost uncovered");
@@ -336,6 +354,8 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
                   }
                }
       }
+      gt[l].finish();
+   }
 
    // levels placed in the composite layout, and the composite over all patches
    for (int l = 0; l < nlev; l++) {
@@ -349,8 +369,7 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
          pl.side_base[a] = H->soff[a][p0];
          pl.nside_total[a] = H->nside[a];
       }
-      if (level_create_placed(ndim, H->boxes.data() + p0, H->pbeg[l + 1] - p0, pl, gd[l], gs[l],
-                              &H->lev[l]))
+      if (level_create_placed(ndim, H->boxes.data() + p0, H->pbeg[l + 1] - p0, pl, gt[l], &H->lev[l]))
          return hier_fail(H, "level placement failed");
    }
    {
@@ -358,12 +377,11 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
       pl.ncg_total = H->ncg;
       pl.ncell_total = H->ncell;
       for (int a = 0; a < 3; a++) pl.nside_total[a] = H->nside[a];
-      std::vector<long long> none;
       std::vector<int> patch_lev((size_t)np);
       for (int l = 0; l < nlev; l++)
          for (int q = H->pbeg[l]; q < H->pbeg[l + 1]; q++) patch_lev[q] = l;
       pl.patch_lev = patch_lev.data();
-      if (level_create_placed(ndim, H->boxes.data(), np, pl, none, none, &H->comp))
+      if (level_create_placed(ndim, H->boxes.data(), np, pl, GhostTable(), &H->comp))
          return hier_fail(H, "composite placement failed");
    }
    for (int l = 1; l < nlev; l++) {
@@ -628,13 +646,15 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
       };
       std::vector<CfCorr> corr, icorr;
       if (records(keys, corr) || records(ikeys, icorr)) return -1;
-      if (H->cff[l].upload(faces) || H->cfc[l - 1].upload(corr) || H->fff[l].upload(ffaces) ||
-          H->cfi[l - 1].upload(icorr))
-         return hier_fail(H, "upload failed");
+      const size_t ncf = faces.size(), ncc = corr.size();
       faces.insert(faces.end(), ffaces.begin(), ffaces.end());
       corr.insert(corr.end(), icorr.begin(), icorr.end());
       if (H->facf[l].upload(faces) || H->facc[l - 1].upload(corr))
          return hier_fail(H, "upload failed");
+      H->cff[l] = H->facf[l].part(0, ncf);
+      H->fff[l] = H->facf[l].part(ncf, faces.size() - ncf);
+      H->cfc[l - 1] = H->facc[l - 1].part(0, ncc);
+      H->cfi[l - 1] = H->facc[l - 1].part(ncc, corr.size() - ncc);
    }
 
    // weights: cell volume relative to level 0, zero under a finer level
@@ -1500,7 +1520,7 @@ static int fac_comp_residual(const FacCtx<T>& X, int l, T* res, T* u, const T* f
       // fine fluxes: the uncovered cells next to coarse-fine faces, then the
       // covered cells inside the fine patches
       for (int t = 0; t < 2 && l + 1 < H.nlev; t++) {
-         const DevVec<CfCorr>& tab = t == 0 ? H.cfc[l] : H.cfi[l];
+         const DevSpan<CfCorr>& tab = t == 0 ? H.cfc[l] : H.cfi[l];
          if (tab.n == 0) continue;
          double af, ac;
          corr_areas(H, l, af, ac);
@@ -1511,7 +1531,7 @@ static int fac_comp_residual(const FacCtx<T>& X, int l, T* res, T* u, const T* f
          AMPE_HIP_CHECK(hipGetLastError());
       }
       for (int t = 0; t < 2 && l > 0; t++) {
-         const DevVec<CfFace>& tab = t == 0 ? H.cff[l] : H.fff[l];
+         const DevSpan<CfFace>& tab = t == 0 ? H.cff[l] : H.fff[l];
          if (tab.n == 0) continue;
          hipLaunchKernelGGL(k_oflux_save<T>, grid1(tab.n), dim3(256), 0, X.s, um,
                             B.kind == 1 ? B.S : nullptr, B.D, B.D_const, tab.p, tab.n, di[0],

@@ -88,6 +88,29 @@ struct Level {
    const double* wt = nullptr;
 };
 
+// A ghost gather with the face ghosts (those next to an interior cell's face)
+// first, each part in the order it is added: the parts fill the table from its
+// two ends, so that nothing is copied to join them.
+struct GhostTable {
+   std::vector<long long> dst, src;
+   long long nface = 0, ntail = 0;
+   // at most n entries
+   void reserve(long long n)
+   {
+      dst.resize((size_t)n);
+      src.resize((size_t)n);
+   }
+   void add(bool face, long long d, long long s)
+   {
+      const size_t i = face ? (size_t)nface++ : dst.size() - (size_t)++ntail;
+      dst[i] = d;
+      src[i] = s;
+   }
+   void finish();
+   // how far position i lies outside n cells
+   static int outside(int i, int n) { return i < 0 ? -i : (i >= n ? i - n + 1 : 0); }
+};
+
 int level_create(int ndim, const ampe_box* boxes, int npatch, int ghost,
                  const ampe_box* periodic, Level** out);
 void level_destroy(Level* L);
@@ -96,15 +119,14 @@ void level_destroy(Level* L);
 // blocks from cell_base inside each component block of ncg_total cells, its
 // faces from side_base[d] inside direction block d of a side field with
 // nside_total[d] faces per direction, interior (compact) offsets from
-// int_base; ghost width 1; gd / gs: its ghost gather (composite indices).
+// int_base; ghost width 1; gt: its ghost gather (composite indices).
 struct LevelPlacement {
    long long cell_base = 0, ncg_total = 0, int_base = 0, ncell_total = 0;
    long long side_base[3] = {0, 0, 0}, nside_total[3] = {0, 0, 0};
    const int* patch_lev = nullptr;  // PatchDev::lev per patch (null: 0)
 };
 int level_create_placed(int ndim, const ampe_box* boxes, int npatch, const LevelPlacement& pl,
-                        const std::vector<long long>& gd, const std::vector<long long>& gs,
-                        Level** out);
+                        const GhostTable& gt, Level** out);
 
 // Ghost gather for ncomp component blocks (double or float fields); split:
 // the blocks are stored in the row parity-split layout (split_col), which

@@ -66,57 +66,21 @@ static void xcd_order(std::vector<Tile>& tiles)
    }
 }
 
+void GhostTable::finish()
+{
+   std::reverse(dst.end() - ntail, dst.end());
+   std::reverse(src.end() - ntail, src.end());
+   dst.erase(dst.begin() + nface, dst.end() - ntail);
+   src.erase(src.begin() + nface, src.end() - ntail);
+}
+
 // Work lists, device copies of the patch table and the ghost gather, and
 // the reduction buffers of a level whose patch table L->hp is complete.
-static int level_upload(Level* L, const std::vector<long long>& gd0,
-                        const std::vector<long long>& gs0, Level** out)
+static int level_upload(Level* L, const GhostTable& gt, Level** out)
 {
    const int ndim = L->ndim, npatch = L->npatch;
-   // the ghost gather with the face ghosts first (an entry's patch: the last
-   // whose block starts at or before it; the tables list patch after patch)
-   std::vector<long long> gd, gs;
-   {
-      const size_t ne = gd0.size();
-      std::vector<long long> rd, rs;
-      gd.reserve(ne);
-      gs.reserve(ne);
-      rd.reserve(ne);
-      rs.reserve(ne);
-      int p = 0, x = 0, y = 0, z = 0;  // the entry's position in its patch's ghosted box
-      long long at = -1;               // and the entry before it
-      for (size_t e = 0; e < ne; e++) {
-         const bool same = at >= 0 && gd0[e] >= at &&
-                           (p + 1 == npatch || gd0[e] < L->hp[p + 1].cell_off);
-         while (p + 1 < npatch && L->hp[p + 1].cell_off <= gd0[e]) p++;
-         const PatchDev& d = L->hp[p];
-         if (same && gd0[e] - at <= d.sy) {
-            // the tables run through a box row by row: mostly one step or one row
-            x += (int)(gd0[e] - at);
-            if (x >= d.sy) {
-               x -= d.sy;
-               if (++y == d.ny + 2 * L->g) {
-                  y = 0;
-                  z++;
-               }
-            }
-         } else {
-            const long long loc = gd0[e] - d.cell_off, row = loc % d.sz;
-            x = (int)(row % d.sy);
-            y = (int)(row / d.sy);
-            z = (int)(loc / d.sz);
-         }
-         at = gd0[e];
-         auto outside = [](int i, int n) { return i < 0 ? -i : (i >= n ? i - n + 1 : 0); };
-         const int ox = outside(x - L->g, d.nx), oy = outside(y - L->g, d.ny),
-                   oz = ndim == 3 ? outside(z - L->gz, d.nz) : 0;
-         const bool face = ox + oy + oz == 1;
-         (face ? gd : rd).push_back(gd0[e]);
-         (face ? gs : rs).push_back(gs0[e]);
-      }
-      L->nghost_face = (long long)gd.size();
-      gd.insert(gd.end(), rd.begin(), rd.end());
-      gs.insert(gs.end(), rs.begin(), rs.end());
-   }
+   const std::vector<long long>&gd = gt.dst, &gs = gt.src;
+   L->nghost_face = gt.nface;
    // work lists
    std::vector<Tile> ct, ft, zt, mt;
    for (int p = 0; p < npatch; p++) {
@@ -162,7 +126,6 @@ static int level_upload(Level* L, const std::vector<long long>& gd0,
    if (e == hipSuccess) e = hipHostMalloc(&L->hpinned, sizeof(double) * 64);
    if (e == hipSuccess) e = hipMalloc(&L->iscratch, sizeof(int) * 64);
    if (e == hipSuccess) e = hipMalloc(&L->kks_part, sizeof(double) * kKksPartDoubles);
-   if (e == hipSuccess) e = hipMemset(L->kks_part, 0, sizeof(double) * kKksPartDoubles);
    if (e == hipSuccess)
       e = hipMemcpy(L->dp, L->hp.data(), sizeof(PatchDev) * npatch, hipMemcpyHostToDevice);
    if (e == hipSuccess)
@@ -278,7 +241,8 @@ int level_create(int ndim, const ampe_box* boxes, int npatch, int ghost,
    L->nside_tot = soff[0] + soff[1] + soff[2];
 
    // ghost gather: each ghost cell copies the interior cell it images
-   std::vector<long long> gd, gs;
+   GhostTable gt;
+   gt.reserve(L->ncg - L->ncell);
    for (int p = 0; p < npatch; p++) {
       const PatchDev& d = L->hp[p];
       int g = ghost, gz = L->gz;
@@ -321,18 +285,20 @@ int level_create(int ndim, const ampe_box* boxes, int npatch, int ghost,
                   sk = std::min(std::max(k, 0), d.nz - 1);
                }
                const PatchDev& e = L->hp[src_p];
-               gd.push_back(d.cell_off + (i + g) + (long long)(j + g) * d.sy +
-                            (long long)(k + gz) * d.sz);
-               gs.push_back(e.cell_off + (si + g) + (long long)(sj + g) * e.sy +
-                            (long long)(sk + gz) * e.sz);
+               gt.add(GhostTable::outside(i, d.nx) + GhostTable::outside(j, d.ny) +
+                              GhostTable::outside(k, d.nz) == 1,
+                      d.cell_off + (i + g) + (long long)(j + g) * d.sy +
+                          (long long)(k + gz) * d.sz,
+                      e.cell_off + (si + g) + (long long)(sj + g) * e.sy +
+                          (long long)(sk + gz) * e.sz);
             }
    }
-   return level_upload(L, gd, gs, out);
+   gt.finish();
+   return level_upload(L, gt, out);
 }
 
 int level_create_placed(int ndim, const ampe_box* boxes, int npatch, const LevelPlacement& pl,
-                        const std::vector<long long>& gd, const std::vector<long long>& gs,
-                        Level** out)
+                        const GhostTable& gt, Level** out)
 {
    if ((ndim != 2 && ndim != 3) || npatch <= 0 || !boxes) {
       set_error("level_create_placed: bad arguments");
@@ -391,7 +357,7 @@ int level_create_placed(int ndim, const ampe_box* boxes, int npatch, const Level
       delete L;
       return -1;
    }
-   return level_upload(L, gd, gs, out);
+   return level_upload(L, gt, out);
 }
 
 void level_destroy(Level* L)
