@@ -27,7 +27,7 @@ def _boxes(shape, split):
     return out
 
 
-def _run(shape, split, periodic, sweeps, fused, seed=3):
+def _run(shape, split, periodic, sweeps, fused, seed=3, take=4):
     import torch
     from ampe_amd import hip as H
     ndim = len(shape)
@@ -42,12 +42,13 @@ def _run(shape, split, periodic, sweeps, fused, seed=3):
                                            for _ in range(ncomp)])).to(dev)
     z = torch.from_numpy(np.concatenate([lev.to_ghosted(rng.normal(size=shape))
                                          for _ in range(ncomp)])).to(dev)
+    ncomp = take  # of the same four components
     ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
     H.check(H.lib().ampe_ghost_fill(lev.h, ptr(sm), 1, None))
     dx = (C.c_double * 3)(0.5, 0.25, 0.75)
     H.check(H.lib().ampe_quat_smooth(lev.h, ptr(fc), ptr(sm), 0.3, dx, ncomp, ptr(rhs), ptr(z),
                                      sweeps, fused, None))
-    zz = z.cpu().numpy().reshape(ncomp, -1)
+    zz = z.cpu().numpy().reshape(4, -1)
     return np.stack([_interior(lev, zz[m], ndim) for m in range(ncomp)])
 
 
@@ -78,3 +79,13 @@ def test_fused_sweep_bit_identical(dev, shape, split, periodic, sweeps):
     b = _run(shape, split, periodic, sweeps, fused=1)
     assert np.isfinite(a).all()
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape,split,periodic", [((40, 48), 21, False), ((12, 18, 70), 30, True)])
+@pytest.mark.parametrize("take", [1, 2, 3])
+def test_components_by_themselves(dev, shape, split, periodic, take):
+    """One, two and four components have kernels of their own, other counts a
+    loop: a component's values do not depend on how many are swept with it."""
+    a = _run(shape, split, periodic, 2, fused=0)
+    b = _run(shape, split, periodic, 2, fused=0, take=take)
+    assert np.isfinite(b).all() and np.array_equal(a[:take], b[:take])
