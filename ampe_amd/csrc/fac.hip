@@ -878,6 +878,25 @@ __global__ void __launch_bounds__(256) k_set_resrestrict(LevelArgs ca, LevelArgs
       set_resrestrict<T, NDIM, 1, SPLIT, WRAP>(ca, fa, p, o, dinv, hinv2, rhs, x, bc, m);
 }
 
+// The same of one block by itself, of a known kind with QL components: the
+// elliptic rows by themselves take 144 registers, with the orientation's in the same
+// kernel 213.  192^3, FP64: elliptic block 46 us (60 as a set of one), orientation
+// block of two components 157 us (196, one after the other).
+template <typename T, int NDIM, int KIND, int QL>
+__global__ void __launch_bounds__(256) k_block_resrestrict(LevelArgs ca, LevelArgs fa,
+                                                           SweepSlot<T> o, T di0, T di1, T di2,
+                                                           T hi0, T hi1, T hi2,
+                                                           const T* __restrict__ rhs,
+                                                           const T* __restrict__ x,
+                                                           T* __restrict__ bc)
+{
+   CellPos p;
+   if (!cell_pos(ca, 0, p)) return;
+   const T dinv[3] = {di0, di1, di2}, hinv2[3] = {hi0, hi1, hi2};
+   o.kind = KIND;
+   set_resrestrict<T, NDIM, QL, false, false>(ca, fa, p, o, dinv, hinv2, rhs, x, bc, 0);
+}
+
 // ------------------------------------------------------------ launchers
 static dim3 tblock() { return dim3(TX, TY); }
 static dim3 cblock() { return dim3(TX / 2, TY); }
@@ -1148,11 +1167,33 @@ int launch_residual(const Level& L, const EllOp<T>& op, const double* dx, const 
    return 0;
 }
 
+template <typename T, class ND, class KIND, class QL>
+static int block_resrestrict(ND, KIND, QL, const Level& coarse, const Level& fine,
+                             const SweepSlot<T>& o, const double* dx, const T* rhs, const T* x,
+                             T* b, hipStream_t s)
+{
+   T di[3], hi[3];
+   recip(dx, di);
+   recip2(dx, hi);
+   hipLaunchKernelGGL((k_block_resrestrict<T, ND::value, KIND::value, QL::value>),
+                      dim3(coarse.ncell_tiles), tblock(), 0, s, level_args(coarse),
+                      level_args(fine), o, di[0], di[1], di[2], hi[0], hi[1], hi[2], rhs, x, b);
+   AMPE_HIP_CHECK(hipGetLastError());
+   return 0;
+}
+
 template <typename T>
 int launch_ell_resrestrict(const Level& coarse, const Level& fine, const EllOp<T>& op,
                            const double* dx, const T* rhs, const T* u, T* b, hipStream_t s)
 {
-   return launch_set_resrestrict<T>(coarse, fine, ell_set(op), dx, rhs, u, b, SetForm{}, s);
+   using I0 = std::integral_constant<int, 0>;
+   using I1 = std::integral_constant<int, 1>;
+   const SweepSlot<T> o = ell_set(op).s[0];
+   if (fine.ndim == 3)
+      return block_resrestrict<T>(std::integral_constant<int, 3>(), I0(), I1(), coarse, fine, o, dx,
+                                  rhs, u, b, s);
+   return block_resrestrict<T>(std::integral_constant<int, 2>(), I0(), I1(), coarse, fine, o, dx,
+                               rhs, u, b, s);
 }
 
 template <typename T>
@@ -1233,8 +1274,18 @@ int launch_quat_resrestrict(const Level& coarse, const Level& fine, const T* fc,
                             double gamma, const double* dx, int ncomp, const T* rhs, const T* z,
                             T* b, hipStream_t s)
 {
-   return launch_set_resrestrict<T>(coarse, fine, quat_set(fc, sm, gamma, ncomp), dx, rhs, z, b,
-                                    SetForm{}, s);
+   if (ncomp != 1 && ncomp != 2 && ncomp != 4) {
+      set_error("launch_quat_resrestrict: one, two or four components");
+      return -1;
+   }
+   const SweepSet<T> set = quat_set(fc, sm, gamma, ncomp);
+   int rc = 0;
+   quat_dispatch(fine.ndim, ncomp, [&](auto nd, auto ql) {
+      if constexpr (decltype(ql)::value > 0)
+         rc = block_resrestrict<T>(nd, std::integral_constant<int, 1>(), ql, coarse, fine, set.s[0],
+                                   dx, rhs, z, b, s);
+   });
+   return rc;
 }
 
 #define AMPE_INST(T)                                                                     \

@@ -228,3 +228,40 @@ def test_red_residual_restriction_elliptic(dev, shape, split, variant):
     assert np.abs(inter[black]).max() < 1e-12 * np.abs(inter[~black]).max()
     bf, br = b_full.cpu().numpy(), b_red.cpu().numpy()
     assert np.abs(br - bf).max() < 1e-12 * np.abs(bf).max()
+
+
+@pytest.mark.parametrize("shape,split", [((24, 36), 20), ((8, 12, 20), None), ((8, 12, 20), 12)])
+@pytest.mark.parametrize("take", [1, 2])
+def test_red_restriction_of_fewer_components(dev, shape, split, take):
+    """One, two and four components have kernels of their own: the red-only
+    coarse right-hand side of a component does not depend on how many are
+    restricted with it, and matches the full residual's."""
+    import ctypes as C
+    import torch
+    from ampe_amd import hip as H
+    ndim = len(shape)
+    ext = list(shape[::-1]) + [1] * (3 - ndim)
+    cuts = [(0, ext[0] - 1)] if split is None else [(0, split - 1), (split, ext[0] - 1)]
+    boxes = [_box((lo, 0, 0), (hi, ext[1] - 1, ext[2] - 1)) for lo, hi in cuts]
+    full = H.boxes_of(shape, ndim)
+    fine = H.Level(ndim, boxes, 1, periodic=full)
+    coarse = H.Level(ndim, _halved(boxes), 1, periodic=_halved([full])[0])
+    rng = np.random.default_rng(11)
+    fc = torch.from_numpy(-rng.uniform(0.5, 1.5, fine.nside_tot)).to(dev)
+    sm, rhs, z = (torch.from_numpy(np.concatenate(
+        [fine.to_ghosted(f(size=shape)) for _ in range(k)])).to(dev)
+        for f, k in ((lambda size: rng.uniform(0.5, 1.5, size), 1), (rng.normal, 4), (rng.normal, 4)))
+    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    L = H.lib()
+    H.check(L.ampe_ghost_fill(fine.h, ptr(sm), 1, None))
+    dx = (C.c_double * 3)(0.5, 0.25, 0.75)
+    H.check(L.ampe_quat_smooth(fine.h, ptr(fc), ptr(sm), 0.3, dx, 4, ptr(rhs), ptr(z), 1, 0, None))
+    out = {}
+    for n, red in ((4, 1), (take, 1), (take, 0)):
+        b, res = torch.zeros(4 * coarse.ncg, dtype=torch.float64, device=dev), torch.zeros_like(z)
+        H.check(L.ampe_quat_residual_restrict(coarse.h, fine.h, ptr(fc), ptr(sm), 0.3, dx, n,
+                                              ptr(rhs), ptr(z), ptr(res), ptr(b), red, None))
+        out[n, red] = b.cpu().numpy()[:take * coarse.ncg]
+    assert np.abs(out[take, 1]).max() > 0 and np.array_equal(out[take, 1], out[4, 1])
+    # the black residuals left out are rounding of rows of size one
+    assert np.abs(out[take, 1] - out[take, 0]).max() < 1e-12 * np.abs(out[take, 0]).max()
