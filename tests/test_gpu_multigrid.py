@@ -155,6 +155,25 @@ def test_refine_add(dev, ndim, order):
         assert set(np.round(got, 12)) <= set(np.round(cint, 12))
 
 
+@pytest.mark.parametrize("ndim", [2, 3])
+@pytest.mark.parametrize("order", [0, 1])
+def test_refine_add_components(dev, ndim, order):
+    """Several components at once: each as by itself, to the last bit."""
+    from ampe_amd import hip as H
+    import torch
+    fine, coarse = _levels(ndim)
+    rng = np.random.default_rng(2)
+    c = torch.from_numpy(rng.normal(size=3 * coarse.ncg)).to(dev)
+    f = torch.from_numpy(rng.normal(size=3 * fine.ncg)).to(dev)
+    g = f.clone()
+    H.check(H.lib().ampe_refine_add(fine.h, coarse.h, 3, order, _ptr(c), _ptr(f), None))
+    for m in range(3):
+        H.check(H.lib().ampe_refine_add(fine.h, coarse.h, 1, order,
+                                        C.c_void_p(c.data_ptr() + 8 * m * coarse.ncg),
+                                        C.c_void_p(g.data_ptr() + 8 * m * fine.ncg), None))
+    assert torch.equal(f, g) and not torch.equal(f[:fine.ncg], f[fine.ncg:2 * fine.ncg])
+
+
 def test_refine_rejects_level_that_is_not_halved(dev):
     from ampe_amd import hip as H
     import torch
