@@ -466,7 +466,8 @@ int ampe_fac_residual_restrict(const ampe_level* coarse, const ampe_level* fine,
    if (ampe::ghost_fill(F, u, 1, s)) return -1;
    if (red_only) {
       AMPE_REQUIRE(ampe::red_residual_ok(F, 1),
-                   "red_only needs a periodic fine level with even, non-negative patch corners");
+                   "red_only needs a periodic fine level covered by its patches, of even extents, with "
+                   "even, non-negative patch corners");
       return ampe::launch_ell_resrestrict<double>(*coarse->L, F, o, op->dx, rhs, u, b, s);
    }
    AMPE_REQUIRE(res, "null residual buffer");
@@ -721,8 +722,8 @@ int ampe_quat_residual_restrict(const ampe_level* coarse, const ampe_level* fine
    if (ampe::ghost_fill(F, z, ncomp, s)) return -1;
    if (red_only) {
       AMPE_REQUIRE(ampe::red_residual_ok(F, ncomp),
-                   "red_only needs a periodic fine level with even, non-negative patch "
-                   "corners and one, two or four components");
+                   "red_only needs a periodic fine level covered by its patches, of even extents, "
+                   "with even, non-negative patch corners, and one, two or four components");
       return ampe::launch_quat_resrestrict<double>(*coarse->L, F, fc, sm, gamma, dx, ncomp, rhs,
                                                    z, b, s);
    }

@@ -97,10 +97,8 @@ int mg_prolong_add(const Level& fine, const Level& coarse, int ncomp, int order,
                    T* xf, hipStream_t s, bool split = false, bool wrap = false);
 // coarse holds the boxes of fine halved, patch by patch (even corners/extents)
 bool is_coarsening(const Level& coarse, const Level& fine);
-// After red-black sweeps ending with the black colour, the orientation
-// residual vanishes on black cells when every black cell's neighbours are
-// red: one checkerboard over the patches (non-negative, even patch corners)
-// and periodic ghosts; one, two or four components.
+// After red-black sweeps ending with the black colour a block's residual
+// vanishes on black cells (checker_ok); one, two or four components.
 bool red_residual_ok(const Level& L, int ncomp);
 
 // Orientation field (ql <= 4 components) coarsened by the normalised volume

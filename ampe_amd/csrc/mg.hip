@@ -380,21 +380,12 @@ int mg_setup_quat(Mg<T>& m, const T* fc0, const T* sm0, hipStream_t s)
 
 // ------------------------------------------------------------ cycles
 // The residual after red-black sweeps ending with the black colour vanishes
-// on black cells when every black cell's neighbours are red: one checkerboard
-// over the patches (non-negative, even patch corners: the colour rule of the
-// sweeps then depends on global indices only) and periodic ghosts (zero-slope
-// ghosts copy a cell's own value into its row).  One, two or four components.
+// on black cells when every black cell's neighbours are red (checker_ok: a
+// zero-slope ghost, at a bounded side or next to cells no patch covers, copies a
+// cell's own value into its row).  One, two or four components.
 bool red_residual_ok(const Level& L, int ncomp)
 {
-   if (!L.periodic || (ncomp != 1 && ncomp != 2 && ncomp != 4)) return false;
-   for (int a = 0; a < L.ndim; a++) {
-      int ext = L.pbox.hi[a] - L.pbox.lo[a] + 1;
-      if (L.pbox.lo[a] < 0 || (L.pbox.lo[a] & 1) || (ext & 1)) return false;
-   }
-   for (const PatchDev& d : L.hp)
-      for (int a = 0; a < L.ndim; a++)
-         if (d.lo[a] < 0 || (d.lo[a] & 1)) return false;
-   return true;
+   return checker_ok(L) && (ncomp == 1 || ncomp == 2 || ncomp == 4);
 }
 
 // The set's operators on level l.

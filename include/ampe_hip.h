@@ -582,7 +582,8 @@ int ampe_fac_residual(const ampe_level* level, const ampe_elliptic_op* op,
  * restriction.  red_only = 1: u comes out of red-black sweeps ending with the
  * black colour, whose residual vanishes on black cells, so only the red
  * cells' residuals are formed, per coarse cell (res unused); needs a periodic
- * fine level with even, non-negative patch corners. */
+ * fine level covered by its patches, of even extents, with even, non-negative
+ * patch corners. */
 int ampe_fac_residual_restrict(const ampe_level* coarse, const ampe_level* fine,
                                const ampe_elliptic_op* op, const double* rhs, double* u,
                                double* res, double* b, int red_only, ampe_stream_t stream);
@@ -613,8 +614,9 @@ int ampe_refine_add(const ampe_level* fine, const ampe_level* coarse, int ncomp,
  * blocks), then the restriction.  red_only = 1: z comes out of red-black
  * sweeps ending with the black colour, whose residual vanishes on black
  * cells, so only the red cells' residuals are formed, per coarse cell, and
- * res is not used; needs a periodic fine level with even, non-negative patch
- * corners (one checkerboard) and ncomp 1, 2 or 4. */
+ * res is not used; needs a periodic fine level covered by its patches, of even
+ * extents, with even, non-negative patch corners (one checkerboard) and ncomp
+ * 1, 2 or 4. */
 int ampe_quat_residual_restrict(const ampe_level* coarse, const ampe_level* fine,
                                 const double* fc, const double* sm, double gamma,
                                 const double dx[3], int ncomp, const double* rhs, double* z,

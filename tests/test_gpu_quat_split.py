@@ -265,3 +265,36 @@ def test_red_restriction_of_fewer_components(dev, shape, split, take):
     assert np.abs(out[take, 1]).max() > 0 and np.array_equal(out[take, 1], out[4, 1])
     # the black residuals left out are rounding of rows of size one
     assert np.abs(out[take, 1] - out[take, 0]).max() < 1e-12 * np.abs(out[take, 0]).max()
+
+
+def test_red_restriction_needs_covered_level(dev):
+    """A periodic level with cells no patch covers: the ghosts beside them copy
+    the cell's own value into its row, so black residuals do not vanish after
+    the black sweep (the full residual shows them), and the restriction of the
+    red ones alone is refused."""
+    import ctypes as C
+    import torch
+    from ampe_amd import hip as H
+    shape = (16, 20)
+    dom, cdom = H.boxes_of((16, 32), 2), H.boxes_of((8, 16), 2)
+    fine = H.Level(2, [H.boxes_of(shape, 2)], 1, periodic=dom)
+    coarse = H.Level(2, [H.boxes_of((8, 10), 2)], 1, periodic=cdom)
+    rng = np.random.default_rng(5)
+    op = H.EllipticOp(None, -0.7, None, 1.0, None, 1.0, (C.c_double * 3)(1, 1, 1))
+    rhs, u = (torch.from_numpy(fine.to_ghosted(rng.normal(size=shape))).to(dev) for _ in range(2))
+    fc = torch.from_numpy(-rng.uniform(0.5, 1.5, fine.nside_tot)).to(dev)
+    sm = torch.ones_like(u)
+    res, b = torch.zeros_like(u), torch.zeros(coarse.ncg, dtype=torch.float64, device=dev)
+    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    L = H.lib()
+    H.check(L.ampe_fac_smooth(fine.h, C.byref(op), ptr(rhs), ptr(u), 1, -1.0, None, None))
+    H.check(L.ampe_fac_residual_restrict(coarse.h, fine.h, C.byref(op), ptr(rhs), ptr(u), ptr(res),
+                                         ptr(b), 0, None))
+    r = np.abs(_domain(fine, res.cpu().numpy(), shape))
+    black = (np.indices(shape).sum(axis=0) % 2) == 1
+    assert r[black].max() > 1e-3 * r[~black].max()
+    assert L.ampe_fac_residual_restrict(coarse.h, fine.h, C.byref(op), ptr(rhs), ptr(u), None,
+                                        ptr(b), 1, None) < 0
+    dx = (C.c_double * 3)(1, 1, 1)
+    assert L.ampe_quat_residual_restrict(coarse.h, fine.h, ptr(fc), ptr(sm), 0.3, dx, 1, ptr(rhs),
+                                         ptr(u), None, ptr(b), 1, None) < 0
