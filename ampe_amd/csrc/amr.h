@@ -49,7 +49,7 @@ int hier_weight_sum(Hier* H, double* sum);
 int hier_nlev(const Hier* H);
 // coarsenData of an integrator state (phase, composition: CONSERVATIVE_COARSEN;
 // orientation: QuatWeightedAverage) and its ghosts by LINEAR_REFINE
-int hier_sim_sync_fill(Hier* H, double* y, int nc, int nord, int ic, int ncs, int iq, int qlen,
+int hier_sim_sync_fill(Hier* H, double* y, int nc, int nord, int ncs, int iq, int qlen,
                        hipStream_t s);
 int hier_ghost_fill(const Hier& H, double* f, int ncomp, int cf, hipStream_t s);
 int hier_coarsen(const Hier& H, double* f, int ncomp, int quatnorm, hipStream_t s);

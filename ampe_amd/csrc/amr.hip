@@ -1825,14 +1825,13 @@ int hier_weight_sum(Hier* H, double* sum)
    return 0;
 }
 
-int hier_sim_sync_fill(Hier* H, double* y, int nc, int nord, int ic, int ncs, int iq, int qlen,
+int hier_sim_sync_fill(Hier* H, double* y, int nc, int nord, int ncs, int iq, int qlen,
                        hipStream_t s)
 {
    if (iq >= 0 && qlen != 4) {
       set_error("hier_sim_sync_fill: four orientation components");
       return -1;
    }
-   (void)ic;
    const int rows = nord + ncs + (iq >= 0 ? 1 : 0);
    for (int l = H->nlev - 2; l >= 0; l--) {
       if (H->crs_dst[l].n == 0) continue;

@@ -42,6 +42,28 @@ struct SetForm {
    bool split = false, wrap = false;
    int from = 0;
 };
+// The split layout is the FP32 vectors'.
+template <typename T>
+constexpr bool kCanSplit = false;
+template <>
+inline constexpr bool kCanSplit<float> = true;
+// Calls f with split as std::integral_constant, where the element type has it; -1
+// where it has not.
+template <typename T, class F>
+int split_dispatch(bool split, F&& f)
+{
+   if constexpr (kCanSplit<T>) {
+      if (split) {
+         f(std::true_type());
+         return 0;
+      }
+   } else if (split) {
+      set_error("the row parity-split layout is for FP32 vectors");
+      return -1;
+   }
+   f(std::false_type());
+   return 0;
+}
 constexpr int kMaxSlots = 16;
 template <typename T>
 struct SweepSet {

@@ -482,8 +482,9 @@ __global__ void __launch_bounds__(256) k_quat_rbgs_shell(LevelArgs a, const T* _
    }
 }
 
-// Residual of one cell, every component (QL as in quat_rbgs_cell); returns
-// the sum of the squared residuals (double).
+// Residual of one cell, every component (QL > 0: all loads of QL components
+// before the first of them is used); returns the sum of the squared residuals
+// (double).
 template <typename T, int NDIM, int QL, bool SPLIT>
 __device__ __forceinline__ double quat_residual_cell(const LevelArgs& a, const CellPos& c,
                                                      const T* __restrict__ fc,
@@ -1010,15 +1011,15 @@ int launch_set_sweep(const Level& L, const SweepSet<T>& set, const double* dx, c
       else
          go(nd, sp, wr, std::integral_constant<int, 0>());
    };
-   auto by_form = [&](auto nd) {
-      bool_dispatch(form.split, [&](auto sp) {
-         bool_dispatch(form.wrap, [&](auto wr) { by_from(nd, sp, wr); });
+   const int rc = split_dispatch<T>(form.split, [&](auto sp) {
+      bool_dispatch(form.wrap, [&](auto wr) {
+         if (L.ndim == 3)
+            by_from(std::integral_constant<int, 3>(), sp, wr);
+         else
+            by_from(std::integral_constant<int, 2>(), sp, wr);
       });
-   };
-   if (L.ndim == 3)
-      by_form(std::integral_constant<int, 3>());
-   else
-      by_form(std::integral_constant<int, 2>());
+   });
+   if (rc) return rc;
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -1037,12 +1038,13 @@ int launch_set_residual(const Level& L, const SweepSet<T>& set, const double* dx
                          tblock(), 0, s, la, set, di[0], di[1], di[2], hi[0], hi[1], hi[2], rhs, x,
                          res);
    };
-   bool_dispatch(split, [&](auto sp) {
+   const int rc = split_dispatch<T>(split, [&](auto sp) {
       if (L.ndim == 3)
          go(std::integral_constant<int, 3>(), sp);
       else
          go(std::integral_constant<int, 2>(), sp);
    });
+   if (rc) return rc;
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -1063,7 +1065,7 @@ int launch_set_resrestrict(const Level& coarse, const Level& fine, const SweepSe
                          g, tblock(), 0, s, ca, fa, set, di[0], di[1], di[2], hi[0], hi[1], hi[2],
                          rhs, x, b);
    };
-   bool_dispatch(form.split, [&](auto sp) {
+   const int rc = split_dispatch<T>(form.split, [&](auto sp) {
       bool_dispatch(form.wrap, [&](auto wr) {
          if (fine.ndim == 3)
             go(std::integral_constant<int, 3>(), sp, wr);
@@ -1071,6 +1073,7 @@ int launch_set_resrestrict(const Level& coarse, const Level& fine, const SweepSe
             go(std::integral_constant<int, 2>(), sp, wr);
       });
    });
+   if (rc) return rc;
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -1255,16 +1258,15 @@ int launch_quat_residual(const Level& L, const T* fc, const T* sm, double gamma,
    dim3 g(L.ncell_tiles);
    T hi[3];
    recip2(dx, hi);
-   auto go = [&](auto ndim, auto ql) {
-      constexpr int ND = decltype(ndim)::value, Q = decltype(ql)::value;
-      if (split)
-         hipLaunchKernelGGL((k_quat_residual<T, ND, Q, true>), g, tblock(), 0, s, la, fc, sm,
-                            (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res, part);
-      else
-         hipLaunchKernelGGL((k_quat_residual<T, ND, Q, false>), g, tblock(), 0, s, la, fc, sm,
-                            (T)gamma, hi[0], hi[1], hi[2], ncomp, rhs, z, res, part);
-   };
-   quat_dispatch(L.ndim, ncomp, go);
+   const int rc = split_dispatch<T>(split, [&](auto sp) {
+      quat_dispatch(L.ndim, ncomp, [&](auto ndim, auto ql) {
+         hipLaunchKernelGGL((k_quat_residual<T, decltype(ndim)::value, decltype(ql)::value,
+                                             decltype(sp)::value>),
+                            g, tblock(), 0, s, la, fc, sm, (T)gamma, hi[0], hi[1], hi[2], ncomp,
+                            rhs, z, res, part);
+      });
+   });
+   if (rc) return rc;
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -1305,16 +1307,18 @@ int launch_quat_resrestrict(const Level& coarse, const Level& fine, const T* fc,
                                     int, const T*, T*, int, hipStream_t);                \
    template int launch_quat_residual<T>(const Level&, const T*, const T*, double,         \
                                         const double*, int, const T*, const T*, T*,      \
-                                        double*, hipStream_t, bool);                     \
-   template int launch_ell_resrestrict<T>(const Level&, const Level&, const EllOp<T>&,     \
-                                          const double*, const T*, const T*, T*, hipStream_t); \
-   template int launch_quat_resrestrict<T>(const Level&, const Level&, const T*, const T*, \
-                                           double, const double*, int, const T*,         \
-                                           const T*, T*, hipStream_t);                   \
-   template int launch_quat_rbgs_fused<T>(const Level&, const T*, const T*, double,       \
-                                          const double*, int, const T*, const T*, T*,    \
-                                          hipStream_t);
+                                        double*, hipStream_t, bool);
 AMPE_INST(double)
 AMPE_INST(float)
+// by the entry points alone
+template int launch_ell_resrestrict<double>(const Level&, const Level&, const EllOp<double>&,
+                                            const double*, const double*, const double*, double*,
+                                            hipStream_t);
+template int launch_quat_resrestrict<double>(const Level&, const Level&, const double*,
+                                             const double*, double, const double*, int,
+                                             const double*, const double*, double*, hipStream_t);
+template int launch_quat_rbgs_fused<double>(const Level&, const double*, const double*, double,
+                                            const double*, int, const double*, const double*,
+                                            double*, hipStream_t);
 
 }  // namespace ampe

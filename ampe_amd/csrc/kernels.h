@@ -98,26 +98,6 @@ __device__ __forceinline__ bool cell_pos_col(const LevelArgs& a, int kk, CellPos
    return true;
 }
 
-// Pair mapping of a tile onto a workgroup of TX/2 x TY threads: thread
-// (tx, ty) takes the cell 2 tx + io of its row, so the lanes of a half-wave
-// hold cells of one column parity (io = 0 and 1 in turn cover the tile).
-// Plane t.k + kk; false when outside the box.
-__device__ __forceinline__ bool cell_pos_pair(const LevelArgs& a, int kk, int io, CellPos& c)
-{
-   const Tile t = a.T[tile_index(a)];
-   c.pd = a.P[t.patch];
-   c.i = t.i0 + 2 * (int)threadIdx.x + io;  // t.i0 is a multiple of TX (even)
-   c.j = t.j0 + (int)threadIdx.y;
-   c.k = t.k + kk;
-   if (c.i >= c.pd.nx || c.j >= c.pd.ny || c.k >= c.pd.nz) return false;
-   c.st[0] = 1;
-   c.st[1] = c.pd.sy;
-   c.st[2] = c.pd.sz;
-   c.c0 = c.pd.cell_off + (c.i + a.g) + (long long)(c.j + a.g) * c.pd.sy +
-          (long long)(c.k + a.gz) * c.pd.sz;
-   return true;
-}
-
 // Row parity-split layout of a ghosted cell block: inside every row of sy
 // cells the even ghosted columns come first, then the odd ones, so the cells
 // of one red-black colour in a row are contiguous (a colour sweep writes and
@@ -232,9 +212,6 @@ int launch_rhs_all(const Level& L, const ampe_model_params& p, const RhsLev& k, 
 int launch_conc_coeffs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
                            const double* phi, const double* cl, const double* cs, double* Dc,
                            double* Dphi, hipStream_t s);
-int launch_conc_rhs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
-                        const double* c, const double* phi, const double* Dc, const double* Dphi,
-                        double* rhs, hipStream_t s);
 int launch_phase_rhs(const Level& L, const ampe_model_params& p, const double* phi,
                      const double* q, const double* cl, const double* cs, double* rhs,
                      hipStream_t s);

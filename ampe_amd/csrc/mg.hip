@@ -114,12 +114,12 @@ __global__ void __launch_bounds__(256) k_prolong_add(LevelArgs fa, LevelArgs ca,
    }
 }
 
-// The split-layout prolongation per coarse cell: a thread adds the
+// The split-layout interpolation per coarse cell: a thread adds the
 // correction to the 2^NDIM children of its coarse cell (consecutive lanes:
 // consecutive coarse cells, so for each child offset the fine updates are
 // contiguous in the split layout), each child's value by the formula and
 // summation order of the natural form.
-template <typename T, int NDIM, int ORDER, bool WRAP>
+template <typename T, int NDIM, bool WRAP>
 __global__ void __launch_bounds__(256) k_prolong_add_cc(LevelArgs fa, LevelArgs ca,
                                                         const T* __restrict__ xc,
                                                         T* __restrict__ xf)
@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(256) k_prolong_add_cc(LevelArgs fa, LevelArgs 
    for (int e = 0; e < (NDIM == 3 ? 8 : 4); e++) {
       const long long oj = nbr_off<WRAP>(p.j, p.pd.ny, sy, (e >> 1) & 1);
       const long long ok = NDIM == 3 ? nbr_off<WRAP>(p.k, p.pd.nz, p.pd.sz, e >> 2) : 0;
-      y[fo[e]] = old[e] + prolong_value<T, NDIM, ORDER>(x, c0, (e & 1) ? cp : cm, oj, ok);
+      y[fo[e]] = old[e] + prolong_value<T, NDIM, 1>(x, c0, (e & 1) ? cp : cm, oj, ok);
    }
 }
 
@@ -165,14 +165,13 @@ int mg_restrict_cell(const Level& coarse, const Level& fine, int ncomp, const T*
       hipLaunchKernelGGL((k_restrict_cell<T, decltype(nd)::value, decltype(sp)::value>), g, b, 0,
                          s, ca, fa, ncomp, f, c);
    };
-   using I2 = std::integral_constant<int, 2>;
-   using I3 = std::integral_constant<int, 3>;
-   using ST = std::true_type;
-   using SF = std::false_type;
-   if (coarse.ndim == 3)
-      split ? go(I3(), ST()) : go(I3(), SF());
-   else
-      split ? go(I2(), ST()) : go(I2(), SF());
+   const int rc = split_dispatch<T>(split, [&](auto sp) {
+      if (coarse.ndim == 3)
+         go(std::integral_constant<int, 3>(), sp);
+      else
+         go(std::integral_constant<int, 2>(), sp);
+   });
+   if (rc) return rc;
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -202,26 +201,33 @@ int mg_prolong_add(const Level& fine, const Level& coarse, int ncomp, int order,
    dim3 gf(fine.ncell_tiles, order == 0 ? 1 : ncomp);
    dim3 gc(coarse.ncell_tiles, ncomp), b(TX, TY);
    LevelArgs fa = level_args(fine), ca = level_args(coarse);
-   auto go = [&](auto nd, auto od, auto wr) {
-      constexpr int ND = decltype(nd)::value, OD = decltype(od)::value;
+   if (split && order == 0) {
+      set_error("mg_prolong_add: the split layout has the interpolated form only");
+      return -1;
+   }
+   auto go = [&](auto nd, auto sp, auto wr) {
+      constexpr int ND = decltype(nd)::value;
       constexpr bool WR = decltype(wr)::value;
-      if (split)
-         hipLaunchKernelGGL((k_prolong_add_cc<T, ND, OD, WR>), gc, b, 0, s, fa, ca, xc, xf);
+      if constexpr (decltype(sp)::value)
+         hipLaunchKernelGGL((k_prolong_add_cc<T, ND, WR>), gc, b, 0, s, fa, ca, xc, xf);
+      else if (order == 0)
+         hipLaunchKernelGGL((k_prolong_add<T, ND, 0, false>), gf, b, 0, s, fa, ca, ncomp, xc, xf);
       else
-         hipLaunchKernelGGL((k_prolong_add<T, ND, OD, WR>), gf, b, 0, s, fa, ca, ncomp, xc, xf);
+         hipLaunchKernelGGL((k_prolong_add<T, ND, 1, WR>), gf, b, 0, s, fa, ca, ncomp, xc, xf);
    };
-   auto by = [&](auto nd) {
-      if (order == 0)
-         go(nd, std::integral_constant<int, 0>(), std::false_type());
-      else if (wrap)
-         go(nd, std::integral_constant<int, 1>(), std::true_type());
+   const int rc = split_dispatch<T>(split, [&](auto sp) {
+      auto by_wrap = [&](auto nd) {
+         if (wrap)
+            go(nd, sp, std::true_type());
+         else
+            go(nd, sp, std::false_type());
+      };
+      if (fine.ndim == 3)
+         by_wrap(std::integral_constant<int, 3>());
       else
-         go(nd, std::integral_constant<int, 1>(), std::false_type());
-   };
-   if (fine.ndim == 3)
-      by(std::integral_constant<int, 3>());
-   else
-      by(std::integral_constant<int, 2>());
+         by_wrap(std::integral_constant<int, 2>());
+   });
+   if (rc) return rc;
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -415,7 +421,7 @@ static SweepSet<T> level_set(const Mg<T>& m, const SweepSet<T>& set, int l)
 // zero.  On one checkerboard the first two colours then start from what they
 // know (SetForm::from) and nothing is cleared; elsewhere a colour may read its
 // own colour across the boundary, and x is cleared.  A level that wraps fills
-// no ghosts.  nv: length of x.
+// no ghosts.
 template <typename T>
 int set_smooth(const Level& L, const SweepSet<T>& set, const double* dx, int ncomp, const T* b,
                T* x, int sweeps, bool zero, bool split, hipStream_t s)
@@ -505,11 +511,11 @@ int mg_enable_split(Mg<T>& m, hipStream_t s)
                              hipStream_t);                                                   \
    template int mg_restrict_cell<T>(const Level&, const Level&, int, const T*, T*,           \
                                     hipStream_t, bool);                                      \
-   template int mg_enable_split<T>(Mg<T>&, hipStream_t);                                     \
    template int mg_restrict_side<T>(const Level&, const Level&, const T*, T*, hipStream_t);  \
    template int mg_prolong_add<T>(const Level&, const Level&, int, int, const T*, T*,        \
                                   hipStream_t, bool, bool);
 AMPE_MG_INST(float)
 AMPE_MG_INST(double)
+template int mg_enable_split<float>(Mg<float>&, hipStream_t);
 
 }  // namespace ampe

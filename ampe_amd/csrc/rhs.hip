@@ -75,26 +75,26 @@ __global__ void __launch_bounds__(256) k_quat_modulus(LevelArgs a, ampe_model_pa
    gmod[c.c0] = quat_cell_modulus<NDIM>(p, k, q, a.ncg, c.st, c.c0);
 }
 
-// GNI: store 1 / |grad q| of the face (grad_normi) instead of |grad q|^2.
-template <int NDIM, bool GNI>
+// Any number of components.
+template <int NDIM>
 __global__ void __launch_bounds__(256) k_quat_face_norm2(LevelArgs a, ampe_model_params p,
-                                                         RhsLev kl, const double* __restrict__ q,
+                                                         RhsConst k, const double* __restrict__ q,
                                                          double* __restrict__ n2)
 {
    CellPos c;
    if (!cell_pos(a, 1, c)) return;
    if (NDIM == 2 && c.k > 0) return;
-   const RhsConst& k = kl.k[c.pd.lev];
    for (int d = 0; d < NDIM; d++) {
       bool ok = (c.i < c.pd.nx + (d == 0)) && (c.j < c.pd.ny + (d == 1)) &&
                 (NDIM == 2 || c.k < c.pd.nz + (d == 2));
       if (!ok) continue;
-      const double v = quat_face_norm2<NDIM>(p, k, q, a.ncg, c.st, d, c.c0 - c.st[d], c.c0);
-      n2[face_idx(a, c.pd, d, c.i, c.j, c.k)] = GNI ? face_gni(p, k, v) : v;
+      n2[face_idx(a, c.pd, d, c.i, c.j, c.k)] =
+          quat_face_norm2<NDIM>(p, k, q, a.ncg, c.st, d, c.c0 - c.st[d], c.c0);
    }
 }
 
-// The same in 3-D for four components.  A workgroup marches up a column of KM
+// The same in 3-D for four components; GNI: 1 / |grad q| of the face (grad_normi)
+// instead of |grad q|^2.  A workgroup marches up a column of KM
 // planes of its tile: four planes of the tile's q with a one-cell halo sit in
 // LDS (k - 1, k, k + 1 and the one being loaded), so that each value is read
 // once, and a cell's centred differences serve all its faces: across a face
@@ -556,7 +556,7 @@ __global__ void __launch_bounds__(256) k_conc_coeffs(LevelArgs a, ampe_model_par
 // concentrationflux (2d/concentrationrhs.m4:15-82) + computerhsconcentration
 // (2d/concentrationrhs.m4:326-367)
 template <int NDIM>
-__global__ void __launch_bounds__(256) k_conc_rhs(LevelArgs a, ampe_model_params p, RhsLev kl,
+__global__ void __launch_bounds__(256) k_conc_rhs(LevelArgs a, ampe_model_params p, RhsConst k,
                                                   const double* __restrict__ cc,
                                                   const double* __restrict__ phi,
                                                   const double* __restrict__ Dc,
@@ -564,7 +564,6 @@ __global__ void __launch_bounds__(256) k_conc_rhs(LevelArgs a, ampe_model_params
                                                   double* __restrict__ rhs)
 {
    AMPE_COLUMN_BEGIN(a, c)
-   const RhsConst& k = kl.k[c.pd.lev];
    const long long c0 = c.c0;
    const int ijk[3] = {c.i, c.j, c.k};
    double s = 0.0;
@@ -893,16 +892,18 @@ static int quat_face_norms(const Level& L, const ampe_model_params& p, const Rhs
 {
    dim3 g(L.nface_tiles), b = tile_block();
    LevelArgs a = level_args(L, true);
-   if (L.ndim == 3 && p.qlen == 4)
-      hipLaunchKernelGGL(k_quat_face_norm2_march<GNI>, dim3(L.nmarch_tiles), b, 0, s,
-                         level_args_march(L), p, k, q, n2);
-   else if (L.ndim == 3)
-      hipLaunchKernelGGL((k_quat_face_norm2<3, GNI>), g, b, 0, s, a, p, k, q, n2);
-   else if (p.qlen == 4)
-      hipLaunchKernelGGL(k_quat_face_norm2_tile<GNI>, dim3(L.ncell_tiles), b, 0, s, level_args(L),
-                         p, k, q, n2);
-   else
-      hipLaunchKernelGGL((k_quat_face_norm2<2, GNI>), g, b, 0, s, a, p, k, q, n2);
+   if (GNI || p.qlen == 4) {  // (the integrator has four components)
+      if (L.ndim == 3)
+         hipLaunchKernelGGL(k_quat_face_norm2_march<GNI>, dim3(L.nmarch_tiles), b, 0, s,
+                            level_args_march(L), p, k, q, n2);
+      else
+         hipLaunchKernelGGL(k_quat_face_norm2_tile<GNI>, dim3(L.ncell_tiles), b, 0, s,
+                            level_args(L), p, k, q, n2);
+   } else if (L.ndim == 3) {
+      hipLaunchKernelGGL(k_quat_face_norm2<3>, g, b, 0, s, a, p, k.k[0], q, n2);
+   } else {
+      hipLaunchKernelGGL(k_quat_face_norm2<2>, g, b, 0, s, a, p, k.k[0], q, n2);
+   }
    AMPE_HIP_CHECK(hipGetLastError());
    return 0;
 }
@@ -1046,19 +1047,12 @@ int launch_conc_coeffs(const Level& L, const ampe_model_params& p, const double*
    return launch_conc_coeffs_lev(L, p, rhs_lev(p), phi, cl, cs, Dc, Dphi, s);
 }
 
-int launch_conc_rhs_lev(const Level& L, const ampe_model_params& p, const RhsLev& k,
-                        const double* c, const double* phi, const double* Dc, const double* Dphi,
-                        double* rhs, hipStream_t s)
-{
-   AMPE_DISPATCH(L, k_conc_rhs, L.ncol_tiles, level_args_col(L), p, k, c, phi, Dc, Dphi, rhs);
-   return 0;
-}
-
 int launch_conc_rhs(const Level& L, const ampe_model_params& p, const double* c,
                     const double* phi, const double* Dc, const double* Dphi, double* rhs,
                     hipStream_t s)
 {
-   return launch_conc_rhs_lev(L, p, rhs_lev(p), c, phi, Dc, Dphi, rhs, s);
+   AMPE_DISPATCH(L, k_conc_rhs, L.ncol_tiles, level_args_col(L), p, rhs_const(p), c, phi, Dc, Dphi, rhs);
+   return 0;
 }
 
 int launch_ebs_coeffs(const Level& L, const ampe_model_params& p, const double* phi, double* DL,

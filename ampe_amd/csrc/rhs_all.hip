@@ -174,8 +174,9 @@ __device__ __forceinline__ void rhs_tail(const LevelArgs& a, const ampe_model_pa
    put(yc, c0, ic, p.conc_mobility * s);
 }
 
-// One cell per thread; the anisotropic flux (four transcendentals a face) is
-// evaluated once per x and y face through LDS (k_phase_rhs_faces).
+// One cell per thread; the anisotropic flux (square roots, a division and a
+// power a face) is evaluated once per x and y face through LDS
+// (k_phase_rhs_faces).
 template <int NDIM, int FLUX, int FE, int CONC, bool FIN>
 __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params p, RhsLev kl,
                                                  const double* __restrict__ phi,
@@ -232,8 +233,7 @@ __global__ void __launch_bounds__(256) k_rhs_all(LevelArgs a, ampe_model_params 
          double fhi = phase_face_flux<NDIM, FLUX>(p, k, phi, q, a.ncg, c.st, 2, c0, c0 + sz);
          r = r + (fhi - flo) * k.dxinv[2];
       }
-      rhs_tail<NDIM, FE, CONC, FIN>(a, p, k, c, r, phi, q, cc, cl, cs, gni, Dc, Dphi,
-                               yp, yq, yc, fin, iq,
+      rhs_tail<NDIM, FE, CONC, FIN>(a, p, k, c, r, phi, q, cc, cl, cs, gni, Dc, Dphi, yp, yq, yc, fin, iq,
                                     ic);
    } else {
       CellPos c;
@@ -259,12 +259,12 @@ int launch_rhs_all(const Level& L, const ampe_model_params& p, const RhsLev& k, 
                    int iq, int ic, const double* cl, const double* cs, const double* gni,
                    double* Dc, double* Dphi, int conc, double* rhs, hipStream_t s, const KryFin* fin)
 {
-   if (fin && conc > 1) {
-      set_error("rhs: a full evaluation's values are stored");
+   const int fe = ic >= 0 ? p.fe_model : kFeNone;
+   if (fin && conc != (ic >= 0 ? 1 : 0)) {
+      set_error("rhs: a full evaluation's values, or an EBS composition's, are stored");
       return -1;
    }
    const KryFin kf = fin ? *fin : KryFin{};
-   const int fe = ic >= 0 ? p.fe_model : kFeNone;
    const double* q = iq >= 0 ? y + (long long)iq * L.ncg : nullptr;
    const double* cc = ic >= 0 ? y + (long long)ic * L.ncg : nullptr;
    double* yq = iq >= 0 ? rhs + (long long)iq * L.ncg : nullptr;
@@ -277,7 +277,8 @@ int launch_rhs_all(const Level& L, const ampe_model_params& p, const RhsLev& k, 
                          Dc, Dphi, rhs, yq, yc, kf, iq, ic);
    };
    auto go = [&](auto nd, auto fl, auto f, auto cn) {
-      if constexpr (decltype(cn)::value < 2) {
+      // (values are passed on by evaluations whose composition, if any, is formed here)
+      if constexpr (decltype(cn)::value == (decltype(f)::value == kFeNone ? 0 : 1)) {
          if (fin) return go2(nd, fl, f, cn, std::true_type());
       }
       go2(nd, fl, f, cn, std::false_type());

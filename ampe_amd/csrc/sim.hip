@@ -420,7 +420,7 @@ int sim_set_state_composite(Sim* S, const double* y_host)
    hipStream_t st = S->stream;
    AMPE_HIP_CHECK(hipMemcpy(S->y, y_host, sizeof(double) * S->nv, hipMemcpyHostToDevice));
    int ql = S->iq >= 0 ? S->p.qlen : 0;
-   if (hier_sim_sync_fill(S->hier, S->y, S->nc, S->nord, S->ic, S->ncs, S->iq, ql, st)) return -1;
+   if (hier_sim_sync_fill(S->hier, S->y, S->nc, S->nord, S->ncs, S->iq, ql, st)) return -1;
    std::memset(&S->st, 0, sizeof(S->st));
    if (S->ic >= 0) {
       const double* cc = S->y + (long long)S->ic * S->ng;
@@ -533,7 +533,7 @@ static int hier_rhs_eval(Sim* S, double* y, double* ydot, bool fd)
    bool recompute = !fd || !S->s.lag_quat_sidegrad;
    S->st.nfe++;
    int ql = S->iq >= 0 ? p.qlen : 0;
-   if (hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ic, S->ncs, S->iq, ql, st)) return -1;
+   if (hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ncs, S->iq, ql, st)) return -1;
    const double* phi = y;
    const double* c = S->ic >= 0 ? y + (long long)S->ic * S->ng : nullptr;
    if (S->tern) {
@@ -556,7 +556,7 @@ static int hier_psetup(Sim* S, double* y, double gamma, bool fresh)
    hipStream_t st = S->stream;
    S->st.npe++;
    int ql = S->iq >= 0 ? p.qlen : 0;
-   if (!fresh && hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ic, S->ncs, S->iq, ql, st))
+   if (!fresh && hier_sim_sync_fill(S->hier, y, S->nc, S->nord, S->ncs, S->iq, ql, st))
       return -1;
    const double* phi = y;
    const double* q = S->iq >= 0 ? y + (long long)S->iq * S->ng : nullptr;
