@@ -68,6 +68,11 @@ static int sim_check(const ampe_model_params& p, const ampe_solver_params& s)
       set_error("sim_create: qlen must be 4");
       return -1;
    }
+   if (p.with_conc && p.fe_model != AMPE_FE_QUADRATIC && p.fe_model != AMPE_FE_CALPHAD_BINARY &&
+       p.fe_model != AMPE_FE_KKS_DILUTE && p.fe_model != AMPE_FE_QUADRATIC_TERNARY_3PH) {
+      set_error("sim_create: unknown free-energy model");
+      return -1;
+   }
    if (p.phi_mobility_type == AMPE_PHI_MOB_KIM && !p.with_conc) {
       set_error("sim_create: Kim's phase mobility needs a composition field");
       return -1;
