@@ -2266,6 +2266,9 @@ int ampe_hier_phase_rhs(const ampe_hier* h, const ampe_model_params* p0, const d
                         ampe_stream_t stream)
 {
    AMPE_HREQ(h && p0 && phi && rhs, "null argument");
+   AMPE_HREQ(!p0->evolve_quat || q, "orientation field required");
+   AMPE_HREQ(p0->flux_type != AMPE_FLUX_ANISOTROPIC || q, "anisotropy needs q");
+   AMPE_HREQ(!p0->with_conc || (cl && cs), "phase concentrations required");
    return ampe::hier_phase_rhs(*h->H, *p0, phi, q, cl, cs, rhs, hstream(stream));
 }
 

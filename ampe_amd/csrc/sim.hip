@@ -77,6 +77,11 @@ static int sim_check(const ampe_model_params& p, const ampe_solver_params& s)
       set_error("sim_create: Kim's phase mobility needs a composition field");
       return -1;
    }
+   // (several orders have a flux of their own)
+   if (p.flux_type == AMPE_FLUX_ANISOTROPIC && !p.evolve_quat && p.norderp <= 1) {
+      set_error("sim_create: the anisotropic flux needs an orientation field");
+      return -1;
+   }
    if (p.conc_rhs_form != AMPE_CONC_RHS_KKS && p.conc_rhs_form != AMPE_CONC_RHS_EBS) {
       set_error("sim_create: unknown composition rhs form");
       return -1;
