@@ -51,12 +51,17 @@ struct DevVec {
    T* p = nullptr;
    long long n = 0;
    DevSpan<T> part(size_t from, size_t count) const { return {p + from, (long long)count}; }
-   int upload(const std::vector<T>& h)
+   // h, and h2 behind it
+   int upload(const std::vector<T>& h, const std::vector<T>& h2 = {})
    {
-      n = (long long)h.size();
+      n = (long long)(h.size() + h2.size());
       if (n == 0) return 0;
-      AMPE_HIP_CHECK(hipMalloc((void**)&p, sizeof(T) * h.size()));
-      AMPE_HIP_CHECK(hipMemcpy(p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
+      AMPE_HIP_CHECK(hipMalloc((void**)&p, sizeof(T) * (size_t)n));
+      if (!h.empty())
+         AMPE_HIP_CHECK(hipMemcpy(p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice));
+      if (!h2.empty())
+         AMPE_HIP_CHECK(hipMemcpy(p + h.size(), h2.data(), sizeof(T) * h2.size(),
+                                  hipMemcpyHostToDevice));
       return 0;
    }
    void release()
@@ -646,15 +651,12 @@ int hier_create(int ndim, int nlev, const int* npatch, const ampe_box* boxes, co
       };
       std::vector<CfCorr> corr, icorr;
       if (records(keys, corr) || records(ikeys, icorr)) return -1;
-      const size_t ncf = faces.size(), ncc = corr.size();
-      faces.insert(faces.end(), ffaces.begin(), ffaces.end());
-      corr.insert(corr.end(), icorr.begin(), icorr.end());
-      if (H->facf[l].upload(faces) || H->facc[l - 1].upload(corr))
+      if (H->facf[l].upload(faces, ffaces) || H->facc[l - 1].upload(corr, icorr))
          return hier_fail(H, "upload failed");
-      H->cff[l] = H->facf[l].part(0, ncf);
-      H->fff[l] = H->facf[l].part(ncf, faces.size() - ncf);
-      H->cfc[l - 1] = H->facc[l - 1].part(0, ncc);
-      H->cfi[l - 1] = H->facc[l - 1].part(ncc, corr.size() - ncc);
+      H->cff[l] = H->facf[l].part(0, faces.size());
+      H->fff[l] = H->facf[l].part(faces.size(), ffaces.size());
+      H->cfc[l - 1] = H->facc[l - 1].part(0, corr.size());
+      H->cfi[l - 1] = H->facc[l - 1].part(corr.size(), icorr.size());
    }
 
    // weights: cell volume relative to level 0, zero under a finer level
