@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(256)
 // face closing each row and column, in LDS, then every cell takes the
 // divergence from there (z faces, 3-D: both per cell).  The per-cell form
 // evaluates every face twice, once from each side; the anisotropic flux has
-// about four transcendentals per face.  Same values as phase_rhs_cell.
+// square roots, a division and a power per face.  Same values as phase_rhs_cell.
 template <int NDIM, int FLUX, int FE>
 __global__ void __launch_bounds__(256) k_phase_rhs_faces(LevelArgs a, ampe_model_params p,
                                                          RhsConst k,

@@ -33,7 +33,8 @@ __device__ __forceinline__ void quatmult4(const double* a, const double* b, doub
 // precision is 1.1e-15 at most for kn = 4 and 1.7e-15 for 6 (angle form 3.9e-15 and
 // 9.1e-15), 0.2e-15 and 0.3e-15 in the mean square (0.5e-15 and 0.9e-15), over
 // 4 10^5 directions and angles, half of them with qa near 1.
-// 1500 x 1130 dendrite, full right-hand side: 85 us (98 in the angle form).
+// 1500 x 1130 dendrite, full right-hand side: 81 us (98 in the angle form with
+// the logarithm of k_e taken in every cell).
 __device__ __forceinline__ void aniso_angle(double gx, double gy, double qa, bool twice, int kn,
                                             double& cs, double& sn)
 {

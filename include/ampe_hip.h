@@ -241,8 +241,8 @@ typedef struct ampe_solver_params {
                            * correction (dsm = ||acor||_wrms tq2 <= 1), step and
                            * order selection after each step, first step dt_init
                            * (else dt), largest step dt (max_step_size) */
-   int mg_quat_natural;   /* FP32 multigrid: 0 (default) stores the orientation block's
-                           * multigrid vectors row parity-split (inside each ghosted row
+   int mg_quat_natural;   /* FP32 multigrid with an orientation field: 0 (default) stores
+                           * its vectors row parity-split (inside each ghosted row
                            * the even columns, then the odd ones), so one red-black
                            * colour reads and writes whole lines; 1 keeps the natural
                            * layout.  Same values either way. */
