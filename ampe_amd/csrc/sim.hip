@@ -221,6 +221,12 @@ static int sim_finish(Sim* S, Sim** out)
       sim_destroy(S);
       return -1;
    }
+   // lagged evaluations before the first full one: no gradient (y is zero)
+   if (S->iq >= 0 && (S->hier ? hier_quat_gni(*S->hier, p, S->y, S->gni, S->stream)
+                              : launch_quat_gni(L, p, rhs_lev(p), S->y, S->gni, S->stream))) {
+      sim_destroy(S);
+      return -1;
+   }
    S->h = first_step(s);
    *out = S;
    return 0;

@@ -152,3 +152,34 @@ def test_types(dev, kw):
     for level in ("odd2", "two3"):
         nd = 3 if level == "two3" else 2
         _check(level, P.two_grain_params(ndim=nd, **kw))
+
+
+@pytest.mark.parametrize("nd,floor", [(2, b"m"), (3, b"t"), (3, b"s")])
+def test_lagged_before_any_full(dev, nd, floor):
+    """A lagged evaluation of a new integrator takes no face gradients: the
+    orientation's right-hand side is the separate entry point's with |grad q|^2 = 0
+    on every face (the floor's coefficient)."""
+    import torch
+    from ampe_amd import hip as H
+    shape = (9, 12, 70)[3 - nd:]
+    box = H.boxes_of(shape, nd)
+    p = P.two_grain_params(ndim=nd, with_conc=0, floor_type=floor)
+    sim = H.Sim(p, P.solver_defaults(dt=1e-3), [box], periodic=box)
+    lev = H.Level(nd, [box], 1, periodic=box)
+    rng = np.random.Generator(np.random.Philox(6))
+    phi, q = rng.uniform(0.1, 0.9, shape), rng.normal(size=(4,) + shape)
+    q /= np.sqrt((q ** 2).sum(0))
+    y = torch.from_numpy(np.concatenate([lev.to_ghosted(a) for a in [phi, *q]])).to(dev)
+    got = torch.zeros_like(y)
+    n2 = torch.zeros(lev.nside_tot, dtype=torch.float64, device=dev)
+    want = torch.zeros(4 * lev.ncg, dtype=torch.float64, device=dev)
+    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
+    torch.cuda.synchronize()
+    H.check(H.lib().ampe_rhs_eval(sim.h, 0.0, ptr(y), ptr(got), 1))  # fills y's ghosts
+    torch.cuda.synchronize()
+    H.check(H.lib().ampe_quat_rhs(lev.h, C.byref(p), ptr(y), ptr(y[lev.ncg:]), ptr(n2), ptr(want),
+                                  None))
+    a, b = got.cpu().numpy()[lev.ncg:].reshape(4, -1), want.cpu().numpy().reshape(4, -1)
+    for m in range(4):
+        u, v = (lev.ghost_view(x[m], 0)[(slice(1, -1),) * nd] for x in (a, b))
+        assert np.abs(v).max() > 0 and np.array_equal(u, v)
