@@ -2,7 +2,7 @@
 vectors up to ten, a loop above) against the oracle's integrator, both
 orthogonalisations; and classical against modified Gram-Schmidt, which share the
 solution up to rounding, where their kernels differ in form: levels of one tile,
-of few (each step sums the products of the one before) and of more than 1024 (a
+of few (each pass sums the products of the one before) and of more than 1024 (a
 reduction in between), odd numbers of components, FP32 solutions read in the
 row parity-split layout and in the plain one, FP64 ones, patch hierarchies are in
 the hierarchy tests.
