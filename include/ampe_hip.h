@@ -777,9 +777,9 @@ int ampe_kks_batch_noalloc(const ampe_model_params* p, const ampe_calphad_tdep* 
  * Gram-Schmidt, left block preconditioner, difference-quotient Jv) driving
  * the kernels above -- the QuatIntegrator/CVODESolver callback loop
  * (source/QuatIntegrator.cc:2096-2233, 3134-3771;
- * source/samrai/CVODESolver.cc:150-247).  Refused: combinations no kernel forms, among them a composition
- * field with an unknown fe_model and the anisotropic flux without an orientation
- * field. */
+ * source/samrai/CVODESolver.cc:150-247).  Refused: combinations no kernel
+ * forms, among them a composition field with an unknown fe_model and the
+ * anisotropic flux without an orientation field. */
 typedef struct ampe_sim ampe_sim;
 int ampe_sim_create(const ampe_model_params* p, const ampe_solver_params* s,
                     const ampe_box* boxes, int npatch,
